@@ -66,7 +66,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
         s.nPad = next_pow2(s.nScan);
         s.L = ilog2(s.nPad);
         s.na = q.method == kABM ? 4 * q.n : q.n;
-        sys_[i].core.reset(new ScanCore(q.method, q.n, q.m, q.p, !q.C, !q.D, s.nPad, opt, arena));
+        sys_[i].core.reset(new ScanCore(q.method, q.n, q.m, q.p, !q.C, !q.D, s.nPad, opt, arena, false));
         ScanCore& c = *sys_[i].core;
         if (!c.Sks32_.get()) sys_[i].copies.alloc(2 * ks_half(s.nPad, s.na), arena);
         s.lc = c.chunk_log(s.nScan, s.nPad, true);

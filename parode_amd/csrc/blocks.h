@@ -1,0 +1,95 @@
+// Block responses: the scan with T steps at a time.
+//
+// The map x_{e+1} = M x_e + v_e is linear and time-invariant, so over a block
+// of T = 2^lb steps the state at the block's end and the T outputs inside it
+// are fixed linear functions of the state at its start and of the block's
+// input samples.  A solve then is
+//   pass 1: per block, its response from zero at its end  (one product with Q)
+//   scan:   the states at the blocks' starts (n_a values a block)
+//   pass 2: per block, its T outputs                      (one product with
+//           [O H]: the outputs' responses to the state and to the samples)
+// in place of T dependent steps, and no state inside a block is formed.
+//
+// To make a block need only its own samples, the state is shifted by the
+// samples that an element and its successors share: with the direct terms
+//   Z_e = X_e - sum_{r < taps} D_r u_{e,r},
+// Z_{e+1} = M Z_e + G u_e, where u_e are the s samples that element e adds
+// (RK4: rows 2e and 2e + 1, taps = 1; ABM: one row, taps = 4), and
+// y_e = C x(Z_e) + sum_{r < taps} F_r u_{e,r}.
+//
+// Everything is FP64 on the matrix cores (v_mfma_f64_16x16x4f64).
+// Tables (device, row-major; m inputs, p outputs, kb = s T m):
+//   PT [L][na][na]     transposed powers, PT_l = (M^(2^l))^T
+//   QT [kb][na]        row (s i + q) m + j: (M^(T-1-i) G_q)[:, j]
+//   OT [na][T p]       column i p + o: row o of C E M^i (E: the state block read)
+//   Ht [(s (T-1) + taps) m][p]  row d m + j, d = window row - s i + s (T - 1):
+//                      the response of output o of step i to input j
+//   DL [taps m][na]    the shift of the state
+// The factors of column (i, o) for window value k = row m + j are
+// Ht[(k + s (T-1-i) m) p + o]: linear in k, so pass 2 needs no row index.
+#pragma once
+#include "kernels.h"
+
+namespace parode {
+namespace k {
+
+struct BlockShape {
+    int method = 0, n = 0, m = 0, p = 0, na = 0;
+    bool useC = false, useD = false;   // useC false: the outputs are the states (p = n)
+    bool mirror = false;               // the reference's float rounding of the map
+    int lb = 0, T = 0;                 // steps per block
+    int L = 0;                         // powers in PT
+    int s = 0, taps = 0;
+    int kb() const { return s * T * m; }
+    int kh() const { return (s * (T - 1) + taps) * m; }
+};
+
+// Block responses of one system: tables and states carved by ScanCore.
+struct BlockBufs {
+    double *PT = nullptr, *QT = nullptr, *OT = nullptr, *Ht = nullptr, *DL = nullptr;
+    double* Z = nullptr;    // [blocks + 1][na]: aggregates, then the blocks' start states
+    double* Z2 = nullptr;   // [groups + 1][na]: the same for groups of blocks
+};
+
+// Where a batch's samples lie: window row r of block b is the sample row
+// b T sL + r g (sL sample rows a step, g = sL / s); rows past `last` (in window
+// rows) are not there and count as zero.
+struct BlockInput {
+    const void* U = nullptr;
+    bool isDouble = false;
+    long sL = 0;
+    long last = 0;
+};
+
+// Steps per block for a shape and horizon, 0: this shape keeps the general
+// path (see the rule at its definition).
+int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long nScan, long nPad);
+BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bool mirror, int lb,
+                       int L);
+// How a pass is tiled (kBlockAuto: by the rule at launch_pass).
+enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit16 = 3 };
+// Groups of blocks that the scan of nb blocks makes first (0: none).
+long block_groups(int na, long nb);
+
+// M, G, the direct terms and (x0 given) the seed: x0, or with the ABM start-up
+// the states x_0..x_3 and their three outputs.
+void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+               const float* B, const float* C, const float* D, const float* x0, const void* U,
+               bool uDouble, double* seed, float* Y);
+// PT up to P_lb, QT, OT, Ht
+void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C);
+// the blocks' responses from zero (and, with powers, the rest of PT)
+void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, bool powers, int tiling = kBlockAuto);
+// the blocks' start states from the seed (in X); Z[nb] is the state after them
+void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                long nb, const double* seed);
+// seedOut = the state (in X) after the blocks
+void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, double* seedOut);
+void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, long nReal, const double* seed, const float* D, float* Y,
+                 int tiling = kBlockAuto);
+
+}  // namespace k
+}  // namespace parode

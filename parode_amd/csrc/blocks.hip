@@ -1,0 +1,1356 @@
+// Kernels of the block responses (blocks.h).
+#include "blocks.h"
+#include "launch.h"
+
+#include <algorithm>
+
+namespace parode {
+namespace k {
+
+// The kernels that hold a whole map in one work-group's LDS.
+constexpr int kBN = 64;             // states (n_a), outputs a step
+constexpr int kBP = kBN + 1;        // LDS pitch
+constexpr int kBM = 32;             // inputs
+
+// ------------------------------------------------------------------ products
+// One 16 x 16 tile of X Y from LDS (v_mfma_f64_16x16x4f64): lane l holds
+// X[i0 + l%16][k + l/16] and Y[k + l/16][j0 + l%16] (YT: Y given transposed);
+// D: register v of lane l is row i0 + 4v + l/16, column j0 + l%16.
+template <bool YT>
+__device__ __forceinline__ doublex4 lds_tile(const double* X, int px, const double* Y, int py,
+                                             int i0, int j0, int kk)
+{
+    const int l16 = threadIdx.x & 15, q4 = (threadIdx.x >> 4) & 3;
+    doublex4 acc = {0.0, 0.0, 0.0, 0.0};
+    const double* xr = X + (i0 + l16) * px + q4;
+    const double* yr = YT ? Y + (j0 + l16) * py + q4 : Y + q4 * py + j0 + l16;
+    const int ys = YT ? 1 : py;
+    for (int k = 0; k < kk; k += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[k], yr[k * ys], acc, 0, 0, 0);
+    return acc;
+}
+
+// ------------------------------------------------------------------- the map
+struct BlkMap {
+    BlockShape s;
+    double h;
+    Rk4Coef rk;
+    AbmCoef ab;
+    const float *A, *B, *C, *D, *x0;
+    const void* U;
+    double *PT, *QT, *Ht, *DL, *seed;
+    float* Y;
+    long gx;
+};
+
+// Z = X Y with the reference's rounding: float products, sequential float sums.
+__device__ __forceinline__ void lds_mul_seq(int r, int kk, int c, const float* X, int px,
+                                            const float* Y, int py, float* Z, int pz)
+{
+#pragma clang fp contract(off)
+    for (int t = threadIdx.x; t < r * c; t += 1024) {
+        const int i = t / c, j = t - i * c;
+        float v = 0.0f;
+        for (int q = 0; q < kk; ++q) {
+            const float pr = X[i * px + q] * Y[q * py + j];
+            v = v + pr;
+        }
+        Z[i * pz + j] = v;
+    }
+}
+
+// One work-group makes a small system's map (n_a <= 64, m <= 32) in LDS: the
+// step map M, the block input G, the direct terms F and the state's shift D
+// (blocks.h).  RK4 by Horner's scheme, M = I + hA (I + hA/2 (I + hA/3 (I +
+// hA/4))), beside the products A^k B; with the reference's rounding by its own
+// products A^2, A^3, A^4.  A chain of a few dependent 64 x 64 products: latency.
+__device__ __forceinline__ void d_blk_map_rk4(const BlkMap& a, double* lds)
+{
+#pragma clang fp contract(off)
+    const BlockShape& s = a.s;
+    const int n = s.n, m = s.m, p = s.p, tid = threadIdx.x, wave = tid >> 6;
+    const int n16 = (n + 15) & ~15, m16 = (m + 15) & ~15, nt = n16 / 16, mt = m16 / 16;
+    constexpr int KP = kBM + 1;
+    double* As = lds;
+    double* Ts = lds + kBN * kBP;
+    double* Kb[4];
+    for (int q = 0; q < 4; ++q) Kb[q] = lds + 2 * kBN * kBP + q * kBN * KP;
+    const int l16 = tid & 15, q4 = (tid >> 4) & 3;
+    for (int t = tid; t < n16 * m16; t += 1024) {
+        const int i = t / m16, j = t - i * m16;
+        const bool in = i < n && j < m;
+        Kb[0][i * KP + j] = in ? (double)a.B[(long)i * m + j] : 0.0;
+        for (int q = 1; q < 4; ++q) Kb[q][i * KP + j] = 0.0;
+    }
+    if (s.mirror) {
+        float* A1 = reinterpret_cast<float*>(As);
+        float* A2 = A1 + kBN * kBP;
+        float* A3 = reinterpret_cast<float*>(Ts);
+        float* A4 = A3 + kBN * kBP;
+        float* Bf = reinterpret_cast<float*>(Kb[0]);   // B, AB, A2B, A3B in float
+        for (int t = tid; t < n * n; t += 1024) A1[t / n * kBP + t % n] = a.A[t];
+        __syncthreads();
+        for (int t = tid; t < n * m; t += 1024) Bf[t / m * KP + t % m] = a.B[t];
+        __syncthreads();
+        float* AB = Bf + kBN * KP;
+        float* A2B = AB + kBN * KP;
+        float* A3B = A2B + kBN * KP;
+        lds_mul_seq(n, n, n, A1, kBP, A1, kBP, A2, kBP);
+        lds_mul_seq(n, n, m, A1, kBP, Bf, KP, AB, KP);
+        __syncthreads();
+        lds_mul_seq(n, n, n, A2, kBP, A1, kBP, A3, kBP);
+        lds_mul_seq(n, n, m, A2, kBP, Bf, KP, A2B, KP);
+        __syncthreads();
+        lds_mul_seq(n, n, n, A1, kBP, A3, kBP, A4, kBP);
+        lds_mul_seq(n, n, m, A3, kBP, Bf, KP, A3B, KP);
+        __syncthreads();
+        // the combinations (RungeKutta4thOrder.cpp:48-57), in registers first:
+        // the float products share their LDS with what follows
+        double mv[4], bv[2][3];
+        for (int u = 0; u < 4; ++u) {
+            const int t = tid + u * 1024;
+            mv[u] = 0.0;
+            if (t >= n * n) continue;
+            const int i = t / n, j = t - i * n, x = i * kBP + j;
+            double v = ((i == j) ? 1.0 : 0.0) + a.rk.h * (double)A1[x];
+            v = v + a.rk.c2 * (double)A2[x];
+            v = v + a.rk.c3 * (double)A3[x];
+            v = v + a.rk.c4 * (double)A4[x];
+            mv[u] = (double)(float)v;
+        }
+        for (int u = 0; u < 2; ++u) {
+            const int t = tid + u * 1024;
+            if (t >= n * m) continue;
+            const int x = t / m * KP + t % m;
+            const double b = Bf[x], ab = AB[x], a2b = A2B[x], a3b = A3B[x];
+            bv[u][0] = (double)(float)((1.0 / 6.0) * (((a.rk.h * b + a.rk.s1 * ab) + a.rk.s2 * a2b) + a.rk.s3 * a3b));
+            bv[u][1] = (double)(float)((1.0 / 6.0) * ((a.rk.t0 * b + a.rk.t1 * ab) + a.rk.t2 * a2b));
+            bv[u][2] = (double)(float)(a.rk.u0 * b);
+        }
+        __syncthreads();
+        for (int t = tid; t < n16 * n16; t += 1024) Ts[t / n16 * kBP + t % n16] = 0.0;
+        for (int t = tid; t < n16 * m16; t += 1024)
+            for (int q = 0; q < 4; ++q) Kb[q][t / m16 * KP + t % m16] = 0.0;
+        __syncthreads();
+        for (int u = 0; u < 4; ++u) {
+            const int t = tid + u * 1024;
+            if (t < n * n) Ts[t / n * kBP + t % n] = mv[u];
+        }
+        for (int u = 0; u < 2; ++u) {
+            const int t = tid + u * 1024;
+            if (t >= n * m) continue;
+            const int x = t / m * KP + t % m;
+            for (int q = 0; q < 3; ++q) Kb[q == 2 ? 3 : q][x] = bv[u][q];
+        }
+        __syncthreads();
+    } else {
+        for (int t = tid; t < n16 * n16; t += 1024) {
+            const int i = t / n16, j = t - i * n16;
+            const double v = (i < n && j < n) ? (double)a.A[(long)i * n + j] : 0.0;
+            As[i * kBP + j] = v;
+            Ts[i * kBP + j] = (i == j ? 1.0 : 0.0) + (a.h / 4.0) * v;
+        }
+        __syncthreads();
+        for (int st = 3; st >= 1; --st) {
+            // tiles of A T, then of A (A^k B); a wave has at most two items
+            doublex4 acc[2];
+            const int items = nt * nt + nt * mt;
+            for (int u = 0; u < 2; ++u) {
+                const int w = wave + 16 * u;
+                if (w < nt * nt)
+                    acc[u] = lds_tile<false>(As, kBP, Ts, kBP, w / nt * 16, w % nt * 16, n16);
+                else if (w < items)
+                    acc[u] = lds_tile<false>(As, kBP, Kb[3 - st], KP, (w - nt * nt) / mt * 16,
+                                             (w - nt * nt) % mt * 16, n16);
+            }
+            __syncthreads();
+            const double c = a.h / (double)st;
+            for (int u = 0; u < 2; ++u) {
+                const int w = wave + 16 * u;
+                if (w < nt * nt) {
+                    for (int v = 0; v < 4; ++v) {
+                        const int i = w / nt * 16 + 4 * v + q4, j = w % nt * 16 + l16;
+                        Ts[i * kBP + j] = (i == j ? 1.0 : 0.0) + c * acc[u][v];
+                    }
+                } else if (w < items) {
+                    for (int v = 0; v < 4; ++v) {
+                        const int i = (w - nt * nt) / mt * 16 + 4 * v + q4;
+                        const int j = (w - nt * nt) % mt * 16 + l16;
+                        Kb[4 - st][i * KP + j] = acc[u][v];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        for (int t = tid; t < n16 * m16; t += 1024) {
+            const int x = t / m16 * KP + t % m16;
+            const double b = Kb[0][x], ab = Kb[1][x], a2b = Kb[2][x], a3b = Kb[3][x];
+            Kb[0][x] = (1.0 / 6.0) * (((a.rk.h * b + a.rk.s1 * ab) + a.rk.s2 * a2b) + a.rk.s3 * a3b);
+            Kb[1][x] = (1.0 / 6.0) * ((a.rk.t0 * b + a.rk.t1 * ab) + a.rk.t2 * a2b);
+            Kb[3][x] = a.rk.u0 * b;
+        }
+        __syncthreads();
+    }
+    // Ts = M; Kb[0], Kb[1], Kb[3] = the three input blocks of a step.
+    // G = [B1 + M B3 | B2], the shift and the direct term from B3
+    double* GT = a.QT + (long)s.s * (s.T - 1) * m * n;
+    for (int w = wave; w < nt * mt; w += 16) {
+        const int i0 = w / mt * 16, j0 = w % mt * 16;
+        const doublex4 acc = lds_tile<false>(Ts, kBP, Kb[3], KP, i0, j0, n16);
+        for (int v = 0; v < 4; ++v) {
+            const int i = i0 + 4 * v + q4, j = j0 + l16;
+            if (i >= n || j >= m) continue;
+            GT[(long)j * n + i] = Kb[0][i * KP + j] + acc[v];
+            GT[(long)(m + j) * n + i] = Kb[1][i * KP + j];
+        }
+    }
+    for (int t = tid; t < n * n; t += 1024) a.PT[t] = Ts[(t % n) * kBP + t / n];
+    for (int t = tid; t < m * n; t += 1024) a.DL[t] = Kb[3][(t % n) * KP + t / n];
+    double* F = a.Ht + (long)s.s * (s.T - 1) * m * p;
+    for (int t = tid; t < m * p; t += 1024) {
+        const int j = t / p, o = t - j * p;
+        double v = 0.0;
+        if (s.useC)
+            for (int i = 0; i < n; ++i) v = fma((double)a.C[(long)o * n + i], Kb[3][i * KP + j], v);
+        else
+            v = Kb[3][o * KP + j];
+        F[t] = v + (s.useD ? (double)a.D[(long)o * m + j] : 0.0);
+    }
+}
+
+// The ABM companion of a small system (n <= 16): its dense block row R, the
+// blocks V_0 = B_4, V_t = B_{4-t} + sum_{i < t} M_{4-t+i} V_i (M_b: R's blocks,
+// oldest first; B_q: the step's input blocks), which give
+// G = [V_1; V_2; V_3; V_4], D_r = [0 (r blocks); V_0 .. V_{3-r}], F_r = C V_{3-r}.
+__device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
+{
+#pragma clang fp contract(off)
+    const BlockShape& s = a.s;
+    const int n = s.n, m = s.m, p = s.p, na = s.na, tid = threadIdx.x;
+    constexpr int AP = 17, KP = kBM + 1;
+    double* A1 = lds;                  // [16][AP]
+    double* A2 = A1 + 16 * AP;
+    double* B1 = A2 + 16 * AP;         // [16][KP]
+    double* AB = B1 + 16 * KP;
+    double* R = AB + 16 * KP;          // [16][kBP]
+    double* V = R + 16 * kBP;          // [5][16][KP]
+    for (int t = tid; t < n * n; t += 1024) A1[t / n * AP + t % n] = a.A[t];
+    for (int t = tid; t < n * m; t += 1024) B1[t / m * KP + t % m] = a.B[t];
+    __syncthreads();
+    for (int t = tid; t < n * (n + m); t += 1024) {
+        const int i = t / (n + m), j = t - i * (n + m);
+        const double* y = j < n ? A1 + j : B1 + (j - n);
+        const int py = j < n ? AP : KP;
+        double v = 0.0;
+        if (s.mirror) {
+            float f = 0.0f;
+            for (int q = 0; q < n; ++q) {
+                const float pr = (float)A1[i * AP + q] * (float)y[q * py];
+                f = f + pr;
+            }
+            v = f;
+        } else {
+            for (int q = 0; q < n; ++q) v = fma(A1[i * AP + q], y[q * py], v);
+        }
+        if (j < n)
+            A2[i * AP + j] = v;
+        else
+            AB[i * KP + j - n] = v;
+    }
+    __syncthreads();
+    auto rnd = [&](double v) { return s.mirror ? (double)(float)v : v; };
+    const AbmCoef& c = a.ab;
+    for (int t = tid; t < n * n; t += 1024) {
+        const int i = t / n, j = t - i * n;
+        const double id = (i == j) ? 1.0 : 0.0, x = A1[i * AP + j], x2 = A2[i * AP + j];
+        R[i * kBP + j] = rnd(c.a3A2 * x2);
+        R[i * kBP + n + j] = rnd(c.a2A * x + c.a2A2 * x2);
+        R[i * kBP + 2 * n + j] = rnd(c.a1A * x + c.a1A2 * x2);
+        R[i * kBP + 3 * n + j] = rnd((id + c.a0A * x) + c.a0A2 * x2);
+    }
+    auto bq = [&](int q, int i, int j) {   // the step's input block q
+        const double b = B1[i * KP + j], ab = AB[i * KP + j];
+        return q == 0 ? rnd(c.b3AB * ab) : q == 1 ? rnd(c.b2B * b + c.b2AB * ab)
+             : q == 2 ? rnd(c.b1B * b + c.b1AB * ab) : q == 3 ? rnd(c.b0B * b + c.b0AB * ab)
+             : rnd(c.bm1 * b);
+    };
+    for (int st = 0; st < 5; ++st) {
+        __syncthreads();
+        for (int t = tid; t < n * m; t += 1024) {
+            const int i = t / m, j = t - i * m;
+            double v = bq(4 - st, i, j);
+            for (int b = 0; b < st; ++b)
+                for (int q = 0; q < n; ++q)
+                    v = fma(R[i * kBP + (4 - st + b) * n + q], V[(b * 16 + q) * KP + j], v);
+            V[(st * 16 + i) * KP + j] = v;
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < na * na; t += 1024) {
+        const int j = t / na, i = t - j * na;   // PT[j][i] = M[i][j]
+        a.PT[t] = i < 3 * n ? (j == i + n ? 1.0 : 0.0) : R[(i - 3 * n) * kBP + j];
+    }
+    double* GT = a.QT + (long)(s.T - 1) * m * na;
+    for (int t = tid; t < m * na; t += 1024) {
+        const int j = t / na, x = t - j * na, b = x / n, i = x - b * n;
+        GT[t] = V[((b + 1) * 16 + i) * KP + j];
+    }
+    for (int t = tid; t < 4 * m * na; t += 1024) {
+        const int rj = t / na, x = t - rj * na, r = rj / m, j = rj - r * m, b = x / n, i = x - b * n;
+        a.DL[t] = b >= r ? V[((b - r) * 16 + i) * KP + j] : 0.0;
+    }
+    double* F = a.Ht + (long)(s.T - 1) * m * p;
+    for (int t = tid; t < 4 * m * p; t += 1024) {
+        const int rj = t / p, o = t - rj * p, r = rj / m, j = rj - r * m;
+        double v = 0.0;
+        if (s.useC)
+            for (int i = 0; i < n; ++i)
+                v = fma((double)a.C[(long)o * n + i], V[((3 - r) * 16 + i) * KP + j], v);
+        else
+            v = V[((3 - r) * 16 + o) * KP + j];
+        F[t] = v + (r == 3 && s.useD ? (double)a.D[(long)o * m + j] : 0.0);
+    }
+}
+
+// The seed of a plan's solve (work-group 1): x0, or the ABM start-up states
+// and the outputs of the first three (inputs: rows 0, 2, 4 of the h/2 grid).
+template <typename TU>
+__device__ __forceinline__ void d_blk_seed(const VBlock vb, const BlkMap& a)
+{
+    const BlockShape& s = a.s;
+    const TU* U = static_cast<const TU*>(a.U);
+    if (s.method == 0) {
+        for (int i = threadIdx.x; i < s.n; i += 1024) a.seed[i] = (double)a.x0[i];
+        return;
+    }
+    d_abm_startup<TU>(vb, s.mirror, s.n, s.m, a.h, true, a.A, a.B, a.x0, U, a.seed);
+    for (int t = threadIdx.x; t < 3 * s.p; t += 1024) {
+        const int e = t / s.p, o = t - e * s.p;
+        double v = 0.0;
+        if (s.useC)
+            for (int i = 0; i < s.n; ++i)
+                v = fma((double)a.C[(long)o * s.n + i], a.seed[e * s.n + i], v);
+        else
+            v = a.seed[e * s.n + o];
+        if (s.useD)
+            for (int j = 0; j < s.m; ++j)
+                v = fma((double)a.D[(long)o * s.m + j], (double)U[(long)2 * e * s.m + j], v);
+        a.Y[t] = (float)v;
+    }
+}
+
+template <typename TU>
+__device__ __forceinline__ void d_blk_map(const VBlock vb, const BlkMap& a, double* lds)
+{
+    if (vb.x == 1)
+        d_blk_seed<TU>(vb, a);
+    else if (a.s.method == 0)
+        d_blk_map_rk4(a, lds);
+    else
+        d_blk_map_abm(a, lds);
+}
+
+constexpr int kMapLds = 2 * kBN * kBP + 4 * kBN * (kBM + 1);   // doubles
+
+template <typename TU>
+__global__ __launch_bounds__(1024) void k_blk_map(const BlkMap a)
+{
+    __shared__ double lds[kMapLds];
+    d_blk_map<TU>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, lds);
+}
+
+// ---------------------------------------------------------------- the tables
+struct BlkTables {
+    BlockShape s;
+    const float* C;
+    double *PT, *QT, *OT, *Ht;
+    int ni, nq;   // steps of a slice of OT (and Ht), of a slice of QT
+    long gx;
+};
+
+// P <- P^2 in LDS (and, with R, the rows of R by P or P^T): every tile from the
+// old values, a barrier, the new values, a barrier.  Sixteen waves, two tiles
+// of P^2 and rows each.  from/to: the rows of R that are read and written.
+template <bool ROWS, bool YT>
+__device__ __forceinline__ void lds_step(double* P, int n16, double* R, int from, int to, int rows,
+                                         bool square)
+{
+    const int wave = threadIdx.x >> 6, l16 = threadIdx.x & 15, q4 = (threadIdx.x >> 4) & 3;
+    const int nt = n16 / 16, sq = square ? nt * nt : 0, rt = (rows + 15) / 16;
+    const int items = sq + (ROWS ? rt * nt : 0);
+    doublex4 acc[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int w = wave + 16 * u;
+        if (w < sq)
+            acc[u] = lds_tile<false>(P, kBP, P, kBP, w / nt * 16, w % nt * 16, n16);
+        else if (w < items)
+            acc[u] = lds_tile<YT>(R + from * kBP, kBP, P, kBP, (w - sq) / nt * 16,
+                                  (w - sq) % nt * 16, n16);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int w = wave + 16 * u;
+        if (w >= items) continue;
+        const bool isR = w >= sq;
+        const int x = isR ? w - sq : w, i0 = x / nt * 16, j = x % nt * 16 + l16;
+        for (int v = 0; v < 4; ++v) {
+            const int i = i0 + 4 * v + q4;
+            if (!isR)
+                P[i * kBP + j] = acc[u][v];
+            else if (i < rows)
+                R[(to + i) * kBP + j] = acc[u][v];
+        }
+    }
+    __syncthreads();
+}
+
+// Tables of a small system (n_a, p, s m <= 64).  Work-group 0 squares P_0 up
+// to P_lb; the others each make a slice of OT and Ht (ni steps) or of QT (nq
+// steps) and square P_l for themselves, since passing it between work-groups
+// would cost a launch per level.  A slice of steps [i0, i0 + 2^a) takes the
+// levels below a by doubling its rows and the others by the bits of i0 (the
+// powers commute).  Time: lb dependent products of 64 x 64 in one compute unit.
+__device__ __forceinline__ void d_blk_tables(const VBlock vb, const BlkTables& a, double* P,
+                                             double* R, double* G)
+{
+    const BlockShape& s = a.s;
+    const int na = s.na, n16 = (na + 15) & ~15, tid = threadIdx.x, m = s.m, p = s.p;
+    const int sm = s.s * m, nO = s.T / a.ni;
+    const long nn = (long)na * na;
+    const double* GT = a.QT + (long)(s.T - 1) * sm * na;
+    for (int t = tid; t < n16 * n16; t += 1024) {
+        const int r = t / n16, c = t - r * n16;
+        P[r * kBP + c] = (r < na && c < na) ? a.PT[(long)r * na + c] : 0.0;
+    }
+    if (vb.x == 0) {
+        __syncthreads();
+        for (int l = 0; l < s.lb; ++l) {
+            lds_step<false, false>(P, n16, nullptr, 0, 0, 0, true);
+            double* out = a.PT + (l + 1) * nn;
+            for (int t = tid; t < nn; t += 1024) out[t] = P[t / na * kBP + t % na];
+        }
+        return;
+    }
+    const bool isO = vb.x <= nO;
+    const int w = (int)vb.x - 1 - (isO ? 0 : nO);
+    const int ns = isO ? a.ni : a.nq, per = isO ? p : sm, i0 = w * ns, rows = ns * per;
+    const int off = na - s.n;
+    for (int t = tid; t < kBN * n16; t += 1024) {
+        const int r = t / n16, c = t - r * n16;
+        double v = 0.0;
+        if (r < per) {
+            if (!isO)
+                v = c < na ? GT[(long)r * na + c] : 0.0;
+            else if (c >= off && c < na)
+                v = s.useC ? (double)a.C[(long)r * s.n + c - off] : (c - off == r ? 1.0 : 0.0);
+        }
+        R[r * kBP + c] = v;
+        if (isO) G[r * kBP + c] = (r < sm && c < na) ? GT[(long)r * na + c] : 0.0;
+    }
+    __syncthreads();
+    for (int l = 0; l < s.lb; ++l) {
+        const bool more = l + 1 < s.lb;
+        const bool dbl = (1 << l) < ns;
+        const bool mul = dbl || ((i0 >> l) & 1);
+        const int cnt = dbl ? per << l : rows;
+        // rows of OT are multiplied by P_l (PT transposed), rows of QT by P_l^T
+        if (!mul)
+            lds_step<false, false>(P, n16, nullptr, 0, 0, 0, more);
+        else if (isO)
+            lds_step<true, true>(P, n16, R, 0, dbl ? cnt : 0, cnt, more);
+        else
+            lds_step<true, false>(P, n16, R, 0, dbl ? cnt : 0, cnt, more);
+    }
+    if (!isO) {
+        for (int t = tid; t < rows * na; t += 1024) {
+            const int r = t / na, c = t - r * na, i = r / sm;
+            if (i0 + i > 0)   // (step 0 is G itself, which the map made)
+                a.QT[((long)(s.T - 1 - i0 - i) * sm + (r - i * sm)) * na + c] = R[r * kBP + c];
+        }
+        return;
+    }
+    const long cols = (long)s.T * p;
+    for (int t = tid; t < rows * na; t += 1024) {
+        const int c = t / rows, r = t - c * rows;
+        a.OT[c * cols + (long)i0 * p + r] = R[r * kBP + c];
+    }
+    // Ht of step k: (C E M^k) G, [s m][p], for a lag of k + 1 steps
+    const int wave = tid >> 6, l16 = tid & 15, q4 = (tid >> 4) & 3;
+    const int ct = (sm + 15) / 16, rt = (rows + 15) / 16;
+    for (int x = wave; x < rt * ct; x += 16) {
+        const doublex4 acc = lds_tile<true>(R, kBP, G, kBP, x / ct * 16, x % ct * 16, n16);
+        const int j = x % ct * 16 + l16;
+        for (int v = 0; v < 4; ++v) {
+            const int r = x / ct * 16 + 4 * v + q4, i = r / p, k = i0 + i;
+            if (r < rows && j < sm && k <= s.T - 2)
+                a.Ht[((long)(s.T - 2 - k) * sm + j) * p + (r - i * p)] = acc[v];
+        }
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_blk_tables(const BlkTables a)
+{
+    __shared__ double P[kBN * kBP], R[kBN * kBP], G[kBN * kBP];
+    d_blk_tables(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, P, R, G);
+}
+
+// ---------------------------------------------------------------- the passes
+// Pass 1 (OUT false): Z[b][:] = window of block b times QT.
+// Pass 2 (OUT true):  Y[b T p ...] = [Z_b, window of block b] times [OT; Ht].
+// Both are products of Nb rows; the window part of pass 2 is causal: column
+// (i, o) takes the window's first (s i + taps) m values only.
+struct BlkPass {
+    int na, m, p, s, T, taps;
+    int cols, kz, ku;       // columns; K of the state part and of the window part
+    long nb, nReal;
+    const void* U;
+    long blockU;            // samples between blocks' windows
+    int gm;                 // samples skipped after each window row
+    unsigned magic;         // of m (k / m by multiply-high; m = 1: k itself)
+    long last;              // last window row that is there
+    const double *Z, *OT, *BU;   // BU: QT or Ht
+    double* S;              // pass 1's output
+    float* Y;               // pass 2's output
+    const double* seed;     // pass 2, RK4: the first state, and D (or null)
+    const float* D;
+    double* PT;             // pass 1: work-group gx * gy squares P_lb .. P_{L-2}
+    int lb, L;
+    long gx, gy;
+};
+
+__device__ __forceinline__ bool not_finite(double v) { return !(fabs(v) <= 1.7976931348623157e308); }
+
+// offset of window value k of a block (its samples start at u)
+__device__ __forceinline__ long win(const BlkPass& a, int k)
+{
+    if (a.gm == 0) return k;
+    const int r = a.m == 1 ? k : (int)__umulhi((unsigned)k, a.magic);
+    return k + (long)r * a.gm;
+}
+// window values of block b that are there
+__device__ __forceinline__ int win_len(const BlkPass& a, long b)
+{
+    const long rows = a.last + 1 - b * a.s * a.T;
+    const long k = (rows < 0 ? 0 : rows) * a.m;
+    return k < a.ku ? (int)k : a.ku;
+}
+
+// RK4's first outputs depend on x_0 alone (and u_0 through D)
+__device__ __forceinline__ bool first_output(const BlkPass& a, long b, int col)
+{
+    return a.taps == 1 && b == 0 && col < a.p;
+}
+
+// One output of pass 2, term by term and only over the samples it depends on:
+// for tiles that hold a sample that is not finite, which the tile's products
+// would carry (times zero) into the outputs before it.
+template <typename TU>
+__device__ double blk_output(const BlkPass& a, long b, int col)
+{
+    const int i = col / a.p, o = col - i * a.p;
+    double y = 0.0;
+    const TU* u = static_cast<const TU*>(a.U) + b * a.blockU;
+    if (first_output(a, b, col)) {   // from x_0 itself, not from x_0 less a shift by u_0
+        for (int k = 0; k < a.kz; ++k) y = fma(a.seed[k], a.OT[(long)k * a.cols + col], y);
+        if (a.D)
+            for (int k = 0; k < a.m; ++k) y = fma((double)u[k], (double)a.D[(long)o * a.m + k], y);
+        return y;
+    }
+    for (int k = 0; k < a.kz; ++k) y = fma(a.Z[b * a.na + k], a.OT[(long)k * a.cols + col], y);
+    const double* h = a.BU + (long)a.s * (a.T - 1 - i) * a.m * a.p + o;
+    int ke = (a.s * i + a.taps) * a.m;
+    const int kl = win_len(a, b);
+    ke = ke < kl ? ke : kl;
+    for (int k = 0; k < ke; ++k) y = fma((double)u[win(a, k)], h[(long)k * a.p], y);
+    return y;
+}
+
+__device__ __forceinline__ void blk_store(const BlkPass& a, bool out, long b, int col, double v)
+{
+    if (!out) {
+        a.S[b * a.na + col] = v;
+    } else if (b * a.T + col / a.p < a.nReal) {
+        a.Y[b * a.cols + col] = (float)v;
+    }
+}
+
+// Few tiles: 16 x 16 tiles whose K is split over NW waves, operands straight
+// from the caches, eight k-steps of loads in flight; the waves' partial tiles
+// meet in LDS.  Bound by the latency of those loads; used while the 64 x 64
+// tiles would not fill the compute units.
+template <typename TU, bool OUT, int NW>
+__device__ __forceinline__ void d_blk_split(const VBlock vb, const BlkPass& a, double* part,
+                                            int* bad)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
+    const long b0 = vb.y * 16;
+    const int j0 = (int)vb.x * 16;
+    const long b = b0 + l16 < a.nb ? b0 + l16 : a.nb - 1;
+    const int col = j0 + l16 < a.cols ? j0 + l16 : a.cols - 1;
+    const TU* u = static_cast<const TU*>(a.U) + b * a.blockU;
+    const int kl = win_len(a, b);
+    int kcol = a.ku, kEnd = a.ku, kMin = a.ku, stride = a.na;
+    const double* h = a.BU + col;
+    if (OUT) {
+        const int jl = j0 + 15 < a.cols ? j0 + 15 : a.cols - 1;
+        const int i = col / a.p;
+        kcol = (a.s * i + a.taps) * a.m;
+        kEnd = (a.s * (jl / a.p) + a.taps) * a.m;
+        kMin = (a.s * (j0 / a.p) + a.taps) * a.m;
+        stride = a.p;
+        h = a.BU + (long)a.s * (a.T - 1 - i) * a.m * a.p + (col - i * a.p);
+        if (threadIdx.x == 0) *bad = 0;
+        __syncthreads();
+    }
+    const int zs = OUT ? (a.kz + 3) / 4 : 0, us = (kEnd + 3) / 4, per = (zs + us + NW - 1) / NW;
+    const int kb = wave * per, ke = kb + per < zs + us ? kb + per : zs + us;
+    doublex4 acc = {0.0, 0.0, 0.0, 0.0};
+    constexpr int UN = 8;
+    int k = kb;
+    if (OUT) {
+        const double* z = a.Z + b * a.na;
+        const int kz = ke < zs ? ke : zs;
+        for (; k < kz; k += UN) {
+            double x[UN], y[UN];
+#pragma unroll
+            for (int t = 0; t < UN; ++t) {
+                const int j = (k + t) * 4 + q4;
+                const bool in = k + t < kz && j < a.kz;
+                x[t] = in ? z[j] : 0.0;
+                y[t] = in ? a.OT[(long)j * a.cols + col] : 0.0;
+            }
+#pragma unroll
+            for (int t = 0; t < UN; ++t)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], y[t], acc, 0, 0, 0);
+        }
+        k = kb > zs ? kb : zs;
+    }
+    bool nf = false;
+    if (OUT && first_output(a, b0, j0)) kMin = 0;
+    for (; k < ke; k += UN) {
+        double x[UN], y[UN];
+#pragma unroll
+        for (int t = 0; t < UN; ++t) {
+            const int j = (k - zs + t) * 4 + q4;
+            const bool in = k + t < ke;
+            x[t] = (in && j < kl && j < kEnd) ? (double)u[win(a, j)] : 0.0;
+            y[t] = (in && j < kcol) ? h[(long)j * stride] : 0.0;
+            if (OUT) nf = nf || (j >= kMin && not_finite(x[t]));
+        }
+#pragma unroll
+        for (int t = 0; t < UN; ++t)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], y[t], acc, 0, 0, 0);
+    }
+    if (OUT && nf) *bad = 1;
+    if (wave > 0) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[((wave - 1) * 4 + v) * 64 + lane] = acc[v];
+    }
+    __syncthreads();
+    if (OUT && *bad) {
+        for (int t = threadIdx.x; t < 256; t += NW * 64) {
+            const long bb = b0 + t / 16;
+            const int cc = j0 + t % 16;
+            if (bb < a.nb && cc < a.cols) blk_store(a, true, bb, cc, blk_output<TU>(a, bb, cc));
+        }
+        return;
+    }
+    if (wave > 0) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        double y = acc[v];
+#pragma unroll
+        for (int g = 1; g < NW; ++g) y += part[((g - 1) * 4 + v) * 64 + lane];
+        const long bb = b0 + 4 * v + q4;
+        if (bb < a.nb && j0 + l16 < a.cols) blk_store(a, OUT, bb, j0 + l16, y);
+    }
+}
+
+// Many tiles: 64 x 64 tiles, four waves of 2 x 2 matrix-core tiles, K in slices
+// of 16 (first the states, then the window) staged in LDS and double buffered.
+constexpr int kPT = 64, kPK = 16;
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+struct BlkTileLds {
+    double A[2][kPT][kPK + 1];
+    double B[2][kPK][kPT + 1];
+    int bad;
+};
+
+template <typename TU, bool OUT>
+__device__ __forceinline__ void d_blk_tile(const VBlock vb, const BlkPass& a, BlkTileLds& L)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, q4 = lane >> 4;
+    const int wr = wave >> 1, wc = wave & 1;
+    const long b0 = vb.y * kPT;
+    const int j0 = (int)vb.x * kPT;
+    const int ar = tid >> 2, ak = (tid & 3) * 4;     // A slice: row, first of four k
+    const int bk = tid >> 4, bj = (tid & 15) * 4;    // B slice: k, first of four columns
+    const bool realA = b0 + ar < a.nb;
+    const long ab = realA ? b0 + ar : a.nb - 1;
+    const TU* u = static_cast<const TU*>(a.U) + ab * a.blockU;
+    const double* z = OUT ? a.Z + ab * a.na : nullptr;
+    int kl = realA ? win_len(a, ab) : 0;
+    int kEnd = a.ku, kMin = a.ku, stride = a.na;
+    int kcol[4];
+    long hb[4];                                      // offset of the column's factors in BU
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int col = j0 + bj + q;
+        kcol[q] = col < a.cols ? a.ku : 0;
+        hb[q] = col;
+        if (OUT && col < a.cols) {
+            const int i = col / a.p;
+            kcol[q] = (a.s * i + a.taps) * a.m;
+            hb[q] = (long)a.s * (a.T - 1 - i) * a.m * a.p + (col - i * a.p);
+        }
+    }
+    if (OUT) {
+        const int jl = j0 + kPT - 1 < a.cols ? j0 + kPT - 1 : a.cols - 1;
+        kEnd = (a.s * (jl / a.p) + a.taps) * a.m;
+        kMin = (a.s * (j0 / a.p) + a.taps) * a.m;
+        if (first_output(a, b0, j0)) kMin = 0;
+        stride = a.p;
+        kl = kl < kEnd ? kl : kEnd;   // (the last slice may reach past the tile's samples)
+        if (tid == 0) L.bad = 0;
+    }
+    const int kz = OUT ? a.kz : 0, zs = (kz + kPK - 1) / kPK;
+    const int slices = zs + (kEnd + kPK - 1) / kPK;
+    bool nf = false;
+    double ra[4], rb[4];
+    auto load = [&](int sl) {
+        if (OUT && sl < zs) {
+            const int k = sl * kPK + ak;
+            if (k + 4 <= kz) {
+                const double2u v0 = *reinterpret_cast<const double2u*>(z + k);
+                const double2u v1 = *reinterpret_cast<const double2u*>(z + k + 2);
+                ra[0] = v0.x;
+                ra[1] = v0.y;
+                ra[2] = v1.x;
+                ra[3] = v1.y;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) ra[q] = k + q < kz ? z[k + q] : 0.0;
+            }
+            const int kk = sl * kPK + bk;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = j0 + bj + q;
+                rb[q] = (kk < kz && col < a.cols) ? a.OT[(long)kk * a.cols + col] : 0.0;
+            }
+            return;
+        }
+        const int k = (sl - zs) * kPK + ak;
+        if (sizeof(TU) == 8 && a.gm == 0 && k + 4 <= kl) {
+            const double2u v0 = *reinterpret_cast<const double2u*>(u + k);
+            const double2u v1 = *reinterpret_cast<const double2u*>(u + k + 2);
+            ra[0] = v0.x;
+            ra[1] = v0.y;
+            ra[2] = v1.x;
+            ra[3] = v1.y;
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ra[q] = k + q < kl ? (double)u[win(a, k + q)] : 0.0;
+        }
+        if (OUT && k + 4 > kMin) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) nf = nf || not_finite(ra[q]);
+        }
+        const int kk = (sl - zs) * kPK + bk;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            rb[q] = kk < kcol[q] ? a.BU[hb[q] + (long)kk * stride] : 0.0;
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            L.A[buf][ar][ak + q] = ra[q];
+            L.B[buf][bk][bj + q] = rb[q];
+        }
+    };
+    doublex4 acc[2][2];
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj) acc[ti][tj] = doublex4{0.0, 0.0, 0.0, 0.0};
+    load(0);
+    store(0);
+    __syncthreads();
+    int buf = 0;
+    for (int sl = 0; sl < slices; ++sl) {
+        const bool more = sl + 1 < slices;
+        if (more) load(sl + 1);
+#pragma unroll
+        for (int ks = 0; ks < kPK; ks += 4) {
+            double x[2], y[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                x[t] = L.A[buf][wr * 32 + t * 16 + l16][ks + q4];
+                y[t] = L.B[buf][ks + q4][wc * 32 + t * 16 + l16];
+            }
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj)
+                    acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[ti], y[tj], acc[ti][tj],
+                                                                      0, 0, 0);
+        }
+        if (more) store(buf ^ 1);
+        __syncthreads();
+        buf ^= 1;
+    }
+    if (OUT) {
+        if (nf) L.bad = 1;
+        __syncthreads();
+        if (L.bad) {
+            for (int t = tid; t < kPT * kPT; t += 256) {
+                const long bb = b0 + t / kPT;
+                const int cc = j0 + t % kPT;
+                if (bb < a.nb && cc < a.cols)
+                    blk_store(a, true, bb, cc, blk_output<TU>(a, bb, cc));
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int tj = 0; tj < 2; ++tj) {
+        const int col = j0 + wc * 32 + tj * 16 + l16;
+        if (col >= a.cols) continue;
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const long bb = b0 + wr * 32 + ti * 16 + 4 * v + q4;
+                if (bb < a.nb) blk_store(a, OUT, bb, col, acc[ti][tj][v]);
+            }
+    }
+}
+
+// P_{l+1} = P_l^2 for l = lb .. L-2 of a small system, beside pass 1's tiles.
+template <int NW>
+__device__ __forceinline__ void d_blk_powers(int na, int lb, int L, double* PT, double* P)
+{
+    const int n16 = (na + 15) & ~15, nt = n16 / 16, tid = threadIdx.x, wave = tid >> 6;
+    const int l16 = tid & 15, q4 = (tid >> 4) & 3;
+    const long nn = (long)na * na;
+    for (int t = tid; t < n16 * n16; t += NW * 64) {
+        const int r = t / n16, c = t - r * n16;
+        P[r * kBP + c] = (r < na && c < na) ? PT[lb * nn + (long)r * na + c] : 0.0;
+    }
+    __syncthreads();
+    constexpr int U = 16 / NW < 1 ? 1 : 16 / NW;
+    for (int l = lb; l + 1 < L; ++l) {
+        doublex4 acc[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int w = wave + NW * q;
+            if (w < nt * nt)
+                acc[q] = lds_tile<false>(P, kBP, P, kBP, w / nt * 16, w % nt * 16, n16);
+        }
+        __syncthreads();
+        double* out = PT + (l + 1) * nn;
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+            const int w = wave + NW * q;
+            if (w >= nt * nt) continue;
+            for (int v = 0; v < 4; ++v) {
+                const int r = w / nt * 16 + 4 * v + q4, c = w % nt * 16 + l16;
+                P[r * kBP + c] = acc[q][v];
+                if (r < na && c < na) out[(long)r * na + c] = acc[q][v];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// The work-group's tile: consecutive work-groups go to different XCDs, each
+// with its own L2, so the tiles of one row block (which read the same samples)
+// are given to one XCD.  Row blocks past the last full eight keep plain order.
+__device__ __forceinline__ VBlock blk_place(long idx, long gx, long gy)
+{
+    const long full = gy / 8 * 8 * gx;
+    if (idx >= full) return VBlock{idx % gx, idx / gx, gx};
+    const long t = idx / 8;
+    return VBlock{t % gx, t / gx * 8 + idx % 8, gx};
+}
+
+template <typename TU, bool OUT, int NW>
+__global__ __launch_bounds__(NW * 64) void k_blk_split(const BlkPass a)
+{
+    constexpr int kPart = (NW - 1) * 256;
+    constexpr int kLds = OUT || kPart > kBN * kBP ? kPart : kBN * kBP;
+    __shared__ double lds[kLds];
+    __shared__ int bad;
+    if (!OUT && (long)blockIdx.x == a.gx * a.gy) {
+        d_blk_powers<NW>(a.na, a.lb, a.L, a.PT, lds);
+        return;
+    }
+    d_blk_split<TU, OUT, NW>(blk_place(blockIdx.x, a.gx, a.gy), a, lds, &bad);
+}
+
+template <typename TU, bool OUT>
+__global__ __launch_bounds__(256) void k_blk_tile(const BlkPass a)
+{
+    __shared__ BlkTileLds L;
+    static_assert(sizeof(BlkTileLds) >= kBN * kBP * sizeof(double), "room for the powers");
+    if (!OUT && (long)blockIdx.x == a.gx * a.gy) {
+        d_blk_powers<4>(a.na, a.lb, a.L, a.PT, &L.A[0][0][0]);
+        return;
+    }
+    d_blk_tile<TU, OUT>(blk_place(blockIdx.x, a.gx, a.gy), a, L);
+}
+
+// ------------------------------------------------------------------ the scan
+// Start states of Nb blocks: E_0 = Z_0, E_{b+1} = P E_b + S_b with P = P_l0.
+// The blocks are taken as up to 16 R groups of Lg consecutive ones, one group a
+// row of the matrix-core tiles; a wave holds 16 columns of P in registers.
+//   kScanAll  (one work-group): every group from zero; then the groups' start
+//             states by doubling, y_g += P_{l0 + lg + k} y_{g - 2^k}; then every
+//             group from its start state, writing E (in place of S)
+//   kScanUp   the groups' responses from zero to Zg (work-groups of 16 groups)
+//   kScanDown the groups from their start states in Zg, writing E
+// E[Nb] is the state after the last block.  Bound by the chain of 2 Lg + log2
+// steps, each a 16 x n_a x n_a product and an exchange through LDS.
+enum { kScanAll, kScanUp, kScanDown };
+struct BlkScan {
+    int na, l0, lg, L;
+    long nb;
+    const double* PT;
+    double *E, *Zg;
+    // the seed in X and its shift to Z (kScanAll)
+    const double *seed, *DL;
+    const void* U;
+    bool uDouble;
+    int km, m, gm, gx_;     // taps m; samples skipped after each window row
+    unsigned magic;
+    long last;
+    int R;                  // row tiles of a work-group
+    long gx;
+};
+
+// Z_0 = X_0 - sum_r D_r u_r
+__device__ __forceinline__ double blk_shift(const BlkScan& a, long row0, long at, int i)
+{
+    double v = 0.0;
+    const double* Ud = static_cast<const double*>(a.U);
+    const float* Uf = static_cast<const float*>(a.U);
+    for (int k = 0; k < a.km; ++k) {
+        const int r = a.m == 1 ? k : (int)__umulhi((unsigned)k, a.magic);
+        if (row0 + r > a.last) break;
+        const long o = at + k + (long)r * a.gm;
+        v = fma(a.DL[(long)k * a.na + i], a.uDouble ? Ud[o] : (double)Uf[o], v);
+    }
+    return v;
+}
+
+template <int MODE>
+__device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, double* lds)
+{
+    const int na = a.na, n16 = (na + 15) & ~15, nct = n16 / 16, pitch = n16 + 1;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q4 = lane >> 4;
+    const int rt = wave / nct, ct = wave - rt * nct, rows = 16 * a.R, nth = 64 * nct * a.R;
+    const long Lg = 1L << a.lg, g0 = vb.x * rows;
+    double* x0 = lds;                       // [rows][pitch], double buffered
+    double* x1 = lds + rows * pitch;
+    const long nn = (long)na * na;
+    const int col = ct * 16 + l16;
+    double p[kBN / 4];
+    auto load_p = [&](int l) {
+        const double* P = a.PT + l * nn;
+#pragma unroll
+        for (int u = 0; u < kBN / 4; ++u) {
+            const int k = 4 * u + q4;
+            p[u] = (k < na && col < na) ? P[(long)k * na + col] : 0.0;
+        }
+    };
+    // rows of x (this wave's row tile shifted up by d rows, zero above) times P
+    auto product = [&](const double* x, doublex4 acc, int d) {
+        const int r = rt * 16 + l16 - d;
+        const double* xr = x + (r > 0 ? r : 0) * pitch + q4;
+        const bool in = r >= 0;
+#pragma unroll
+        for (int u = 0; u < kBN / 4; ++u) {
+            if (4 * u >= n16) break;
+            const double v = in ? xr[4 * u] : 0.0;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, p[u], acc, 0, 0, 0);
+        }
+        return acc;
+    };
+    // this lane's groups (rows rt 16 + 4 v + q4) and its element of block e
+    long e0[4];
+    bool ok[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        e0[v] = (g0 + rt * 16 + 4 * v + q4) * Lg;
+        ok[v] = e0[v] < a.nb && col < na;
+    }
+    auto elem = [&](int v, long j) {
+        const long e = e0[v] + j;
+        return (ok[v] && j < Lg && e < a.nb) ? a.E[e * na + col] : 0.0;
+    };
+    auto put = [&](double* x, int v, double y) { x[(rt * 16 + 4 * v + q4) * pitch + col] = y; };
+    load_p(a.l0);
+    double* cur = x0;
+    double* nxt = x1;
+    auto flip = [&]() {
+        __syncthreads();
+        double* t = cur;
+        cur = nxt;
+        nxt = t;
+    };
+    doublex4 s;
+    if (MODE != kScanDown) {
+        // from zero: the first step takes S_0 as it is
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            put(cur, v, elem(v, 0));
+            s[v] = elem(v, 1);
+        }
+        __syncthreads();
+        for (long j = 1; j < Lg; ++j) {
+            doublex4 sn;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sn[v] = elem(v, j + 1);
+            const doublex4 y = product(cur, s, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                put(nxt, v, y[v]);
+                s[v] = sn[v];
+            }
+            flip();
+        }
+        if (MODE == kScanUp) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const long g = g0 + rt * 16 + 4 * v + q4;
+                if (ok[v]) a.Zg[g * na + col] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
+            }
+            return;
+        }
+        // the groups' start states: row g holds the response of group g - 1,
+        // row 0 the seed
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int g = rt * 16 + 4 * v + q4;
+            double y = 0.0;
+            if (g > 0) y = cur[(g - 1) * pitch + col];
+            if (g == 0 && col < na) y = a.seed[col] - blk_shift(a, 0, 0, col);
+            put(nxt, v, y);
+        }
+        flip();
+        const long groups = (a.nb + Lg - 1) / Lg;
+        for (int k = 0; (1L << k) < groups; ++k) {
+            load_p(a.l0 + a.lg + k);
+            doublex4 y;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y[v] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
+            y = product(cur, y, 1 << k);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) put(nxt, v, y[v]);
+            flip();
+        }
+        load_p(a.l0);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const long g = g0 + rt * 16 + 4 * v + q4;
+            put(cur, v, ok[v] ? a.Zg[g * na + col] : 0.0);
+        }
+        __syncthreads();
+    }
+    // from the start states: E_e over S_e, each read before it is written
+    doublex4 x;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        x[v] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
+        s[v] = elem(v, 0);
+    }
+    for (long j = 0; j < Lg; ++j) {
+        doublex4 sn;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sn[v] = elem(v, j + 1);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const long e = e0[v] + j;
+            if (ok[v] && e < a.nb) a.E[e * na + col] = x[v];
+        }
+        x = product(cur, s, 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const long e = e0[v] + j;
+            if (ok[v] && e == a.nb - 1) a.E[a.nb * na + col] = x[v];
+            put(nxt, v, x[v]);
+            s[v] = sn[v];
+        }
+        flip();
+    }
+    (void)nth;
+}
+
+template <int MODE>
+__global__ __launch_bounds__(MODE == kScanAll ? 1024 : 256) void k_blk_scan(const BlkScan a)
+{
+    extern __shared__ double scan_lds[];
+    d_blk_scan<MODE>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, scan_lds);
+}
+
+__global__ void k_blk_carry(const BlkScan a, long row0, long at, double* out)
+{
+    for (int i = threadIdx.x; i < a.na; i += blockDim.x)
+        out[i] = a.E[a.nb * a.na + i] + blk_shift(a, row0, at, i);
+}
+
+// ================================================================ host side
+static unsigned magic_of(int m) { return (unsigned)(((1ULL << 32) + m - 1) / m); }
+
+// The rule: which systems run as block responses, and with how many steps per
+// block.  Covered: inputs and outputs present, n_a, p, s m <= 64, m <= 32 (one
+// work-group's LDS holds the map), horizons from 64 points.  More steps per
+// block make the scan shorter (2 n_a^2 products a block, and its chain of
+// dependent steps), fewer make pass 2 cheaper (s m p T / 2 products a step).
+int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long nScan, long nPad)
+{
+    const int na = method == 1 ? 4 * n : n, s = method == 1 ? 1 : 2;
+    if (m < 1 || p < 1 || (!useC && useD)) return 0;
+    if (na > kBN || p > kBN || m > kBM || s * m > kBN || nScan < 64) return 0;
+    int best = 0;
+    double bt = 0.0;
+    for (int lb = 3; lb <= 8; ++lb) {
+        const double T = 1 << lb, N = (double)nScan, nb = N / T;
+        if ((nPad >> lb) < 2) break;
+        // (T m s < 2^16: the window index's multiply-high)
+        if ((long)(s * T + 8) * m >= 65536) break;
+        // microseconds: products at 25 TFLOP/s, the scan's chain, the tables
+        const double pass = N * (2.0 * na * s * m + 2.0 * p * na + 2.0 * s * m * p * (T / 2 + 8)) / 25e6;
+        const double steps = nb <= 512 ? nb / 64 : 2 * 16 + nb / 16 / 64;
+        const double scan = 2 * steps * (0.25 + na * 0.012) + 2 * nb * na * na * 2 / 0.25e6 / (nb <= 512 ? 1 : nb / 512);
+        const double tab = lb * 1.2 + T * (s * m + p) / 64 * 0.05;
+        const double t = pass + scan + tab;
+        if (!best || t < bt) {
+            best = lb;
+            bt = t;
+        }
+    }
+    return best;
+}
+
+BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bool mirror, int lb,
+                       int L)
+{
+    BlockShape s;
+    s.method = method;
+    s.n = n;
+    s.m = m;
+    s.p = useC ? p : n;
+    s.na = method == 1 ? 4 * n : n;
+    s.useC = useC;
+    s.useD = useD;
+    s.mirror = mirror;
+    s.lb = lb;
+    s.T = 1 << lb;
+    s.L = L;
+    s.s = method == 1 ? 1 : 2;
+    s.taps = method == 1 ? 4 : 1;
+    return s;
+}
+
+// One work-group scans up to 512 blocks; more go in groups of 16 (or as many
+// as leave 512 groups).
+static int group_log(long nb)
+{
+    if (nb <= 512) return 0;
+    int lg = 4;
+    while (((nb + (1L << lg) - 1) >> lg) > 512) ++lg;
+    return lg;
+}
+long block_groups(int na, long nb)
+{
+    (void)na;
+    const int lg = group_log(nb);
+    return lg ? (nb + (1L << lg) - 1) >> lg : 0;
+}
+
+void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+               const float* B, const float* C, const float* D, const float* x0, const void* U,
+               bool uDouble, double* seed, float* Y)
+{
+    const BlkMap a{s, h, rk4_coefficients(h), abm_coefficients(h), A, B, C, D, x0, U, b.PT, b.QT,
+                   b.Ht, b.DL, seed, Y, x0 ? 2L : 1L};
+    const size_t lds = s.method == 1 ? 6 * s.n * sizeof(double) + (size_t)s.n * (s.n + 1) * 4 : 0;
+    if (uDouble)
+        hipLaunchKernelGGL(k_blk_map<double>, dim3((unsigned)a.gx), dim3(1024), lds, st, a);
+    else
+        hipLaunchKernelGGL(k_blk_map<float>, dim3((unsigned)a.gx), dim3(1024), lds, st, a);
+    check_launch("block_map");
+}
+
+// steps of a slice: the largest power of two whose rows fit the LDS
+static int slice_steps(int T, int per)
+{
+    int k = 1;
+    while (2 * k <= T && 2 * k * per <= kBN) k *= 2;
+    return k;
+}
+
+void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C)
+{
+    BlkTables a{s, C, b.PT, b.QT, b.OT, b.Ht, slice_steps(s.T, s.p), slice_steps(s.T, s.s * s.m), 0};
+    a.gx = 1 + s.T / a.ni + s.T / a.nq;
+    hipLaunchKernelGGL(k_blk_tables, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
+    check_launch("block_tables");
+}
+
+static BlkPass pass_args(const BlockShape& s, const BlockBufs& b, const BlockInput& in, long nb)
+{
+    BlkPass a{};
+    a.na = s.na;
+    a.m = s.m;
+    a.p = s.p;
+    a.s = s.s;
+    a.T = s.T;
+    a.taps = s.taps;
+    a.nb = nb;
+    a.U = in.U;
+    a.blockU = s.T * in.sL * s.m;
+    a.gm = (int)(in.sL / s.s - 1) * s.m;
+    a.magic = magic_of(s.m);
+    a.last = in.last;
+    a.PT = b.PT;
+    a.lb = s.lb;
+    a.L = s.L;
+    return a;
+}
+
+// 64 x 64 tiles once they give every compute unit one; 16 x 16 below, their K
+// over 16 waves while those tiles are few too.
+template <bool OUT>
+static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, int tiling)
+{
+    const long tx = (a.cols + kPT - 1) / kPT, ty = (a.nb + kPT - 1) / kPT;
+    const long sx = (a.cols + 15) / 16, sy = (a.nb + 15) / 16;
+    const int ksteps = ((OUT ? a.kz : 0) + a.ku) / 4;
+    const bool tile = tiling ? tiling == kBlockTile : tx * ty >= 256;
+    a.gx = tile ? tx : sx;
+    a.gy = tile ? ty : sy;
+    const long blocks = a.gx * a.gy + (powers ? 1 : 0);
+    if (blocks > 0x7fffffffL) throw std::length_error("block pass: too many tiles");
+    const dim3 grid((unsigned)blocks);
+    const bool wide = !tile && (tiling ? tiling == kBlockSplit16 : sx * sy <= 256 && ksteps >= 64);
+#define PARODE_PASS(TU)                                                                   \
+    do {                                                                                  \
+        if (tile)                                                                         \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT>), grid, dim3(256), 0, st, a);         \
+        else if (wide)                                                                    \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 16>), grid, dim3(1024), 0, st, a);   \
+        else                                                                              \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 4>), grid, dim3(256), 0, st, a);     \
+    } while (0)
+    if (uDouble)
+        PARODE_PASS(double);
+    else
+        PARODE_PASS(float);
+#undef PARODE_PASS
+    check_launch("block pass");
+}
+
+void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, bool powers, int tiling)
+{
+    BlkPass a = pass_args(s, b, in, nb);
+    a.cols = s.na;
+    a.kz = 0;
+    a.ku = s.kb();
+    a.BU = b.QT;
+    a.S = b.Z;
+    launch_pass<false>(st, a, in.isDouble, powers, tiling);
+}
+
+void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, long nReal, const double* seed, const float* D, float* Y, int tiling)
+{
+    BlkPass a = pass_args(s, b, in, nb);
+    a.cols = s.T * s.p;
+    a.kz = s.na;
+    a.ku = s.kh();
+    a.nReal = nReal;
+    a.Z = b.Z;
+    a.OT = b.OT;
+    a.BU = b.Ht;
+    a.Y = Y;
+    a.seed = seed;
+    a.D = s.useD ? D : nullptr;
+    launch_pass<true>(st, a, in.isDouble, false, tiling);
+}
+
+static BlkScan scan_args(const BlockShape& s, const BlockBufs& b, const BlockInput& in, long nb,
+                         const double* seed)
+{
+    BlkScan a{};
+    a.na = s.na;
+    a.l0 = s.lb;
+    a.L = s.L;
+    a.nb = nb;
+    a.PT = b.PT;
+    a.E = b.Z;
+    a.Zg = b.Z2;
+    a.seed = seed;
+    a.DL = b.DL;
+    a.U = in.U;
+    a.uDouble = in.isDouble;
+    a.km = s.taps * s.m;
+    a.m = s.m;
+    a.gm = (int)(in.sL / s.s - 1) * s.m;
+    a.magic = magic_of(s.m);
+    a.last = in.last;
+    return a;
+}
+
+void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                long nb, const double* seed)
+{
+    const int nct = (s.na + 15) / 16, pitch = 16 * nct + 1;
+    auto lds = [&](int R) { return (size_t)2 * 16 * R * pitch * sizeof(double); };
+    BlkScan a = scan_args(s, b, in, nb, seed);
+    const int lg = group_log(nb);
+    const long groups = block_groups(s.na, nb);
+    if (lg) {
+        BlkScan u = a;
+        u.lg = lg;
+        u.R = 1;
+        u.gx = (groups + 15) / 16;
+        hipLaunchKernelGGL(k_blk_scan<kScanUp>, dim3((unsigned)u.gx), dim3(64 * nct), lds(1), st, u);
+        check_launch("block scan, up");
+        a.nb = groups;
+        a.E = b.Z2;
+        a.l0 = s.lb + lg;
+    }
+    // as many row tiles as 16 waves (and 64 KB of LDS) hold, no more than the blocks need
+    a.R = 1;
+    while (2 * a.R * nct <= 16 && lds(2 * a.R) <= 65536 && 16L * a.R < a.nb) a.R *= 2;
+    a.lg = 0;
+    while ((16L * a.R << a.lg) < a.nb) ++a.lg;
+    a.gx = 1;
+    hipLaunchKernelGGL(k_blk_scan<kScanAll>, dim3(1), dim3(64 * nct * a.R), lds(a.R), st, a);
+    check_launch("block scan");
+    if (lg) {
+        BlkScan d = scan_args(s, b, in, nb, seed);
+        d.lg = lg;
+        d.R = 1;
+        d.gx = (groups + 15) / 16;
+        hipLaunchKernelGGL(k_blk_scan<kScanDown>, dim3((unsigned)d.gx), dim3(64 * nct), lds(1), st, d);
+        check_launch("block scan, down");
+    }
+}
+
+void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, double* seedOut)
+{
+    const BlkScan a = scan_args(s, b, in, nb, nullptr);
+    hipLaunchKernelGGL(k_blk_carry, dim3(1), dim3(256), 0, st, a, nb * s.s * s.T,
+                       nb * s.T * in.sL * s.m, seedOut);
+    check_launch("block carry");
+}
+
+}  // namespace k
+}  // namespace parode

@@ -8,6 +8,7 @@
 // the reference's MM kernels, left-leaf and root copies collapse into the
 // power table and into the in-place pair update.
 #include "kernels.h"
+#include "launch.h"
 
 #include <algorithm>
 #include <vector>
@@ -18,28 +19,6 @@
 
 namespace parode {
 namespace k {
-
-// The block a kernel body works on: (x, y) and the grid's width in x.  A
-// single-system launch passes its own blockIdx and gridDim; a grouped launch
-// (many systems in one grid) passes the block's place in its system's grid.
-struct VBlock {
-    long x, y, gx;
-};
-
-static void check_launch(const char* what)
-{
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
-        throw std::runtime_error(std::string("kernel launch failed: ") + what + ": " +
-                                 hipGetErrorString(e));
-}
-
-static inline unsigned blocks_for(long work, int block, long cap = 1L << 20)
-{
-    long b = (work + block - 1) / block;
-    if (b < 1) b = 1;
-    return (unsigned)std::min(b, cap);
-}
 
 // ---------------------------------------------------------------- helpers
 template <typename T>
@@ -157,7 +136,6 @@ __global__ void k_gemm_f64_mfma(int r, int kk, int c, const double* __restrict__
 // per SIMD than one-wave-per-tile kernels, whose dependent FP64 MFMAs leave the
 // pipe idle.  Loads are bounds-checked; the next slice is in flight while the
 // current one is multiplied.
-typedef double doublex4 __attribute__((ext_vector_type(4)));
 constexpr int kGemmKsT = 32, kGemmKsKB = 32;
 
 // Leading dimensions of the FP64 GEMMs' operands (X r x kk, Y kk x c, Z r x c,
@@ -3820,94 +3798,6 @@ template void outputs<double, float>(hipStream_t, int, int, int, int, int, bool,
                                      const float*, const float*, const double*, const float*,
                                      long, long, float*);
 
-// ------------------------------------------------------------ ABM start-up
-// Three classic RK4 steps (AdamsMoulton.cpp:96-103).  mirror: float state and
-// float derivative sums (AdamsMoulton.cpp:15-27), stage combinations formed
-// in double and stored to float (odeint runge_kutta4<vector<float>>).
-// When A fits (pitch n + 1, no bank conflicts), it is staged in LDS once: the
-// twelve derivative evaluations are chains of n dependent products per row,
-// which from global memory wait on a load each.
-template <typename TU>
-__device__ __forceinline__ void d_abm_startup(const VBlock vb, bool mirror, int n, int m, double h, bool ldsA,
-                              const float* __restrict__ A, const float* __restrict__ B,
-                              const float* __restrict__ x0, const TU* __restrict__ Uh,
-                              double* __restrict__ X0)
-{
-#pragma clang fp contract(off)
-    extern __shared__ double sh[];
-    double* x = sh;            // n
-    double* xt = sh + n;       // n
-    double* kb = sh + 2 * n;   // 4n: k1..k4
-    float* As = reinterpret_cast<float*>(sh + 6 * n);   // n x (n + 1) when ldsA
-    const double dh = h / 2.0, dt6 = h / 6.0, dt3 = h / 3.0;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-        x[r] = (double)x0[r];
-        X0[r] = (double)x0[r];
-    }
-    if (ldsA)
-        for (int t = threadIdx.x; t < n * n; t += blockDim.x) {
-            const int r = t / n;
-            As[t + r] = A[t];   // row r at r * (n + 1)
-        }
-    __syncthreads();
-    const float* Ar = ldsA ? As : A;
-    const long ap = ldsA ? n + 1 : n;
-    auto deriv = [&](const double* xs, int urow, double* out) {
-        for (int r = threadIdx.x; r < n; r += blockDim.x) {
-            if (mirror) {
-                float f = 0.0f;
-                for (int c = 0; c < n; ++c) {
-                    float pr = Ar[r * ap + c] * (float)xs[c];
-                    f = f + pr;
-                }
-                for (int c = 0; c < m; ++c) {
-                    float pr = B[(long)r * m + c] * (float)Uh[(long)urow * m + c];
-                    f = f + pr;
-                }
-                out[r] = (double)f;
-            } else {
-                double f = 0.0;
-                for (int c = 0; c < n; ++c) f = fma((double)Ar[r * ap + c], xs[c], f);
-                for (int c = 0; c < m; ++c)
-                    f = fma((double)B[(long)r * m + c], (double)Uh[(long)urow * m + c], f);
-                out[r] = f;
-            }
-        }
-        __syncthreads();
-    };
-    auto stage = [&](const double* kk, double coef) {
-        for (int r = threadIdx.x; r < n; r += blockDim.x) {
-            double v = 1.0 * x[r] + coef * kk[r];
-            xt[r] = mirror ? (double)(float)v : v;
-        }
-        __syncthreads();
-    };
-    for (int s = 0; s < 3; ++s) {
-        double* k1 = kb;
-        double* k2 = kb + n;
-        double* k3 = kb + 2 * n;
-        double* k4 = kb + 3 * n;
-        deriv(x, 2 * s, k1);
-        stage(k1, dh);
-        deriv(xt, 2 * s + 1, k2);
-        stage(k2, dh);
-        deriv(xt, 2 * s + 1, k3);
-        stage(k3, h);
-        deriv(xt, 2 * s + 2, k4);
-        for (int r = threadIdx.x; r < n; r += blockDim.x) {
-            double v;
-            if (mirror)
-                v = (double)(float)((((1.0 * x[r] + dt6 * k1[r]) + dt3 * k2[r]) + dt3 * k3[r]) +
-                                    dt6 * k4[r]);
-            else
-                v = x[r] + (h / 6.0) * (k1[r] + 2.0 * k2[r] + 2.0 * k3[r] + k4[r]);
-            x[r] = v;
-            X0[(long)(s + 1) * n + r] = v;
-        }
-        __syncthreads();
-    }
-}
-
 template <typename TU>
 __global__ void k_abm_startup(bool mirror, int n, int m, double h, bool ldsA,
                               const float* __restrict__ A, const float* __restrict__ B,
@@ -4039,26 +3929,6 @@ void sample_family(hipStream_t s, int m, const double* coef, double t0, double d
 namespace g {
 
 namespace {
-
-__device__ __forceinline__ int system_of(const unsigned* __restrict__ start, int nsys)
-{
-    const unsigned b = blockIdx.x;
-    int lo = 0, hi = nsys - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (start[mid] <= b)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return lo;
-}
-
-__device__ __forceinline__ VBlock block_of(const unsigned* __restrict__ start, int s, long gx)
-{
-    const long lb = (long)blockIdx.x - (long)start[s];
-    return VBlock{lb % gx, lb / gx, gx};
-}
 
 // Argument records (one per system of a launch; gx: the system's grid width).
 struct Prep {        // kind 0: out = (double)in; 1: out = v; 2: out[r][c] = in[c][r], c < cols, padded to pp
@@ -4200,11 +4070,6 @@ struct Outputs {
     float* Y;
     long gx;
 };
-
-#define PARODE_GROUP(T)                          \
-    const int sys_ = system_of(st, ns);          \
-    const T& a = args[sys_];                     \
-    const VBlock vb = block_of(st, sys_, a.gx)
 
 __global__ __launch_bounds__(256) void kg_prep(const Prep* __restrict__ args,
                                                const unsigned* __restrict__ st, int ns)
@@ -4436,51 +4301,6 @@ __global__ __launch_bounds__(kOutLanes) void kg_out_kc(const Outputs* __restrict
     PARODE_GROUP(Outputs);
     d_outputs_kc<float, double, JG>(vb, a.n, a.m, a.p, a.pp, a.na, a.oX, a.useC, a.useD, a.N,
                                     a.CT, a.DT, a.X, a.U, a.sO, a.oO, a.Y);
-}
-
-#undef PARODE_GROUP
-
-// The record of the launch (kind, flag) in phase ph, created on first use.
-template <typename A>
-Launch& slot(Phase& ph, int kind, bool flag, int cls)
-{
-    Launch& L = ph[{kind, (flag ? 1 : 0) + 2 * cls}];
-    if (L.kind < 0) {
-        L.kind = kind;
-        L.flag = flag;
-        L.argSize = sizeof(A);
-    }
-    if (L.argSize != sizeof(A)) throw std::logic_error("grouped launch: argument type mismatch");
-    return L;
-}
-
-// Systems whose dynamic LDS differs go to separate launches by size class
-// (up to 8, 16, 32, 48, 64 KiB ...): a launch reserves its largest system's
-// LDS for every work-group, which would cap the occupancy of the others.
-int lds_class(size_t lds)
-{
-    if (lds == 0) return 0;
-    const size_t kib = (lds + 1023) / 1024;
-    return kib <= 8 ? 1 : kib <= 16 ? 2 : kib <= 32 ? 3 : kib <= 48 ? 4 : 5 + (int)((kib - 49) / 16);
-}
-
-template <typename A>
-void append(Phase& ph, int kind, bool flag, const A& a, long blocks, size_t lds = 0,
-            float cost = 0.0f)
-{
-    if (blocks < 1) return;
-    // (the top of the tree runs one 1024-thread work-group per system, one per
-    // CU whatever its LDS: its systems share one launch)
-    const bool oneClass = kind == kTopMfma || kind == kTopSimt;
-    Launch& L = slot<A>(ph, kind, flag, oneClass ? 0 : lds_class(lds));
-    const size_t o = L.args.size();
-    L.args.resize(o + sizeof(A));
-    std::memcpy(L.args.data() + o, &a, sizeof(A));
-    const unsigned long next = (unsigned long)L.start.back() + (unsigned long)blocks;
-    if (next > 0x7fffffffUL) throw std::length_error("grouped launch: too many blocks");
-    L.start.push_back((unsigned)next);
-    L.cost.push_back(cost);
-    L.lds = std::max(L.lds, lds);
 }
 
 }  // namespace

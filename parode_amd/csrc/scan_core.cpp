@@ -16,7 +16,7 @@ int pad8(int c) { return c > 0 ? (c + 7) / 8 * 8 : 8; }
 namespace parode {
 
 ScanCore::ScanCore(int method, int n, int m, int p, bool zC, bool zD, long nPadMax, ScanOptions opt,
-                   Arena* arena)
+                   Arena* arena, bool blocks)
     : method_(method), n_(n), m_(m), p_(p), na_(method == kABM ? 4 * n : n), zC_(zC), zD_(zD),
       nPadMax_(next_pow2(nPadMax < 1 ? 1 : nPadMax)), L_(ilog2(nPadMax_)), opt_(opt)
 {
@@ -24,6 +24,37 @@ ScanCore::ScanCore(int method, int n, int m, int p, bool zC, bool zD, long nPadM
     const size_t nn = (size_t)n * n, nm = (size_t)n * (m > 0 ? m : 1);
     const size_t na2 = (size_t)na_ * na_;
     const int kq = method == kABM ? 5 : 3;
+    if (blocks && level_kernel() == 0) {
+        const bool states = zC && zD;
+        int lb = k::block_steps_log(method, n, m, p, !zC, !zD, nPadMax_, nPadMax_);
+        // as long as its buffers take no more than the general path's
+        const size_t cap = estimate_footprint(method, n, m, nPadMax_, opt, p);
+        for (; lb > 0; --lb) {
+            const k::BlockShape b =
+                k::block_shape(method, n, m, states ? n : p, !zC, !zD,
+                               opt_.precision == kPlain32, lb, L_ + 1);
+            const size_t na = na_, nb = (size_t)(nPadMax_ >> lb);
+            const size_t tab = ((size_t)b.kb() + (size_t)b.T * b.p + (size_t)b.taps * m) * na +
+                               (size_t)b.kh() * b.p;
+            const size_t z = (nb + 1 + k::block_groups(na_, (long)nb) + 1) * na;
+            if (8 * (na2 * (L_ + 1) + tab + z + 3 * na) + 6 * Arena::kAlign > cap) continue;
+            PT64_.alloc(na2 * (L_ + 1), arena);
+            blkTab_.alloc(tab, arena);
+            blkZ_.alloc(z, arena);
+            seed_.alloc(na_, arena);
+            tot_.alloc(na_, arena);
+            seedNext_.alloc(na_, arena);
+            blk_ = b;
+            bb_.PT = PT64_.get();
+            bb_.QT = blkTab_.get();
+            bb_.OT = bb_.QT + (size_t)b.kb() * na;
+            bb_.Ht = bb_.OT + (size_t)b.T * b.p * na;
+            bb_.DL = bb_.Ht + (size_t)b.kh() * b.p;
+            bb_.Z = blkZ_.get();
+            bb_.Z2 = bb_.Z + (nb + 1) * na;
+            return;
+        }
+    }
     if (opt_.precision == kPlain32) {
         prod32_.alloc(4 * nn + 4 * nm, arena);            // A, A2, A3, A4 | B, AB, A2B, A3B (float)
     } else {
@@ -102,7 +133,7 @@ size_t ScanCore::footprint() const
            DT_.bytes() + CT64_.bytes() + DT64_.bytes() +
            PT64_.bytes() + PT32_.bytes() + PTm_.bytes() + Sg_.bytes() + Sks32_.bytes() +
            Sks64_.bytes() + X32_.bytes() + X64_.bytes() + seed_.bytes() +
-           tot_.bytes() + seedNext_.bytes();
+           tot_.bytes() + seedNext_.bytes() + blkTab_.bytes() + blkZ_.bytes();
 }
 
 bool ScanCore::level_is_f64(int l) const
@@ -128,6 +159,11 @@ void ScanCore::build_map(hipStream_t s, const float* dA, const float* dB, double
                          const SideStream* side)
 {
     h_ = h;
+    if (uses_blocks()) {   // made with the tables, which need C and D too
+        dA_ = dA;
+        dB_ = dB;
+        return;
+    }
     const int n = n_, m = m_;
     const size_t nn = (size_t)n * n, nm = (size_t)n * (m > 0 ? m : 1);
     double* MT = PT64_.get();
@@ -213,6 +249,13 @@ void ScanCore::build_map(hipStream_t s, const float* dA, const float* dB, double
 
 void ScanCore::build_powers(hipStream_t s, bool withLast)
 {
+    if (uses_blocks()) {
+        k::block_map(s, blk_, bb_, h_, dA_, dB_, dC_, dD_, nullptr, nullptr, false, nullptr,
+                     nullptr);
+        k::block_tables(s, blk_, bb_, dC_);
+        powersDone_ = false;   // the first batch's pass 1 makes the rest of them
+        return;
+    }
     const size_t na2 = (size_t)na_ * na_;
     // (P^T)^2 = (P^2)^T: squaring the transposed table keeps it transposed
     const bool mm = (level_kernel() & 2) == 0;
@@ -294,6 +337,15 @@ void ScanCore::leaves(hipStream_t s, const void* dU, bool uDouble, long sL, long
     const int kq = method_ == kABM ? 5 : 3;
     const int off = method_ == kABM ? 3 * n_ : 0;
     if (nPad > nPadMax_) throw std::invalid_argument("ScanCore::leaves: batch too long");
+    if (uses_blocks()) {
+        if (oL != 0 || rs * blk_.s != (method_ == kABM ? sL : 2 * rs) || sL % blk_.s != 0)
+            throw std::invalid_argument("ScanCore::leaves: sample layout");
+        in_ = block_input(dU, uDouble, sL, nReal);
+        const long nb = blocks_of(nReal);
+        k::block_pass1(s, blk_, bb_, in_, nb, !powersDone_, block_tiling(1, nb, uDouble));
+        powersDone_ = true;
+        return;
+    }
     if (leafFac_) {
         const bool wz =
             xIsDouble() || !(structured_level0(nReal, nPad) || chunk_log(nReal, nPad) > 0);
@@ -346,6 +398,8 @@ namespace {
 // The autotuned schedule: (n_a, precision, level, pairs, down) -> path
 std::mutex g_schedMu;
 std::map<std::array<long, 5>, int> g_sched;
+// and of the block passes: (n_a, m, p, T, blocks, FP64 samples, pass) -> tiling
+std::map<std::array<long, 7>, int> g_blockSched;
 }  // namespace
 
 int ScanCore::scheduled_path(bool down, int l, long np) const
@@ -359,6 +413,7 @@ void ScanCore::clear_schedule()
 {
     std::lock_guard<std::mutex> lk(g_schedMu);
     g_sched.clear();
+    g_blockSched.clear();
 }
 
 void ScanCore::level(hipStream_t s, bool down, int l, long np)
@@ -494,6 +549,7 @@ static k::LevelRows abm_rows(int n, int level, bool down, bool next)
 
 void ScanCore::sweep_up(hipStream_t s, long nReal, long nPad, hipEvent_t waitTables)
 {
+    if (uses_blocks()) return;   // (sweep_top scans the blocks' states)
     const int lt = top_level(nReal, nPad);
     int l = 0;
     const int lc = chunk_log(nReal, nPad);
@@ -529,6 +585,7 @@ void ScanCore::zero_trajectory(hipStream_t s, long nPad)
 int ScanCore::autotune(hipStream_t s, long nReal, long nPad)
 {
     if (nPad > nPadMax_ || nReal < 1) throw std::invalid_argument("ScanCore::autotune: bad length");
+    if (uses_blocks()) return autotune_blocks(s, nReal);
     const int lt = top_level(nReal, nPad);
     const bool s0 = lt > 0 && structured_level0(nReal, nPad);
     const bool s1 = s0 && structured_level1(nReal, nPad);
@@ -595,6 +652,11 @@ int ScanCore::autotune(hipStream_t s, long nReal, long nPad)
 
 void ScanCore::sweep_top(hipStream_t s, long nReal, long nPad, const double* dSeed, double* dTot)
 {
+    if (uses_blocks()) {
+        batchSeed_ = dSeed;
+        k::block_scan(s, blk_, bb_, in_, blocks_of(nReal), dSeed);
+        return;
+    }
     const int L = ilog2(nPad), lt = top_level(nReal, nPad);
     if (lt >= L) {   // no fused top: the root alone
         if (xIsDouble())
@@ -645,6 +707,7 @@ void ScanCore::down_levels(hipStream_t s, int hi, int lo, long nReal)
 
 void ScanCore::sweep_down(hipStream_t s, long nReal, long nPad)
 {
+    if (uses_blocks()) return;
     const int lt = top_level(nReal, nPad);
     if (const int lc = chunk_log(nReal, nPad)) {   // levels below lc: chunk recurrences
         down_levels(s, lt - 1, lc, nReal);
@@ -667,6 +730,10 @@ void ScanCore::sweep_down(hipStream_t s, long nReal, long nPad)
 void ScanCore::carry(hipStream_t s, long nPad, const double* dSeed, const double* dTot,
                      double* dOut)
 {
+    if (uses_blocks()) {   // (a batch before the last is full)
+        k::block_carry(s, blk_, bb_, in_, nPad >> blk_.lb, dOut);
+        return;
+    }
     k::carry(s, na_, powerT(ilog2(nPad)), dSeed, dTot, dOut);
 }
 
@@ -691,6 +758,14 @@ void ScanCore::prepare_outputs(hipStream_t s, const float* dC, const float* dD, 
 void ScanCore::outputs(hipStream_t s, const float* dC, const float* dD, const void* dU,
                        bool uDouble, long sO, long oO, long N, float* dY, bool prepared)
 {
+    if (uses_blocks()) {
+        if (sO != in_.sL || oO != (method_ == kABM ? 3 * in_.sL : 0) || dU != in_.U ||
+            uDouble != in_.isDouble)
+            throw std::invalid_argument("ScanCore::outputs: sample layout");
+        const long nb = blocks_of(N);
+        k::block_pass2(s, blk_, bb_, in_, nb, N, batchSeed_, dD, dY, block_tiling(2, nb, uDouble));
+        return;
+    }
     const int oX = method_ == kABM ? 3 : 0;
     if (!prepared) prepare_outputs(s, dC, dD, uDouble);
     dC = CT_.get();
@@ -757,6 +832,104 @@ void ScanCore::abm_startup(hipStream_t s, const float* dA, const float* dB, cons
         k::abm_startup<float>(s, mirror, n_, m_, h, dA, dB, dx0, (const float*)dUh, dX0);
 }
 
+// ----------------------------------------------------------- block responses
+k::BlockInput ScanCore::block_input(const void* dU, bool uDouble, long sL, long nReal) const
+{
+    // the last window row that the general path's leaves read, too
+    return k::BlockInput{dU, uDouble, sL, blk_.s * (nReal - 1) + (method_ == kABM ? 4 : 2)};
+}
+
+int ScanCore::block_tiling(int pass, long nb, bool uDouble) const
+{
+    std::lock_guard<std::mutex> lk(g_schedMu);
+    auto it = g_blockSched.find({(long)na_, (long)m_, (long)blk_.p, (long)blk_.T, nb,
+                                 uDouble ? 1L : 0L, (long)pass});
+    return it == g_blockSched.end() ? k::kBlockAuto : it->second;
+}
+
+// Times each tiling of the two passes on samples of zeros.
+int ScanCore::autotune_blocks(hipStream_t s, long nReal)
+{
+    const bool dbl = opt_.precision != kPlain32;
+    const long nb = blocks_of(nReal), sL = 2;
+    k::BlockInput in = block_input(nullptr, dbl, sL, nReal);
+    const size_t vals = (size_t)(in.last + 1) * (sL / blk_.s) * m_;
+    DevArray<double> U(vals);
+    DevArray<float> Y((size_t)nReal * blk_.p);
+    k::fill_f64(s, (long)vals, 0.0, U.get());
+    zero_blocks(s);
+    in.U = U.get();
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    PARODE_HIP(hipEventCreate(&e0));
+    PARODE_HIP(hipEventCreate(&e1));
+    try {
+        for (int pass = 1; pass <= 2; ++pass) {
+            int best = k::kBlockAuto;
+            float bestMs = 0.0f;
+            for (int t : {k::kBlockTile, k::kBlockSplit4, k::kBlockSplit16}) {
+                auto run = [&] {
+                    if (pass == 1)
+                        k::block_pass1(s, blk_, bb_, in, nb, false, t);
+                    else
+                        k::block_pass2(s, blk_, bb_, in, nb, nReal, seed(), nullptr, Y.get(), t);
+                };
+                run();
+                PARODE_HIP(hipEventRecord(e0, s));
+                for (int r = 0; r < 3; ++r) run();
+                PARODE_HIP(hipEventRecord(e1, s));
+                PARODE_HIP(hipEventSynchronize(e1));
+                float ms = 0.0f;
+                PARODE_HIP(hipEventElapsedTime(&ms, e0, e1));
+                if (best == k::kBlockAuto || ms < bestMs) {
+                    best = t;
+                    bestMs = ms;
+                }
+            }
+            std::lock_guard<std::mutex> lk(g_schedMu);
+            g_blockSched[{(long)na_, (long)m_, (long)blk_.p, (long)blk_.T, nb, dbl ? 1L : 0L,
+                          (long)pass}] = best;
+        }
+    } catch (...) {
+        (void)hipStreamSynchronize(s);
+        (void)hipEventDestroy(e0);
+        (void)hipEventDestroy(e1);
+        throw;
+    }
+    PARODE_HIP(hipEventDestroy(e0));
+    PARODE_HIP(hipEventDestroy(e1));
+    return 2;
+}
+
+void ScanCore::zero_blocks(hipStream_t s)
+{
+    k::fill_f64(s, (long)blkTab_.size(), 0.0, blkTab_.get());
+    k::fill_f64(s, (long)blkZ_.size(), 0.0, blkZ_.get());
+}
+
+void ScanCore::solve_blocks(hipStream_t s, long nScan, double h, const float* dA, const float* dB,
+                            const float* dC, const float* dD, const float* dx0, const void* dU,
+                            bool uDouble, float* dY, hipEvent_t* marks)
+{
+    auto tick = [&](int i) {
+        if (marks) PARODE_HIP(hipEventRecord(marks[i], s));
+    };
+    const long nb = blocks_of(nScan);
+    const k::BlockInput in = block_input(dU, uDouble, 2, nScan);
+    tick(0);
+    k::block_map(s, blk_, bb_, h, dA, dB, dC, dD, dx0, dU, uDouble, seed(), dY);
+    k::block_tables(s, blk_, bb_, dC);
+    tick(1);
+    k::block_pass1(s, blk_, bb_, in, nb, true, block_tiling(1, nb, uDouble));
+    tick(2);
+    tick(3);
+    k::block_scan(s, blk_, bb_, in, nb, seed());
+    tick(4);
+    tick(5);
+    k::block_pass2(s, blk_, bb_, in, nb, nScan, seed(), dD,
+                   method_ == kRK4 ? dY : dY + 3L * nOut(), block_tiling(2, nb, uDouble));
+    tick(6);
+}
+
 // ---------------------------------------------------------------- one solve
 void ScanCore::solve(hipStream_t s, long points, double h, const float* dA, const float* dB,
                      const float* dC, const float* dD, const float* dx0, const void* dU,
@@ -767,6 +940,10 @@ void ScanCore::solve(hipStream_t s, long points, double h, const float* dA, cons
     if (nScan < 1 || nPad > nPadMax_) throw std::invalid_argument("ScanCore::solve: bad length");
     if (side && (!side->stream || !side->fork || !side->join))
         throw std::invalid_argument("ScanCore::solve: incomplete side stream");
+    if (uses_blocks()) {
+        solve_blocks(s, nScan, h, dA, dB, dC, dD, dx0, dU, uDouble, dY, marks);
+        return;
+    }
     auto tick = [&](int i) {
         if (marks) PARODE_HIP(hipEventRecord(marks[i], s));
     };

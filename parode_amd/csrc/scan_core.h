@@ -16,6 +16,7 @@
 //                  is dead work and is not performed
 //   outputs      : SystemOutput
 #pragma once
+#include "blocks.h"
 #include "hip_util.h"
 
 #include <vector>
@@ -37,8 +38,11 @@ struct ScanOptions {
 class ScanCore {
 public:
     // Buffers come from hipMalloc, or from `arena` when given (serving).
+    // blocks: the shape may run as block responses (blocks.h) where their rule
+    // takes it and no kernel switch is set; the trajectory X is then not formed
+    // (X() is null).
     ScanCore(int method, int n, int m, int p, bool zC, bool zD, long nPadMax, ScanOptions opt,
-             Arena* arena = nullptr);
+             Arena* arena = nullptr, bool blocks = true);
 
     int method() const { return method_; }
     int n() const { return n_; }
@@ -64,6 +68,13 @@ public:
         hipStream_t stream = nullptr;
         hipEvent_t fork = nullptr, join = nullptr, late = nullptr;
     };
+    bool uses_blocks() const { return blk_.T > 0; }
+    // C and D for block responses (before build_powers; null where absent)
+    void set_outputs(const float* dC, const float* dD)
+    {
+        dC_ = dC;
+        dD_ = dD;
+    }
     void build_map(hipStream_t s, const float* dA, const float* dB, double h,
                    const SideStream* side = nullptr);
     // withLast: also P_L = M^(2^L), which only carry() between batches reads
@@ -145,6 +156,15 @@ private:
     std::vector<int> level_candidates(int l, long np) const;
     void zero_trajectory(hipStream_t s, long nPad);
 
+    void solve_blocks(hipStream_t s, long nScan, double h, const float* dA, const float* dB,
+                      const float* dC, const float* dD, const float* dx0, const void* dU,
+                      bool uDouble, float* dY, hipEvent_t* marks);
+    k::BlockInput block_input(const void* dU, bool uDouble, long sL, long nReal) const;
+    long blocks_of(long nReal) const { return (nReal + blk_.T - 1) / blk_.T; }
+    int block_tiling(int pass, long nb, bool uDouble) const;
+    int autotune_blocks(hipStream_t s, long nReal);
+    void zero_blocks(hipStream_t s);
+
     int method_, n_, m_, p_, na_;
     bool zC_, zD_;
     long nPadMax_;
@@ -178,6 +198,14 @@ private:
         long npOut = 0;
     } ksc_;
     int nap_ = 0, nrp_ = 0;
+    // block responses: tables and the blocks' states; the batch's input
+    k::BlockShape blk_;
+    k::BlockBufs bb_;
+    DevArray<double> blkTab_, blkZ_;
+    k::BlockInput in_;
+    const float *dA_ = nullptr, *dB_ = nullptr, *dC_ = nullptr, *dD_ = nullptr;
+    const double* batchSeed_ = nullptr;
+    bool powersDone_ = false;
     // trajectory
     DevArray<float> X32_;
     DevArray<double> X64_;

@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <iostream>
+#include <typeinfo>
 
 #include "config.h"
 #include "hip_util.h"
@@ -108,7 +109,10 @@ void GPUODESolverFixedStepIterative::CreateScanCore(int method, const matrixf& A
     ScanOptions opt;
     opt.precision = _nPrecision;
     _core.reset(new ScanCore(method, n, m, (int)_nOutputSize, _bZeroC == 1, _bZeroD == 1,
-                             (long)nPadMax, opt));
+                             (long)nPadMax, opt, nullptr,
+                             // (other plug-ins may fill the trajectory themselves)
+                             typeid(*this) == typeid(RungeKutta4thOrder) ||
+                                 typeid(*this) == typeid(AdamsMoulton)));
     _BufferA.reset(new DeviceBuffer(sizeof(float) * n * n, dev));
     _BufferA->MemWrite(A.data(), s);
     _BufferB.reset(new DeviceBuffer(sizeof(float) * n * (m > 0 ? m : 1), dev));
@@ -200,6 +204,8 @@ ErrorCode GPUODESolverFixedStepIterative::SimulateODE(const matrixf& A, const ma
         DeleteGPUFSIObjects();
         return ParODE_NotEnoughResources;
     }
+    _core->set_outputs(_BufferC && !_bZeroC ? (const float*)_BufferC->Get() : nullptr,
+                       _BufferD && !_bZeroD ? (const float*)_BufferD->Get() : nullptr);
     const unsigned long total = _nTotalStepsSimulation, lead = total - _nSteps;
     tVect.resize(total);
     for (unsigned long ii = 0; ii < lead; ++ii) tVect[ii] = (fType)(tStart - (lead - ii) * tStep);
