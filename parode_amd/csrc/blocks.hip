@@ -315,7 +315,7 @@ __device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
 // The seed of a plan's solve (work-group 1): x0, or the ABM start-up states
 // and the outputs of the first three (inputs: rows 0, 2, 4 of the h/2 grid).
 template <typename TU>
-__device__ __forceinline__ void d_blk_seed(const VBlock vb, const BlkMap& a)
+__device__ __forceinline__ void d_blk_seed(const BlkMap& a)
 {
     const BlockShape& s = a.s;
     const TU* U = static_cast<const TU*>(a.U);
@@ -323,7 +323,8 @@ __device__ __forceinline__ void d_blk_seed(const VBlock vb, const BlkMap& a)
         for (int i = threadIdx.x; i < s.n; i += 1024) a.seed[i] = (double)a.x0[i];
         return;
     }
-    d_abm_startup<TU>(vb, s.mirror, s.n, s.m, a.h, true, a.A, a.B, a.x0, U, a.seed);
+    startup_rows<TU, 16>(s.mirror, s.n, s.m, a.h, a.A, a.B, a.x0, U, a.seed);
+    __syncthreads();
     for (int t = threadIdx.x; t < 3 * s.p; t += 1024) {
         const int e = t / s.p, o = t - e * s.p;
         double v = 0.0;
@@ -343,7 +344,7 @@ template <typename TU>
 __device__ __forceinline__ void d_blk_map(const VBlock vb, const BlkMap& a, double* lds)
 {
     if (vb.x == 1)
-        d_blk_seed<TU>(vb, a);
+        d_blk_seed<TU>(a);
     else if (a.s.method == 0)
         d_blk_map_rk4(a, lds);
     else
@@ -1177,11 +1178,10 @@ void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h
 {
     const BlkMap a{s, h, rk4_coefficients(h), abm_coefficients(h), A, B, C, D, x0, U, b.PT, b.QT,
                    b.Ht, b.DL, seed, Y, x0 ? 2L : 1L};
-    const size_t lds = s.method == 1 ? 6 * s.n * sizeof(double) + (size_t)s.n * (s.n + 1) * 4 : 0;
     if (uDouble)
-        hipLaunchKernelGGL(k_blk_map<double>, dim3((unsigned)a.gx), dim3(1024), lds, st, a);
+        hipLaunchKernelGGL(k_blk_map<double>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     else
-        hipLaunchKernelGGL(k_blk_map<float>, dim3((unsigned)a.gx), dim3(1024), lds, st, a);
+        hipLaunchKernelGGL(k_blk_map<float>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     check_launch("block_map");
 }
 

@@ -35,6 +35,31 @@ Rk4Coef rk4_coefficients(double h);
 AbmCoef abm_coefficients(double h);
 AbmFactors abm_chunk_factors(double h);
 
+// Leading dimensions of the FP64 GEMMs' operands (X r x kk, Y kk x c, Z r x c,
+// row-major), an optional addend, Z[i][j] = (X Y)[i][j] + add[(i - shift) lda +
+// j] for i >= shift (the ABM companion's shifted blocks, a scan's other
+// operand), an optional copy of X (kk = c) to cp with Z's leading dimension,
+// and an optional split of Z's columns: column j goes to block j / zp, zs values
+// further each, column j % zp of it.  The addend and the copy may lie in Z's own
+// buffer: each value of them is read, then written, by one lane.
+struct GemmLd {
+    int ldx, ldy, ldz;
+    const double* add = nullptr;
+    int lda = 0, shift = 0;
+    double* cp = nullptr;
+    int zp = 0;
+    long zs = 0;
+};
+struct GemmOp {
+    int r, kk, c;
+    const double *X, *Y;
+    double* Z;
+    GemmLd ld;
+};
+// Independent FP64 products in one launch (at most kGemmMulti).
+constexpr int kGemmMulti = 8;
+void gemm_multi(hipStream_t s, const GemmOp* ops, int count);
+
 // Z = X * Y.  mirror = true: float products, sequential-k float accumulation,
 // no fused multiply-add (the rounding of uBLAS prod() on matrix<float>).
 void gemm_seq_f32(hipStream_t s, int r, int kk, int c, const float* X, const float* Y, float* Z);
@@ -275,6 +300,7 @@ void add_gemm(Phase& ph, int r, int kk, int c, const double* X, const double* Y,
 // add[(i - shift) ldz + j] on the rows i >= shift
 void add_gemm_ld(Phase& ph, int r, int kk, int c, const double* X, int ldx, const double* Y,
                  int ldy, double* Z, int ldz, const double* add, int shift);
+void add_gemm_op(Phase& ph, const GemmOp& op);
 void add_rk4_combine(Phase& ph, int n, int m, double h, const double* A, const double* A2,
                      const double* A3, const double* A4, const double* B, const double* AB,
                      const double* A2B, const double* A3B, double* MT, double* Bbar);

@@ -52,26 +52,40 @@ template void transpose<float>(hipStream_t, int, int, const float*, float*);
 template void transpose<double>(hipStream_t, int, int, const double*, double*);
 
 // ------------------------------------------------------------------ GEMMs
-__global__ void k_gemm_seq_f32(int r, int kk, int c, const float* __restrict__ X,
-                               const float* __restrict__ Y, float* __restrict__ Z)
+// A work-group's 16 x 16 outputs, K staged in LDS 64 at a time: each output is
+// still one sequential float sum, but its operands wait on one round of loads
+// per 64 terms instead of a load per term (n = 64: 12 -> 4 us).
+__global__ __launch_bounds__(256) void k_gemm_seq_f32(int r, int kk, int c,
+                                                      const float* __restrict__ X,
+                                                      const float* __restrict__ Y,
+                                                      float* __restrict__ Z)
 {
 #pragma clang fp contract(off)
-    long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long)r * c) return;
-    int i = (int)(idx / c), j = (int)(idx % c);
+    __shared__ float xs[16][65], ys[64][17];
+    const int ti = threadIdx.x >> 4, tj = threadIdx.x & 15;
+    const int i0 = (int)blockIdx.y * 16, j0 = (int)blockIdx.x * 16;
     float t = 0.0f;
-    for (int q = 0; q < kk; ++q) {
-        float pr = X[(long)i * kk + q] * Y[(long)q * c + j];
-        t = t + pr;
+    for (int q0 = 0; q0 < kk; q0 += 64) {
+        const int kn = kk - q0 < 64 ? kk - q0 : 64;
+        __syncthreads();
+        for (int u = threadIdx.x; u < 16 * 64; u += 256) {
+            const int xi = u >> 6, xq = u & 63, yq = u >> 4, yj = u & 15;
+            xs[xi][xq] = (i0 + xi < r && xq < kn) ? X[(long)(i0 + xi) * kk + q0 + xq] : 0.0f;
+            ys[yq][yj] = (j0 + yj < c && yq < kn) ? Y[(long)(q0 + yq) * c + j0 + yj] : 0.0f;
+        }
+        __syncthreads();
+        for (int q = 0; q < kn; ++q) {
+            const float pr = xs[ti][q] * ys[q][tj];
+            t = t + pr;
+        }
     }
-    Z[idx] = t;
+    if (i0 + ti < r && j0 + tj < c) Z[(long)(i0 + ti) * c + j0 + tj] = t;
 }
 
 void gemm_seq_f32(hipStream_t s, int r, int kk, int c, const float* X, const float* Y, float* Z)
 {
-    long work = (long)r * c;
-    hipLaunchKernelGGL(k_gemm_seq_f32, dim3(blocks_for(work, 256)), dim3(256), 0, s, r, kk, c, X,
-                       Y, Z);
+    hipLaunchKernelGGL(k_gemm_seq_f32, dim3((c + 15) / 16, (r + 15) / 16), dim3(256), 0, s, r, kk,
+                       c, X, Y, Z);
     check_launch("gemm_seq_f32");
 }
 
@@ -138,18 +152,22 @@ __global__ void k_gemm_f64_mfma(int r, int kk, int c, const double* __restrict__
 // current one is multiplied.
 constexpr int kGemmKsT = 32, kGemmKsKB = 32;
 
-// Leading dimensions of the FP64 GEMMs' operands (X r x kk, Y kk x c, Z r x c,
-// row-major), and an optional addend: Z[i][j] = (X Y)[i][j] + add[(i - shift)
-// ldz + j] for i >= shift (the ABM companion's shifted blocks).
-struct GemmLd {
-    int ldx, ldy, ldz;
-    const double* add;
-    int shift;
-};
-__host__ __device__ inline GemmLd gemm_ld(int kk, int c) { return GemmLd{kk, c, c, nullptr, 0}; }
-__device__ __forceinline__ double gemm_out(const GemmLd& ld, int i, int j, double v)
+__host__ __device__ inline GemmLd gemm_ld(int kk, int c) { return GemmLd{kk, c, c}; }
+// One value of Z = X Y: the addend, the copy of X and Z's place (GemmLd).
+__device__ __forceinline__ void gemm_put(const GemmLd& ld, const double* __restrict__ X,
+                                         double* __restrict__ Z, int i, int j, double v)
 {
-    return (ld.add && i >= ld.shift) ? v + ld.add[(long)(i - ld.shift) * ld.ldz + j] : v;
+    if (ld.add && i >= ld.shift) v += ld.add[(long)(i - ld.shift) * ld.lda + j];
+    if (ld.cp) {
+        const double x = X[(long)i * ld.ldx + j];
+        ld.cp[(long)i * ld.ldz + j] = x;
+    }
+    if (ld.zp) {
+        const int b = j / ld.zp;
+        Z[b * ld.zs + (long)i * ld.ldz + (j - b * ld.zp)] = v;
+    } else {
+        Z[(long)i * ld.ldz + j] = v;
+    }
 }
 
 template <int KSPLIT>
@@ -216,7 +234,7 @@ __device__ __forceinline__ void d_gemm_f64_ks(const VBlock vb, int r, int kk, in
 #pragma unroll
         for (int g = 1; g < KSPLIT; ++g) y += part[(((g - 1) * 4 + wq) * 4 + v) * 64 + lane];
         const int i = i0 + wr * 16 + 4 * v + q4, j = j0 + wc * 16 + l16;
-        if (i < r && j < c) Z[(long)i * ld.ldz + j] = gemm_out(ld, i, j, y);
+        if (i < r && j < c) gemm_put(ld, X, Z, i, j, y);
     }
 }
 
@@ -314,7 +332,7 @@ __device__ __forceinline__ void d_gemm_f64_t64(const VBlock vb, int r, int kk, i
             for (int v = 0; v < 4; ++v) {
                 const int i = i0 + wr * 32 + ti * 16 + 4 * v + q4;
                 const int j = j0 + wc * 32 + tj * 16 + l16;
-                if (i < r && j < c) Z[(long)i * ld.ldz + j] = gemm_out(ld, i, j, acc[ti][tj][v]);
+                if (i < r && j < c) gemm_put(ld, X, Z, i, j, acc[ti][tj][v]);
             }
 }
 
@@ -388,7 +406,7 @@ __device__ __forceinline__ void d_gemm_f64_mfma(const VBlock vb, int r, int kk, 
         for (int v = 0; v < 4; ++v) {
             const double sum = acc[v] + part[0][v][lane] + part[1][v][lane] + part[2][v][lane];
             const int i = i0 + 4 * v + q4, j = j0 + l16;
-            if (i < r && j < c) Z[(long)i * ld.ldz + j] = gemm_out(ld, i, j, sum);
+            if (i < r && j < c) gemm_put(ld, X, Z, i, j, sum);
         }
     }
 }
@@ -400,6 +418,53 @@ __global__ __launch_bounds__(256) void k_gemm_f64_mfma(int r, int kk, int c,
 {
     d_gemm_f64_mfma(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, r, kk, c, X, Y, Z,
                     gemm_ld(kk, c));
+}
+
+// The tiling of a product: 64 x 64 tiles where they are many (from 96 of them;
+// a product of fewer keeps more compute units busy as 16 x 16 tiles whose K is
+// split over four waves).
+__host__ __device__ inline bool gemm_tiles64(int r, int kk, int c)
+{
+    return gemm_wide(r, kk, c) && (long)((r + 63) / 64) * ((c + 63) / 64) >= 96;
+}
+struct GemmMulti {
+    unsigned start[kGemmMulti + 1];
+    int count;
+    GemmOp op[kGemmMulti];
+};
+
+__global__ __launch_bounds__(256) void k_gemm_multi(const GemmMulti a)
+{
+    int q = 0;
+    while (q + 1 < a.count && blockIdx.x >= a.start[q + 1]) ++q;
+    const GemmOp& o = a.op[q];
+    const long lb = (long)blockIdx.x - a.start[q];
+    if (gemm_tiles64(o.r, o.kk, o.c)) {
+        const long gx = (o.c + 63) / 64;
+        d_gemm_f64_t64(VBlock{lb % gx, lb / gx, gx}, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld);
+    } else {
+        const long gx = (o.c + 15) / 16;
+        d_gemm_f64_mfma(VBlock{lb % gx, lb / gx, gx}, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld);
+    }
+}
+
+void gemm_multi(hipStream_t s, const GemmOp* ops, int count)
+{
+    GemmMulti a{};
+    if (count > kGemmMulti) throw std::invalid_argument("gemm_multi: too many products");
+    for (int q = 0; q < count; ++q) {
+        const GemmOp& o = ops[q];
+        if (o.r <= 0 || o.c <= 0) continue;
+        const int t = gemm_tiles64(o.r, o.kk, o.c) ? 64 : 16;
+        const unsigned long n = (unsigned long)((o.r + t - 1) / t) * ((o.c + t - 1) / t);
+        if (a.start[a.count] + n > 0x7fffffffUL) throw std::length_error("gemm_multi: too many tiles");
+        a.op[a.count] = o;
+        a.start[a.count + 1] = a.start[a.count] + (unsigned)n;
+        ++a.count;
+    }
+    if (a.count == 0) return;
+    hipLaunchKernelGGL(k_gemm_multi, dim3(a.start[a.count]), dim3(256), 0, s, a);
+    check_launch("gemm_multi");
 }
 
 __device__ __forceinline__ void d_cast_f32_f64(const VBlock vb, long count, const float* __restrict__ in, double* __restrict__ out)
@@ -3808,9 +3873,26 @@ __global__ void k_abm_startup(bool mirror, int n, int m, double h, bool ldsA,
 }
 
 template <typename TU>
+__global__ __launch_bounds__(1024) void k_startup_rows(bool mirror, int n, int m, double h,
+                                                       const float* __restrict__ A,
+                                                       const float* __restrict__ B,
+                                                       const float* __restrict__ x0,
+                                                       const TU* __restrict__ Uh,
+                                                       double* __restrict__ X0)
+{
+    d_startup_rows<TU>(mirror, n, m, h, A, B, x0, Uh, X0);
+}
+
+template <typename TU>
 void abm_startup(hipStream_t s, bool mirror, int n, int m, double h, const float* A,
                  const float* B, const float* x0, const TU* Uh, double* X0)
 {
+    if (startup_rows_fit(n, m)) {
+        hipLaunchKernelGGL((k_startup_rows<TU>), dim3(1), dim3(1024), 0, s, mirror, n, m, h, A, B,
+                           x0, Uh, X0);
+        check_launch("startup_rows");
+        return;
+    }
     size_t lds = (size_t)6 * n * sizeof(double);
     const size_t ldsA = (size_t)n * (n + 1) * sizeof(float);
     const bool useA = lds + ldsA <= 65536;
@@ -3990,7 +4072,6 @@ struct Sample {
 struct Startup {
     int n, m;
     double h;
-    bool ldsA;
     const float *A, *B, *x0;
     const double* Uh;
     double* X0;
@@ -4153,11 +4234,12 @@ __global__ __launch_bounds__(256) void kg_sample(const Sample* __restrict__ args
     d_sample_family(vb, a.m, a.coef, a.t0, a.dt, 0, a.S, a.sigma, a.seed, a.out);
 }
 
-__global__ __launch_bounds__(256) void kg_startup(const Startup* __restrict__ args,
-                                                  const unsigned* __restrict__ st, int ns)
+__global__ __launch_bounds__(1024) void kg_startup(const Startup* __restrict__ args,
+                                                   const unsigned* __restrict__ st, int ns)
 {
     PARODE_GROUP(Startup);
-    d_abm_startup<double>(vb, false, a.n, a.m, a.h, a.ldsA, a.A, a.B, a.x0, a.Uh, a.X0);
+    (void)vb;
+    d_startup_rows<double>(false, a.n, a.m, a.h, a.A, a.B, a.x0, a.Uh, a.X0);
 }
 
 // The outputs of the ABM start-up states x_0, x_1, x_2 (the first n-blocks of
@@ -4370,7 +4452,7 @@ void add_gemm_ld(Phase& ph, int r, int kk, int c, const double* X, int ldx, cons
                  int ldy, double* Z, int ldz, const double* add, int shift)
 {
     if (r <= 0 || c <= 0) return;
-    const GemmLd ld{ldx, ldy, ldz, add, shift};
+    const GemmLd ld{ldx, ldy, ldz, add, ldz, shift};
     // (a work-group's matrix-core instructions per wave: kk for a 64 x 64 tile,
     // kk / 16 for a K-split 16 x 16 tile)
     if (gemm_wide(r, kk, c)) {
@@ -4380,6 +4462,15 @@ void add_gemm_ld(Phase& ph, int r, int kk, int c, const double* X, int ldx, cons
         const long gx = (c + 15) / 16, gy = (r + 15) / 16;
         append(ph, kGemm, false, Gemm{r, kk, c, X, Y, Z, ld, gx}, gx * gy, 0, kk / 16.0f);
     }
+}
+
+void add_gemm_op(Phase& ph, const GemmOp& o)
+{
+    if (o.r <= 0 || o.c <= 0) return;
+    const int t = gemm_wide(o.r, o.kk, o.c) ? kG64 : 16;
+    const long gx = (o.c + t - 1) / t, gy = (o.r + t - 1) / t;
+    append(ph, kGemm, false, Gemm{o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld, gx}, gx * gy, 0,
+           t == kG64 ? (float)o.kk : o.kk / 16.0f);
 }
 
 void add_rk4_combine(Phase& ph, int n, int m, double h, const double* A, const double* A2,
@@ -4443,11 +4534,9 @@ void add_sample(Phase& ph, int m, const double* coef, double t0, double dt, long
 void add_startup(Phase& ph, int n, int m, double h, const float* A, const float* B,
                  const float* x0, const double* Uh, double* X0)
 {
-    size_t lds = (size_t)6 * n * sizeof(double);
-    const size_t ldsA = (size_t)n * (n + 1) * sizeof(float);
-    const bool useA = lds + ldsA <= 65536;
-    if (useA) lds += ldsA;
-    append(ph, kStartup, false, Startup{n, m, h, useA, A, B, x0, Uh, X0, 1}, 1, lds);
+    // (the grouped path covers n, m <= 256)
+    if (!startup_rows_fit(n, m)) throw std::invalid_argument("grouped start-up: too wide");
+    append(ph, kStartup, false, Startup{n, m, h, A, B, x0, Uh, X0, 1}, 1, 0, (float)n);
 }
 
 void add_start_outputs(Phase& ph, int n, int m, int p, int pp, bool useC, bool useD,
@@ -4687,7 +4776,7 @@ void run(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dSta
     case kPowersSmall: PARODE_RUN(kg_powers_small, Powers, 1024); break;
     case kTables: PARODE_RUN(kg_tables, Tables, 256); break;
     case kSample: PARODE_RUN(kg_sample, Sample, 256); break;
-    case kStartup: PARODE_RUN(kg_startup, Startup, 256); break;
+    case kStartup: PARODE_RUN(kg_startup, Startup, 1024); break;
     case kStartOut: PARODE_RUN(kg_start_outputs, StartOut, 256); break;
     case kLeavesPlain: PARODE_RUN(kg_leaves<false>, Leaves, 256); break;
     case kLeavesFac: PARODE_RUN(kg_leaves<true>, Leaves, 256); break;
