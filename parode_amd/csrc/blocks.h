@@ -40,6 +40,7 @@ struct BlockShape {
     int lb = 0, T = 0;                 // steps per block
     int L = 0;                         // powers in PT
     int s = 0, taps = 0;
+    bool wide = false;   // the map does not fit one work-group: made by products over many
     int kb() const { return s * T * m; }
     int kh() const { return (s * (T - 1) + taps) * m; }
 };
@@ -48,7 +49,9 @@ struct BlockShape {
 struct BlockBufs {
     double *PT = nullptr, *QT = nullptr, *OT = nullptr, *Ht = nullptr, *DL = nullptr;
     double* Z = nullptr;    // [blocks + 1][na]: aggregates, then the blocks' start states
-    double* Z2 = nullptr;   // [groups + 1][na]: the same for groups of blocks
+    double* Z2 = nullptr;   // [groups + 1][na]: the same for groups of blocks (wide: for
+                            // every level of the tree over the blocks)
+    double* W = nullptr;    // wide: the map's intermediate products
 };
 
 // Where a batch's samples lie: window row r of block b is the sample row
@@ -71,22 +74,71 @@ enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit
 // Groups of blocks that the scan of nb blocks makes first (0: none).
 long block_groups(int na, long nb);
 
+// doubles in QT, OT, Ht and DL together; in Z2 for at most nb blocks; in W
+size_t block_table_values(const BlockShape& s);
+size_t block_z2_values(const BlockShape& s, long nb);
+size_t block_scratch_values(const BlockShape& s);
+BlockBufs block_carve(const BlockShape& s, double* PT, double* tab, double* z, long nb, double* w);
+
+// ---- wide maps: the launches that make the tables, as operations by phase (an
+// operation reads what lower phases wrote)
+struct BlkElem {        // element-wise stages of a wide map
+    enum Stage { kPrep, kComb, kAsm };
+    BlockShape s;
+    int stage = 0;
+    double h = 0.0;
+    Rk4Coef rk;
+    AbmCoef ab;
+    const float *A, *B, *C, *D, *x0;
+    double *PT, *QT, *OT, *DL, *seed;
+    double *A64, *B64, *A2, *A3, *A4, *AB, *A2B, *A3B, *CT, *DT, *B1, *VT;
+    long count = 0;     // elements
+    long gx = 0;
+};
+struct SeqOp {          // Z = X Y in the reference's float rounding
+    int r, kk, c;
+    const float *X, *Y;
+    float* Z;
+};
+struct BlockSink {
+    virtual void gemm(int phase, const GemmOp& op) = 0;
+    virtual void elem(int phase, const BlkElem& e) = 0;
+    virtual void seq(int phase, const SeqOp& op) = 0;
+    virtual ~BlockSink() = default;
+};
+// Emits a wide map's operations.  Returns the phase before which pass 1's
+// table is not complete.  The powers up to P_last (P_0 .. P_{last}) are made;
+// those that pass 1's tables do not need come at the phases they can.
+int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A, const float* B,
+               const float* C, const float* D, const float* x0, double* seed, int last,
+               BlockSink& sink);
+// The tree over the blocks' states of a wide map: up products (level k from 0),
+// then the seed, then down products from level top - 1 to 0.  Returns top.
+int block_tree_levels(long nb);
+GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k);
+GemmOp block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int k);
+void block_elem(hipStream_t st, const BlkElem& e);
+
 // M, G, the direct terms and (x0 given) the seed: x0, or with the ABM start-up
-// the states x_0..x_3 and their three outputs.
+// the states x_0..x_3 and their three outputs.  (Maps that are not wide.)
 void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
                const float* B, const float* C, const float* D, const float* x0, const void* U,
                bool uDouble, double* seed, float* Y);
+// the outputs of the ABM start-up states (X0: x_0 .. x_3)
+void block_start_outputs(hipStream_t st, const BlockShape& s, const float* C, const float* D,
+                         const double* X0, const void* U, bool uDouble, float* Y);
 // PT up to P_lb, QT, OT, Ht
 void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C);
 // the blocks' responses from zero (and, with powers, the rest of PT)
 void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                  long nb, bool powers, int tiling = kBlockAuto);
 // the blocks' start states from the seed (in X); Z[nb] is the state after them
+// (wide: tot receives the blocks' response from zero instead, if not null)
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                long nb, const double* seed);
+                long nb, const double* seed, double* tot = nullptr);
 // seedOut = the state (in X) after the blocks
 void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                 long nb, double* seedOut);
+                 long nb, const double* seed, const double* tot, double* seedOut);
 void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                  long nb, long nReal, const double* seed, const float* D, float* Y,
                  int tiling = kBlockAuto);

@@ -3,6 +3,7 @@
 #include "launch.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace parode {
 namespace k {
@@ -312,6 +313,33 @@ __device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
     }
 }
 
+// The outputs of the ABM start-up states x_0, x_1, x_2 (inputs: rows 0, 2, 4 of
+// the h/2 grid; AdamsMoulton.cpp:106-116), FP64 sums.
+template <typename TU>
+__device__ __forceinline__ void d_start_outputs(const BlockShape& s, const float* C, const float* D,
+                                                const double* X0, const TU* U, float* Y)
+{
+    for (int t = threadIdx.x; t < 3 * s.p; t += blockDim.x) {
+        const int e = t / s.p, o = t - e * s.p;
+        double v = 0.0;
+        if (s.useC)
+            for (int i = 0; i < s.n; ++i) v = fma((double)C[(long)o * s.n + i], X0[e * s.n + i], v);
+        else
+            v = X0[e * s.n + o];
+        if (s.useD)
+            for (int j = 0; j < s.m; ++j)
+                v = fma((double)D[(long)o * s.m + j], (double)U[(long)2 * e * s.m + j], v);
+        Y[t] = (float)v;
+    }
+}
+template <typename TU>
+__global__ __launch_bounds__(1024) void k_blk_start_outputs(BlockShape s, const float* C,
+                                                            const float* D, const double* X0,
+                                                            const TU* U, float* Y)
+{
+    d_start_outputs<TU>(s, C, D, X0, U, Y);
+}
+
 // The seed of a plan's solve (work-group 1): x0, or the ABM start-up states
 // and the outputs of the first three (inputs: rows 0, 2, 4 of the h/2 grid).
 template <typename TU>
@@ -325,19 +353,7 @@ __device__ __forceinline__ void d_blk_seed(const BlkMap& a)
     }
     startup_rows<TU, 16>(s.mirror, s.n, s.m, a.h, a.A, a.B, a.x0, U, a.seed);
     __syncthreads();
-    for (int t = threadIdx.x; t < 3 * s.p; t += 1024) {
-        const int e = t / s.p, o = t - e * s.p;
-        double v = 0.0;
-        if (s.useC)
-            for (int i = 0; i < s.n; ++i)
-                v = fma((double)a.C[(long)o * s.n + i], a.seed[e * s.n + i], v);
-        else
-            v = a.seed[e * s.n + o];
-        if (s.useD)
-            for (int j = 0; j < s.m; ++j)
-                v = fma((double)a.D[(long)o * s.m + j], (double)U[(long)2 * e * s.m + j], v);
-        a.Y[t] = (float)v;
-    }
+    d_start_outputs<TU>(s, a.C, a.D, a.seed, U, a.Y);
 }
 
 template <typename TU>
@@ -1102,38 +1118,215 @@ __global__ void k_blk_carry(const BlkScan a, long row0, long at, double* out)
         out[i] = a.E[a.nb * a.na + i] + blk_shift(a, row0, at, i);
 }
 
+// wide maps: the tree's root takes the shifted seed (its response from zero goes
+// to tot), and the state after the blocks is P_L Z_0 plus that response
+__device__ __forceinline__ void d_blk_root(const BlkScan& a, double* root, double* tot)
+{
+    for (int i = threadIdx.x; i < a.na; i += blockDim.x) {
+        if (tot) tot[i] = root[i];
+        root[i] = a.seed[i] - blk_shift(a, 0, 0, i);
+    }
+}
+__global__ __launch_bounds__(1024) void k_blk_root(const BlkScan a, double* root, double* tot)
+{
+    d_blk_root(a, root, tot);
+}
+__global__ __launch_bounds__(256) void k_blk_carry_wide(const BlkScan a, const double* P,
+                                                        const double* tot, long row0, long at,
+                                                        double* out)
+{
+    extern __shared__ double z[];
+    for (int i = threadIdx.x; i < a.na; i += 256) z[i] = a.seed[i] - blk_shift(a, 0, 0, i);
+    __syncthreads();
+    const int i = (int)blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.na) return;
+    double v = tot[i] + blk_shift(a, row0, at, i);
+    for (int k = 0; k < a.na; ++k) v = fma(P[(long)k * a.na + i], z[k], v);
+    out[i] = v;
+}
+
+// ---------------------------------------------------------------- wide maps
+// The element-wise stages between the products: FP64 copies and the transposed
+// outputs (prep), the step's combinations (comb; RungeKutta4thOrder.cpp:48-57,
+// AdamsMoulton.cpp:258-316), the ABM block input and shift (asm).
+template <typename TI>
+__device__ __forceinline__ void blk_comb(const BlkElem& a, long x)
+{
+#pragma clang fp contract(off)
+    const BlockShape& s = a.s;
+    const int n = s.n, m = s.m, na = s.na;
+    // with the reference's rounding the products are floats, and A, B the inputs
+    const TI* A = s.mirror ? reinterpret_cast<const TI*>(a.A) : reinterpret_cast<const TI*>(a.A64);
+    const TI* B = s.mirror ? reinterpret_cast<const TI*>(a.B) : reinterpret_cast<const TI*>(a.B64);
+    const TI *A2 = reinterpret_cast<const TI*>(a.A2), *A3 = reinterpret_cast<const TI*>(a.A3),
+             *A4 = reinterpret_cast<const TI*>(a.A4), *AB = reinterpret_cast<const TI*>(a.AB),
+             *A2B = reinterpret_cast<const TI*>(a.A2B), *A3B = reinterpret_cast<const TI*>(a.A3B);
+    auto rnd = [&](double v) { return s.mirror ? (double)(float)v : v; };
+    const long np = (long)na * na;
+    if (s.method == 0) {
+        const Rk4Coef& k = a.rk;
+        if (x < np) {
+            const int j = (int)(x / n), i = (int)(x - (long)j * n);
+            const long t = (long)i * n + j;
+            double v = ((i == j) ? 1.0 : 0.0) + k.h * (double)A[t];
+            v = v + k.c2 * (double)A2[t];
+            v = v + k.c3 * (double)A3[t];
+            v = v + k.c4 * (double)A4[t];
+            a.PT[x] = rnd(v);
+            return;
+        }
+        x -= np;
+        const int j = (int)(x / n), i = (int)(x - (long)j * n);
+        const long t = (long)i * m + j;
+        const double b = B[t], ab = AB[t], a2b = A2B[t], a3b = A3B[t];
+        a.B1[x] = rnd((1.0 / 6.0) * (((k.h * b + k.s1 * ab) + k.s2 * a2b) + k.s3 * a3b));
+        a.QT[((long)s.s * (s.T - 1) * m + m + j) * n + i] =
+            rnd((1.0 / 6.0) * ((k.t0 * b + k.t1 * ab) + k.t2 * a2b));
+        a.DL[x] = rnd(k.u0 * b);
+        return;
+    }
+    const AbmCoef& c = a.ab;
+    if (x < np) {
+        const int j = (int)(x / na), i = (int)(x - (long)j * na);   // PT[j][i] = M[i][j]
+        double v;
+        if (i < 3 * n) {
+            v = j == i + n ? 1.0 : 0.0;
+        } else {
+            const int r = i - 3 * n, b = j / n, q = j - b * n;
+            const double y = A[(long)r * n + q], y2 = A2[(long)r * n + q], id = r == q ? 1.0 : 0.0;
+            v = b == 0 ? rnd(c.a3A2 * y2) : b == 1 ? rnd(c.a2A * y + c.a2A2 * y2)
+              : b == 2 ? rnd(c.a1A * y + c.a1A2 * y2) : rnd((id + c.a0A * y) + c.a0A2 * y2);
+        }
+        a.PT[x] = v;
+        return;
+    }
+    x -= np;
+    const int j = (int)(x / n), i = (int)(x - (long)j * n);
+    const long t = (long)i * m + j, mn = (long)m * n;
+    const double b = B[t], ab = AB[t];
+    a.B1[x] = rnd(c.b3AB * ab);
+    a.B1[mn + x] = rnd(c.b2B * b + c.b2AB * ab);
+    a.B1[2 * mn + x] = rnd(c.b1B * b + c.b1AB * ab);
+    a.B1[3 * mn + x] = rnd(c.b0B * b + c.b0AB * ab);
+    a.VT[(long)j * 5 * n + i] = rnd(c.bm1 * b);
+}
+
+__device__ __forceinline__ void d_blk_elem(const VBlock vb, const BlkElem& a)
+{
+    const BlockShape& s = a.s;
+    const int n = s.n, m = s.m, p = s.p, na = s.na;
+    for (long x = vb.x * 256 + threadIdx.x; x < a.count; x += vb.gx * 256) {
+        if (a.stage == BlkElem::kComb) {
+            if (s.mirror)
+                blk_comb<float>(a, x);
+            else
+                blk_comb<double>(a, x);
+        } else if (a.stage == BlkElem::kPrep) {
+            long t = x;
+            if (t < (long)n * n) {
+                a.A64[t] = (double)a.A[t];
+                continue;
+            }
+            t -= (long)n * n;
+            if (t < (long)n * m) {
+                a.B64[t] = (double)a.B[t];
+                continue;
+            }
+            t -= (long)n * m;
+            if (t < (long)m * p) {
+                a.DT[t] = s.useD ? (double)a.D[(t % p) * m + t / p] : 0.0;
+                continue;
+            }
+            t -= (long)m * p;
+            if (t < (long)na * p) {     // O of step 0, and C^T
+                const int k = (int)(t / p), o = (int)(t - (long)k * p), i = k - (na - n);
+                double v = 0.0;
+                if (i >= 0) {
+                    v = s.useC ? (double)a.C[(long)o * n + i] : (i == o ? 1.0 : 0.0);
+                    a.CT[(long)i * p + o] = v;
+                }
+                a.OT[(long)k * s.T * p + o] = v;
+                continue;
+            }
+            t -= (long)na * p;
+            a.seed[t] = (double)a.x0[t];
+        } else {
+            long t = x;
+            if (t < (long)m * na) {
+                const int j = (int)(t / na), i = (int)(t - (long)j * na);
+                a.QT[(long)(s.T - 1) * m * na + t] = a.VT[(long)j * 5 * n + n + i];
+                continue;
+            }
+            t -= (long)m * na;
+            const int rj = (int)(t / na), y = (int)(t - (long)rj * na);
+            const int r = rj / m, j = rj - r * m, b = y / n, i = y - b * n;
+            a.DL[t] = b >= r ? a.VT[(long)j * 5 * n + (b - r) * n + i] : 0.0;
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_blk_elem(const BlkElem a)
+{
+    d_blk_elem(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a);
+}
+
 // ================================================================ host side
 static unsigned magic_of(int m) { return (unsigned)(((1ULL << 32) + m - 1) / m); }
 
+// One work-group's LDS holds the map.
+static bool fits_one(int method, int n, int m, int p)
+{
+    const int na = method == 1 ? 4 * n : n, s = method == 1 ? 1 : 2;
+    return na <= kBN && p <= kBN && m <= kBM && s * m <= kBN;
+}
+
 // The rule: which systems run as block responses, and with how many steps per
-// block.  Covered: inputs and outputs present, n_a, p, s m <= 64, m <= 32 (one
-// work-group's LDS holds the map), horizons from 64 points.  More steps per
+// block: the fastest by the model below, if it beats the general path's.
+// Covered: inputs and outputs present, horizons from 64 points.  More steps per
 // block make the scan shorter (2 n_a^2 products a block, and its chain of
-// dependent steps), fewer make pass 2 cheaper (s m p T / 2 products a step).
+// dependent steps), fewer make pass 2 (s m p T / 2 products a step) and the
+// tables (2 n_a^2 (s m + p) T) cheaper.
 int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long nScan, long nPad)
 {
     const int na = method == 1 ? 4 * n : n, s = method == 1 ? 1 : 2;
-    if (m < 1 || p < 1 || (!useC && useD)) return 0;
-    if (na > kBN || p > kBN || m > kBM || s * m > kBN || nScan < 64) return 0;
+    if (m < 1 || p < 1 || (!useC && useD) || nScan < 64) return 0;
+    if (!useC) p = n;
+    const bool one = fits_one(method, n, m, p);
+    if (n > 1024 || (long)m * p > (1L << 20)) return 0;
     int best = 0;
     double bt = 0.0;
+    const double N = (double)nScan, na2 = (double)na * na;
     for (int lb = 3; lb <= 8; ++lb) {
-        const double T = 1 << lb, N = (double)nScan, nb = N / T;
+        const double T = 1 << lb, nb = N / T;
         if ((nPad >> lb) < 2) break;
         // (T m s < 2^16: the window index's multiply-high)
         if ((long)(s * T + 8) * m >= 65536) break;
-        // microseconds: products at 25 TFLOP/s, the scan's chain, the tables
-        const double pass = N * (2.0 * na * s * m + 2.0 * p * na + 2.0 * s * m * p * (T / 2 + 8)) / 25e6;
-        const double steps = nb <= 512 ? nb / 64 : 2 * 16 + nb / 16 / 64;
-        const double scan = 2 * steps * (0.25 + na * 0.012) + 2 * nb * na * na * 2 / 0.25e6 / (nb <= 512 ? 1 : nb / 512);
-        const double tab = lb * 1.2 + T * (s * m + p) / 64 * 0.05;
+        // microseconds: FP64 products at 25 (few tiles) or 40 TFLOP/s, the
+        // scan's chain, the tables
+        const double pass = N * (2.0 * na * s * m + 2.0 * p * na +
+                                 2.0 * s * m * p * (T / 2 + 32.0 / p + 2)) / (one ? 25e6 : 40e6);
+        double scan, tab;
+        if (one) {
+            const double steps = nb <= 512 ? nb / 64 : 2 * 16 + nb / 16 / 64;
+            scan = 2 * steps * (0.25 + na * 0.012) + 2 * nb * na2 * 2 / 0.25e6 / (nb <= 512 ? 1 : nb / 512);
+            tab = lb * 1.2 + T * (s * m + p) / 64 * 0.05;
+        } else {
+            scan = 4 * na2 * nb / 40e6 + 2 * 5.0 * std::max(1.0, std::log2(nb));
+            tab = 2 * na2 * (s * m + p) * T / 40e6 + 5.0 * lb;
+        }
         const double t = pass + scan + tab;
         if (!best || t < bt) {
             best = lb;
             bt = t;
         }
     }
-    return best;
+    if (!best || one) return best;
+    // the general path: two chunk passes (or tree levels) in FP32, FP64 leaves
+    // and outputs, levels
+    const double step = method == 1 ? 8.0 * n * n : 4.0 * n * n;
+    const double general = N * (step / 45e6 + (2.0 * n * m * (method == 1 ? 2 : 3) + 2.0 * p * (n + m)) / 15e6) +
+                           10.0 * std::log2(N);
+    return bt < general ? best : 0;
 }
 
 BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bool mirror, int lb,
@@ -1153,7 +1346,253 @@ BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bo
     s.L = L;
     s.s = method == 1 ? 1 : 2;
     s.taps = method == 1 ? 4 : 1;
+    s.wide = !fits_one(method, n, m, s.p);
     return s;
+}
+
+size_t block_table_values(const BlockShape& s)
+{
+    return ((size_t)s.kb() + (size_t)s.T * s.p + (size_t)s.taps * s.m) * s.na +
+           (size_t)s.kh() * s.p;
+}
+
+// (wide) rows of the tree's levels above the blocks, an even number each
+static long tree_rows(long n) { return (n + 1) / 2 * 2; }
+
+size_t block_z2_values(const BlockShape& s, long nb)
+{
+    long rows = 0;
+    if (s.wide)
+        for (long n = nb; n > 1; n = (n + 1) / 2) rows += tree_rows((n + 1) / 2);
+    else
+        rows = block_groups(s.na, nb) + 1;
+    return (size_t)(rows + 1) * s.na;
+}
+
+size_t block_scratch_values(const BlockShape& s)
+{
+    if (!s.wide) return 0;
+    const size_t n = s.n, m = s.m, p = s.p;
+    return 4 * n * n + 4 * n * m + n * p + m * p + 9 * m * n;
+}
+
+BlockBufs block_carve(const BlockShape& s, double* PT, double* tab, double* z, long nb, double* w)
+{
+    BlockBufs b;
+    b.PT = PT;
+    b.QT = tab;
+    b.OT = b.QT + (size_t)s.kb() * s.na;
+    b.Ht = b.OT + (size_t)s.T * s.p * s.na;
+    b.DL = b.Ht + (size_t)s.kh() * s.p;
+    b.Z = z;
+    b.Z2 = z + (size_t)(tree_rows(nb) + 1) * s.na;
+    b.W = w;
+    return b;
+}
+
+void block_elem(hipStream_t st, const BlkElem& e)
+{
+    if (e.count <= 0) return;
+    hipLaunchKernelGGL(k_blk_elem, dim3((unsigned)e.gx), dim3(256), 0, st, e);
+    check_launch("block elem");
+}
+
+// Whether an ABM map's squarings take block column 0 by a product and the
+// others by the companion's recurrence (56 n^3 flop in four dependent launches)
+// rather than the whole square (128 n^3 in one): from n = 128, where the
+// products' time exceeds the launches'.
+static bool structured_square(const BlockShape& s) { return s.method == 1 && s.n > 128; }
+
+int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A, const float* B,
+               const float* C, const float* D, const float* x0, double* seed, int last,
+               BlockSink& sink)
+{
+    const int n = s.n, m = s.m, p = s.p, na = s.na, sm = s.s * m, T = s.T;
+    const size_t nn = (size_t)n * n, nm = (size_t)n * m;
+    const size_t na2 = (size_t)na * na;
+    BlkElem e{};
+    e.s = s;
+    e.h = h;
+    e.rk = rk4_coefficients(h);
+    e.ab = abm_coefficients(h);
+    e.A = A;
+    e.B = B;
+    e.C = C;
+    e.D = D;
+    e.x0 = x0;
+    e.PT = b.PT;
+    e.QT = b.QT;
+    e.OT = b.OT;
+    e.DL = b.DL;
+    e.seed = seed;
+    e.A64 = b.W;
+    e.A2 = e.A64 + nn;
+    e.A3 = e.A2 + nn;
+    e.A4 = e.A3 + nn;
+    e.B64 = e.A4 + nn;
+    e.AB = e.B64 + nm;
+    e.A2B = e.AB + nm;
+    e.A3B = e.A2B + nm;
+    e.CT = e.A3B + nm;
+    e.DT = e.CT + (size_t)n * p;
+    e.B1 = e.DT + (size_t)m * p;
+    e.VT = e.B1 + 4 * nm;
+    auto elem = [&](int phase, int stage, long count) {
+        e.stage = stage;
+        e.count = count;
+        e.gx = std::min<long>((count + 255) / 256, 1024);
+        sink.elem(phase, e);
+    };
+    const bool rk4 = s.method == 0;
+    elem(0, BlkElem::kPrep, (long)(nn + nm) + (long)m * p + (long)na * p + (rk4 && x0 ? n : 0));
+    int base;
+    if (s.mirror) {
+        auto f = [](double* v) { return reinterpret_cast<float*>(v); };
+        sink.seq(1, SeqOp{n, n, n, A, A, f(e.A2)});
+        sink.seq(1, SeqOp{n, n, m, A, B, f(e.AB)});
+        if (rk4) {
+            sink.seq(2, SeqOp{n, n, n, f(e.A2), A, f(e.A3)});
+            sink.seq(2, SeqOp{n, n, m, f(e.A2), B, f(e.A2B)});
+            sink.seq(3, SeqOp{n, n, n, A, f(e.A3), f(e.A4)});
+            sink.seq(3, SeqOp{n, n, m, f(e.A3), B, f(e.A3B)});
+        }
+        base = rk4 ? 4 : 2;
+    } else {
+        auto mul = [&](int phase, int c, const double* X, const double* Y, double* Z) {
+            sink.gemm(phase, GemmOp{n, n, c, X, Y, Z, gemm_ld(n, c)});
+        };
+        mul(1, n, e.A64, e.A64, e.A2);
+        mul(1, m, e.A64, e.B64, e.AB);
+        if (rk4) {
+            mul(2, n, e.A2, e.A64, e.A3);
+            mul(2, n, e.A2, e.A2, e.A4);
+            mul(2, m, e.A2, e.B64, e.A2B);
+            mul(2, m, e.A2, e.AB, e.A3B);
+        }
+        base = rk4 ? 3 : 2;
+    }
+    elem(base, BlkElem::kComb, (long)na2 + (long)nm);
+    double* GT = b.QT + (size_t)sm * (T - 1) * na;
+    double* F = b.Ht + (size_t)s.s * (T - 1) * m * p;
+    const long cols = (long)T * p;
+    int ready;                       // the phase at which G can be read
+    const double* G = GT;
+    int ldg = na;
+    if (rk4) {
+        // G's first half: B1 + M B3 (transposed); F = D + C B3
+        GemmLd ld{n, n, n};
+        ld.add = e.B1;
+        ld.lda = n;
+        sink.gemm(base + 1, GemmOp{m, n, n, b.DL, b.PT, GT, ld});
+        GemmLd lf{n, p, p};
+        lf.add = e.DT;
+        lf.lda = p;
+        sink.gemm(base + 1, GemmOp{m, n, p, b.DL, e.CT, F, lf});
+        ready = base + 2;
+    } else {
+        // V_t^T = B_{4-t}^T + [V_0 .. V_{t-1}]^T [M_{4-t} .. M_3]^T
+        for (int t = 1; t < 5; ++t) {
+            GemmLd ld{5 * n, na, 5 * n};
+            ld.add = e.B1 + (size_t)(4 - t) * nm;
+            ld.lda = n;
+            sink.gemm(base + t, GemmOp{m, t * n, n, e.VT,
+                                       b.PT + (size_t)(4 - t) * n * na + 3 * n, e.VT + t * n, ld});
+        }
+        ready = base + 5;
+        elem(ready, BlkElem::kAsm, (long)m * na + 4L * m * na);
+        for (int r = 0; r < 4; ++r) {
+            GemmLd lf{5 * n, p, p};
+            if (r == 3) {
+                lf.add = e.DT;
+                lf.lda = p;
+            }
+            sink.gemm(ready, GemmOp{m, n, p, e.VT + (3 - r) * n, e.CT, F + (size_t)r * m * p, lf});
+        }
+        G = e.VT + n;                // (GT itself is copied in phase `ready`)
+        ldg = 5 * n;
+    }
+    // powers, and the tables by doubling
+    const bool st = structured_square(s);
+    const int spp = st ? 4 : 1;
+    int q = ready - 1;
+    for (int l = 0; l < last || l < s.lb; ++l) {
+        const int ph = base + 1 + spp * l;   // P_l can be read
+        const double* P = b.PT + l * na2;
+        if (l < last) {
+            double* P2 = b.PT + (l + 1) * na2;
+            if (!st) {
+                sink.gemm(ph, GemmOp{na, na, na, P, P, P2, gemm_ld(na, na)});
+            } else {
+                sink.gemm(ph, GemmOp{na, na, n, P, P, P2, GemmLd{na, na, na}});
+                for (int c = 1; c < 4; ++c) {
+                    GemmLd ld{na, na, na};
+                    ld.add = P2 + (c - 1) * n;
+                    ld.lda = na;
+                    ld.shift = n;
+                    sink.gemm(ph + c, GemmOp{na, n, n, b.PT + 3 * n,
+                                             P2 + 3L * n * na + (c - 1) * n, P2 + c * n, ld});
+                }
+            }
+        }
+        if (l >= s.lb) continue;
+        const int k = 1 << l;
+        sink.gemm(ph, GemmOp{na, na, k * p, P, b.OT, b.OT + (long)k * p,
+                             GemmLd{na, (int)cols, (int)cols}});
+        q = std::max(q + 1, ph);
+        sink.gemm(q, GemmOp{k * sm, na, na, l == 0 ? G : b.QT + (size_t)(T - k) * sm * na, P,
+                            b.QT + (size_t)(T - 2 * k) * sm * na,
+                            GemmLd{l == 0 ? ldg : na, na, na}});
+    }
+    GemmLd lh{ldg, (int)cols, p};
+    lh.zp = p;
+    lh.zs = -(long)sm * p;
+    sink.gemm(std::max(ready, base + 2 + spp * (s.lb - 1)),
+              GemmOp{sm, na, (T - 1) * p, G, b.OT, b.Ht + (size_t)(T - 2) * sm * p, lh});
+    return q + 1;
+}
+
+int block_tree_levels(long nb)
+{
+    int k = 0;
+    for (long n = nb; n > 1; n = (n + 1) / 2) ++k;
+    return k;
+}
+// the states of level k of the tree (level 0: the blocks) and their count
+static double* tree_level(const BlockShape& s, const BlockBufs& b, long nb, int k, long& count)
+{
+    double* at = b.Z;
+    double* next = b.Z2;
+    count = nb;
+    for (int i = 0; i < k; ++i) {
+        count = (count + 1) / 2;
+        at = next;
+        next += tree_rows(count) * s.na;
+    }
+    return at;
+}
+GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k)
+{
+    long c0, c1;
+    double* S0 = tree_level(s, b, nb, k, c0);
+    double* S1 = tree_level(s, b, nb, k + 1, c1);
+    const int na = s.na;
+    GemmLd ld{2 * na, na, na};
+    ld.add = S0 + na;
+    ld.lda = 2 * na;
+    return GemmOp{(int)(c0 / 2), na, na, S0, b.PT + (size_t)(s.lb + k) * na * na, S1, ld};
+}
+// in place: E[2i] over S[2i], which is first added to E[2i + 1]
+GemmOp block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int k)
+{
+    long c0, c1;
+    double* S0 = tree_level(s, b, nb, k, c0);
+    double* E1 = tree_level(s, b, nb, k + 1, c1);
+    const int na = s.na;
+    GemmLd ld{na, na, 2 * na};
+    ld.add = S0;
+    ld.lda = 2 * na;
+    ld.cp = S0;
+    return GemmOp{(int)c1, na, na, E1, b.PT + (size_t)(s.lb + k) * na * na, S0 + na, ld};
 }
 
 // One work-group scans up to 512 blocks; more go in groups of 16 (or as many
@@ -1183,6 +1622,18 @@ void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h
     else
         hipLaunchKernelGGL(k_blk_map<float>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     check_launch("block_map");
+}
+
+void block_start_outputs(hipStream_t st, const BlockShape& s, const float* C, const float* D,
+                         const double* X0, const void* U, bool uDouble, float* Y)
+{
+    if (uDouble)
+        hipLaunchKernelGGL(k_blk_start_outputs<double>, dim3(1), dim3(1024), 0, st, s, C, D, X0,
+                           (const double*)U, Y);
+    else
+        hipLaunchKernelGGL(k_blk_start_outputs<float>, dim3(1), dim3(1024), 0, st, s, C, D, X0,
+                           (const float*)U, Y);
+    check_launch("block start outputs");
 }
 
 // steps of a slice: the largest power of two whose rows fit the LDS
@@ -1307,8 +1758,25 @@ static BlkScan scan_args(const BlockShape& s, const BlockBufs& b, const BlockInp
 }
 
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                long nb, const double* seed)
+                long nb, const double* seed, double* tot)
 {
+    if (s.wide) {
+        const int top = block_tree_levels(nb);
+        for (int k = 0; k < top; ++k) {
+            const GemmOp op = block_tree_up(s, b, nb, k);
+            gemm_multi(st, &op, 1);
+        }
+        long one;
+        double* root = tree_level(s, b, nb, top, one);
+        hipLaunchKernelGGL(k_blk_root, dim3(1), dim3(1024), 0, st, scan_args(s, b, in, nb, seed),
+                           root, tot);
+        check_launch("block root");
+        for (int k = top - 1; k >= 0; --k) {
+            const GemmOp op = block_tree_down(s, b, nb, k);
+            gemm_multi(st, &op, 1);
+        }
+        return;
+    }
     const int nct = (s.na + 15) / 16, pitch = 16 * nct + 1;
     auto lds = [&](int R) { return (size_t)2 * 16 * R * pitch * sizeof(double); };
     BlkScan a = scan_args(s, b, in, nb, seed);
@@ -1344,9 +1812,17 @@ void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const B
 }
 
 void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                 long nb, double* seedOut)
+                 long nb, const double* seed, const double* tot, double* seedOut)
 {
-    const BlkScan a = scan_args(s, b, in, nb, nullptr);
+    const BlkScan a = scan_args(s, b, in, nb, seed);
+    if (s.wide) {   // (nb is a power of two here)
+        hipLaunchKernelGGL(k_blk_carry_wide, dim3((s.na + 255) / 256), dim3(256),
+                           s.na * sizeof(double), st, a,
+                           b.PT + (size_t)(s.lb + block_tree_levels(nb)) * s.na * s.na, tot,
+                           nb * s.s * s.T, nb * s.T * in.sL * s.m, seedOut);
+        check_launch("block carry");
+        return;
+    }
     hipLaunchKernelGGL(k_blk_carry, dim3(1), dim3(256), 0, st, a, nb * s.s * s.T,
                        nb * s.T * in.sL * s.m, seedOut);
     check_launch("block carry");

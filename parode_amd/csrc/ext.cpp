@@ -46,7 +46,9 @@ struct Plan {
     const parode::ScanCore::SideStream* side_stream()
     {
         if (!side.stream) {
-            PARODE_HIP(hipStreamCreate(&side.stream));
+            // (not blocking: the null stream's launches would wait for it and it for
+            // them; the events order it against the plan's stream)
+            PARODE_HIP(hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking));
             PARODE_HIP(hipEventCreateWithFlags(&side.fork, hipEventDisableTiming));
             PARODE_HIP(hipEventCreateWithFlags(&side.join, hipEventDisableTiming));
             PARODE_HIP(hipEventCreateWithFlags(&side.late, hipEventDisableTiming));

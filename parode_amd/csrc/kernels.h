@@ -50,6 +50,7 @@ struct GemmLd {
     int zp = 0;
     long zs = 0;
 };
+__host__ __device__ inline GemmLd gemm_ld(int kk, int c) { return GemmLd{kk, c, c}; }
 struct GemmOp {
     int r, kk, c;
     const double *X, *Y;

@@ -152,7 +152,6 @@ __global__ void k_gemm_f64_mfma(int r, int kk, int c, const double* __restrict__
 // current one is multiplied.
 constexpr int kGemmKsT = 32, kGemmKsKB = 32;
 
-__host__ __device__ inline GemmLd gemm_ld(int kk, int c) { return GemmLd{kk, c, c}; }
 // One value of Z = X Y: the addend, the copy of X and Z's place (GemmLd).
 __device__ __forceinline__ void gemm_put(const GemmLd& ld, const double* __restrict__ X,
                                          double* __restrict__ Z, int i, int j, double v)

@@ -33,25 +33,20 @@ ScanCore::ScanCore(int method, int n, int m, int p, bool zC, bool zD, long nPadM
             const k::BlockShape b =
                 k::block_shape(method, n, m, states ? n : p, !zC, !zD,
                                opt_.precision == kPlain32, lb, L_ + 1);
-            const size_t na = na_, nb = (size_t)(nPadMax_ >> lb);
-            const size_t tab = ((size_t)b.kb() + (size_t)b.T * b.p + (size_t)b.taps * m) * na +
-                               (size_t)b.kh() * b.p;
-            const size_t z = (nb + 1 + k::block_groups(na_, (long)nb) + 1) * na;
-            if (8 * (na2 * (L_ + 1) + tab + z + 3 * na) + 6 * Arena::kAlign > cap) continue;
+            const size_t na = na_;
+            const long nb = nPadMax_ >> lb;
+            const size_t tab = k::block_table_values(b), w = k::block_scratch_values(b);
+            const size_t z = (size_t)(nb + 2) * na + k::block_z2_values(b, nb);
+            if (8 * (na2 * (L_ + 1) + tab + z + w + 3 * na) + 8 * Arena::kAlign > cap) continue;
             PT64_.alloc(na2 * (L_ + 1), arena);
             blkTab_.alloc(tab, arena);
             blkZ_.alloc(z, arena);
+            if (w) blkW_.alloc(w, arena);
             seed_.alloc(na_, arena);
             tot_.alloc(na_, arena);
             seedNext_.alloc(na_, arena);
             blk_ = b;
-            bb_.PT = PT64_.get();
-            bb_.QT = blkTab_.get();
-            bb_.OT = bb_.QT + (size_t)b.kb() * na;
-            bb_.Ht = bb_.OT + (size_t)b.T * b.p * na;
-            bb_.DL = bb_.Ht + (size_t)b.kh() * b.p;
-            bb_.Z = blkZ_.get();
-            bb_.Z2 = bb_.Z + (nb + 1) * na;
+            bb_ = k::block_carve(b, PT64_.get(), blkTab_.get(), blkZ_.get(), nb, blkW_.get());
             return;
         }
     }
@@ -133,7 +128,8 @@ size_t ScanCore::footprint() const
            DT_.bytes() + CT64_.bytes() + DT64_.bytes() +
            PT64_.bytes() + PT32_.bytes() + PTm_.bytes() + Sg_.bytes() + Sks32_.bytes() +
            Sks64_.bytes() + X32_.bytes() + X64_.bytes() + seed_.bytes() +
-           tot_.bytes() + seedNext_.bytes() + blkTab_.bytes() + blkZ_.bytes();
+           tot_.bytes() + seedNext_.bytes() + blkTab_.bytes() + blkZ_.bytes() +
+           blkW_.bytes();
 }
 
 bool ScanCore::level_is_f64(int l) const
@@ -250,6 +246,11 @@ void ScanCore::build_map(hipStream_t s, const float* dA, const float* dB, double
 void ScanCore::build_powers(hipStream_t s, bool withLast)
 {
     if (uses_blocks()) {
+        if (blk_.wide) {
+            wide_tables(s, dA_, dB_, dC_, dD_, nullptr, withLast, nullptr);
+            powersDone_ = true;
+            return;
+        }
         k::block_map(s, blk_, bb_, h_, dA_, dB_, dC_, dD_, nullptr, nullptr, false, nullptr,
                      nullptr);
         k::block_tables(s, blk_, bb_, dC_);
@@ -654,7 +655,7 @@ void ScanCore::sweep_top(hipStream_t s, long nReal, long nPad, const double* dSe
 {
     if (uses_blocks()) {
         batchSeed_ = dSeed;
-        k::block_scan(s, blk_, bb_, in_, blocks_of(nReal), dSeed);
+        k::block_scan(s, blk_, bb_, in_, blocks_of(nReal), dSeed, dTot);
         return;
     }
     const int L = ilog2(nPad), lt = top_level(nReal, nPad);
@@ -731,7 +732,7 @@ void ScanCore::carry(hipStream_t s, long nPad, const double* dSeed, const double
                      double* dOut)
 {
     if (uses_blocks()) {   // (a batch before the last is full)
-        k::block_carry(s, blk_, bb_, in_, nPad >> blk_.lb, dOut);
+        k::block_carry(s, blk_, bb_, in_, nPad >> blk_.lb, dSeed, dTot, dOut);
         return;
     }
     k::carry(s, na_, powerT(ilog2(nPad)), dSeed, dTot, dOut);
@@ -904,29 +905,94 @@ void ScanCore::zero_blocks(hipStream_t s)
 {
     k::fill_f64(s, (long)blkTab_.size(), 0.0, blkTab_.get());
     k::fill_f64(s, (long)blkZ_.size(), 0.0, blkZ_.get());
+    k::fill_f64(s, na_, 0.0, seed());
+}
+
+namespace {
+// A wide map's operations, kept by phase: a phase's products are one launch.
+struct Phases : k::BlockSink {
+    struct Phase {
+        std::vector<k::GemmOp> gemm;
+        std::vector<k::BlkElem> elem;
+        std::vector<k::SeqOp> seq;
+    };
+    std::vector<Phase> ph;
+    Phase& at(int p)
+    {
+        if ((int)ph.size() <= p) ph.resize(p + 1);
+        return ph[p];
+    }
+    void gemm(int p, const k::GemmOp& o) override { at(p).gemm.push_back(o); }
+    void elem(int p, const k::BlkElem& e) override { at(p).elem.push_back(e); }
+    void seq(int p, const k::SeqOp& o) override { at(p).seq.push_back(o); }
+    void run(hipStream_t s, int from, int to) const
+    {
+        for (int p = from; p < to && p < (int)ph.size(); ++p) {
+            for (auto& o : ph[p].seq) k::gemm_seq_f32(s, o.r, o.kk, o.c, o.X, o.Y, o.Z);
+            for (auto& e : ph[p].elem) k::block_elem(s, e);
+            for (size_t i = 0; i < ph[p].gemm.size(); i += k::kGemmMulti)
+                k::gemm_multi(s, ph[p].gemm.data() + i,
+                              (int)std::min<size_t>(k::kGemmMulti, ph[p].gemm.size() - i));
+        }
+    }
+};
+}  // namespace
+
+// The tables of a wide map.  With side, the powers that only the tree reads are
+// queued on side->stream (forked from s once pass 1's tables are queued; the
+// caller joins).
+void ScanCore::wide_tables(hipStream_t s, const float* dA, const float* dB, const float* dC,
+                           const float* dD, const float* dx0, bool withLast,
+                           const SideStream* side)
+{
+    Phases ph;
+    const int done = k::block_emit(blk_, bb_, h_, dA, dB, dC, dD, dx0, seed(),
+                                   withLast ? L_ : L_ - 1, ph);
+    ph.run(s, 0, done);
+    if (side) {
+        PARODE_HIP(hipEventRecord(side->fork, s));
+        PARODE_HIP(hipStreamWaitEvent(side->stream, side->fork, 0));
+        s = side->stream;
+    }
+    ph.run(s, done, (int)ph.ph.size());
 }
 
 void ScanCore::solve_blocks(hipStream_t s, long nScan, double h, const float* dA, const float* dB,
                             const float* dC, const float* dD, const float* dx0, const void* dU,
-                            bool uDouble, float* dY, hipEvent_t* marks)
+                            bool uDouble, float* dY, hipEvent_t* marks, const SideStream* side)
 {
     auto tick = [&](int i) {
         if (marks) PARODE_HIP(hipEventRecord(marks[i], s));
     };
     const long nb = blocks_of(nScan);
     const k::BlockInput in = block_input(dU, uDouble, 2, nScan);
+    float* yScan = method_ == kRK4 ? dY : dY + 3L * nOut();
+    h_ = h;
     tick(0);
-    k::block_map(s, blk_, bb_, h, dA, dB, dC, dD, dx0, dU, uDouble, seed(), dY);
-    k::block_tables(s, blk_, bb_, dC);
-    tick(1);
-    k::block_pass1(s, blk_, bb_, in, nb, true, block_tiling(1, nb, uDouble));
+    if (blk_.wide) {
+        // beside pass 1: the powers that only the tree reads, and the start-up
+        wide_tables(s, dA, dB, dC, dD, dx0, false, side);
+        hipStream_t ps = side ? side->stream : s;
+        if (method_ == kABM) {
+            abm_startup(ps, dA, dB, dx0, dU, uDouble, h, seed());
+            k::block_start_outputs(ps, blk_, dC, dD, seed(), dU, uDouble, dY);
+        }
+        if (side) PARODE_HIP(hipEventRecord(side->join, ps));
+        tick(1);
+        k::block_pass1(s, blk_, bb_, in, nb, false, block_tiling(1, nb, uDouble));
+        if (side) PARODE_HIP(hipStreamWaitEvent(s, side->join, 0));
+    } else {
+        k::block_map(s, blk_, bb_, h, dA, dB, dC, dD, dx0, dU, uDouble, seed(), dY);
+        k::block_tables(s, blk_, bb_, dC);
+        tick(1);
+        k::block_pass1(s, blk_, bb_, in, nb, true, block_tiling(1, nb, uDouble));
+    }
     tick(2);
     tick(3);
     k::block_scan(s, blk_, bb_, in, nb, seed());
     tick(4);
     tick(5);
-    k::block_pass2(s, blk_, bb_, in, nb, nScan, seed(), dD,
-                   method_ == kRK4 ? dY : dY + 3L * nOut(), block_tiling(2, nb, uDouble));
+    k::block_pass2(s, blk_, bb_, in, nb, nScan, seed(), dD, yScan, block_tiling(2, nb, uDouble));
     tick(6);
 }
 
@@ -941,7 +1007,7 @@ void ScanCore::solve(hipStream_t s, long points, double h, const float* dA, cons
     if (side && (!side->stream || !side->fork || !side->join))
         throw std::invalid_argument("ScanCore::solve: incomplete side stream");
     if (uses_blocks()) {
-        solve_blocks(s, nScan, h, dA, dB, dC, dD, dx0, dU, uDouble, dY, marks);
+        solve_blocks(s, nScan, h, dA, dB, dC, dD, dx0, dU, uDouble, dY, marks, side);
         return;
     }
     auto tick = [&](int i) {

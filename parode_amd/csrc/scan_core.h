@@ -158,7 +158,9 @@ private:
 
     void solve_blocks(hipStream_t s, long nScan, double h, const float* dA, const float* dB,
                       const float* dC, const float* dD, const float* dx0, const void* dU,
-                      bool uDouble, float* dY, hipEvent_t* marks);
+                      bool uDouble, float* dY, hipEvent_t* marks, const SideStream* side);
+    void wide_tables(hipStream_t s, const float* dA, const float* dB, const float* dC,
+                     const float* dD, const float* dx0, bool withLast, const SideStream* side);
     k::BlockInput block_input(const void* dU, bool uDouble, long sL, long nReal) const;
     long blocks_of(long nReal) const { return (nReal + blk_.T - 1) / blk_.T; }
     int block_tiling(int pass, long nb, bool uDouble) const;
@@ -201,7 +203,7 @@ private:
     // block responses: tables and the blocks' states; the batch's input
     k::BlockShape blk_;
     k::BlockBufs bb_;
-    DevArray<double> blkTab_, blkZ_;
+    DevArray<double> blkTab_, blkZ_, blkW_;
     k::BlockInput in_;
     const float *dA_ = nullptr, *dB_ = nullptr, *dC_ = nullptr, *dD_ = nullptr;
     const double* batchSeed_ = nullptr;

@@ -45,7 +45,10 @@ def _oracle(s, U, states):
     (0, 17, 31, 33, 2049), (0, 63, 32, 2, 777), (0, 64, 32, 64, 9001), (0, 64, 1, 1, 70001),
     (0, 65, 33, 9, 1500), (0, 5, 2, 3, 300007),
     (1, 1, 1, 1, 67), (1, 4, 2, 1, 131), (1, 15, 32, 64, 1030), (1, 16, 7, 15, 40003),
-    (1, 17, 3, 2, 600), (1, 3, 5, 4, 270001)])
+    (1, 17, 3, 2, 600), (1, 3, 5, 4, 270001),
+    # maps made by products over many work-groups
+    (0, 96, 40, 70, 1100), (0, 128, 16, 16, 20000), (0, 130, 1, 1, 64), (0, 200, 25, 7, 3001),
+    (1, 33, 4, 4, 7000), (1, 64, 8, 8, 30003), (1, 129, 5, 9, 2500)])
 @pytest.mark.parametrize("precision", [api.PLAIN32, api.MIXED, api.FP64])
 def test_block_shapes_meet_the_bars(method, n, m, p, steps, precision):
     s = synth.make_system(method, n, m, p, -5.0, -0.1, 1e-3, steps, seed=31 * n + steps,
@@ -62,7 +65,7 @@ def test_block_shapes_meet_the_bars(method, n, m, p, steps, precision):
     assert err <= BAR[precision]
 
 
-@pytest.mark.parametrize("method,n,steps", [(0, 1, 64), (0, 48, 5001), (0, 64, 999), (1, 16, 2500),
+@pytest.mark.parametrize("method,n,steps", [(0, 1, 64), (0, 48, 5001), (0, 64, 999), (0, 70, 3000), (1, 16, 2500), (1, 20, 1500),
                                             (1, 5, 100)])
 def test_states_as_outputs(method, n, steps):
     s = synth.make_system(method, n, 3, 2, -5.0, -0.1, 1e-3, steps, seed=9 * n)
@@ -72,7 +75,7 @@ def test_states_as_outputs(method, n, steps):
 
 
 @pytest.mark.parametrize("method,n,m,p,steps,row", [
-    (0, 6, 2, 3, 2000, 1501), (0, 6, 2, 3, 2000, 0), (0, 40, 3, 40, 60000, 77777),
+    (0, 6, 2, 3, 2000, 1501), (0, 6, 2, 3, 2000, 0), (0, 40, 3, 40, 60000, 77777), (0, 80, 3, 5, 9000, 8191), (1, 40, 2, 3, 9000, 8190),
     (1, 8, 2, 3, 3000, 2466), (1, 12, 1, 30, 40000, 40404)])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 def test_a_sample_that_is_not_finite_reaches_only_what_depends_on_it(method, n, m, p, steps, row,
