@@ -48,11 +48,13 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
     ScanOptions opt;
     opt.precision = kMixed;
     // stages, in order; the squarings and the tree levels get one phase per level
-    enum { kSmp = 0, kIn, kR1, kR2, kR3, kComb, kPost, kPow0 };
-    int maxL = 0, upSteps = 0;
+    enum { kSmp = 0, kIn, kR1, kR2, kR3, kComb, kPost, kBlk0 };
+    int maxL = 0, upSteps = 0, blkSteps = 0, blkRest = 0;
     struct Shape {
         long nScan, nPad;
         int L, na, lc, lt;
+        BlockPhases ops;   // of a wide map that runs as block responses
+        int ready = 0;     // the phase of ops before which pass 1's table is not complete
     };
     std::vector<Shape> sh(systems.size());
     sys_.resize(systems.size());
@@ -66,8 +68,22 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
         s.nPad = next_pow2(s.nScan);
         s.L = ilog2(s.nPad);
         s.na = q.method == kABM ? 4 * q.n : q.n;
-        sys_[i].core.reset(new ScanCore(q.method, q.n, q.m, q.p, !q.C, !q.D, s.nPad, opt, arena, false));
+        sys_[i].core.reset(new ScanCore(q.method, q.n, q.m, q.p, !q.C, !q.D, s.nPad, opt, arena));
         ScanCore& c = *sys_[i].core;
+        if (c.uses_blocks()) {
+            const long nb = c.blocks_of(s.nScan);
+            if (c.blk_.wide) {
+                s.ready = k::block_emit(c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0, c.seed(),
+                                        s.L - 1, s.ops);
+                upSteps = std::max(upSteps, k::block_tree_levels(nb));
+                blkSteps = std::max(blkSteps, s.ready);
+                blkRest = std::max(blkRest, (int)s.ops.ph.size() - s.ready);
+            } else {
+                upSteps = std::max(upSteps, 1);
+                blkSteps = std::max(blkSteps, 2);
+            }
+            continue;
+        }
         if (!c.Sks32_.get()) sys_[i].copies.alloc(2 * ks_half(s.nPad, s.na), arena);
         s.lc = c.chunk_log(s.nScan, s.nPad, true);
         s.lt = c.top_level(s.nScan, s.nPad);
@@ -77,6 +93,9 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
         maxL = std::max(maxL, s.L);
         upSteps = std::max(upSteps, s.lt - s.lc);
     }
+    // the tables of block responses, what only their tree reads, the general
+    // path's powers
+    const int kBlk1 = kBlk0 + blkSteps, kPow0 = kBlk1 + std::max(blkRest, 0);
     const int kTables = kPow0 + 4 * maxL, kStart = kTables + 1, kLeaves = kStart + 1,
               kChunk1 = kLeaves + 1, kUp0 = kChunk1 + 1, kTop = kUp0 + upSteps,
               kGather = kTop + 1, kDown0 = kGather + 1, kChunk2 = kDown0 + upSteps,
@@ -87,6 +106,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
     phases_.resize(kOut + kOutSets);
     outPhase_ = kOut;
     auto stage_of = [&](int ph) {
+        if (ph >= kBlk0 && ph < kPow0) return kStagePowers;
         if (ph <= kIn) return kStageInputs;
         if (ph <= kPost) return kStageMap;
         if (ph < kTables) return kStagePowers;
@@ -108,6 +128,44 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
         ScanCore& c = *sys_[i].core;
         const int n = q.n, m = q.m, p = q.p, na = s.na, L = s.L;
         const bool abm = q.method == kABM;
+        if (c.uses_blocks()) {
+            if (q.coef)
+                k::g::add_sample(P[kSmp], m, q.coef, q.t0, 0.5 * q.h, 2 * q.points + 1, q.sigma,
+                                 q.seed, q.U);
+            const k::BlockInput bin = c.block_input(q.U, true, 2, s.nScan);
+            const long nb = c.blocks_of(s.nScan);
+            float* yScan = q.Y;
+            if (abm) {
+                k::g::add_startup(P[kStart], n, m, q.h, q.A, q.B, q.x0, q.U, c.seed());
+                k::g::add_block_start_outputs(P[kOut], c.blk_, q.C, q.D, c.seed(), q.U, q.Y);
+                yScan = q.Y + 3L * p;
+            }
+            if (c.blk_.wide) {
+                for (int t = 0; t < (int)s.ops.ph.size(); ++t) {
+                    k::g::Phase& ph = P[t < s.ready ? kBlk0 + t : kBlk1 + t - s.ready];
+                    for (auto& e : s.ops.ph[t].elem) k::g::add_block_elem(ph, e);
+                    for (auto& o : s.ops.ph[t].gemm) k::g::add_gemm_op(ph, o);
+                }
+                const int top = k::block_tree_levels(nb);
+                for (int t = 0; t < top; ++t) {
+                    k::g::add_gemm_op(P[kUp0 + upSteps - (top - t)],
+                                      k::block_tree_up(c.blk_, c.bb_, nb, t));
+                    k::g::add_gemm_op(P[kDown0 + top - 1 - t],
+                                      k::block_tree_down(c.blk_, c.bb_, nb, t));
+                }
+                k::g::add_block_root(P[kTop], c.blk_, c.bb_, bin, nb, c.seed());
+            } else {
+                k::g::add_block_map(P[kBlk0], c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0,
+                                    c.seed());
+                k::g::add_block_tables(P[kBlk0 + 1], c.blk_, c.bb_, q.C);
+                k::g::add_block_scan(P[kUp0 + upSteps - 1], P[kTop], P[kDown0], c.blk_, c.bb_, bin,
+                                     nb, c.seed());
+            }
+            k::g::add_block_pass1(P[kChunk1], c.blk_, c.bb_, bin, nb);
+            k::g::add_block_pass2(P[kChunk2], c.blk_, c.bb_, bin, nb, s.nScan, c.seed(), q.D,
+                                  yScan);
+            return;
+        }
         const size_t nn = (size_t)n * n, nm = (size_t)n * m, na2 = (size_t)na * na;
         double* A = c.A64_.get();
         double* B = c.B64_.get();
@@ -318,10 +376,12 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
             // powers and level tables on the side stream, beside the input
             // samples, the ABM start-up, the leaves and the first chunk pass;
             // the rest after both (roles: 0 copies and map, 5 samples, 1
-            // powers and tables, 4 start-up, 2 leaves and chunks, 3 the rest)
+            // powers and tables, 4 start-up, 2 leaves and chunks, 3 the rest;
+            // block responses: 6 what pass 1 reads, 1 what only their tree does)
             const int pos = (int)pi;
             const int role = pos == kSmp     ? 5
                              : pos <= kPost  ? 0
+                             : pos < kBlk1   ? 6
                              : pos < kStart  ? 1
                              : pos == kStart ? 4
                              : pos <= kChunk1 ? 2
@@ -463,17 +523,22 @@ void BatchSolve::run(hipStream_t s, void* hostStage, void* devDesc, bool upload,
         queue(s, 0, fan);
         PARODE_HIP(hipEventRecord(side->fork, s));
         PARODE_HIP(hipStreamWaitEvent(side->stream, side->fork, 0));
-        queue(side->stream, 1, nullptr);
-        PARODE_HIP(hipEventRecord(side->join, side->stream));
+        // (the host queues both streams: what pass 1 waits for first, then the
+        // samples, so that neither stream waits for the other's many launches)
+        queue(side->stream, 6, nullptr);
+        if (side->late) PARODE_HIP(hipEventRecord(side->late, side->stream));
         queue(s, 5, fan);
         queue(s, 4, fan);
+        queue(side->stream, 1, nullptr);
+        PARODE_HIP(hipEventRecord(side->join, side->stream));
+        PARODE_HIP(hipStreamWaitEvent(s, side->late ? side->late : side->join, 0));
         queue(s, 2, fan);
         PARODE_HIP(hipStreamWaitEvent(s, side->join, 0));
         queue(s, 3, fan);
         return;
     }
     if (!marks) {
-        for (int role : {0, 5, 1, 4, 2, 3}) queue(s, role, fan);
+        for (int role : {0, 5, 6, 1, 4, 2, 3}) queue(s, role, fan);
         return;
     }
     int stage = 0;
@@ -512,6 +577,7 @@ struct Group {
         fan.destroy();
         if (side.fork) (void)hipEventDestroy(side.fork);
         if (side.join) (void)hipEventDestroy(side.join);
+        if (side.late) (void)hipEventDestroy(side.late);
         if (side.stream) (void)hipStreamDestroy(side.stream);
         for (hipEvent_t e : marks)
             if (e) (void)hipEventDestroy(e);
@@ -590,9 +656,10 @@ int ParODE_GroupExecute(void* group, void* stream)
     try {
         PARODE_HIP(hipSetDevice(g->device));
         if (!g->side.stream) {
-            PARODE_HIP(hipStreamCreate(&g->side.stream));
+            PARODE_HIP(hipStreamCreateWithFlags(&g->side.stream, hipStreamNonBlocking));
             PARODE_HIP(hipEventCreateWithFlags(&g->side.fork, hipEventDisableTiming));
             PARODE_HIP(hipEventCreateWithFlags(&g->side.join, hipEventDisableTiming));
+            PARODE_HIP(hipEventCreateWithFlags(&g->side.late, hipEventDisableTiming));
         }
         if (!g->fan.start) g->fan.create();
         g->batch->run(static_cast<hipStream_t>(stream), g->stage, g->desc, !g->uploaded, nullptr,

@@ -143,5 +143,25 @@ void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
                  long nb, long nReal, const double* seed, const float* D, float* Y,
                  int tiling = kBlockAuto);
 
+// ---- the same launches for many systems in one grid (FP64 samples)
+namespace g {
+void add_block_map(Phase& ph, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                   const float* B, const float* C, const float* D, const float* x0, double* seed);
+void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, const float* C);
+void add_block_elem(Phase& ph, const BlkElem& e);
+void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, const float* D,
+                             const double* X0, const double* U, float* Y);
+void add_block_pass1(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                     long nb);
+void add_block_pass2(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                     long nb, long nReal, const double* seed, const float* D, float* Y);
+// the scan of a map that is not wide: up and down are used when the blocks go in groups
+void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, const BlockBufs& b,
+                    const BlockInput& in, long nb, const double* seed);
+// the root of a wide map's tree
+void add_block_root(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                    long nb, const double* seed);
+}  // namespace g
+
 }  // namespace k
 }  // namespace parode

@@ -966,7 +966,8 @@ __device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, do
 {
     const int na = a.na, n16 = (na + 15) & ~15, nct = n16 / 16, pitch = n16 + 1;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q4 = lane >> 4;
-    const int rt = wave / nct, ct = wave - rt * nct, rows = 16 * a.R, nth = 64 * nct * a.R;
+    const int rt = wave / nct, ct = wave - rt * nct, rows = 16 * a.R;
+    if (rt >= a.R) return;   // (a grouped launch has waves for its widest system)
     const long Lg = 1L << a.lg, g0 = vb.x * rows;
     double* x0 = lds;                       // [rows][pitch], double buffered
     double* x1 = lds + rows * pitch;
@@ -1102,7 +1103,6 @@ __device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, do
         }
         flip();
     }
-    (void)nth;
 }
 
 template <int MODE>
@@ -1611,12 +1611,19 @@ long block_groups(int na, long nb)
     return lg ? (nb + (1L << lg) - 1) >> lg : 0;
 }
 
+static BlkMap map_args(const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                       const float* B, const float* C, const float* D, const float* x0,
+                       const void* U, double* seed, float* Y)
+{
+    return BlkMap{s, h, rk4_coefficients(h), abm_coefficients(h), A, B, C, D, x0, U, b.PT, b.QT,
+                  b.Ht, b.DL, seed, Y, x0 ? 2L : 1L};
+}
+
 void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
                const float* B, const float* C, const float* D, const float* x0, const void* U,
                bool uDouble, double* seed, float* Y)
 {
-    const BlkMap a{s, h, rk4_coefficients(h), abm_coefficients(h), A, B, C, D, x0, U, b.PT, b.QT,
-                   b.Ht, b.DL, seed, Y, x0 ? 2L : 1L};
+    const BlkMap a = map_args(s, b, h, A, B, C, D, x0, U, seed, Y);
     if (uDouble)
         hipLaunchKernelGGL(k_blk_map<double>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     else
@@ -1644,10 +1651,16 @@ static int slice_steps(int T, int per)
     return k;
 }
 
-void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C)
+static BlkTables table_args(const BlockShape& s, const BlockBufs& b, const float* C)
 {
     BlkTables a{s, C, b.PT, b.QT, b.OT, b.Ht, slice_steps(s.T, s.p), slice_steps(s.T, s.s * s.m), 0};
     a.gx = 1 + s.T / a.ni + s.T / a.nq;
+    return a;
+}
+
+void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C)
+{
+    const BlkTables a = table_args(s, b, C);
     hipLaunchKernelGGL(k_blk_tables, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     check_launch("block_tables");
 }
@@ -1673,21 +1686,32 @@ static BlkPass pass_args(const BlockShape& s, const BlockBufs& b, const BlockInp
     return a;
 }
 
-// 64 x 64 tiles once they give every compute unit one; 16 x 16 below, their K
-// over 16 waves while those tiles are few too.
-template <bool OUT>
-static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, int tiling)
+// The tiling of a pass over one system: 64 x 64 tiles once they give every
+// compute unit one; 16 x 16 below, their K over 16 waves while those tiles are
+// few too.  In a grouped launch (grouped) the other systems fill the GPU, so
+// the 64 x 64 tiles' higher rate counts from fewer of them.
+static int pass_tiling(const BlkPass& a, bool out, bool grouped)
 {
     const long tx = (a.cols + kPT - 1) / kPT, ty = (a.nb + kPT - 1) / kPT;
     const long sx = (a.cols + 15) / 16, sy = (a.nb + 15) / 16;
-    const int ksteps = ((OUT ? a.kz : 0) + a.ku) / 4;
-    const bool tile = tiling ? tiling == kBlockTile : tx * ty >= 256;
-    a.gx = tile ? tx : sx;
-    a.gy = tile ? ty : sy;
-    const long blocks = a.gx * a.gy + (powers ? 1 : 0);
-    if (blocks > 0x7fffffffL) throw std::length_error("block pass: too many tiles");
-    const dim3 grid((unsigned)blocks);
-    const bool wide = !tile && (tiling ? tiling == kBlockSplit16 : sx * sy <= 256 && ksteps >= 64);
+    if (tx * ty >= (grouped ? 24 : 256)) return kBlockTile;
+    return sx * sy <= 256 && ((out ? a.kz : 0) + a.ku) / 4 >= 64 ? kBlockSplit16 : kBlockSplit4;
+}
+static void pass_grid(BlkPass& a, int tiling)
+{
+    const int t = tiling == kBlockTile ? kPT : 16;
+    a.gx = (a.cols + t - 1) / t;
+    a.gy = (a.nb + t - 1) / t;
+    if (a.gx * a.gy >= 0x7fffffffL) throw std::length_error("block pass: too many tiles");
+}
+
+template <bool OUT>
+static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, int tiling)
+{
+    if (!tiling) tiling = pass_tiling(a, OUT, false);
+    pass_grid(a, tiling);
+    const dim3 grid((unsigned)(a.gx * a.gy + (powers ? 1 : 0)));
+    const bool tile = tiling == kBlockTile, wide = tiling == kBlockSplit16;
 #define PARODE_PASS(TU)                                                                   \
     do {                                                                                  \
         if (tile)                                                                         \
@@ -1705,8 +1729,7 @@ static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, in
     check_launch("block pass");
 }
 
-void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                 long nb, bool powers, int tiling)
+static BlkPass pass1_args(const BlockShape& s, const BlockBufs& b, const BlockInput& in, long nb)
 {
     BlkPass a = pass_args(s, b, in, nb);
     a.cols = s.na;
@@ -1714,11 +1737,10 @@ void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
     a.ku = s.kb();
     a.BU = b.QT;
     a.S = b.Z;
-    launch_pass<false>(st, a, in.isDouble, powers, tiling);
+    return a;
 }
-
-void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                 long nb, long nReal, const double* seed, const float* D, float* Y, int tiling)
+static BlkPass pass2_args(const BlockShape& s, const BlockBufs& b, const BlockInput& in, long nb,
+                          long nReal, const double* seed, const float* D, float* Y)
 {
     BlkPass a = pass_args(s, b, in, nb);
     a.cols = s.T * s.p;
@@ -1731,7 +1753,19 @@ void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
     a.Y = Y;
     a.seed = seed;
     a.D = s.useD ? D : nullptr;
-    launch_pass<true>(st, a, in.isDouble, false, tiling);
+    return a;
+}
+
+void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, bool powers, int tiling)
+{
+    launch_pass<false>(st, pass1_args(s, b, in, nb), in.isDouble, powers, tiling);
+}
+
+void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                 long nb, long nReal, const double* seed, const float* D, float* Y, int tiling)
+{
+    launch_pass<true>(st, pass2_args(s, b, in, nb, nReal, seed, D, Y), in.isDouble, false, tiling);
 }
 
 static BlkScan scan_args(const BlockShape& s, const BlockBufs& b, const BlockInput& in, long nb,
@@ -1757,6 +1791,37 @@ static BlkScan scan_args(const BlockShape& s, const BlockBufs& b, const BlockInp
     return a;
 }
 
+static size_t scan_lds_bytes(const BlkScan& a)
+{
+    return (size_t)2 * 16 * a.R * ((a.na + 15) / 16 * 16 + 1) * sizeof(double);
+}
+
+// The scan's launches: u and d when the blocks go in groups (returns true), a
+// over the blocks or the groups.
+static bool scan_plan(BlkScan a0, const BlockBufs& b, BlkScan& u, BlkScan& a, BlkScan& d)
+{
+    const int nct = (a0.na + 15) / 16, lg = group_log(a0.nb);
+    a = a0;
+    a.R = 1;
+    if (lg) {
+        u = a0;
+        u.lg = lg;
+        u.R = 1;
+        const long groups = block_groups(a0.na, a0.nb);
+        u.gx = (groups + 15) / 16;
+        d = u;
+        a.nb = groups;
+        a.E = b.Z2;
+        a.l0 = a0.l0 + lg;
+    }
+    // as many row tiles as 16 waves (and 64 KB of LDS) hold, no more than the blocks need
+    while (2 * a.R * nct <= 16 && 2 * scan_lds_bytes(a) <= 65536 && 16L * a.R < a.nb) a.R *= 2;
+    a.lg = 0;
+    while ((16L * a.R << a.lg) < a.nb) ++a.lg;
+    a.gx = 1;
+    return lg > 0;
+}
+
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                 long nb, const double* seed, double* tot)
 {
@@ -1777,36 +1842,20 @@ void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const B
         }
         return;
     }
-    const int nct = (s.na + 15) / 16, pitch = 16 * nct + 1;
-    auto lds = [&](int R) { return (size_t)2 * 16 * R * pitch * sizeof(double); };
-    BlkScan a = scan_args(s, b, in, nb, seed);
-    const int lg = group_log(nb);
-    const long groups = block_groups(s.na, nb);
-    if (lg) {
-        BlkScan u = a;
-        u.lg = lg;
-        u.R = 1;
-        u.gx = (groups + 15) / 16;
-        hipLaunchKernelGGL(k_blk_scan<kScanUp>, dim3((unsigned)u.gx), dim3(64 * nct), lds(1), st, u);
+    BlkScan u, a, d;
+    const bool groups = scan_plan(scan_args(s, b, in, nb, seed), b, u, a, d);
+    const int nct = (s.na + 15) / 16;
+    if (groups) {
+        hipLaunchKernelGGL(k_blk_scan<kScanUp>, dim3((unsigned)u.gx), dim3(64 * nct),
+                           scan_lds_bytes(u), st, u);
         check_launch("block scan, up");
-        a.nb = groups;
-        a.E = b.Z2;
-        a.l0 = s.lb + lg;
     }
-    // as many row tiles as 16 waves (and 64 KB of LDS) hold, no more than the blocks need
-    a.R = 1;
-    while (2 * a.R * nct <= 16 && lds(2 * a.R) <= 65536 && 16L * a.R < a.nb) a.R *= 2;
-    a.lg = 0;
-    while ((16L * a.R << a.lg) < a.nb) ++a.lg;
-    a.gx = 1;
-    hipLaunchKernelGGL(k_blk_scan<kScanAll>, dim3(1), dim3(64 * nct * a.R), lds(a.R), st, a);
+    hipLaunchKernelGGL(k_blk_scan<kScanAll>, dim3(1), dim3(64 * nct * a.R), scan_lds_bytes(a), st,
+                       a);
     check_launch("block scan");
-    if (lg) {
-        BlkScan d = scan_args(s, b, in, nb, seed);
-        d.lg = lg;
-        d.R = 1;
-        d.gx = (groups + 15) / 16;
-        hipLaunchKernelGGL(k_blk_scan<kScanDown>, dim3((unsigned)d.gx), dim3(64 * nct), lds(1), st, d);
+    if (groups) {
+        hipLaunchKernelGGL(k_blk_scan<kScanDown>, dim3((unsigned)d.gx), dim3(64 * nct),
+                           scan_lds_bytes(d), st, d);
         check_launch("block scan, down");
     }
 }
@@ -1827,6 +1876,204 @@ void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
                        nb * s.T * in.sL * s.m, seedOut);
     check_launch("block carry");
 }
+
+// ---------------------------------------------------------- grouped launches
+namespace g {
+
+namespace {
+
+struct StartOutB {
+    BlockShape s;
+    const float *C, *D;
+    const double *X0, *U;
+    float* Y;
+    long gx;
+};
+struct RootB {
+    BlkScan a;
+    double* root;
+    long gx;
+};
+
+__global__ __launch_bounds__(1024) void kg_blk_map(const BlkMap* __restrict__ args,
+                                                   const unsigned* __restrict__ st, int ns)
+{
+    PARODE_GROUP(BlkMap);
+    __shared__ double lds[kMapLds];
+    d_blk_map<double>(vb, a, lds);
+}
+__global__ __launch_bounds__(1024) void kg_blk_tables(const BlkTables* __restrict__ args,
+                                                      const unsigned* __restrict__ st, int ns)
+{
+    PARODE_GROUP(BlkTables);
+    __shared__ double P[kBN * kBP], R[kBN * kBP], G[kBN * kBP];
+    d_blk_tables(vb, a, P, R, G);
+}
+__global__ __launch_bounds__(256) void kg_blk_elem(const BlkElem* __restrict__ args,
+                                                   const unsigned* __restrict__ st, int ns)
+{
+    PARODE_GROUP(BlkElem);
+    d_blk_elem(vb, a);
+}
+__global__ __launch_bounds__(256) void kg_blk_start_outputs(const StartOutB* __restrict__ args,
+                                                            const unsigned* __restrict__ st, int ns)
+{
+    PARODE_GROUP(StartOutB);
+    (void)vb;
+    d_start_outputs<double>(a.s, a.C, a.D, a.X0, a.U, a.Y);
+}
+// (a system's last work-group of pass 1 squares the rest of its powers, if any)
+template <bool OUT, int NW>
+__global__ __launch_bounds__(NW * 64) void kg_blk_split(const BlkPass* __restrict__ args,
+                                                        const unsigned* __restrict__ st, int ns)
+{
+    constexpr int kPart = (NW - 1) * 256;
+    constexpr int kLds = OUT || kPart > kBN * kBP ? kPart : kBN * kBP;
+    __shared__ double lds[kLds];
+    __shared__ int bad;
+    const int sys = system_of(st, ns);
+    const BlkPass& a = args[sys];
+    const long idx = (long)blockIdx.x - (long)st[sys];
+    if (!OUT && idx == a.gx * a.gy) {
+        d_blk_powers<NW>(a.na, a.lb, a.L, a.PT, lds);
+        return;
+    }
+    d_blk_split<double, OUT, NW>(blk_place(idx, a.gx, a.gy), a, lds, &bad);
+}
+template <bool OUT>
+__global__ __launch_bounds__(256) void kg_blk_tile(const BlkPass* __restrict__ args,
+                                                   const unsigned* __restrict__ st, int ns)
+{
+    __shared__ BlkTileLds L;
+    const int sys = system_of(st, ns);
+    const BlkPass& a = args[sys];
+    const long idx = (long)blockIdx.x - (long)st[sys];
+    if (!OUT && idx == a.gx * a.gy) {
+        d_blk_powers<4>(a.na, a.lb, a.L, a.PT, &L.A[0][0][0]);
+        return;
+    }
+    d_blk_tile<double, OUT>(blk_place(idx, a.gx, a.gy), a, L);
+}
+template <int MODE>
+__global__ __launch_bounds__(MODE == kScanAll ? 1024 : 256) void kg_blk_scan(
+    const BlkScan* __restrict__ args, const unsigned* __restrict__ st, int ns)
+{
+    extern __shared__ double scan_lds[];
+    PARODE_GROUP(BlkScan);
+    d_blk_scan<MODE>(vb, a, scan_lds);
+}
+__global__ __launch_bounds__(256) void kg_blk_root(const RootB* __restrict__ args,
+                                                   const unsigned* __restrict__ st, int ns)
+{
+    PARODE_GROUP(RootB);
+    (void)vb;
+    d_blk_root(a.a, a.root, nullptr);
+}
+
+void add_pass(Phase& ph, BlkPass a, bool out, bool powers)
+{
+    const int t = pass_tiling(a, out, true);
+    pass_grid(a, t);
+    const float cost = (float)((out ? a.kz : 0) + a.ku);
+    append(ph, t == kBlockTile ? kBlkTile : t == kBlockSplit16 ? kBlkSplit16 : kBlkSplit4, out, a,
+           a.gx * a.gy + (powers ? 1 : 0), 0, cost);
+}
+
+}  // namespace
+
+void add_block_map(Phase& ph, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                   const float* B, const float* C, const float* D, const float* x0, double* seed)
+{
+    // (an ABM start-up reads the input samples: it has a launch of its own)
+    const BlkMap a = map_args(s, b, h, A, B, C, D, s.method == 0 ? x0 : nullptr, nullptr, seed,
+                              nullptr);
+    append(ph, kBlkMap, false, a, a.gx, 0, (float)s.na);
+}
+void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, const float* C)
+{
+    const BlkTables a = table_args(s, b, C);
+    append(ph, kBlkTables, false, a, a.gx, 0, (float)s.na * s.lb);
+}
+void add_block_elem(Phase& ph, const BlkElem& e)
+{
+    if (e.count <= 0) return;
+    append(ph, kBlkElem, false, e, e.gx);
+}
+void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, const float* D,
+                             const double* X0, const double* U, float* Y)
+{
+    append(ph, kBlkStartOut, false, StartOutB{s, C, D, X0, U, Y, 1}, 1);
+}
+void add_block_pass1(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                     long nb)
+{
+    add_pass(ph, pass1_args(s, b, in, nb), false, !s.wide);
+}
+void add_block_pass2(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                     long nb, long nReal, const double* seed, const float* D, float* Y)
+{
+    add_pass(ph, pass2_args(s, b, in, nb, nReal, seed, D, Y), true, false);
+}
+void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, const BlockBufs& b,
+                    const BlockInput& in, long nb, const double* seed)
+{
+    BlkScan u, a, d;
+    if (scan_plan(scan_args(s, b, in, nb, seed), b, u, a, d)) {
+        append(up, kBlkScanUp, false, u, u.gx, scan_lds_bytes(u), (float)(s.na << u.lg));
+        append(down, kBlkScanDown, false, d, d.gx, scan_lds_bytes(d), (float)(s.na << d.lg));
+    }
+    append(all, kBlkScanAll, false, a, 1, scan_lds_bytes(a), (float)(s.na << a.lg));
+}
+void add_block_root(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
+                    long nb, const double* seed)
+{
+    long one;
+    double* root = tree_level(s, b, nb, block_tree_levels(nb), one);
+    append(ph, kBlkRoot, false, RootB{scan_args(s, b, in, nb, seed), root, 1}, 1, 0, (float)s.na);
+}
+
+bool run_blocks(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dStart)
+{
+    const int ns = L.nsys();
+    const dim3 grid(L.blocks());
+    const size_t lds = L.lds;
+#define PARODE_RUN(KERNEL, T, THREADS)                                                        \
+    hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), lds, s, static_cast<const T*>(dArgs),   \
+                       dStart, ns)
+    switch (L.kind) {
+    case kBlkMap: PARODE_RUN(kg_blk_map, BlkMap, 1024); break;
+    case kBlkTables: PARODE_RUN(kg_blk_tables, BlkTables, 1024); break;
+    case kBlkElem: PARODE_RUN(kg_blk_elem, BlkElem, 256); break;
+    case kBlkStartOut: PARODE_RUN(kg_blk_start_outputs, StartOutB, 256); break;
+    case kBlkTile:
+        if (L.flag)
+            PARODE_RUN(kg_blk_tile<true>, BlkPass, 256);
+        else
+            PARODE_RUN(kg_blk_tile<false>, BlkPass, 256);
+        break;
+    case kBlkSplit4:
+        if (L.flag)
+            PARODE_RUN((kg_blk_split<true, 4>), BlkPass, 256);
+        else
+            PARODE_RUN((kg_blk_split<false, 4>), BlkPass, 256);
+        break;
+    case kBlkSplit16:
+        if (L.flag)
+            PARODE_RUN((kg_blk_split<true, 16>), BlkPass, 1024);
+        else
+            PARODE_RUN((kg_blk_split<false, 16>), BlkPass, 1024);
+        break;
+    case kBlkScanUp: PARODE_RUN(kg_blk_scan<kScanUp>, BlkScan, 256); break;
+    case kBlkScanAll: PARODE_RUN(kg_blk_scan<kScanAll>, BlkScan, 1024); break;
+    case kBlkScanDown: PARODE_RUN(kg_blk_scan<kScanDown>, BlkScan, 256); break;
+    case kBlkRoot: PARODE_RUN(kg_blk_root, RootB, 256); break;
+    default: return false;
+    }
+#undef PARODE_RUN
+    return true;
+}
+
+}  // namespace g
 
 }  // namespace k
 }  // namespace parode

@@ -266,7 +266,10 @@ enum Kind {
     kDense16, kDense32, kDense48, kDense64, kDense96, kDense128, kDense160, kDense192, kDense224,
     kDense256,
     kLevel32, kLevel32W, kLevel32Delta, kLevel32DeltaW, kLevelG, kLevelGDelta, kLevel64, kGather, kTopMfma, kTopSimt, kRoot,
-    kOutputsLanes, kOutputsKc8, kOutputsKc16, kOutputsKc24, kOutputsKc32, kOutputsMfma
+    kOutputsLanes, kOutputsKc8, kOutputsKc16, kOutputsKc24, kOutputsKc32, kOutputsMfma,
+    // block responses (flag: pass 2)
+    kBlkMap, kBlkTables, kBlkElem, kBlkStartOut, kBlkTile, kBlkSplit4, kBlkSplit16, kBlkScanUp,
+    kBlkScanAll, kBlkScanDown, kBlkRoot
 };
 struct Launch {
     int kind = -1;
@@ -344,6 +347,8 @@ void add_root(Phase& ph, int na, long last, const double* seed, float* X, double
 bool add_outputs(Phase& ph, int n, int m, int p, int pp, int na, int oX, bool useC, bool useD,
                  long N, const double* CT, const double* DT, const float* X, const double* U,
                  long sO, long oO, float* Y);
+// The launches of blocks.hip (false: not one of them).
+bool run_blocks(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dStart);
 // Launches L with its records at dArgs and its block table at dStart (device).
 void run(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dStart);
 }  // namespace g

@@ -4820,7 +4820,9 @@ void run(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dSta
     case kOutputsKc16: PARODE_RUN(kg_out_kc<16>, Outputs, kOutLanes); break;
     case kOutputsKc24: PARODE_RUN(kg_out_kc<24>, Outputs, kOutLanes); break;
     case kOutputsKc32: PARODE_RUN(kg_out_kc<32>, Outputs, kOutLanes); break;
-    default: throw std::logic_error("grouped launch: unknown kernel");
+    default:
+        if (!run_blocks(s, L, dArgs, dStart))
+            throw std::logic_error("grouped launch: unknown kernel");
     }
 #undef PARODE_RUN2
 #undef PARODE_RUN

@@ -908,35 +908,16 @@ void ScanCore::zero_blocks(hipStream_t s)
     k::fill_f64(s, na_, 0.0, seed());
 }
 
-namespace {
-// A wide map's operations, kept by phase: a phase's products are one launch.
-struct Phases : k::BlockSink {
-    struct Phase {
-        std::vector<k::GemmOp> gemm;
-        std::vector<k::BlkElem> elem;
-        std::vector<k::SeqOp> seq;
-    };
-    std::vector<Phase> ph;
-    Phase& at(int p)
-    {
-        if ((int)ph.size() <= p) ph.resize(p + 1);
-        return ph[p];
+void BlockPhases::run(hipStream_t s, int from, int to) const
+{
+    for (int p = from; p < to && p < (int)ph.size(); ++p) {
+        for (auto& o : ph[p].seq) k::gemm_seq_f32(s, o.r, o.kk, o.c, o.X, o.Y, o.Z);
+        for (auto& e : ph[p].elem) k::block_elem(s, e);
+        for (size_t i = 0; i < ph[p].gemm.size(); i += k::kGemmMulti)
+            k::gemm_multi(s, ph[p].gemm.data() + i,
+                          (int)std::min<size_t>(k::kGemmMulti, ph[p].gemm.size() - i));
     }
-    void gemm(int p, const k::GemmOp& o) override { at(p).gemm.push_back(o); }
-    void elem(int p, const k::BlkElem& e) override { at(p).elem.push_back(e); }
-    void seq(int p, const k::SeqOp& o) override { at(p).seq.push_back(o); }
-    void run(hipStream_t s, int from, int to) const
-    {
-        for (int p = from; p < to && p < (int)ph.size(); ++p) {
-            for (auto& o : ph[p].seq) k::gemm_seq_f32(s, o.r, o.kk, o.c, o.X, o.Y, o.Z);
-            for (auto& e : ph[p].elem) k::block_elem(s, e);
-            for (size_t i = 0; i < ph[p].gemm.size(); i += k::kGemmMulti)
-                k::gemm_multi(s, ph[p].gemm.data() + i,
-                              (int)std::min<size_t>(k::kGemmMulti, ph[p].gemm.size() - i));
-        }
-    }
-};
-}  // namespace
+}
 
 // The tables of a wide map.  With side, the powers that only the tree reads are
 // queued on side->stream (forked from s once pass 1's tables are queued; the
@@ -945,7 +926,7 @@ void ScanCore::wide_tables(hipStream_t s, const float* dA, const float* dB, cons
                            const float* dD, const float* dx0, bool withLast,
                            const SideStream* side)
 {
-    Phases ph;
+    BlockPhases ph;
     const int done = k::block_emit(blk_, bb_, h_, dA, dB, dC, dD, dx0, seed(),
                                    withLast ? L_ : L_ - 1, ph);
     ph.run(s, 0, done);

@@ -35,6 +35,25 @@ struct ScanOptions {
     int deltaLevels = 0;  // mixed: lowest levels applied as X + (P - I) X
 };
 
+// A wide map's operations, kept by phase (a phase's products are one launch).
+struct BlockPhases : k::BlockSink {
+    struct Phase {
+        std::vector<k::GemmOp> gemm;
+        std::vector<k::BlkElem> elem;
+        std::vector<k::SeqOp> seq;
+    };
+    std::vector<Phase> ph;
+    Phase& at(int p)
+    {
+        if ((int)ph.size() <= p) ph.resize(p + 1);
+        return ph[p];
+    }
+    void gemm(int p, const k::GemmOp& o) override { at(p).gemm.push_back(o); }
+    void elem(int p, const k::BlkElem& e) override { at(p).elem.push_back(e); }
+    void seq(int p, const k::SeqOp& o) override { at(p).seq.push_back(o); }
+    void run(hipStream_t s, int from, int to) const;
+};
+
 class ScanCore {
 public:
     // Buffers come from hipMalloc, or from `arena` when given (serving).

@@ -152,6 +152,7 @@ Server::Server(int lanes, size_t deviceBytes, size_t pinnedBytes, int precision)
         PARODE_HIP(hipStreamCreateWithFlags(&sd.stream, hipStreamNonBlocking));
         PARODE_HIP(hipEventCreateWithFlags(&sd.fork, hipEventDisableTiming));
         PARODE_HIP(hipEventCreateWithFlags(&sd.join, hipEventDisableTiming));
+        PARODE_HIP(hipEventCreateWithFlags(&sd.late, hipEventDisableTiming));
         fans_[l].create();
     }
     st_.arenaBytes = arena_->capacity();
@@ -170,6 +171,7 @@ Server::~Server()
     for (auto& sd : sides_) {
         if (sd.fork) (void)hipEventDestroy(sd.fork);
         if (sd.join) (void)hipEventDestroy(sd.join);
+        if (sd.late) (void)hipEventDestroy(sd.late);
         if (sd.stream) (void)hipStreamDestroy(sd.stream);
     }
     for (auto& f : fans_) f.destroy();
