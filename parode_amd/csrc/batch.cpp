@@ -75,7 +75,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
             if (c.blk_.wide) {
                 s.ready = k::block_emit(c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0, c.seed(),
                                         s.L - 1, s.ops);
-                upSteps = std::max(upSteps, k::block_tree_levels(nb));
+                upSteps = std::max(upSteps, k::block_tree_up_levels(nb));
                 blkSteps = std::max(blkSteps, s.ready);
                 blkRest = std::max(blkRest, (int)s.ops.ph.size() - s.ready);
             } else {
@@ -146,13 +146,13 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
                     for (auto& e : s.ops.ph[t].elem) k::g::add_block_elem(ph, e);
                     for (auto& o : s.ops.ph[t].gemm) k::g::add_gemm_op(ph, o);
                 }
-                const int top = k::block_tree_levels(nb);
-                for (int t = 0; t < top; ++t) {
+                const int top = k::block_tree_up_levels(nb);
+                for (int t = 0; t < top; ++t)
                     k::g::add_gemm_op(P[kUp0 + upSteps - (top - t)],
                                       k::block_tree_up(c.blk_, c.bb_, nb, t));
-                    k::g::add_gemm_op(P[kDown0 + top - 1 - t],
-                                      k::block_tree_down(c.blk_, c.bb_, nb, t));
-                }
+                for (int t = 0; t < k::block_tree_down_steps(c.blk_, nb); ++t)
+                    for (auto& o : k::block_tree_down(c.blk_, c.bb_, nb, t))
+                        k::g::add_gemm_op(P[kDown0 + t], o);
                 k::g::add_block_root(P[kTop], c.blk_, c.bb_, bin, nb, c.seed());
             } else {
                 k::g::add_block_map(P[kBlk0], c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0,

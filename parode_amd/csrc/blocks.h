@@ -41,6 +41,15 @@ struct BlockShape {
     int L = 0;                         // powers in PT
     int s = 0, taps = 0;
     bool wide = false;   // the map does not fit one work-group: made by products over many
+    // Where P_l lies in PT (in matrices).  Wide: from P_lb on the powers lie in
+    // threes, P_l^3, P_{l+1}, P_l (l - lb even): the factors of a radix-4 level
+    // of the tree, stacked.
+    int slot(int l) const
+    {
+        return !wide || l < lb ? l : lb + 3 * ((l - lb) / 2) + ((l - lb) & 1 ? 1 : 2);
+    }
+    int slots() const { return wide ? lb + 3 * ((L - lb) / 2 + 1) : L; }
+    bool radix4() const { return wide && na <= 256; }
     int kb() const { return s * T * m; }
     int kh() const { return (s * (T - 1) + taps) * m; }
 };
@@ -48,7 +57,8 @@ struct BlockShape {
 // Block responses of one system: tables and states carved by ScanCore.
 struct BlockBufs {
     double *PT = nullptr, *QT = nullptr, *OT = nullptr, *Ht = nullptr, *DL = nullptr;
-    double* Z = nullptr;    // [blocks + 1][na]: aggregates, then the blocks' start states
+    double* Z = nullptr;    // [blocks + 1][na]: aggregates
+    double* E = nullptr;    // the blocks' start states (Z's place unless wide)
     double* Z2 = nullptr;   // [groups + 1][na]: the same for groups of blocks (wide: for
                             // every level of the tree over the blocks)
     double* W = nullptr;    // wide: the map's intermediate products
@@ -74,9 +84,9 @@ enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit
 // Groups of blocks that the scan of nb blocks makes first (0: none).
 long block_groups(int na, long nb);
 
-// doubles in QT, OT, Ht and DL together; in Z2 for at most nb blocks; in W
+// doubles in QT, OT, Ht and DL together; in the states for at most nb blocks; in W
 size_t block_table_values(const BlockShape& s);
-size_t block_z2_values(const BlockShape& s, long nb);
+size_t block_state_values(const BlockShape& s, long nb);
 size_t block_scratch_values(const BlockShape& s);
 BlockBufs block_carve(const BlockShape& s, double* PT, double* tab, double* z, long nb, double* w);
 
@@ -108,15 +118,20 @@ struct BlockSink {
 };
 // Emits a wide map's operations.  Returns the phase before which pass 1's
 // table is not complete.  The powers up to P_last (P_0 .. P_{last}) are made;
-// those that pass 1's tables do not need come at the phases they can.
+// those that pass 1's tables do not need come at the phases they can.  ready, if
+// given, receives for each power the phase from which it can be read.
 int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A, const float* B,
                const float* C, const float* D, const float* x0, double* seed, int last,
-               BlockSink& sink);
-// The tree over the blocks' states of a wide map: up products (level k from 0),
-// then the seed, then down products from level top - 1 to 0.  Returns top.
-int block_tree_levels(long nb);
+               BlockSink& sink, std::vector<int>* ready = nullptr);
+// The tree over the blocks' states of a wide map: up products by pairs (level k
+// from 0, with the power lb + k), the root's seed, down products (step j from 0).
+int block_tree_up_levels(long nb);
+int block_tree_down_steps(const BlockShape& s, long nb);
 GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k);
-GemmOp block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int k);
+std::vector<GemmOp> block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int j);
+// the root and the down steps
+void block_tree_finish(hipStream_t st, const BlockShape& s, const BlockBufs& b,
+                       const BlockInput& in, long nb, const double* seed, double* tot = nullptr);
 void block_elem(hipStream_t st, const BlkElem& e);
 
 // M, G, the direct terms and (x0 given) the seed: x0, or with the ABM start-up

@@ -688,40 +688,50 @@ __device__ __forceinline__ void d_blk_split(const VBlock vb, const BlkPass& a, d
 // Many tiles: 64 x 64 tiles, four waves of 2 x 2 matrix-core tiles, K in slices
 // of 16 (first the states, then the window) staged in LDS and double buffered.
 constexpr int kPT = 64, kPK = 16;
-typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
-struct BlkTileLds {
+struct BlkStage {
     double A[2][kPT][kPK + 1];
-    double B[2][kPK][kPT + 1];
+    double B[2][kPK][kPT + 8];
+};
+template <int KS>
+struct BlkTileLds {
+    BlkStage stage[KS];
     int bad;
 };
 
-template <typename TU, bool OUT>
-__device__ __forceinline__ void d_blk_tile(const VBlock vb, const BlkPass& a, BlkTileLds& L)
+template <typename TU, bool OUT, int KS>
+__device__ __forceinline__ void d_blk_tile(const VBlock vb, const BlkPass& a, BlkTileLds<KS>& Ls)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, q4 = lane >> 4;
+    const int grp = KS > 1 ? (int)threadIdx.x >> 8 : 0;
+    BlkStage& L = Ls.stage[grp];
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, q4 = lane >> 4;
     const int wr = wave >> 1, wc = wave & 1;
     const long b0 = vb.y * kPT;
     const int j0 = (int)vb.x * kPT;
     const int ar = tid >> 2, ak = (tid & 3) * 4;     // A slice: row, first of four k
     const int bk = tid >> 4, bj = (tid & 15) * 4;    // B slice: k, first of four columns
-    const bool realA = b0 + ar < a.nb;
-    const long ab = realA ? b0 + ar : a.nb - 1;
+    // rows past nb repeat the last one (their products are not stored)
+    const long ab = b0 + ar < a.nb ? b0 + ar : a.nb - 1;
     const TU* u = static_cast<const TU*>(a.U) + ab * a.blockU;
-    const double* z = OUT ? a.Z + ab * a.na : nullptr;
-    int kl = realA ? win_len(a, ab) : 0;
-    int kEnd = a.ku, kMin = a.ku, stride = a.na;
+    const int kz = OUT ? a.kz : 0, zs = (kz + kPK - 1) / kPK;
+    int kl = win_len(a, ab), kEnd = a.ku, kMin = a.ku, stride = a.na;
+    // the thread's four columns (those past the last repeat it): their factors
+    // in BU at hb[q] + k stride, zero from k = kcol[q] on
     int kcol[4];
-    long hb[4];                                      // offset of the column's factors in BU
+    long hb[4];
+    const bool cols4 = j0 + bj + 4 <= a.cols;
+    const int c0 = cols4 ? j0 + bj : a.cols - 1;
+    bool run4 = cols4;                               // one run of four factors
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int col = j0 + bj + q;
-        kcol[q] = col < a.cols ? a.ku : 0;
-        hb[q] = col;
-        if (OUT && col < a.cols) {
+        const int col = j0 + bj + q < a.cols ? j0 + bj + q : a.cols - 1;
+        kcol[q] = a.ku;
+        hb[q] = col + (long)bk * stride;
+        if (OUT) {
             const int i = col / a.p;
             kcol[q] = (a.s * i + a.taps) * a.m;
-            hb[q] = (long)a.s * (a.T - 1 - i) * a.m * a.p + (col - i * a.p);
+            hb[q] = ((long)a.s * (a.T - 1 - i) * a.m + bk) * a.p + (col - i * a.p);
         }
+        run4 = run4 && hb[q] == hb[0] + q && kcol[q] == kcol[0];
     }
     if (OUT) {
         const int jl = j0 + kPT - 1 < a.cols ? j0 + kPT - 1 : a.cols - 1;
@@ -730,54 +740,59 @@ __device__ __forceinline__ void d_blk_tile(const VBlock vb, const BlkPass& a, Bl
         if (first_output(a, b0, j0)) kMin = 0;
         stride = a.p;
         kl = kl < kEnd ? kl : kEnd;   // (the last slice may reach past the tile's samples)
-        if (tid == 0) L.bad = 0;
+        if (threadIdx.x == 0) Ls.bad = 0;
     }
-    const int kz = OUT ? a.kz : 0, zs = (kz + kPK - 1) / kPK;
     const int slices = zs + (kEnd + kPK - 1) / kPK;
+    // window rows lie in a row of samples when four values never cross one
+    const bool wide4 = sizeof(TU) == 8 && (a.gm == 0 || (a.m & 3) == 0);
+    const double* z = OUT ? a.Z + ab * a.na + ak : nullptr;
+    const double* ot = OUT ? a.OT + (long)bk * a.cols : nullptr;
     bool nf = false;
     double ra[4], rb[4];
     auto load = [&](int sl) {
         if (OUT && sl < zs) {
-            const int k = sl * kPK + ak;
-            if (k + 4 <= kz) {
-                const double2u v0 = *reinterpret_cast<const double2u*>(z + k);
-                const double2u v1 = *reinterpret_cast<const double2u*>(z + k + 2);
-                ra[0] = v0.x;
-                ra[1] = v0.y;
-                ra[2] = v1.x;
-                ra[3] = v1.y;
+            const int k0 = sl * kPK;
+            const double* o = ot + (long)k0 * a.cols;
+            if (k0 + kPK <= kz) {
+                load4(z + k0, ra);
+                if (cols4) {
+                    load4(o + c0, rb);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        rb[q] = o[j0 + bj + q < a.cols ? j0 + bj + q : a.cols - 1];
+                }
             } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) ra[q] = k + q < kz ? z[k + q] : 0.0;
-            }
-            const int kk = sl * kPK + bk;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int col = j0 + bj + q;
-                rb[q] = (kk < kz && col < a.cols) ? a.OT[(long)kk * a.cols + col] : 0.0;
+                for (int q = 0; q < 4; ++q) {
+                    ra[q] = k0 + ak + q < kz ? z[k0 + q] : 0.0;
+                    rb[q] = k0 + bk < kz ? o[j0 + bj + q < a.cols ? j0 + bj + q : a.cols - 1] : 0.0;
+                }
             }
             return;
         }
-        const int k = (sl - zs) * kPK + ak;
-        if (sizeof(TU) == 8 && a.gm == 0 && k + 4 <= kl) {
-            const double2u v0 = *reinterpret_cast<const double2u*>(u + k);
-            const double2u v1 = *reinterpret_cast<const double2u*>(u + k + 2);
-            ra[0] = v0.x;
-            ra[1] = v0.y;
-            ra[2] = v1.x;
-            ra[3] = v1.y;
+        const int k0 = (sl - zs) * kPK, k = k0 + ak;
+        if (wide4 && k + 4 <= kl) {
+            load4(reinterpret_cast<const double*>(u) + win(a, k), ra);
         } else {
 #pragma unroll
             for (int q = 0; q < 4; ++q) ra[q] = k + q < kl ? (double)u[win(a, k + q)] : 0.0;
         }
-        if (OUT && k + 4 > kMin) {
+        const double* h = a.BU + (long)k0 * stride;
+        if (k0 + kPK <= kMin || (!OUT && k0 + kPK <= kEnd)) {   // every factor is there
+            if (run4) {
+                load4(h + hb[0], rb);
+            } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) nf = nf || not_finite(ra[q]);
+                for (int q = 0; q < 4; ++q) rb[q] = h[hb[q]];
+            }
+            return;
         }
-        const int kk = (sl - zs) * kPK + bk;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            rb[q] = kk < kcol[q] ? a.BU[hb[q] + (long)kk * stride] : 0.0;
+        for (int q = 0; q < 4; ++q) {
+            if (OUT) nf = nf || not_finite(ra[q]);
+            rb[q] = k0 + bk < kcol[q] ? h[hb[q]] : 0.0;
+        }
     };
     auto store = [&](int buf) {
 #pragma unroll
@@ -791,43 +806,75 @@ __device__ __forceinline__ void d_blk_tile(const VBlock vb, const BlkPass& a, Bl
     for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
         for (int tj = 0; tj < 2; ++tj) acc[ti][tj] = doublex4{0.0, 0.0, 0.0, 0.0};
-    load(0);
-    store(0);
+    // group g takes the slices g, g + KS, ...
+    const int rounds = (slices + KS - 1) / KS;
+    if (grp < slices) {
+        load(grp);
+        store(0);
+    }
     __syncthreads();
     int buf = 0;
-    for (int sl = 0; sl < slices; ++sl) {
-        const bool more = sl + 1 < slices;
-        if (more) load(sl + 1);
+    for (int t0 = 0; t0 < rounds; ++t0) {
+        const int sl = t0 * KS + grp;
+        const bool more = sl + KS < slices;
+        if (more) load(sl + KS);
+        if (sl < slices) {
 #pragma unroll
-        for (int ks = 0; ks < kPK; ks += 4) {
-            double x[2], y[2];
+            for (int ks = 0; ks < kPK; ks += 4) {
+                double x[2], y[2];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                x[t] = L.A[buf][wr * 32 + t * 16 + l16][ks + q4];
-                y[t] = L.B[buf][ks + q4][wc * 32 + t * 16 + l16];
+                for (int t = 0; t < 2; ++t) {
+                    x[t] = L.A[buf][wr * 32 + t * 16 + l16][ks + q4];
+                    y[t] = L.B[buf][ks + q4][wc * 32 + t * 16 + l16];
+                }
+#pragma unroll
+                for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                    for (int tj = 0; tj < 2; ++tj)
+                        acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[ti], y[tj],
+                                                                          acc[ti][tj], 0, 0, 0);
             }
-#pragma unroll
-            for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-                for (int tj = 0; tj < 2; ++tj)
-                    acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[ti], y[tj], acc[ti][tj],
-                                                                      0, 0, 0);
         }
         if (more) store(buf ^ 1);
         __syncthreads();
         buf ^= 1;
     }
     if (OUT) {
-        if (nf) L.bad = 1;
+        if (nf) Ls.bad = 1;
         __syncthreads();
-        if (L.bad) {
-            for (int t = tid; t < kPT * kPT; t += 256) {
+        if (Ls.bad) {
+            for (int t = threadIdx.x; t < kPT * kPT; t += 256 * KS) {
                 const long bb = b0 + t / kPT;
                 const int cc = j0 + t % kPT;
                 if (bb < a.nb && cc < a.cols)
                     blk_store(a, true, bb, cc, blk_output<TU>(a, bb, cc));
             }
             return;
+        }
+    }
+    if (KS > 1) {   // the groups' partial tiles, added in group order
+        if (grp > 0) {
+            double* part = &L.A[0][0][0];            // 16 values a thread
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        part[((ti * 2 + tj) * 4 + v) * 256 + tid] = acc[ti][tj][v];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 1; g < KS; ++g) {
+            const double* pg = &Ls.stage[g].A[0][0][0];
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[ti][tj][v] += pg[((ti * 2 + tj) * 4 + v) * 256 + tid];
         }
     }
 #pragma unroll
@@ -906,16 +953,16 @@ __global__ __launch_bounds__(NW * 64) void k_blk_split(const BlkPass a)
     d_blk_split<TU, OUT, NW>(blk_place(blockIdx.x, a.gx, a.gy), a, lds, &bad);
 }
 
-template <typename TU, bool OUT>
-__global__ __launch_bounds__(256) void k_blk_tile(const BlkPass a)
+template <typename TU, bool OUT, int KS>
+__global__ __launch_bounds__(256 * KS) void k_blk_tile(const BlkPass a)
 {
-    __shared__ BlkTileLds L;
-    static_assert(sizeof(BlkTileLds) >= kBN * kBP * sizeof(double), "room for the powers");
+    __shared__ BlkTileLds<KS> L;
+    static_assert(sizeof(BlkStage) >= kBN * kBP * sizeof(double), "room for the powers");
     if (!OUT && (long)blockIdx.x == a.gx * a.gy) {
-        d_blk_powers<4>(a.na, a.lb, a.L, a.PT, &L.A[0][0][0]);
+        d_blk_powers<4 * KS>(a.na, a.lb, a.L, a.PT, &L.stage[0].A[0][0][0]);
         return;
     }
-    d_blk_tile<TU, OUT>(blk_place(blockIdx.x, a.gx, a.gy), a, L);
+    d_blk_tile<TU, OUT, KS>(blk_place(blockIdx.x, a.gx, a.gy), a, L);
 }
 
 // ------------------------------------------------------------------ the scan
@@ -1120,16 +1167,18 @@ __global__ void k_blk_carry(const BlkScan a, long row0, long at, double* out)
 
 // wide maps: the tree's root takes the shifted seed (its response from zero goes
 // to tot), and the state after the blocks is P_L Z_0 plus that response
-__device__ __forceinline__ void d_blk_root(const BlkScan& a, double* root, double* tot)
+__device__ __forceinline__ void d_blk_root(const BlkScan& a, const double* S, double* E,
+                                           double* tot)
 {
     for (int i = threadIdx.x; i < a.na; i += blockDim.x) {
-        if (tot) tot[i] = root[i];
-        root[i] = a.seed[i] - blk_shift(a, 0, 0, i);
+        if (tot) tot[i] = S[i];
+        E[i] = a.seed[i] - blk_shift(a, 0, 0, i);
     }
 }
-__global__ __launch_bounds__(1024) void k_blk_root(const BlkScan a, double* root, double* tot)
+__global__ __launch_bounds__(1024) void k_blk_root(const BlkScan a, const double* S, double* E,
+                                                   double* tot)
 {
-    d_blk_root(a, root, tot);
+    d_blk_root(a, S, E, tot);
 }
 __global__ __launch_bounds__(256) void k_blk_carry_wide(const BlkScan a, const double* P,
                                                         const double* tot, long row0, long at,
@@ -1325,7 +1374,7 @@ int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long 
     // and outputs, levels
     const double step = method == 1 ? 8.0 * n * n : 4.0 * n * n;
     const double general = N * (step / 45e6 + (2.0 * n * m * (method == 1 ? 2 : 3) + 2.0 * p * (n + m)) / 15e6) +
-                           10.0 * std::log2(N);
+                           10.0 * std::log2(N) + (n <= 256 ? std::min(N / 512, 256.0) * 1.5 : N * step / 45e6);
     return bt < general ? best : 0;
 }
 
@@ -1356,17 +1405,64 @@ size_t block_table_values(const BlockShape& s)
            (size_t)s.kh() * s.p;
 }
 
-// (wide) rows of the tree's levels above the blocks, an even number each
-static long tree_rows(long n) { return (n + 1) / 2 * 2; }
-
-size_t block_z2_values(const BlockShape& s, long nb)
+// The tree over a wide map's blocks.  Up, level k + 1 holds the responses of
+// pairs of level k: a launch a level, beside which the next power's squaring
+// runs.  Down, a step takes the start states from level k to the two levels
+// below it at once (n_a <= 256: half the launches, whose products are shorter
+// than a launch; a step's third power costs n_a^3 and its second products
+// n_a^2, too much for wider maps) or to the one below.  A level's states are
+// padded to whole nodes of four.
+struct TreeLevel {
+    long n;        // states of the level
+    size_t s, e;   // responses and start states, in states from b.Z2 (level 0: b.Z, b.E)
+};
+static long tree_rows(long n) { return (n + 3) / 4 * 4; }
+static std::vector<TreeLevel> tree_of(long nb)
 {
-    long rows = 0;
-    if (s.wide)
-        for (long n = nb; n > 1; n = (n + 1) / 2) rows += tree_rows((n + 1) / 2);
-    else
-        rows = block_groups(s.na, nb) + 1;
-    return (size_t)(rows + 1) * s.na;
+    std::vector<TreeLevel> t;
+    size_t at = 0;
+    for (long n = nb;; n = (n + 1) / 2) {
+        const size_t rows = t.empty() ? 0 : (size_t)tree_rows(n);
+        t.push_back(TreeLevel{n, at, at + rows});
+        at += 2 * rows;
+        if (n <= 1) return t;
+    }
+}
+static double* tree_s(const BlockShape& s, const BlockBufs& b, const std::vector<TreeLevel>& t, int k)
+{
+    return k == 0 ? b.Z : b.Z2 + t[k].s * s.na;
+}
+static double* tree_e(const BlockShape& s, const BlockBufs& b, const std::vector<TreeLevel>& t, int k)
+{
+    return k == 0 ? b.E : b.Z2 + t[k].e * s.na;
+}
+int block_tree_up_levels(long nb) { return (int)tree_of(nb).size() - 1; }
+// the levels that the down steps go to, from the top
+static std::vector<int> tree_steps(const BlockShape& s, int top)
+{
+    std::vector<int> to;
+    // pairs of levels lie at even distances from level 0 (their powers' stacks)
+    for (int k = top; k > 0;) {
+        k -= s.radix4() && k % 2 == 0 ? 2 : 1;
+        to.push_back(k);
+    }
+    return to;
+}
+int block_tree_down_steps(const BlockShape& s, long nb)
+{
+    return (int)tree_steps(s, block_tree_up_levels(nb)).size();
+}
+
+// Z (and E): whole nodes and one state more; then Z2
+static size_t state_rows0(const BlockShape& s, long nb)
+{
+    return s.wide ? (size_t)tree_rows(nb) : (size_t)nb + 1;
+}
+size_t block_state_values(const BlockShape& s, long nb)
+{
+    if (!s.wide) return (state_rows0(s, nb) + block_groups(s.na, nb) + 1) * s.na;
+    const std::vector<TreeLevel> t = tree_of(nb);
+    return (2 * state_rows0(s, nb) + t.back().e + (nb > 1 ? 4 : 0)) * s.na;
 }
 
 size_t block_scratch_values(const BlockShape& s)
@@ -1385,7 +1481,8 @@ BlockBufs block_carve(const BlockShape& s, double* PT, double* tab, double* z, l
     b.Ht = b.OT + (size_t)s.T * s.p * s.na;
     b.DL = b.Ht + (size_t)s.kh() * s.p;
     b.Z = z;
-    b.Z2 = z + (size_t)(tree_rows(nb) + 1) * s.na;
+    b.E = s.wide ? z + state_rows0(s, nb) * s.na : z;
+    b.Z2 = b.E + state_rows0(s, nb) * s.na;
     b.W = w;
     return b;
 }
@@ -1405,7 +1502,7 @@ static bool structured_square(const BlockShape& s) { return s.method == 1 && s.n
 
 int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A, const float* B,
                const float* C, const float* D, const float* x0, double* seed, int last,
-               BlockSink& sink)
+               BlockSink& sink, std::vector<int>* readyAt)
 {
     const int n = s.n, m = s.m, p = s.p, na = s.na, sm = s.s * m, T = s.T;
     const size_t nn = (size_t)n * n, nm = (size_t)n * m;
@@ -1515,11 +1612,12 @@ int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A
     const bool st = structured_square(s);
     const int spp = st ? 4 : 1;
     int q = ready - 1;
-    for (int l = 0; l < last || l < s.lb; ++l) {
+    for (int l = 0; l <= last || l < s.lb; ++l) {
         const int ph = base + 1 + spp * l;   // P_l can be read
-        const double* P = b.PT + l * na2;
+        if (readyAt) readyAt->push_back(ph);
+        const double* P = b.PT + s.slot(l) * na2;
         if (l < last) {
-            double* P2 = b.PT + (l + 1) * na2;
+            double* P2 = b.PT + s.slot(l + 1) * na2;
             if (!st) {
                 sink.gemm(ph, GemmOp{na, na, na, P, P, P2, gemm_ld(na, na)});
             } else {
@@ -1534,6 +1632,10 @@ int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A
                 }
             }
         }
+        // the third power of a radix-4 level
+        if (s.radix4() && l > s.lb && ((l - s.lb) & 1))
+            sink.gemm(ph, GemmOp{na, na, na, P, b.PT + s.slot(l - 1) * na2,
+                                 b.PT + (s.slot(l - 1) - 2) * na2, gemm_ld(na, na)});
         if (l >= s.lb) continue;
         const int k = 1 << l;
         sink.gemm(ph, GemmOp{na, na, k * p, P, b.OT, b.OT + (long)k * p,
@@ -1551,48 +1653,44 @@ int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A
     return q + 1;
 }
 
-int block_tree_levels(long nb)
-{
-    int k = 0;
-    for (long n = nb; n > 1; n = (n + 1) / 2) ++k;
-    return k;
-}
-// the states of level k of the tree (level 0: the blocks) and their count
-static double* tree_level(const BlockShape& s, const BlockBufs& b, long nb, int k, long& count)
-{
-    double* at = b.Z;
-    double* next = b.Z2;
-    count = nb;
-    for (int i = 0; i < k; ++i) {
-        count = (count + 1) / 2;
-        at = next;
-        next += tree_rows(count) * s.na;
-    }
-    return at;
-}
+// S'[i] = S[2i] P + S[2i + 1] (a last state without a pair is no other's left
+// neighbour: not formed)
 GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k)
 {
-    long c0, c1;
-    double* S0 = tree_level(s, b, nb, k, c0);
-    double* S1 = tree_level(s, b, nb, k + 1, c1);
+    const std::vector<TreeLevel> t = tree_of(nb);
     const int na = s.na;
+    double* S = tree_s(s, b, t, k);
     GemmLd ld{2 * na, na, na};
-    ld.add = S0 + na;
+    ld.add = S + na;
     ld.lda = 2 * na;
-    return GemmOp{(int)(c0 / 2), na, na, S0, b.PT + (size_t)(s.lb + k) * na * na, S1, ld};
+    return GemmOp{(int)(t[k].n / 2), na, na, S, b.PT + (size_t)s.slot(s.lb + k) * na * na,
+                  tree_s(s, b, t, k + 1), ld};
 }
-// in place: E[2i] over S[2i], which is first added to E[2i + 1]
-GemmOp block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int k)
+// E[R i] = E'[i], E[R i + j] = E'[i] P^j + sum_{q < j} S[R i + q] P^(j-1-q), R = 2 or 4
+std::vector<GemmOp> block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int j0)
 {
-    long c0, c1;
-    double* S0 = tree_level(s, b, nb, k, c0);
-    double* E1 = tree_level(s, b, nb, k + 1, c1);
-    const int na = s.na;
-    GemmLd ld{na, na, 2 * na};
-    ld.add = S0;
-    ld.lda = 2 * na;
-    ld.cp = S0;
-    return GemmOp{(int)c1, na, na, E1, b.PT + (size_t)(s.lb + k) * na * na, S0 + na, ld};
+    const std::vector<TreeLevel> t = tree_of(nb);
+    const int na = s.na, top = (int)t.size() - 1;
+    const std::vector<int> to = tree_steps(s, top);
+    const int from = j0 == 0 ? top : to[j0 - 1], k = to[j0], R = 1 << (from - k);
+    const double* S = tree_s(s, b, t, k);
+    double* E = tree_e(s, b, t, k);
+    std::vector<GemmOp> ops;
+    for (int j = 1; j < R; ++j) {
+        GemmLd ld{na, na, R * na};
+        ld.add = S + (j - 1) * na;
+        ld.lda = R * na;
+        if (j == 1) {
+            ld.cp = E;
+        } else {
+            ld.X2 = S;
+            ld.ldx2 = R * na;
+            ld.k1 = na;
+        }
+        ops.push_back(GemmOp{(int)t[from].n, j * na, na, tree_e(s, b, t, from),
+                             b.PT + (size_t)(s.slot(s.lb + k) - (j - 1)) * na * na, E + j * na, ld});
+    }
+    return ops;
 }
 
 // One work-group scans up to 512 blocks; more go in groups of 16 (or as many
@@ -1686,15 +1784,17 @@ static BlkPass pass_args(const BlockShape& s, const BlockBufs& b, const BlockInp
     return a;
 }
 
-// The tiling of a pass over one system: 64 x 64 tiles once they give every
-// compute unit one; 16 x 16 below, their K over 16 waves while those tiles are
-// few too.  In a grouped launch (grouped) the other systems fill the GPU, so
-// the 64 x 64 tiles' higher rate counts from fewer of them.
+// The tiling of a pass over one system: 64 x 64 tiles from 64 of them (50 001
+// points, n_a = 37: 135 us a solve against 169 when they start at 16; 16 x 16
+// from 256 tiles on: 20 us more at n_a = 48, 2^18 points), 16 x 16 below, their K
+// over 16 waves while those tiles are few too.  In a grouped launch the other
+// systems fill the GPU and the wide tiles' higher rate counts from fewer of
+// them (512 systems: 45.3 ms from 16 tiles, 48.0 from 64).
 static int pass_tiling(const BlkPass& a, bool out, bool grouped)
 {
     const long tx = (a.cols + kPT - 1) / kPT, ty = (a.nb + kPT - 1) / kPT;
     const long sx = (a.cols + 15) / 16, sy = (a.nb + 15) / 16;
-    if (tx * ty >= (grouped ? 24 : 256)) return kBlockTile;
+    if (tx * ty >= (grouped ? 16 : 64)) return kBlockTile;
     return sx * sy <= 256 && ((out ? a.kz : 0) + a.ku) / 4 >= 64 ? kBlockSplit16 : kBlockSplit4;
 }
 static void pass_grid(BlkPass& a, int tiling)
@@ -1714,8 +1814,12 @@ static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, in
     const bool tile = tiling == kBlockTile, wide = tiling == kBlockSplit16;
 #define PARODE_PASS(TU)                                                                   \
     do {                                                                                  \
-        if (tile)                                                                         \
-            hipLaunchKernelGGL((k_blk_tile<TU, OUT>), grid, dim3(256), 0, st, a);         \
+        if (tile && a.gx * a.gy <= 384)                                                   \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 4>), grid, dim3(1024), 0, st, a);     \
+        else if (tile && a.gx * a.gy <= 768)                                              \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 2>), grid, dim3(512), 0, st, a);      \
+        else if (tile)                                                                    \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 1>), grid, dim3(256), 0, st, a);      \
         else if (wide)                                                                    \
             hipLaunchKernelGGL((k_blk_split<TU, OUT, 16>), grid, dim3(1024), 0, st, a);   \
         else                                                                              \
@@ -1747,7 +1851,7 @@ static BlkPass pass2_args(const BlockShape& s, const BlockBufs& b, const BlockIn
     a.kz = s.na;
     a.ku = s.kh();
     a.nReal = nReal;
-    a.Z = b.Z;
+    a.Z = b.E;
     a.OT = b.OT;
     a.BU = b.Ht;
     a.Y = Y;
@@ -1822,24 +1926,29 @@ static bool scan_plan(BlkScan a0, const BlockBufs& b, BlkScan& u, BlkScan& a, Bl
     return lg > 0;
 }
 
+void block_tree_finish(hipStream_t st, const BlockShape& s, const BlockBufs& b,
+                       const BlockInput& in, long nb, const double* seed, double* tot)
+{
+    const std::vector<TreeLevel> t = tree_of(nb);
+    const int top = (int)t.size() - 1;
+    hipLaunchKernelGGL(k_blk_root, dim3(1), dim3(1024), 0, st, scan_args(s, b, in, nb, seed),
+                       tree_s(s, b, t, top), tree_e(s, b, t, top), tot);
+    check_launch("block root");
+    for (int j = 0; j < block_tree_down_steps(s, nb); ++j) {
+        const std::vector<GemmOp> ops = block_tree_down(s, b, nb, j);
+        gemm_multi(st, ops.data(), (int)ops.size());
+    }
+}
+
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                 long nb, const double* seed, double* tot)
 {
     if (s.wide) {
-        const int top = block_tree_levels(nb);
-        for (int k = 0; k < top; ++k) {
+        for (int k = 0; k < block_tree_up_levels(nb); ++k) {
             const GemmOp op = block_tree_up(s, b, nb, k);
             gemm_multi(st, &op, 1);
         }
-        long one;
-        double* root = tree_level(s, b, nb, top, one);
-        hipLaunchKernelGGL(k_blk_root, dim3(1), dim3(1024), 0, st, scan_args(s, b, in, nb, seed),
-                           root, tot);
-        check_launch("block root");
-        for (int k = top - 1; k >= 0; --k) {
-            const GemmOp op = block_tree_down(s, b, nb, k);
-            gemm_multi(st, &op, 1);
-        }
+        block_tree_finish(st, s, b, in, nb, seed, tot);
         return;
     }
     BlkScan u, a, d;
@@ -1867,7 +1976,7 @@ void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
     if (s.wide) {   // (nb is a power of two here)
         hipLaunchKernelGGL(k_blk_carry_wide, dim3((s.na + 255) / 256), dim3(256),
                            s.na * sizeof(double), st, a,
-                           b.PT + (size_t)(s.lb + block_tree_levels(nb)) * s.na * s.na, tot,
+                           b.PT + (size_t)s.slot(s.lb + block_tree_up_levels(nb)) * s.na * s.na, tot,
                            nb * s.s * s.T, nb * s.T * in.sL * s.m, seedOut);
         check_launch("block carry");
         return;
@@ -1891,7 +2000,8 @@ struct StartOutB {
 };
 struct RootB {
     BlkScan a;
-    double* root;
+    const double* S;
+    double* E;
     long gx;
 };
 
@@ -1944,15 +2054,15 @@ template <bool OUT>
 __global__ __launch_bounds__(256) void kg_blk_tile(const BlkPass* __restrict__ args,
                                                    const unsigned* __restrict__ st, int ns)
 {
-    __shared__ BlkTileLds L;
+    __shared__ BlkTileLds<1> L;
     const int sys = system_of(st, ns);
     const BlkPass& a = args[sys];
     const long idx = (long)blockIdx.x - (long)st[sys];
     if (!OUT && idx == a.gx * a.gy) {
-        d_blk_powers<4>(a.na, a.lb, a.L, a.PT, &L.A[0][0][0]);
+        d_blk_powers<4>(a.na, a.lb, a.L, a.PT, &L.stage[0].A[0][0][0]);
         return;
     }
-    d_blk_tile<double, OUT>(blk_place(idx, a.gx, a.gy), a, L);
+    d_blk_tile<double, OUT, 1>(blk_place(idx, a.gx, a.gy), a, L);
 }
 template <int MODE>
 __global__ __launch_bounds__(MODE == kScanAll ? 1024 : 256) void kg_blk_scan(
@@ -1967,7 +2077,7 @@ __global__ __launch_bounds__(256) void kg_blk_root(const RootB* __restrict__ arg
 {
     PARODE_GROUP(RootB);
     (void)vb;
-    d_blk_root(a.a, a.root, nullptr);
+    d_blk_root(a.a, a.S, a.E, nullptr);
 }
 
 void add_pass(Phase& ph, BlkPass a, bool out, bool powers)
@@ -2027,9 +2137,10 @@ void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, con
 void add_block_root(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                     long nb, const double* seed)
 {
-    long one;
-    double* root = tree_level(s, b, nb, block_tree_levels(nb), one);
-    append(ph, kBlkRoot, false, RootB{scan_args(s, b, in, nb, seed), root, 1}, 1, 0, (float)s.na);
+    const std::vector<TreeLevel> t = tree_of(nb);
+    const int top = (int)t.size() - 1;
+    append(ph, kBlkRoot, false, RootB{scan_args(s, b, in, nb, seed), tree_s(s, b, t, top),
+                                      tree_e(s, b, t, top), 1}, 1, 0, (float)s.na);
 }
 
 bool run_blocks(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dStart)

@@ -49,6 +49,9 @@ struct GemmLd {
     double* cp = nullptr;
     int zp = 0;
     long zs = 0;
+    // X's columns from k1 on are those of X2 (leading dimension ldx2), if not null
+    const double* X2 = nullptr;
+    int ldx2 = 0, k1 = 0;
 };
 __host__ __device__ inline GemmLd gemm_ld(int kk, int c) { return GemmLd{kk, c, c}; }
 struct GemmOp {

@@ -174,12 +174,11 @@ __device__ __forceinline__ void d_gemm_f64_ks(const VBlock vb, int r, int kk, in
                                                               const double* __restrict__ X,
                                                               const double* __restrict__ Y,
                                                               double* __restrict__ Z,
-                                                              const GemmLd ld)
+                                                              const GemmLd ld, double* gsm)
 {
     constexpr int T = kGemmKsT, KB = kGemmKsKB, AP = KB + 1, BP = T + 1, NT = 256 * KSPLIT;
     constexpr int PA = T * KB / NT, PB = KB * T / NT;
     static_assert(PA >= 1 && PB >= 1 && 4 * KSPLIT <= KB, "tile, slice and split");
-    extern __shared__ double gsm[];
     double* As = gsm;                      // [T][AP]
     double* Bs = gsm + T * AP;             // [KB][BP]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -188,12 +187,15 @@ __device__ __forceinline__ void d_gemm_f64_ks(const VBlock vb, int r, int kk, in
     const int i0 = vb.y * T, j0 = vb.x * T;
     const int ar = tid / (KB / PA), ak = (tid % (KB / PA)) * PA;
     const int bk = tid / (T / PB), bj = (tid % (T / PB)) * PB;
+    const int k1 = ld.X2 ? ld.k1 : kk;     // X2's first k
     double ra[PA], rb[PB];
     auto load = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < PA; ++q) {
             const int gi = i0 + ar, gk = k0 + ak + q;
-            ra[q] = (gi < r && gk < kk) ? X[(long)gi * ld.ldx + gk] : 0.0;
+            ra[q] = (gi < r && gk < kk) ? (gk < k1 ? X[(long)gi * ld.ldx + gk]
+                                                   : ld.X2[(long)gi * ld.ldx2 + gk - k1])
+                                        : 0.0;
         }
 #pragma unroll
         for (int q = 0; q < PB; ++q) {
@@ -243,8 +245,9 @@ __global__ __launch_bounds__(256 * KSPLIT) void k_gemm_f64_ks(int r, int kk, int
                                                               const double* __restrict__ Y,
                                                               double* __restrict__ Z)
 {
+    extern __shared__ double gsm[];
     d_gemm_f64_ks<KSPLIT>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, r, kk, c, X, Y, Z,
-                          gemm_ld(kk, c));
+                          gemm_ld(kk, c), gsm);
 }
 
 // FP64 GEMM on 64 x 64 tiles of Z for the squarings of the power tables: four
@@ -252,7 +255,10 @@ __global__ __launch_bounds__(256 * KSPLIT) void k_gemm_f64_ks(int r, int kk, int
 // independent accumulators, each operand fragment used twice), K in slices of
 // 16 staged in LDS (odd pitches), double buffered: the next slice's loads are
 // in flight while the current one is multiplied, one barrier per slice.  Twice
-// the arithmetic per byte of operands of the 32 x 32 tiles.
+// the arithmetic per byte of operands of the 32 x 32 tiles.  With KS > 1, KS
+// groups of four waves share the tile's K: a compute unit with one work-group
+// of four waves waits on every slice's barrier and loads (10 of the 50 TFLOP/s
+// of four work-groups per unit at K = 1024).
 constexpr int kG64 = 64, kG64KB = 16;
 
 // 64 x 64 tiles once the padding of the edge tiles costs less than the 16 x 16
@@ -262,26 +268,55 @@ __host__ __device__ constexpr bool gemm_wide(int r, int kk, int c)
     return r >= 96 && c >= 96 && kk >= 64;
 }
 
+struct GemmStage {   // (pitches: operand reads of a wave fall in distinct banks)
+    double A[2][kG64][kG64KB + 1];
+    double B[2][kG64KB][kG64 + 8];
+};
+
+template <int KS>
 __device__ __forceinline__ void d_gemm_f64_t64(const VBlock vb, int r, int kk, int c,
                                                const double* __restrict__ X,
                                                const double* __restrict__ Y,
-                                               double* __restrict__ Z, const GemmLd ld)
+                                               double* __restrict__ Z, const GemmLd ld, double* lds)
 {
-    __shared__ double As[2][kG64][kG64KB + 1];
-    __shared__ double Bs[2][kG64KB][kG64 + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    GemmStage* stage = reinterpret_cast<GemmStage*>(lds);   // KS of them
+    const int grp = KS > 1 ? (int)threadIdx.x >> 8 : 0;
+    double(*As)[kG64][kG64KB + 1] = stage[grp].A;
+    double(*Bs)[kG64KB][kG64 + 8] = stage[grp].B;
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
     const int wr = wave >> 1, wc = wave & 1, l16 = lane & 15, q4 = lane >> 4;
     const int i0 = (int)vb.y * kG64, j0 = (int)vb.x * kG64;
     const int ar = tid >> 2, ak = (tid & 3) * 4;     // A slice: row, first of four k
     const int bk = tid >> 4, bj = (tid & 15) * 4;    // B slice: k, first of four columns
+    // rows past r repeat the last one (their products are not stored), and so
+    // do the columns of a thread whose four run past c
+    const double* xr = X + (long)(i0 + ar < r ? i0 + ar : r - 1) * ld.ldx + ak;
+    const bool cols4 = j0 + bj + 4 <= c;
+    const double* yr = Y + (long)bk * ld.ldy + (cols4 ? j0 + bj : 0);
+    int yc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) yc[q] = j0 + bj + q < c ? j0 + bj + q : c - 1;
+    const double* xr2 = ld.X2 ? ld.X2 + (long)(i0 + ar < r ? i0 + ar : r - 1) * ld.ldx2 - ld.k1 + ak
+                              : xr;
+    const int k1 = ld.X2 ? ld.k1 : kk;               // X2's first k
     double ra[4], rb[4];
     auto load = [&](int k0) {
+        const bool run = k0 + ak + 4 <= k1 || k0 + ak >= k1;   // four values of one operand
+        if (k0 + kG64KB <= kk && run) {              // a whole slice: 16-byte loads
+            load4((k0 + ak < k1 ? xr : xr2) + k0, ra);
+            const double* y = yr + (long)k0 * ld.ldy;
+            if (cols4) {
+                load4(y, rb);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) rb[q] = y[yc[q]];
+            }
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int gi = i0 + ar, gk = k0 + ak + q;
-            ra[q] = (gi < r && gk < kk) ? X[(long)gi * ld.ldx + gk] : 0.0;
-            const int gk2 = k0 + bk, gj = j0 + bj + q;
-            rb[q] = (gk2 < kk && gj < c) ? Y[(long)gk2 * ld.ldy + gj] : 0.0;
+            ra[q] = k0 + ak + q < kk ? (k0 + ak + q < k1 ? xr : xr2)[k0 + q] : 0.0;
+            rb[q] = k0 + bk < kk ? Y[(long)(k0 + bk) * ld.ldy + yc[q]] : 0.0;
         }
     };
     auto store = [&](int buf) {
@@ -296,31 +331,63 @@ __device__ __forceinline__ void d_gemm_f64_t64(const VBlock vb, int r, int kk, i
     for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
         for (int tj = 0; tj < 2; ++tj) acc[ti][tj] = doublex4{0.0, 0.0, 0.0, 0.0};
-    load(0);
-    store(0);
+    // group g takes the slices g, g + KS, ...
+    const int slices = (kk + kG64KB - 1) / kG64KB, rounds = (slices + KS - 1) / KS;
+    if (grp < slices) {
+        load(grp * kG64KB);
+        store(0);
+    }
     __syncthreads();
     int buf = 0;
-    for (int k0 = 0; k0 < kk; k0 += kG64KB) {
-        const bool more = k0 + kG64KB < kk;
-        if (more) load(k0 + kG64KB);
+    for (int t0 = 0; t0 < rounds; ++t0) {
+        const int sl = t0 * KS + grp;
+        const bool more = sl + KS < slices;
+        if (more) load((sl + KS) * kG64KB);
+        if (sl < slices) {
 #pragma unroll
-        for (int ks = 0; ks < kG64KB; ks += 4) {
-            double a[2], b[2];
+            for (int ks = 0; ks < kG64KB; ks += 4) {
+                double a[2], b[2];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                a[t] = As[buf][wr * 32 + t * 16 + l16][ks + q4];
-                b[t] = Bs[buf][ks + q4][wc * 32 + t * 16 + l16];
+                for (int t = 0; t < 2; ++t) {
+                    a[t] = As[buf][wr * 32 + t * 16 + l16][ks + q4];
+                    b[t] = Bs[buf][ks + q4][wc * 32 + t * 16 + l16];
+                }
+#pragma unroll
+                for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                    for (int tj = 0; tj < 2; ++tj)
+                        acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ti], b[tj],
+                                                                          acc[ti][tj], 0, 0, 0);
             }
-#pragma unroll
-            for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-                for (int tj = 0; tj < 2; ++tj)
-                    acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ti], b[tj], acc[ti][tj],
-                                                                      0, 0, 0);
         }
         if (more) store(buf ^ 1);
         __syncthreads();
         buf ^= 1;
+    }
+    if (KS > 1) {   // the groups' partial tiles, added in group order
+        double* part = &stage[grp].A[0][0][0];   // 16 values a thread
+        if (grp > 0) {
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        part[((ti * 2 + tj) * 4 + v) * 256 + tid] = acc[ti][tj][v];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 1; g < KS; ++g) {
+            const double* pg = &stage[g].A[0][0][0];
+#pragma unroll
+            for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[ti][tj][v] += pg[((ti * 2 + tj) * 4 + v) * 256 + tid];
+        }
     }
     // D[i][j] is in lane j + 16 (i % 4), register i / 4
 #pragma unroll
@@ -367,28 +434,32 @@ void gemm_f64(hipStream_t s, int r, int kk, int c, const double* X, const double
 // four partial tiles are summed through LDS.  Operands come from L2 (the
 // matrices are at most a few MiB).
 
+template <int NW>
 __device__ __forceinline__ void d_gemm_f64_mfma(const VBlock vb, int r, int kk, int c,
                                                        const double* __restrict__ X,
                                                        const double* __restrict__ Y,
-                                                       double* __restrict__ Z, const GemmLd ld)
+                                                       double* __restrict__ Z, const GemmLd ld, double* lds)
 {
-    __shared__ double part[3][4][64];
+    double(*part)[4][64] = reinterpret_cast<double(*)[4][64]>(lds);   // NW - 1 of them
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l16 = lane & 15, q4 = lane >> 4;
     const int i0 = vb.y * 16, j0 = vb.x * 16;
     const int ksteps = (kk + 3) / 4;
-    const int per = (ksteps + 3) / 4;
+    const int per = (ksteps + NW - 1) / NW;
     const int kb = wave * per, ke = (kb + per) < ksteps ? kb + per : ksteps;
     const int ia = i0 + l16, jb = j0 + l16;
+    const int k1 = ld.X2 ? ld.k1 : kk;               // X2's first k
     doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-    constexpr int U = 16;
+    constexpr int U = NW > 4 ? 8 : 16;
     for (int k = kb; k < ke; k += U) {
         double a[U], b[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int kx = (k + u) * 4 + q4;
             const bool ok = k + u < ke && kx < kk;
-            a[u] = (ok && ia < r) ? X[(long)ia * ld.ldx + kx] : 0.0;
+            a[u] = (ok && ia < r) ? (kx < k1 ? X[(long)ia * ld.ldx + kx]
+                                             : ld.X2[(long)ia * ld.ldx2 + kx - k1])
+                                  : 0.0;
             b[u] = (ok && jb < c) ? Y[(long)kx * ld.ldy + jb] : 0.0;
         }
 #pragma unroll
@@ -403,7 +474,9 @@ __device__ __forceinline__ void d_gemm_f64_mfma(const VBlock vb, int r, int kk, 
         // v_mfma_f64_16x16x4_f64 returns D[i][j] in lane j + 16 (i % 4), register i / 4
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const double sum = acc[v] + part[0][v][lane] + part[1][v][lane] + part[2][v][lane];
+            double sum = acc[v];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) sum += part[w - 1][v][lane];
             const int i = i0 + 4 * v + q4, j = j0 + l16;
             if (i < r && j < c) gemm_put(ld, X, Z, i, j, sum);
         }
@@ -415,16 +488,112 @@ __global__ __launch_bounds__(256) void k_gemm_f64_mfma(int r, int kk, int c,
                                                        const double* __restrict__ Y,
                                                        double* __restrict__ Z)
 {
-    d_gemm_f64_mfma(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, r, kk, c, X, Y, Z,
-                    gemm_ld(kk, c));
+    __shared__ double lds[3 * 256];
+    d_gemm_f64_mfma<4>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, r, kk, c, X, Y,
+                       Z, gemm_ld(kk, c), lds);
 }
 
-// The tiling of a product: 64 x 64 tiles where they are many (from 96 of them;
-// a product of fewer keeps more compute units busy as 16 x 16 tiles whose K is
-// split over four waves).
-__host__ __device__ inline bool gemm_tiles64(int r, int kk, int c)
+// FP64 GEMM for products of few tiles: a work-group of NW waves owns one 32 x 32
+// tile of Z, each wave all of it (2 x 2 matrix-core tiles) over its own part of
+// K, operands straight from the caches: no wave waits for another before the
+// partial tiles meet in LDS.  A lane takes two neighbouring k of a block of
+// eight (16-byte loads of X; X and Y agree on the order).  812 x 812 x 203: 11
+// against 21 us with slices staged in LDS.
+template <int NW, int U>
+__device__ __forceinline__ void d_gemm_f64_w32(const VBlock vb, int r, int kk, int c,
+                                               const double* __restrict__ X,
+                                               const double* __restrict__ Y,
+                                               double* __restrict__ Z, const GemmLd ld,
+                                               double* lds)
 {
-    return gemm_wide(r, kk, c) && (long)((r + 63) / 64) * ((c + 63) / 64) >= 96;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
+    const int i0 = (int)vb.y * 32, j0 = (int)vb.x * 32;
+    const int kblocks = (kk + 7) / 8, per = (kblocks + NW - 1) / NW;
+    const int kb = wave * per, ke = kb + per < kblocks ? kb + per : kblocks;
+    const int k1 = ld.X2 ? ld.k1 : kk;               // X2's first k
+    // rows past r and columns past c repeat the last one
+    const double *xr[2], *x2[2];
+    int yc[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int i = i0 + 16 * t + l16 < r ? i0 + 16 * t + l16 : r - 1;
+        xr[t] = X + (long)i * ld.ldx;
+        x2[t] = ld.X2 ? ld.X2 + (long)i * ld.ldx2 - k1 : xr[t];
+        yc[t] = j0 + 16 * t + l16 < c ? j0 + 16 * t + l16 : c - 1;
+    }
+    doublex4 acc[2][2];
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj) acc[ti][tj] = doublex4{0.0, 0.0, 0.0, 0.0};
+    for (int b = kb; b < ke; b += U) {
+        double x[U][2][2], y[U][2][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = (b + u) * 8 + 2 * q4;
+            // a block of eight k of one operand, all in range
+            const bool whole = b + u < ke && (b + u) * 8 + 8 <= kk &&
+                               ((b + u) * 8 + 8 <= k1 || (b + u) * 8 >= k1);
+            if (whole) {
+                const bool first = (b + u) * 8 < k1;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const double2u v = *reinterpret_cast<const double2u*>((first ? xr[t] : x2[t]) + k);
+                    x[u][t][0] = v.x;
+                    x[u][t][1] = v.y;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) y[u][t][h] = Y[(long)(k + h) * ld.ldy + yc[t]];
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bool in = b + u < ke && k + h < kk;
+                        x[u][t][h] = in ? (k + h < k1 ? xr[t] : x2[t])[k + h] : 0.0;
+                        y[u][t][h] = in ? Y[(long)(k + h) * ld.ldy + yc[t]] : 0.0;
+                    }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+                    for (int tj = 0; tj < 2; ++tj)
+                        acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            x[u][ti][h], y[u][tj][h], acc[ti][tj], 0, 0, 0);
+    }
+    // D[i][j] is in lane j + 16 (i % 4), register i / 4; a value's NW parts are
+    // added in wave order, each by one thread
+#pragma unroll
+    for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < 2; ++tj)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                lds[wave * 1024 + (16 * ti + 4 * v + q4) * 32 + 16 * tj + l16] = acc[ti][tj][v];
+    __syncthreads();
+    for (int t = threadIdx.x; t < 1024; t += 64 * NW) {
+        double v = lds[t];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += lds[w * 1024 + t];
+        const int i = i0 + t / 32, j = j0 + t % 32;
+        if (i < r && j < c) gemm_put(ld, X, Z, i, j, v);
+    }
+}
+
+// The tiling of a product launched alone: 64 x 64 tiles where they give nearly
+// every compute unit one (4096 x 256 x 256: 17 us against 19 in tiles of 32; 812^3,
+// 169 tiles: 45 against 35), 16 x 16 where those are at most one for each
+// (256^3: 5.2 against 5.7; 128 x 812 x 812, 408 tiles: 17.7 against 13.4).
+__host__ __device__ inline int gemm_tile(int r, int kk, int c)
+{
+    const long t64 = (long)((r + 63) / 64) * ((c + 63) / 64);
+    const long t16 = (long)((r + 15) / 16) * ((c + 15) / 16);
+    return gemm_wide(r, kk, c) && t64 >= 224 ? 64 : t16 <= 256 ? 16 : 32;
 }
 struct GemmMulti {
     unsigned start[kGemmMulti + 1];
@@ -432,37 +601,56 @@ struct GemmMulti {
     GemmOp op[kGemmMulti];
 };
 
-__global__ __launch_bounds__(256) void k_gemm_multi(const GemmMulti a)
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemm_multi(const GemmMulti a)
 {
+    constexpr int kStage = NW <= 8 ? NW / 4 * (int)(sizeof(GemmStage) / sizeof(double)) : 0;
+    __shared__ double lds[kStage > NW * 1024 ? kStage : NW * 1024];
     int q = 0;
     while (q + 1 < a.count && blockIdx.x >= a.start[q + 1]) ++q;
     const GemmOp& o = a.op[q];
     const long lb = (long)blockIdx.x - a.start[q];
-    if (gemm_tiles64(o.r, o.kk, o.c)) {
-        const long gx = (o.c + 63) / 64;
-        d_gemm_f64_t64(VBlock{lb % gx, lb / gx, gx}, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld);
-    } else {
-        const long gx = (o.c + 15) / 16;
-        d_gemm_f64_mfma(VBlock{lb % gx, lb / gx, gx}, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld);
-    }
+    const int t = gemm_tile(o.r, o.kk, o.c);
+    const long gx = (o.c + t - 1) / t;
+    const VBlock vb{lb % gx, lb / gx, gx};
+    if (t == 32)
+        d_gemm_f64_w32<NW, NW == 16 ? 1 : 2>(vb, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld, lds);
+    else if (t == 16)
+        d_gemm_f64_mfma<NW>(vb, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld, lds);
+    else if constexpr (NW <= 8)
+        d_gemm_f64_t64<NW / 4>(vb, o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld, lds);
 }
 
 void gemm_multi(hipStream_t s, const GemmOp* ops, int count)
 {
     GemmMulti a{};
     if (count > kGemmMulti) throw std::invalid_argument("gemm_multi: too many products");
+    int deep = 0, most = 0;   // the longest K, the widest tile
     for (int q = 0; q < count; ++q) {
         const GemmOp& o = ops[q];
         if (o.r <= 0 || o.c <= 0) continue;
-        const int t = gemm_tiles64(o.r, o.kk, o.c) ? 64 : 16;
+        const int t = gemm_tile(o.r, o.kk, o.c);
         const unsigned long n = (unsigned long)((o.r + t - 1) / t) * ((o.c + t - 1) / t);
         if (a.start[a.count] + n > 0x7fffffffUL) throw std::length_error("gemm_multi: too many tiles");
         a.op[a.count] = o;
         a.start[a.count + 1] = a.start[a.count] + (unsigned)n;
         ++a.count;
+        deep = std::max(deep, o.kk);
+        most = std::max(most, t);
     }
     if (a.count == 0) return;
-    hipLaunchKernelGGL(k_gemm_multi, dim3(a.start[a.count]), dim3(256), 0, s, a);
+    // Waves per tile: 16 on a compute unit (16 to a tile hold 128 KB of LDS, so
+    // one tile to a unit: 812 x 812 x 203, 182 tiles, 14 us against 16 with 8;
+    // 2048 x 256 x 256, 512 tiles, 11.1 against 10.7; 1024 tiles 23 and 19
+    // against 19 with 4).  Tiles of 16 alone have too short a K for 16 waves
+    // below 512.
+    const unsigned tiles = a.start[a.count];
+    if (most != 64 && tiles <= 256 && (most == 32 || deep >= 512))
+        hipLaunchKernelGGL(k_gemm_multi<16>, dim3(tiles), dim3(1024), 0, s, a);
+    else if (most != 16 && tiles <= (most == 64 ? 768 : 512))
+        hipLaunchKernelGGL(k_gemm_multi<8>, dim3(tiles), dim3(512), 0, s, a);
+    else
+        hipLaunchKernelGGL(k_gemm_multi<4>, dim3(tiles), dim3(256), 0, s, a);
     check_launch("gemm_multi");
 }
 
@@ -4177,17 +4365,19 @@ __global__ __launch_bounds__(256) void kg_gemm(const Gemm* __restrict__ args,
                                                const unsigned* __restrict__ st, int ns)
 {
     PARODE_GROUP(Gemm);
+    __shared__ double lds[sizeof(GemmStage) / sizeof(double)];
     if (gemm_wide(a.r, a.kk, a.c))
-        d_gemm_f64_t64(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld);
+        d_gemm_f64_t64<1>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, lds);
     else
-        d_gemm_f64_mfma(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld);
+        d_gemm_f64_mfma<4>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, lds);
 }
 
 __global__ __launch_bounds__(512) void kg_gemm_ks2(const Gemm* __restrict__ args,
                                                    const unsigned* __restrict__ st, int ns)
 {
     PARODE_GROUP(Gemm);
-    d_gemm_f64_ks<2>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld);
+    extern __shared__ double gsm[];
+    d_gemm_f64_ks<2>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, gsm);
 }
 
 __global__ __launch_bounds__(256) void kg_rk4_combine(const Rk4Comb* __restrict__ args,

@@ -12,6 +12,17 @@ namespace parode {
 namespace k {
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));
+// two doubles at any 8-byte address (one 16-byte load: the hardware takes it)
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void load4(const double* p, double (&r)[4])
+{
+    const double2u a = *reinterpret_cast<const double2u*>(p);
+    const double2u b = *reinterpret_cast<const double2u*>(p + 2);
+    r[0] = a.x;
+    r[1] = a.y;
+    r[2] = b.x;
+    r[3] = b.y;
+}
 
 // The block a kernel body works on: (x, y) and the grid's width in x.  A
 // single-system launch passes its own blockIdx and gridDim; a grouped launch

@@ -2,6 +2,7 @@
 
 #include <algorithm>
 #include <array>
+#include <functional>
 #include <mutex>
 #include <map>
 
@@ -36,9 +37,9 @@ ScanCore::ScanCore(int method, int n, int m, int p, bool zC, bool zD, long nPadM
             const size_t na = na_;
             const long nb = nPadMax_ >> lb;
             const size_t tab = k::block_table_values(b), w = k::block_scratch_values(b);
-            const size_t z = (size_t)(nb + 2) * na + k::block_z2_values(b, nb);
-            if (8 * (na2 * (L_ + 1) + tab + z + w + 3 * na) + 8 * Arena::kAlign > cap) continue;
-            PT64_.alloc(na2 * (L_ + 1), arena);
+            const size_t z = k::block_state_values(b, nb);
+            if (8 * (na2 * b.slots() + tab + z + w + 3 * na) + 8 * Arena::kAlign > cap) continue;
+            PT64_.alloc(na2 * b.slots(), arena);
             blkTab_.alloc(tab, arena);
             blkZ_.alloc(z, arena);
             if (w) blkW_.alloc(w, arena);
@@ -247,7 +248,7 @@ void ScanCore::build_powers(hipStream_t s, bool withLast)
 {
     if (uses_blocks()) {
         if (blk_.wide) {
-            wide_tables(s, dA_, dB_, dC_, dD_, nullptr, withLast, nullptr);
+            wide_tables(s, dA_, dB_, dC_, dD_, nullptr, withLast, 0, nullptr);
             powersDone_ = true;
             return;
         }
@@ -919,23 +920,29 @@ void BlockPhases::run(hipStream_t s, int from, int to) const
     }
 }
 
-// The tables of a wide map.  With side, the powers that only the tree reads are
-// queued on side->stream (forked from s once pass 1's tables are queued; the
-// caller joins).
+// The tables of a wide map.  With pass1 (which queues pass 1), also the tree's up
+// products: a launch of them beside each squaring that only the tree reads.
 void ScanCore::wide_tables(hipStream_t s, const float* dA, const float* dB, const float* dC,
-                           const float* dD, const float* dx0, bool withLast,
-                           const SideStream* side)
+                           const float* dD, const float* dx0, bool withLast, long nb,
+                           const std::function<void()>& pass1)
 {
     BlockPhases ph;
+    std::vector<int> ready;
     const int done = k::block_emit(blk_, bb_, h_, dA, dB, dC, dD, dx0, seed(),
-                                   withLast ? L_ : L_ - 1, ph);
-    ph.run(s, 0, done);
-    if (side) {
-        PARODE_HIP(hipEventRecord(side->fork, s));
-        PARODE_HIP(hipStreamWaitEvent(side->stream, side->fork, 0));
-        s = side->stream;
+                                   withLast ? L_ : L_ - 1, ph, &ready);
+    if (!pass1) {
+        ph.run(s, 0, (int)ph.ph.size());
+        return;
     }
-    ph.run(s, done, (int)ph.ph.size());
+    ph.run(s, 0, done);
+    pass1();
+    const int top = k::block_tree_up_levels(nb);
+    int up = 0;
+    for (int p = done; p < (int)ph.ph.size() || up < top; ++p) {
+        BlockPhases::Phase& f = ph.at(p);
+        if (up < top && ready[blk_.lb + up] <= p) f.gemm.push_back(k::block_tree_up(blk_, bb_, nb, up++));
+        ph.run(s, p, p + 1);
+    }
 }
 
 void ScanCore::solve_blocks(hipStream_t s, long nScan, double h, const float* dA, const float* dB,
@@ -951,26 +958,34 @@ void ScanCore::solve_blocks(hipStream_t s, long nScan, double h, const float* dA
     h_ = h;
     tick(0);
     if (blk_.wide) {
-        // beside pass 1: the powers that only the tree reads, and the start-up
-        wide_tables(s, dA, dB, dC, dD, dx0, false, side);
+        // the start-up on the side stream
         hipStream_t ps = side ? side->stream : s;
         if (method_ == kABM) {
+            if (side) {
+                PARODE_HIP(hipEventRecord(side->fork, s));
+                PARODE_HIP(hipStreamWaitEvent(side->stream, side->fork, 0));
+            }
             abm_startup(ps, dA, dB, dx0, dU, uDouble, h, seed());
             k::block_start_outputs(ps, blk_, dC, dD, seed(), dU, uDouble, dY);
+            if (side) PARODE_HIP(hipEventRecord(side->join, ps));
         }
-        if (side) PARODE_HIP(hipEventRecord(side->join, ps));
-        tick(1);
-        k::block_pass1(s, blk_, bb_, in, nb, false, block_tiling(1, nb, uDouble));
-        if (side) PARODE_HIP(hipStreamWaitEvent(s, side->join, 0));
+        wide_tables(s, dA, dB, dC, dD, dx0, false, nb, [&] {
+            tick(1);
+            k::block_pass1(s, blk_, bb_, in, nb, false, block_tiling(1, nb, uDouble));
+            tick(2);
+        });
+        tick(3);
+        if (method_ == kABM && side) PARODE_HIP(hipStreamWaitEvent(s, side->join, 0));
+        k::block_tree_finish(s, blk_, bb_, in, nb, seed());
     } else {
         k::block_map(s, blk_, bb_, h, dA, dB, dC, dD, dx0, dU, uDouble, seed(), dY);
         k::block_tables(s, blk_, bb_, dC);
         tick(1);
         k::block_pass1(s, blk_, bb_, in, nb, true, block_tiling(1, nb, uDouble));
+        tick(2);
+        tick(3);
+        k::block_scan(s, blk_, bb_, in, nb, seed());
     }
-    tick(2);
-    tick(3);
-    k::block_scan(s, blk_, bb_, in, nb, seed());
     tick(4);
     tick(5);
     k::block_pass2(s, blk_, bb_, in, nb, nScan, seed(), dD, yScan, block_tiling(2, nb, uDouble));
