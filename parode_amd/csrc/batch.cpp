@@ -49,7 +49,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
     opt.precision = kMixed;
     // stages, in order; the squarings and the tree levels get one phase per level
     enum { kSmp = 0, kIn, kR1, kR2, kR3, kComb, kPost, kBlk0 };
-    int maxL = 0, upSteps = 0, blkSteps = 0, blkRest = 0;
+    int maxL = 0, upSteps = 0, topSteps = 0, blkSteps = 0, blkRest = 0;
     struct Shape {
         long nScan, nPad;
         int L, na, lc, lt;
@@ -74,8 +74,9 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
             const long nb = c.blocks_of(s.nScan);
             if (c.blk_.wide) {
                 s.ready = k::block_emit(c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0, c.seed(),
-                                        s.L - 1, s.ops);
-                upSteps = std::max(upSteps, k::block_tree_up_levels(nb));
+                                        c.blk_.lb + k::block_tree_up_levels(c.blk_, nb), s.ops);
+                upSteps = std::max(upSteps, k::block_tree_up_levels(c.blk_, nb));
+                topSteps = std::max(topSteps, k::block_tree_top_steps(c.blk_, nb));
                 blkSteps = std::max(blkSteps, s.ready);
                 blkRest = std::max(blkRest, (int)s.ops.ph.size() - s.ready);
             } else {
@@ -98,7 +99,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
     const int kBlk1 = kBlk0 + blkSteps, kPow0 = kBlk1 + std::max(blkRest, 0);
     const int kTables = kPow0 + 4 * maxL, kStart = kTables + 1, kLeaves = kStart + 1,
               kChunk1 = kLeaves + 1, kUp0 = kChunk1 + 1, kTop = kUp0 + upSteps,
-              kGather = kTop + 1, kDown0 = kGather + 1, kChunk2 = kDown0 + upSteps,
+              kTop0 = kTop + 1, kGather = kTop0 + topSteps, kDown0 = kGather + 1, kChunk2 = kDown0 + upSteps,
               kOut = kChunk2 + 1;
     // the outputs in three sets, by the stream that runs the system's second
     // chunk pass (kinds in turn), so that each stream's outputs start when its
@@ -115,7 +116,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
         if (ph == kLeaves) return kStageLeaves;
         if (ph == kChunk1) return kStageChunks1;
         if (ph < kTop) return kStageUp;
-        if (ph == kTop) return kStageTop;
+        if (ph < kGather) return kStageTop;
         if (ph < kChunk2) return kStageDown;
         if (ph == kChunk2) return kStageChunks2;
         return kStageOutputs;
@@ -146,10 +147,12 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
                     for (auto& e : s.ops.ph[t].elem) k::g::add_block_elem(ph, e);
                     for (auto& o : s.ops.ph[t].gemm) k::g::add_gemm_op(ph, o);
                 }
-                const int top = k::block_tree_up_levels(nb);
+                const int top = k::block_tree_up_levels(c.blk_, nb);
                 for (int t = 0; t < top; ++t)
                     k::g::add_gemm_op(P[kUp0 + upSteps - (top - t)],
                                       k::block_tree_up(c.blk_, c.bb_, nb, t));
+                for (int t = 0; t < k::block_tree_top_steps(c.blk_, nb); ++t)
+                    k::g::add_gemm_op(P[kTop0 + t], k::block_tree_top(c.blk_, c.bb_, nb, t));
                 for (int t = 0; t < k::block_tree_down_steps(c.blk_, nb); ++t)
                     for (auto& o : k::block_tree_down(c.blk_, c.bb_, nb, t))
                         k::g::add_gemm_op(P[kDown0 + t], o);
@@ -161,9 +164,9 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
                 k::g::add_block_scan(P[kUp0 + upSteps - 1], P[kTop], P[kDown0], c.blk_, c.bb_, bin,
                                      nb, c.seed());
             }
-            k::g::add_block_pass1(P[kChunk1], c.blk_, c.bb_, bin, nb);
+            k::g::add_block_pass1(P[kChunk1], c.blk_, c.bb_, bin, nb, (int)systems.size());
             k::g::add_block_pass2(P[kChunk2], c.blk_, c.bb_, bin, nb, s.nScan, c.seed(), q.D,
-                                  yScan);
+                                  yScan, (int)systems.size());
             return;
         }
         const size_t nn = (size_t)n * n, nm = (size_t)n * m, na2 = (size_t)na * na;

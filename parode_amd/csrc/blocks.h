@@ -80,7 +80,7 @@ int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long 
 BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bool mirror, int lb,
                        int L);
 // How a pass is tiled (kBlockAuto: by the rule at launch_pass).
-enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit16 = 3 };
+enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit16 = 3, kBlockMid = 4 };
 // Groups of blocks that the scan of nb blocks makes first (0: none).
 long block_groups(int na, long nb);
 
@@ -124,14 +124,17 @@ int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A
                const float* C, const float* D, const float* x0, double* seed, int last,
                BlockSink& sink, std::vector<int>* ready = nullptr);
 // The tree over the blocks' states of a wide map: up products by pairs (level k
-// from 0, with the power lb + k), the root's seed, down products (step j from 0).
-int block_tree_up_levels(long nb);
+// from 0, with the power lb + k), the root's seed, the states at the top one after
+// the other (step i from 0), down products (step j from 0).
+int block_tree_up_levels(const BlockShape& s, long nb);
+int block_tree_top_steps(const BlockShape& s, long nb);
+GemmOp block_tree_top(const BlockShape& s, const BlockBufs& b, long nb, int i);
 int block_tree_down_steps(const BlockShape& s, long nb);
 GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k);
 std::vector<GemmOp> block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int j);
-// the root and the down steps
+// the root, the top and the down steps
 void block_tree_finish(hipStream_t st, const BlockShape& s, const BlockBufs& b,
-                       const BlockInput& in, long nb, const double* seed, double* tot = nullptr);
+                       const BlockInput& in, long nb, const double* seed);
 void block_elem(hipStream_t st, const BlkElem& e);
 
 // M, G, the direct terms and (x0 given) the seed: x0, or with the ABM start-up
@@ -150,10 +153,10 @@ void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
 // the blocks' start states from the seed (in X); Z[nb] is the state after them
 // (wide: tot receives the blocks' response from zero instead, if not null)
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                long nb, const double* seed, double* tot = nullptr);
+                long nb, const double* seed);
 // seedOut = the state (in X) after the blocks
 void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                 long nb, const double* seed, const double* tot, double* seedOut);
+                 long nb, const double* seed, double* seedOut);
 void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                  long nb, long nReal, const double* seed, const float* D, float* Y,
                  int tiling = kBlockAuto);
@@ -167,9 +170,9 @@ void add_block_elem(Phase& ph, const BlkElem& e);
 void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, const float* D,
                              const double* X0, const double* U, float* Y);
 void add_block_pass1(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb);
+                     long nb, int group);
 void add_block_pass2(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb, long nReal, const double* seed, const float* D, float* Y);
+                     long nb, long nReal, const double* seed, const float* D, float* Y, int group);
 // the scan of a map that is not wide: up and down are used when the blocks go in groups
 void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, const BlockBufs& b,
                     const BlockInput& in, long nb, const double* seed);

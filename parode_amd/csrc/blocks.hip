@@ -593,95 +593,144 @@ __device__ __forceinline__ void blk_store(const BlkPass& a, bool out, long b, in
     }
 }
 
-// Few tiles: 16 x 16 tiles whose K is split over NW waves, operands straight
-// from the caches, eight k-steps of loads in flight; the waves' partial tiles
-// meet in LDS.  Bound by the latency of those loads; used while the 64 x 64
-// tiles would not fill the compute units.
-template <typename TU, bool OUT, int NW>
+// Few tiles: 16 R x 16 R tiles whose K is split over NW waves, operands straight
+// from the caches, 16 loads of a wave in flight; the waves' partial tiles meet
+// in LDS.  Bound by the latency of those loads and by the caches (R = 2 halves
+// its bytes per product); used while the 64 x 64 tiles would not fill the
+// compute units.
+template <typename TU, bool OUT, int NW, int R>
 __device__ __forceinline__ void d_blk_split(const VBlock vb, const BlkPass& a, double* part,
                                             int* bad)
 {
+    constexpr int kT = 16 * R, kW = 256 * R * R;   // tile side, values of a partial tile
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, q4 = lane >> 4;
-    const long b0 = vb.y * 16;
-    const int j0 = (int)vb.x * 16;
-    const long b = b0 + l16 < a.nb ? b0 + l16 : a.nb - 1;
-    const int col = j0 + l16 < a.cols ? j0 + l16 : a.cols - 1;
-    const TU* u = static_cast<const TU*>(a.U) + b * a.blockU;
-    const int kl = win_len(a, b);
-    int kcol = a.ku, kEnd = a.ku, kMin = a.ku, stride = a.na;
-    const double* h = a.BU + col;
+    const long b0 = vb.y * kT;
+    const int j0 = (int)vb.x * kT;
+    // a lane's rows and columns (those past the last repeat it): row 16 r + l16
+    // from u[r], its samples zero from k = kl[r] on; the factors of column
+    // 16 r + l16 from h[r], zero from k = kcol[r] on
+    const TU* u[R];
+    const double* h[R];
+    int kl[R], kcol[R], col[R];
+    long row[R];
+    int kEnd = a.ku, kMin = a.ku, stride = a.na;
     if (OUT) {
-        const int jl = j0 + 15 < a.cols ? j0 + 15 : a.cols - 1;
-        const int i = col / a.p;
-        kcol = (a.s * i + a.taps) * a.m;
+        const int jl = j0 + kT - 1 < a.cols ? j0 + kT - 1 : a.cols - 1;
         kEnd = (a.s * (jl / a.p) + a.taps) * a.m;
         kMin = (a.s * (j0 / a.p) + a.taps) * a.m;
         stride = a.p;
-        h = a.BU + (long)a.s * (a.T - 1 - i) * a.m * a.p + (col - i * a.p);
         if (threadIdx.x == 0) *bad = 0;
         __syncthreads();
     }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        row[r] = b0 + 16 * r + l16 < a.nb ? b0 + 16 * r + l16 : a.nb - 1;
+        col[r] = j0 + 16 * r + l16 < a.cols ? j0 + 16 * r + l16 : a.cols - 1;
+        u[r] = static_cast<const TU*>(a.U) + row[r] * a.blockU;
+        const int w = win_len(a, row[r]);
+        kl[r] = w < kEnd ? w : kEnd;
+        kcol[r] = a.ku;
+        h[r] = a.BU + col[r];
+        if (OUT) {
+            const int i = col[r] / a.p;
+            kcol[r] = (a.s * i + a.taps) * a.m;
+            h[r] = a.BU + (long)a.s * (a.T - 1 - i) * a.m * a.p + (col[r] - i * a.p);
+        }
+    }
     const int zs = OUT ? (a.kz + 3) / 4 : 0, us = (kEnd + 3) / 4, per = (zs + us + NW - 1) / NW;
     const int kb = wave * per, ke = kb + per < zs + us ? kb + per : zs + us;
-    doublex4 acc = {0.0, 0.0, 0.0, 0.0};
-    constexpr int UN = 8;
+    doublex4 acc[R][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < R; ++c) acc[r][c] = doublex4{0.0, 0.0, 0.0, 0.0};
+    constexpr int UN = 8 / R;
+    double x[UN][R], y[UN][R];
+    auto multiply = [&] {
+#pragma unroll
+        for (int t = 0; t < UN; ++t)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int c = 0; c < R; ++c)
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t][r], y[t][c], acc[r][c], 0,
+                                                                     0, 0);
+    };
     int k = kb;
     if (OUT) {
-        const double* z = a.Z + b * a.na;
         const int kz = ke < zs ? ke : zs;
         for (; k < kz; k += UN) {
-            double x[UN], y[UN];
 #pragma unroll
             for (int t = 0; t < UN; ++t) {
                 const int j = (k + t) * 4 + q4;
                 const bool in = k + t < kz && j < a.kz;
-                x[t] = in ? z[j] : 0.0;
-                y[t] = in ? a.OT[(long)j * a.cols + col] : 0.0;
-            }
 #pragma unroll
-            for (int t = 0; t < UN; ++t)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], y[t], acc, 0, 0, 0);
+                for (int r = 0; r < R; ++r) {
+                    x[t][r] = in ? a.Z[row[r] * a.na + j] : 0.0;
+                    y[t][r] = in ? a.OT[(long)j * a.cols + col[r]] : 0.0;
+                }
+            }
+            multiply();
         }
         k = kb > zs ? kb : zs;
     }
     bool nf = false;
     if (OUT && first_output(a, b0, j0)) kMin = 0;
     for (; k < ke; k += UN) {
-        double x[UN], y[UN];
 #pragma unroll
         for (int t = 0; t < UN; ++t) {
             const int j = (k - zs + t) * 4 + q4;
             const bool in = k + t < ke;
-            x[t] = (in && j < kl && j < kEnd) ? (double)u[win(a, j)] : 0.0;
-            y[t] = (in && j < kcol) ? h[(long)j * stride] : 0.0;
-            if (OUT) nf = nf || (j >= kMin && not_finite(x[t]));
-        }
+            const int at = win(a, j);
 #pragma unroll
-        for (int t = 0; t < UN; ++t)
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], y[t], acc, 0, 0, 0);
+            for (int r = 0; r < R; ++r) {
+                x[t][r] = (in && j < kl[r]) ? (double)u[r][at] : 0.0;
+                y[t][r] = (in && j < kcol[r]) ? h[r][(long)j * stride] : 0.0;
+                if (OUT) nf = nf || (j >= kMin && not_finite(x[t][r]));
+            }
+        }
+        multiply();
     }
     if (OUT && nf) *bad = 1;
-    if (wave > 0) {
+    // D[i][j] is in lane j + 16 (i % 4), register i / 4
+    if (R > 1 || wave > 0) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) part[((wave - 1) * 4 + v) * 64 + lane] = acc[v];
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < R; ++c)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    part[(R > 1 ? wave : wave - 1) * kW + (16 * r + 4 * v + q4) * kT + 16 * c + l16] =
+                        acc[r][c][v];
     }
     __syncthreads();
     if (OUT && *bad) {
-        for (int t = threadIdx.x; t < 256; t += NW * 64) {
-            const long bb = b0 + t / 16;
-            const int cc = j0 + t % 16;
+        for (int t = threadIdx.x; t < kW; t += NW * 64) {
+            const long bb = b0 + t / kT;
+            const int cc = j0 + t % kT;
             if (bb < a.nb && cc < a.cols) blk_store(a, true, bb, cc, blk_output<TU>(a, bb, cc));
+        }
+        return;
+    }
+    if (R > 1) {   // a value's parts are added in wave order, each by one thread
+        for (int t = threadIdx.x; t < kW; t += NW * 64) {
+            double v = part[t];
+#pragma unroll
+            for (int g = 1; g < NW; ++g) v += part[g * kW + t];
+            const long bb = b0 + t / kT;
+            const int cc = j0 + t % kT;
+            if (bb < a.nb && cc < a.cols) blk_store(a, OUT, bb, cc, v);
         }
         return;
     }
     if (wave > 0) return;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        double y = acc[v];
+        double t = acc[0][0][v];
 #pragma unroll
-        for (int g = 1; g < NW; ++g) y += part[((g - 1) * 4 + v) * 64 + lane];
+        for (int g = 1; g < NW; ++g) t += part[(g - 1) * kW + (4 * v + q4) * kT + l16];
         const long bb = b0 + 4 * v + q4;
-        if (bb < a.nb && j0 + l16 < a.cols) blk_store(a, OUT, bb, j0 + l16, y);
+        if (bb < a.nb && j0 + l16 < a.cols) blk_store(a, OUT, bb, j0 + l16, t);
     }
 }
 
@@ -939,10 +988,10 @@ __device__ __forceinline__ VBlock blk_place(long idx, long gx, long gy)
     return VBlock{t % gx, t / gx * 8 + idx % 8, gx};
 }
 
-template <typename TU, bool OUT, int NW>
+template <typename TU, bool OUT, int NW, int R>
 __global__ __launch_bounds__(NW * 64) void k_blk_split(const BlkPass a)
 {
-    constexpr int kPart = (NW - 1) * 256;
+    constexpr int kPart = R > 1 ? NW * 256 * R * R : (NW - 1) * 256;
     constexpr int kLds = OUT || kPart > kBN * kBP ? kPart : kBN * kBP;
     __shared__ double lds[kLds];
     __shared__ int bad;
@@ -950,11 +999,11 @@ __global__ __launch_bounds__(NW * 64) void k_blk_split(const BlkPass a)
         d_blk_powers<NW>(a.na, a.lb, a.L, a.PT, lds);
         return;
     }
-    d_blk_split<TU, OUT, NW>(blk_place(blockIdx.x, a.gx, a.gy), a, lds, &bad);
+    d_blk_split<TU, OUT, NW, R>(blk_place(blockIdx.x, a.gx, a.gy), a, lds, &bad);
 }
 
 template <typename TU, bool OUT, int KS>
-__global__ __launch_bounds__(256 * KS) void k_blk_tile(const BlkPass a)
+__global__ __launch_bounds__(256 * KS, 4) void k_blk_tile(const BlkPass a)
 {
     __shared__ BlkTileLds<KS> L;
     static_assert(sizeof(BlkStage) >= kBN * kBP * sizeof(double), "room for the powers");
@@ -999,6 +1048,7 @@ __device__ __forceinline__ double blk_shift(const BlkScan& a, long row0, long at
     double v = 0.0;
     const double* Ud = static_cast<const double*>(a.U);
     const float* Uf = static_cast<const float*>(a.U);
+#pragma unroll 1
     for (int k = 0; k < a.km; ++k) {
         const int r = a.m == 1 ? k : (int)__umulhi((unsigned)k, a.magic);
         if (row0 + r > a.last) break;
@@ -1008,10 +1058,14 @@ __device__ __forceinline__ double blk_shift(const BlkScan& a, long row0, long at
     return v;
 }
 
-template <int MODE>
-__device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, double* lds)
+// Loads are unconditional (clamped, and selected where their value is used): a
+// branch around one makes every wait a wait for all of them, and then each step
+// takes a memory latency (2 us at n_a = 48, of which its products are 0.3).
+template <int MODE, int NK>   // NK = (n_a + 15) / 16 * 4 steps of the products
+__device__ __forceinline__ void d_blk_scan_n(const VBlock vb, const BlkScan& a, double* lds)
 {
-    const int na = a.na, n16 = (na + 15) & ~15, nct = n16 / 16, pitch = n16 + 1;
+    constexpr int nct = NK / 4, pitch = 4 * NK + 1;
+    const int na = a.na;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q4 = lane >> 4;
     const int rt = wave / nct, ct = wave - rt * nct, rows = 16 * a.R;
     if (rt >= a.R) return;   // (a grouped launch has waves for its widest system)
@@ -1019,43 +1073,62 @@ __device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, do
     double* x0 = lds;                       // [rows][pitch], double buffered
     double* x1 = lds + rows * pitch;
     const long nn = (long)na * na;
-    const int col = ct * 16 + l16;
-    double p[kBN / 4];
-    auto load_p = [&](int l) {
-        const double* P = a.PT + l * nn;
+    const int col = ct * 16 + l16, ccol = col < na ? col : na - 1;
+    double p[NK];
+    auto fetch_p = [&](int l, double* to) {
+        const double* P = a.PT + l * nn + ccol;
 #pragma unroll
-        for (int u = 0; u < kBN / 4; ++u) {
+        for (int u = 0; u < NK; ++u) {
             const int k = 4 * u + q4;
-            p[u] = (k < na && col < na) ? P[(long)k * na + col] : 0.0;
+            to[u] = P[(long)(k < na ? k : na - 1) * na];
         }
     };
-    // rows of x (this wave's row tile shifted up by d rows, zero above) times P
+    auto use_p = [&](const double* from) {
+#pragma unroll
+        for (int u = 0; u < NK; ++u) p[u] = 4 * u + q4 < na && col < na ? from[u] : 0.0;
+        // (arrived before any loop that reads them: else its every step waits for all loads)
+#pragma unroll
+        for (int u = 0; u < NK; ++u) asm volatile("" : "+v"(p[u]));
+    };
+    // rows of x (this wave's row tile shifted up by d rows, zero above) times P:
+    // CH operands are read before the first of their products (one LDS round
+    // trip, not one for each)
     auto product = [&](const double* x, doublex4 acc, int d) {
+        constexpr int CH = MODE == kScanAll && NK > 8 ? 8 : NK;   // (16 waves: 128 registers each)
         const int r = rt * 16 + l16 - d;
         const double* xr = x + (r > 0 ? r : 0) * pitch + q4;
-        const bool in = r >= 0;
 #pragma unroll
-        for (int u = 0; u < kBN / 4; ++u) {
-            if (4 * u >= n16) break;
-            const double v = in ? xr[4 * u] : 0.0;
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, p[u], acc, 0, 0, 0);
+        for (int u0 = 0; u0 < NK; u0 += CH) {
+            double v[CH];
+#pragma unroll
+            for (int u = 0; u < CH; ++u) v[u] = u0 + u < NK ? xr[4 * (u0 + u)] : 0.0;
+#pragma unroll
+            for (int u = 0; u < CH; ++u)
+                if (u0 + u < NK)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(r >= 0 ? v[u] : 0.0, p[u0 + u], acc,
+                                                               0, 0, 0);
         }
         return acc;
     };
-    // this lane's groups (rows rt 16 + 4 v + q4) and its element of block e
-    long e0[4];
-    bool ok[4];
+    // this lane's groups are rows rt 16 + 4 v + q4; its element of block j of
+    // group v is at at(v, j), the last block's at lim
+    const long g1 = g0 + rt * 16 + q4, first = (g1 << a.lg) * na + ccol;
+    const long lim = (a.nb - 1) * na + ccol;
+    auto at = [&](int v, long j) { return first + (((long)(4 * v) << a.lg) + j) * na; };
+    auto fetch = [&](doublex4& to, long j) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        e0[v] = (g0 + rt * 16 + 4 * v + q4) * Lg;
-        ok[v] = e0[v] < a.nb && col < na;
-    }
-    auto elem = [&](int v, long j) {
-        const long e = e0[v] + j;
-        return (ok[v] && j < Lg && e < a.nb) ? a.E[e * na + col] : 0.0;
+        for (int v = 0; v < 4; ++v) {
+            const long o = at(v, j);
+            to[v] = a.E[o < lim ? o : lim];
+        }
+    };
+    auto select = [&](doublex4 y, long j) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (col >= na || at(v, j) > lim) y[v] = 0.0;
+        return y;
     };
     auto put = [&](double* x, int v, double y) { x[(rt * 16 + 4 * v + q4) * pitch + col] = y; };
-    load_p(a.l0);
     double* cur = x0;
     double* nxt = x1;
     auto flip = [&]() {
@@ -1064,35 +1137,40 @@ __device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, do
         cur = nxt;
         nxt = t;
     };
-    doublex4 s;
+    // the elements of D steps are on their way (D divides L_g: groups over several
+    // work-groups have 16 blocks or more)
+    constexpr int D = MODE == kScanAll ? 1 : 2;
+    doublex4 s[D];
+#pragma unroll
+    for (int q = 0; q < D; ++q) fetch(s[q], q);
+    fetch_p(a.l0, p);
+    use_p(p);
     if (MODE != kScanDown) {
-        // from zero: the first step takes S_0 as it is
+        // from zero
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            put(cur, v, elem(v, 0));
-            s[v] = elem(v, 1);
-        }
+        for (int v = 0; v < 4; ++v) put(cur, v, 0.0);
         __syncthreads();
-        for (long j = 1; j < Lg; ++j) {
-            doublex4 sn;
+#pragma unroll 1
+        for (long j0 = 0; j0 < Lg; j0 += D) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sn[v] = elem(v, j + 1);
-            const doublex4 y = product(cur, s, 0);
+            for (int q = 0; q < D; ++q) {
+                const doublex4 e = select(s[q], j0 + q);
+                fetch(s[q], j0 + q + D);
+                const doublex4 y = product(cur, e, 0);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                put(nxt, v, y[v]);
-                s[v] = sn[v];
+                for (int v = 0; v < 4; ++v) put(nxt, v, y[v]);
+                flip();
             }
-            flip();
         }
         if (MODE == kScanUp) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const long g = g0 + rt * 16 + 4 * v + q4;
-                if (ok[v]) a.Zg[g * na + col] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
-            }
+            for (int v = 0; v < 4; ++v)
+                if (col < na && at(v, 0) <= lim)
+                    a.Zg[(g1 + 4 * v) * na + col] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
             return;
         }
+#pragma unroll
+        for (int q = 0; q < D; ++q) fetch(s[q], q);
         // the groups' start states: row g holds the response of group g - 1,
         // row 0 the seed
 #pragma unroll
@@ -1105,8 +1183,19 @@ __device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, do
         }
         flip();
         const long groups = (a.nb + Lg - 1) / Lg;
+        // the next step's power is on its way (16 waves at NK = 16 have no room for it)
+        constexpr bool kAhead = NK < 16;
+        double pn[kAhead ? NK : 1];
+        if (kAhead && groups > 1) fetch_p(a.l0 + a.lg, pn);
+#pragma unroll 1
         for (int k = 0; (1L << k) < groups; ++k) {
-            load_p(a.l0 + a.lg + k);
+            if (kAhead) {
+                use_p(pn);
+                fetch_p((2L << k) < groups ? a.l0 + a.lg + k + 1 : a.l0, pn);
+            } else {
+                fetch_p(a.l0 + a.lg + k, p);
+                use_p(p);
+            }
             doublex4 y;
 #pragma unroll
             for (int v = 0; v < 4; ++v) y[v] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
@@ -1115,48 +1204,61 @@ __device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, do
             for (int v = 0; v < 4; ++v) put(nxt, v, y[v]);
             flip();
         }
-        load_p(a.l0);
+        if (kAhead) {
+            if (groups > 1) use_p(pn);
+        } else {
+            fetch_p(a.l0, p);
+            use_p(p);
+        }
     } else {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const long g = g0 + rt * 16 + 4 * v + q4;
-            put(cur, v, ok[v] ? a.Zg[g * na + col] : 0.0);
-        }
+        for (int v = 0; v < 4; ++v)
+            put(cur, v, col < na && at(v, 0) <= lim ? a.Zg[(g1 + 4 * v) * na + col] : 0.0);
         __syncthreads();
     }
     // from the start states: E_e over S_e, each read before it is written
     doublex4 x;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        x[v] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
-        s[v] = elem(v, 0);
-    }
-    for (long j = 0; j < Lg; ++j) {
-        doublex4 sn;
+    for (int v = 0; v < 4; ++v) x[v] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
+#pragma unroll 1
+    for (long j0 = 0; j0 < Lg; j0 += D) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sn[v] = elem(v, j + 1);
+        for (int q = 0; q < D; ++q) {
+            const long j = j0 + q;
+            const doublex4 y = select(s[q], j);
+            fetch(s[q], j + D);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const long e = e0[v] + j;
-            if (ok[v] && e < a.nb) a.E[e * na + col] = x[v];
+            for (int v = 0; v < 4; ++v) {
+                const long o = at(v, j);
+                if (col < na && o <= lim) a.E[o] = x[v];
+            }
+            x = product(cur, y, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if (col < na && at(v, j) == lim) a.E[lim + na] = x[v];
+                put(nxt, v, x[v]);
+            }
+            flip();
         }
-        x = product(cur, s, 0);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const long e = e0[v] + j;
-            if (ok[v] && e == a.nb - 1) a.E[a.nb * na + col] = x[v];
-            put(nxt, v, x[v]);
-            s[v] = sn[v];
-        }
-        flip();
     }
 }
 
 template <int MODE>
-__global__ __launch_bounds__(MODE == kScanAll ? 1024 : 256) void k_blk_scan(const BlkScan a)
+__device__ __forceinline__ void d_blk_scan(const VBlock vb, const BlkScan& a, double* lds)
+{
+    switch ((a.na + 15) / 16) {
+    case 1: return d_blk_scan_n<MODE, 4>(vb, a, lds);
+    case 2: return d_blk_scan_n<MODE, 8>(vb, a, lds);
+    case 3: return d_blk_scan_n<MODE, 12>(vb, a, lds);
+    default: return d_blk_scan_n<MODE, 16>(vb, a, lds);
+    }
+}
+
+template <int MODE, int NK>
+__global__ __launch_bounds__(MODE != kScanAll ? 16 * NK : NK == 12 ? 768 : 1024) void k_blk_scan(const BlkScan a)
 {
     extern __shared__ double scan_lds[];
-    d_blk_scan<MODE>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, scan_lds);
+    d_blk_scan_n<MODE, NK>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, scan_lds);
 }
 
 __global__ void k_blk_carry(const BlkScan a, long row0, long at, double* out)
@@ -1165,31 +1267,47 @@ __global__ void k_blk_carry(const BlkScan a, long row0, long at, double* out)
         out[i] = a.E[a.nb * a.na + i] + blk_shift(a, row0, at, i);
 }
 
-// wide maps: the tree's root takes the shifted seed (its response from zero goes
-// to tot), and the state after the blocks is P_L Z_0 plus that response
-__device__ __forceinline__ void d_blk_root(const BlkScan& a, const double* S, double* E,
-                                           double* tot)
+// wide maps: the first state at the tree's top is the seed, shifted.  16 states to
+// a work-group, a state's taps m terms over 16 lanes (one after the other in one
+// work-group: 37 us at 812 states, 100 terms).
+__device__ __forceinline__ void d_blk_root(const VBlock vb, const BlkScan& a, double* E)
 {
-    for (int i = threadIdx.x; i < a.na; i += blockDim.x) {
-        if (tot) tot[i] = S[i];
-        E[i] = a.seed[i] - blk_shift(a, 0, 0, i);
+    __shared__ double part[16][17];
+    const int c = threadIdx.x & 15, g = threadIdx.x >> 4, i = (int)vb.x * 16 + c;
+    double v = 0.0;
+    if (i < a.na) {
+        const double* Ud = static_cast<const double*>(a.U);
+        const float* Uf = static_cast<const float*>(a.U);
+        for (int k = g; k < a.km; k += 16) {
+            const int r = a.m == 1 ? k : (int)__umulhi((unsigned)k, a.magic);
+            if (r > a.last) break;
+            const long o = k + (long)r * a.gm;
+            v = fma(a.DL[(long)k * a.na + i], a.uDouble ? Ud[o] : (double)Uf[o], v);
+        }
     }
+    part[g][c] = v;
+    __syncthreads();
+    if (g || i >= a.na) return;
+#pragma unroll
+    for (int q = 1; q < 16; ++q) v += part[q][c];
+    E[i] = a.seed[i] - v;
 }
-__global__ __launch_bounds__(1024) void k_blk_root(const BlkScan a, const double* S, double* E,
-                                                   double* tot)
+__global__ __launch_bounds__(256) void k_blk_root(const BlkScan a, double* E)
 {
-    d_blk_root(a, S, E, tot);
+    d_blk_root(VBlock{(long)blockIdx.x, 0, (long)gridDim.x}, a, E);
 }
+// The state after all blocks (every node is whole): z P + S from the last node of
+// the tree's top, shifted back.
 __global__ __launch_bounds__(256) void k_blk_carry_wide(const BlkScan a, const double* P,
-                                                        const double* tot, long row0, long at,
-                                                        double* out)
+                                                        const double* e, const double* S,
+                                                        long row0, long at, double* out)
 {
     extern __shared__ double z[];
-    for (int i = threadIdx.x; i < a.na; i += 256) z[i] = a.seed[i] - blk_shift(a, 0, 0, i);
+    for (int i = threadIdx.x; i < a.na; i += 256) z[i] = e[i];
     __syncthreads();
     const int i = (int)blockIdx.x * 256 + threadIdx.x;
     if (i >= a.na) return;
-    double v = tot[i] + blk_shift(a, row0, at, i);
+    double v = S[i] + blk_shift(a, row0, at, i);
     for (int k = 0; k < a.na; ++k) v = fma(P[(long)k * a.na + i], z[k], v);
     out[i] = v;
 }
@@ -1329,6 +1447,15 @@ static bool fits_one(int method, int n, int m, int p)
     return na <= kBN && p <= kBN && m <= kBM && s * m <= kBN;
 }
 
+// One work-group scans up to 512 blocks; more go in groups of 16 (or as many
+// as leave 512 groups).
+static int group_log(long nb)
+{
+    if (nb <= 512) return 0;
+    int lg = 4;
+    while (((nb + (1L << lg) - 1) >> lg) > 512) ++lg;
+    return lg;
+}
 // The rule: which systems run as block responses, and with how many steps per
 // block: the fastest by the model below, if it beats the general path's.
 // Covered: inputs and outputs present, horizons from 64 points.  More steps per
@@ -1350,20 +1477,27 @@ int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long 
         if ((nPad >> lb) < 2) break;
         // (T m s < 2^16: the window index's multiply-high)
         if ((long)(s * T + 8) * m >= 65536) break;
-        // microseconds: FP64 products at 25 (few tiles) or 40 TFLOP/s, the
-        // scan's chain, the tables
-        const double pass = N * (2.0 * na * s * m + 2.0 * p * na +
-                                 2.0 * s * m * p * (T / 2 + 32.0 / p + 2)) / (one ? 25e6 : 40e6);
+        // microseconds: FP64 products at 40 TFLOP/s (25 over few tiles; pass 2 in
+        // tiles of 16 or 32: 6), the scan's chain, the tables
+        const double r1 = one ? 25e6 : 40e6, r2 = one && N * p < 64 * 4096 ? 6e6 : r1;
+        const double pass1 = N * 2.0 * na * s * m / r1;
+        const double pass = pass1 + N * (2.0 * p * na + 2.0 * s * m * p * (T / 2 + 32.0 / p + 2)) / r2;
         double scan, tab;
         if (one) {
-            const double steps = nb <= 512 ? nb / 64 : 2 * 16 + nb / 16 / 64;
-            scan = 2 * steps * (0.25 + na * 0.012) + 2 * nb * na2 * 2 / 0.25e6 / (nb <= 512 ? 1 : nb / 512);
+            // k_blk_scan measured: 13 us + 2.4 a step at n_a = 8, 18 + 3.1 at 48;
+            // groups before it 5 + 0.95 a step and 6 + 1.6 (both ways)
+            const int lg = group_log((long)std::ceil(nb));
+            const double rows = na <= 16 ? 256 : na <= 32 ? 128 : 64;
+            const double Lg = std::exp2(std::max(0.0, std::ceil(std::log2(nb / (1 << lg) / rows))));
+            scan = 12 + 0.13 * na + (2.3 + 0.017 * na) * Lg + (lg ? 6 + (0.85 + 0.016 * na) * (1 << lg) : 0);
             tab = lb * 1.2 + T * (s * m + p) / 64 * 0.05;
         } else {
             scan = 4 * na2 * nb / 40e6 + 2 * 5.0 * std::max(1.0, std::log2(nb));
             tab = 2 * na2 * (s * m + p) * T / 40e6 + 5.0 * lb;
         }
-        const double t = pass + scan + tab;
+        // (what the squarings beside pass 1 take beyond it)
+        const double sq = one ? std::max(0.0, std::log2(nb) * (0.8 + 0.018 * na) - 8 - pass1) : 0.0;
+        const double t = pass + scan + tab + sq;
         if (!best || t < bt) {
             best = lb;
             bt = t;
@@ -1417,7 +1551,15 @@ struct TreeLevel {
     size_t s, e;   // responses and start states, in states from b.Z2 (level 0: b.Z, b.E)
 };
 static long tree_rows(long n) { return (n + 3) / 4 * 4; }
-static std::vector<TreeLevel> tree_of(long nb)
+static bool structured_square(const BlockShape& s);
+// The tree ends at few states, which are taken one after the other: a product of
+// one row each in place of the levels above, and no squarings for those (which
+// the up levels wait for): 8 states where a squaring is four dependent launches
+// (ABM n = 203: 988 us a solve against 1075 with the whole tree, 1000 with 16), 4
+// otherwise (n = 128: 399 against 401, 409 with 8; 512 systems together 44.7 ms
+// against 46.5).
+static long tree_top(const BlockShape& s) { return structured_square(s) ? 8 : 4; }
+static std::vector<TreeLevel> tree_of(const BlockShape& s, long nb)
 {
     std::vector<TreeLevel> t;
     size_t at = 0;
@@ -1425,7 +1567,7 @@ static std::vector<TreeLevel> tree_of(long nb)
         const size_t rows = t.empty() ? 0 : (size_t)tree_rows(n);
         t.push_back(TreeLevel{n, at, at + rows});
         at += 2 * rows;
-        if (n <= 1) return t;
+        if (n <= tree_top(s)) return t;
     }
 }
 static double* tree_s(const BlockShape& s, const BlockBufs& b, const std::vector<TreeLevel>& t, int k)
@@ -1436,7 +1578,7 @@ static double* tree_e(const BlockShape& s, const BlockBufs& b, const std::vector
 {
     return k == 0 ? b.E : b.Z2 + t[k].e * s.na;
 }
-int block_tree_up_levels(long nb) { return (int)tree_of(nb).size() - 1; }
+int block_tree_up_levels(const BlockShape& s, long nb) { return (int)tree_of(s, nb).size() - 1; }
 // the levels that the down steps go to, from the top
 static std::vector<int> tree_steps(const BlockShape& s, int top)
 {
@@ -1450,7 +1592,7 @@ static std::vector<int> tree_steps(const BlockShape& s, int top)
 }
 int block_tree_down_steps(const BlockShape& s, long nb)
 {
-    return (int)tree_steps(s, block_tree_up_levels(nb)).size();
+    return (int)tree_steps(s, block_tree_up_levels(s, nb)).size();
 }
 
 // Z (and E): whole nodes and one state more; then Z2
@@ -1461,7 +1603,7 @@ static size_t state_rows0(const BlockShape& s, long nb)
 size_t block_state_values(const BlockShape& s, long nb)
 {
     if (!s.wide) return (state_rows0(s, nb) + block_groups(s.na, nb) + 1) * s.na;
-    const std::vector<TreeLevel> t = tree_of(nb);
+    const std::vector<TreeLevel> t = tree_of(s, nb);
     return (2 * state_rows0(s, nb) + t.back().e + (nb > 1 ? 4 : 0)) * s.na;
 }
 
@@ -1633,7 +1775,7 @@ int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A
             }
         }
         // the third power of a radix-4 level
-        if (s.radix4() && l > s.lb && ((l - s.lb) & 1))
+        if (s.radix4() && l > s.lb && l < last && ((l - s.lb) & 1))
             sink.gemm(ph, GemmOp{na, na, na, P, b.PT + s.slot(l - 1) * na2,
                                  b.PT + (s.slot(l - 1) - 2) * na2, gemm_ld(na, na)});
         if (l >= s.lb) continue;
@@ -1657,7 +1799,7 @@ int block_emit(const BlockShape& s, const BlockBufs& b, double h, const float* A
 // neighbour: not formed)
 GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k)
 {
-    const std::vector<TreeLevel> t = tree_of(nb);
+    const std::vector<TreeLevel> t = tree_of(s, nb);
     const int na = s.na;
     double* S = tree_s(s, b, t, k);
     GemmLd ld{2 * na, na, na};
@@ -1666,10 +1808,22 @@ GemmOp block_tree_up(const BlockShape& s, const BlockBufs& b, long nb, int k)
     return GemmOp{(int)(t[k].n / 2), na, na, S, b.PT + (size_t)s.slot(s.lb + k) * na * na,
                   tree_s(s, b, t, k + 1), ld};
 }
+// E[i + 1] = E[i] P + S[i] at the tree's top
+int block_tree_top_steps(const BlockShape& s, long nb) { return (int)tree_of(s, nb).back().n - 1; }
+GemmOp block_tree_top(const BlockShape& s, const BlockBufs& b, long nb, int i)
+{
+    const std::vector<TreeLevel> t = tree_of(s, nb);
+    const int na = s.na, top = (int)t.size() - 1;
+    double* E = tree_e(s, b, t, top) + (size_t)i * na;
+    GemmLd ld{na, na, na};
+    ld.add = tree_s(s, b, t, top) + (size_t)i * na;
+    ld.lda = na;
+    return GemmOp{1, na, na, E, b.PT + (size_t)s.slot(s.lb + top) * na * na, E + na, ld};
+}
 // E[R i] = E'[i], E[R i + j] = E'[i] P^j + sum_{q < j} S[R i + q] P^(j-1-q), R = 2 or 4
 std::vector<GemmOp> block_tree_down(const BlockShape& s, const BlockBufs& b, long nb, int j0)
 {
-    const std::vector<TreeLevel> t = tree_of(nb);
+    const std::vector<TreeLevel> t = tree_of(s, nb);
     const int na = s.na, top = (int)t.size() - 1;
     const std::vector<int> to = tree_steps(s, top);
     const int from = j0 == 0 ? top : to[j0 - 1], k = to[j0], R = 1 << (from - k);
@@ -1693,15 +1847,6 @@ std::vector<GemmOp> block_tree_down(const BlockShape& s, const BlockBufs& b, lon
     return ops;
 }
 
-// One work-group scans up to 512 blocks; more go in groups of 16 (or as many
-// as leave 512 groups).
-static int group_log(long nb)
-{
-    if (nb <= 512) return 0;
-    int lg = 4;
-    while (((nb + (1L << lg) - 1) >> lg) > 512) ++lg;
-    return lg;
-}
 long block_groups(int na, long nb)
 {
     (void)na;
@@ -1784,22 +1929,25 @@ static BlkPass pass_args(const BlockShape& s, const BlockBufs& b, const BlockInp
     return a;
 }
 
-// The tiling of a pass over one system: 64 x 64 tiles from 64 of them (50 001
-// points, n_a = 37: 135 us a solve against 169 when they start at 16; 16 x 16
-// from 256 tiles on: 20 us more at n_a = 48, 2^18 points), 16 x 16 below, their K
-// over 16 waves while those tiles are few too.  In a grouped launch the other
-// systems fill the GPU and the wide tiles' higher rate counts from fewer of
-// them (512 systems: 45.3 ms from 16 tiles, 48.0 from 64).
-static int pass_tiling(const BlkPass& a, bool out, bool grouped)
+// The tiling of a pass, alone (group 0) or in a launch of `group` systems: 64 x 64
+// tiles from 64 of them (n_a = 48, 2^18 points: 208 us a solve against 262 from
+// 192; n_a = 37, 50 001 points: 135 against 169 from 16), 16 x 16 while those are
+// at most one for each compute unit, K over 16 waves where it is long (or where
+// a work-group of pass 1 squares powers: 6 squarings of 48 x 48 take 10 us with
+// 16 waves, 34 with 4), 32 x 32 between.  Systems launched together fill the
+// GPU between them: the wider tiles from fewer (64 small systems: 785 us from 32
+// and 64, 897 from 64 and 256; 512 systems 43.3 ms against 48).
+static int pass_tiling(const BlkPass& a, bool out, int group)
 {
     const long tx = (a.cols + kPT - 1) / kPT, ty = (a.nb + kPT - 1) / kPT;
     const long sx = (a.cols + 15) / 16, sy = (a.nb + 15) / 16;
-    if (tx * ty >= (grouped ? 16 : 64)) return kBlockTile;
-    return sx * sy <= 256 && ((out ? a.kz : 0) + a.ku) / 4 >= 64 ? kBlockSplit16 : kBlockSplit4;
+    if (tx * ty >= (group > 1 ? 32 : 64)) return kBlockTile;
+    if (sx * sy > (group > 1 ? std::max(64, 256 / group) : 256)) return kBlockMid;
+    return (!out && a.na > 16) || ((out ? a.kz : 0) + a.ku) / 4 >= 64 ? kBlockSplit16 : kBlockSplit4;
 }
 static void pass_grid(BlkPass& a, int tiling)
 {
-    const int t = tiling == kBlockTile ? kPT : 16;
+    const int t = tiling == kBlockTile ? kPT : tiling == kBlockMid ? 32 : 16;
     a.gx = (a.cols + t - 1) / t;
     a.gy = (a.nb + t - 1) / t;
     if (a.gx * a.gy >= 0x7fffffffL) throw std::length_error("block pass: too many tiles");
@@ -1808,22 +1956,28 @@ static void pass_grid(BlkPass& a, int tiling)
 template <bool OUT>
 static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, int tiling)
 {
-    if (!tiling) tiling = pass_tiling(a, OUT, false);
+    if (!tiling) tiling = pass_tiling(a, OUT, 0);
     pass_grid(a, tiling);
     const dim3 grid((unsigned)(a.gx * a.gy + (powers ? 1 : 0)));
-    const bool tile = tiling == kBlockTile, wide = tiling == kBlockSplit16;
-#define PARODE_PASS(TU)                                                                   \
-    do {                                                                                  \
-        if (tile && a.gx * a.gy <= 384)                                                   \
-            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 4>), grid, dim3(1024), 0, st, a);     \
-        else if (tile && a.gx * a.gy <= 768)                                              \
-            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 2>), grid, dim3(512), 0, st, a);      \
-        else if (tile)                                                                    \
-            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 1>), grid, dim3(256), 0, st, a);      \
-        else if (wide)                                                                    \
-            hipLaunchKernelGGL((k_blk_split<TU, OUT, 16>), grid, dim3(1024), 0, st, a);   \
-        else                                                                              \
-            hipLaunchKernelGGL((k_blk_split<TU, OUT, 4>), grid, dim3(256), 0, st, a);     \
+    const long tiles = a.gx * a.gy;
+#define PARODE_PASS(TU)                                                                     \
+    do {                                                                                    \
+        if (tiling == kBlockTile && tiles <= 384)                                          \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 4>), grid, dim3(1024), 0, st, a);       \
+        else if (tiling == kBlockTile && tiles <= 768)                                     \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 2>), grid, dim3(512), 0, st, a);        \
+        else if (tiling == kBlockTile)                                                      \
+            hipLaunchKernelGGL((k_blk_tile<TU, OUT, 1>), grid, dim3(256), 0, st, a);        \
+        else if (tiling == kBlockMid && tiles <= 256)                                       \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 16, 2>), grid, dim3(1024), 0, st, a);  \
+        else if (tiling == kBlockMid && tiles <= 512)                                       \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 8, 2>), grid, dim3(512), 0, st, a);    \
+        else if (tiling == kBlockMid)                                                       \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 4, 2>), grid, dim3(256), 0, st, a);    \
+        else if (tiling == kBlockSplit16)                                                   \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 16, 1>), grid, dim3(1024), 0, st, a);  \
+        else                                                                                \
+            hipLaunchKernelGGL((k_blk_split<TU, OUT, 4, 1>), grid, dim3(256), 0, st, a);    \
     } while (0)
     if (uDouble)
         PARODE_PASS(double);
@@ -1927,56 +2081,69 @@ static bool scan_plan(BlkScan a0, const BlockBufs& b, BlkScan& u, BlkScan& a, Bl
 }
 
 void block_tree_finish(hipStream_t st, const BlockShape& s, const BlockBufs& b,
-                       const BlockInput& in, long nb, const double* seed, double* tot)
+                       const BlockInput& in, long nb, const double* seed)
 {
-    const std::vector<TreeLevel> t = tree_of(nb);
-    const int top = (int)t.size() - 1;
-    hipLaunchKernelGGL(k_blk_root, dim3(1), dim3(1024), 0, st, scan_args(s, b, in, nb, seed),
-                       tree_s(s, b, t, top), tree_e(s, b, t, top), tot);
+    const std::vector<TreeLevel> t = tree_of(s, nb);
+    hipLaunchKernelGGL(k_blk_root, dim3((unsigned)((s.na + 15) / 16)), dim3(256), 0, st,
+                       scan_args(s, b, in, nb, seed), tree_e(s, b, t, (int)t.size() - 1));
     check_launch("block root");
+    for (int i = 0; i < block_tree_top_steps(s, nb); ++i) {
+        const GemmOp op = block_tree_top(s, b, nb, i);
+        gemm_multi(st, &op, 1);
+    }
     for (int j = 0; j < block_tree_down_steps(s, nb); ++j) {
         const std::vector<GemmOp> ops = block_tree_down(s, b, nb, j);
         gemm_multi(st, ops.data(), (int)ops.size());
     }
 }
 
+template <int MODE>
+static void launch_scan(hipStream_t st, const BlkScan& a)
+{
+    const int nct = (a.na + 15) / 16;
+    const dim3 grid((unsigned)a.gx), wg((unsigned)(64 * nct * a.R));
+    const size_t lds = scan_lds_bytes(a);
+    if (nct == 1)
+        hipLaunchKernelGGL((k_blk_scan<MODE, 4>), grid, wg, lds, st, a);
+    else if (nct == 2)
+        hipLaunchKernelGGL((k_blk_scan<MODE, 8>), grid, wg, lds, st, a);
+    else if (nct == 3)
+        hipLaunchKernelGGL((k_blk_scan<MODE, 12>), grid, wg, lds, st, a);
+    else
+        hipLaunchKernelGGL((k_blk_scan<MODE, 16>), grid, wg, lds, st, a);
+    check_launch("block scan");
+}
+
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                long nb, const double* seed, double* tot)
+                long nb, const double* seed)
 {
     if (s.wide) {
-        for (int k = 0; k < block_tree_up_levels(nb); ++k) {
+        for (int k = 0; k < block_tree_up_levels(s, nb); ++k) {
             const GemmOp op = block_tree_up(s, b, nb, k);
             gemm_multi(st, &op, 1);
         }
-        block_tree_finish(st, s, b, in, nb, seed, tot);
+        block_tree_finish(st, s, b, in, nb, seed);
         return;
     }
     BlkScan u, a, d;
     const bool groups = scan_plan(scan_args(s, b, in, nb, seed), b, u, a, d);
-    const int nct = (s.na + 15) / 16;
-    if (groups) {
-        hipLaunchKernelGGL(k_blk_scan<kScanUp>, dim3((unsigned)u.gx), dim3(64 * nct),
-                           scan_lds_bytes(u), st, u);
-        check_launch("block scan, up");
-    }
-    hipLaunchKernelGGL(k_blk_scan<kScanAll>, dim3(1), dim3(64 * nct * a.R), scan_lds_bytes(a), st,
-                       a);
-    check_launch("block scan");
-    if (groups) {
-        hipLaunchKernelGGL(k_blk_scan<kScanDown>, dim3((unsigned)d.gx), dim3(64 * nct),
-                           scan_lds_bytes(d), st, d);
-        check_launch("block scan, down");
-    }
+    if (groups) launch_scan<kScanUp>(st, u);
+    launch_scan<kScanAll>(st, a);
+    if (groups) launch_scan<kScanDown>(st, d);
 }
 
 void block_carry(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                 long nb, const double* seed, const double* tot, double* seedOut)
+                 long nb, const double* seed, double* seedOut)
 {
     const BlkScan a = scan_args(s, b, in, nb, seed);
     if (s.wide) {   // (nb is a power of two here)
+        const std::vector<TreeLevel> t = tree_of(s, nb);
+        const int top = (int)t.size() - 1;
+        const size_t at = (size_t)(t[top].n - 1) * s.na;
         hipLaunchKernelGGL(k_blk_carry_wide, dim3((s.na + 255) / 256), dim3(256),
                            s.na * sizeof(double), st, a,
-                           b.PT + (size_t)s.slot(s.lb + block_tree_up_levels(nb)) * s.na * s.na, tot,
+                           b.PT + (size_t)s.slot(s.lb + top) * s.na * s.na,
+                           tree_e(s, b, t, top) + at, tree_s(s, b, t, top) + at,
                            nb * s.s * s.T, nb * s.T * in.sL * s.m, seedOut);
         check_launch("block carry");
         return;
@@ -2000,7 +2167,6 @@ struct StartOutB {
 };
 struct RootB {
     BlkScan a;
-    const double* S;
     double* E;
     long gx;
 };
@@ -2033,11 +2199,11 @@ __global__ __launch_bounds__(256) void kg_blk_start_outputs(const StartOutB* __r
     d_start_outputs<double>(a.s, a.C, a.D, a.X0, a.U, a.Y);
 }
 // (a system's last work-group of pass 1 squares the rest of its powers, if any)
-template <bool OUT, int NW>
+template <bool OUT, int NW, int R>
 __global__ __launch_bounds__(NW * 64) void kg_blk_split(const BlkPass* __restrict__ args,
                                                         const unsigned* __restrict__ st, int ns)
 {
-    constexpr int kPart = (NW - 1) * 256;
+    constexpr int kPart = R > 1 ? NW * 256 * R * R : (NW - 1) * 256;
     constexpr int kLds = OUT || kPart > kBN * kBP ? kPart : kBN * kBP;
     __shared__ double lds[kLds];
     __shared__ int bad;
@@ -2048,11 +2214,11 @@ __global__ __launch_bounds__(NW * 64) void kg_blk_split(const BlkPass* __restric
         d_blk_powers<NW>(a.na, a.lb, a.L, a.PT, lds);
         return;
     }
-    d_blk_split<double, OUT, NW>(blk_place(idx, a.gx, a.gy), a, lds, &bad);
+    d_blk_split<double, OUT, NW, R>(blk_place(idx, a.gx, a.gy), a, lds, &bad);
 }
 template <bool OUT>
-__global__ __launch_bounds__(256) void kg_blk_tile(const BlkPass* __restrict__ args,
-                                                   const unsigned* __restrict__ st, int ns)
+__global__ __launch_bounds__(256, 4) void kg_blk_tile(const BlkPass* __restrict__ args,
+                                                      const unsigned* __restrict__ st, int ns)
 {
     __shared__ BlkTileLds<1> L;
     const int sys = system_of(st, ns);
@@ -2076,16 +2242,20 @@ __global__ __launch_bounds__(256) void kg_blk_root(const RootB* __restrict__ arg
                                                    const unsigned* __restrict__ st, int ns)
 {
     PARODE_GROUP(RootB);
-    (void)vb;
-    d_blk_root(a.a, a.S, a.E, nullptr);
+    d_blk_root(vb, a.a, a.E);
 }
 
-void add_pass(Phase& ph, BlkPass a, bool out, bool powers)
+void add_pass(Phase& ph, BlkPass a, bool out, bool powers, int group)
 {
-    const int t = pass_tiling(a, out, true);
+    const int t = pass_tiling(a, out, group);
     pass_grid(a, t);
     const float cost = (float)((out ? a.kz : 0) + a.ku);
-    append(ph, t == kBlockTile ? kBlkTile : t == kBlockSplit16 ? kBlkSplit16 : kBlkSplit4, out, a,
+    append(ph,
+           t == kBlockTile      ? kBlkTile
+           : t == kBlockMid     ? kBlkMid
+           : t == kBlockSplit16 ? kBlkSplit16
+                                : kBlkSplit4,
+           out, a,
            a.gx * a.gy + (powers ? 1 : 0), 0, cost);
 }
 
@@ -2115,14 +2285,14 @@ void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, con
     append(ph, kBlkStartOut, false, StartOutB{s, C, D, X0, U, Y, 1}, 1);
 }
 void add_block_pass1(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb)
+                     long nb, int group)
 {
-    add_pass(ph, pass1_args(s, b, in, nb), false, !s.wide);
+    add_pass(ph, pass1_args(s, b, in, nb), false, !s.wide, group);
 }
 void add_block_pass2(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb, long nReal, const double* seed, const float* D, float* Y)
+                     long nb, long nReal, const double* seed, const float* D, float* Y, int group)
 {
-    add_pass(ph, pass2_args(s, b, in, nb, nReal, seed, D, Y), true, false);
+    add_pass(ph, pass2_args(s, b, in, nb, nReal, seed, D, Y), true, false, group);
 }
 void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, const BlockBufs& b,
                     const BlockInput& in, long nb, const double* seed)
@@ -2137,10 +2307,11 @@ void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, con
 void add_block_root(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                     long nb, const double* seed)
 {
-    const std::vector<TreeLevel> t = tree_of(nb);
+    const std::vector<TreeLevel> t = tree_of(s, nb);
     const int top = (int)t.size() - 1;
-    append(ph, kBlkRoot, false, RootB{scan_args(s, b, in, nb, seed), tree_s(s, b, t, top),
-                                      tree_e(s, b, t, top), 1}, 1, 0, (float)s.na);
+    const long gx = (s.na + 15) / 16;
+    append(ph, kBlkRoot, false, RootB{scan_args(s, b, in, nb, seed), tree_e(s, b, t, top), gx}, gx, 0,
+           (float)(s.taps * s.m));
 }
 
 bool run_blocks(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dStart)
@@ -2164,15 +2335,21 @@ bool run_blocks(hipStream_t s, const Launch& L, const void* dArgs, const unsigne
         break;
     case kBlkSplit4:
         if (L.flag)
-            PARODE_RUN((kg_blk_split<true, 4>), BlkPass, 256);
+            PARODE_RUN((kg_blk_split<true, 4, 1>), BlkPass, 256);
         else
-            PARODE_RUN((kg_blk_split<false, 4>), BlkPass, 256);
+            PARODE_RUN((kg_blk_split<false, 4, 1>), BlkPass, 256);
+        break;
+    case kBlkMid:
+        if (L.flag)
+            PARODE_RUN((kg_blk_split<true, 8, 2>), BlkPass, 512);
+        else
+            PARODE_RUN((kg_blk_split<false, 8, 2>), BlkPass, 512);
         break;
     case kBlkSplit16:
         if (L.flag)
-            PARODE_RUN((kg_blk_split<true, 16>), BlkPass, 1024);
+            PARODE_RUN((kg_blk_split<true, 16, 1>), BlkPass, 1024);
         else
-            PARODE_RUN((kg_blk_split<false, 16>), BlkPass, 1024);
+            PARODE_RUN((kg_blk_split<false, 16, 1>), BlkPass, 1024);
         break;
     case kBlkScanUp: PARODE_RUN(kg_blk_scan<kScanUp>, BlkScan, 256); break;
     case kBlkScanAll: PARODE_RUN(kg_blk_scan<kScanAll>, BlkScan, 1024); break;

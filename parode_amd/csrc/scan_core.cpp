@@ -248,7 +248,7 @@ void ScanCore::build_powers(hipStream_t s, bool withLast)
 {
     if (uses_blocks()) {
         if (blk_.wide) {
-            wide_tables(s, dA_, dB_, dC_, dD_, nullptr, withLast, 0, nullptr);
+            wide_tables(s, dA_, dB_, dC_, dD_, nullptr, nPadMax_ >> blk_.lb, nullptr);
             powersDone_ = true;
             return;
         }
@@ -656,7 +656,7 @@ void ScanCore::sweep_top(hipStream_t s, long nReal, long nPad, const double* dSe
 {
     if (uses_blocks()) {
         batchSeed_ = dSeed;
-        k::block_scan(s, blk_, bb_, in_, blocks_of(nReal), dSeed, dTot);
+        k::block_scan(s, blk_, bb_, in_, blocks_of(nReal), dSeed);
         return;
     }
     const int L = ilog2(nPad), lt = top_level(nReal, nPad);
@@ -733,7 +733,7 @@ void ScanCore::carry(hipStream_t s, long nPad, const double* dSeed, const double
                      double* dOut)
 {
     if (uses_blocks()) {   // (a batch before the last is full)
-        k::block_carry(s, blk_, bb_, in_, nPad >> blk_.lb, dSeed, dTot, dOut);
+        k::block_carry(s, blk_, bb_, in_, nPad >> blk_.lb, dSeed, dOut);
         return;
     }
     k::carry(s, na_, powerT(ilog2(nPad)), dSeed, dTot, dOut);
@@ -868,7 +868,7 @@ int ScanCore::autotune_blocks(hipStream_t s, long nReal)
         for (int pass = 1; pass <= 2; ++pass) {
             int best = k::kBlockAuto;
             float bestMs = 0.0f;
-            for (int t : {k::kBlockTile, k::kBlockSplit4, k::kBlockSplit16}) {
+            for (int t : {k::kBlockTile, k::kBlockMid, k::kBlockSplit4, k::kBlockSplit16}) {
                 auto run = [&] {
                     if (pass == 1)
                         k::block_pass1(s, blk_, bb_, in, nb, false, t);
@@ -923,20 +923,20 @@ void BlockPhases::run(hipStream_t s, int from, int to) const
 // The tables of a wide map.  With pass1 (which queues pass 1), also the tree's up
 // products: a launch of them beside each squaring that only the tree reads.
 void ScanCore::wide_tables(hipStream_t s, const float* dA, const float* dB, const float* dC,
-                           const float* dD, const float* dx0, bool withLast, long nb,
+                           const float* dD, const float* dx0, long nb,
                            const std::function<void()>& pass1)
 {
     BlockPhases ph;
     std::vector<int> ready;
+    const int top = k::block_tree_up_levels(blk_, nb);
     const int done = k::block_emit(blk_, bb_, h_, dA, dB, dC, dD, dx0, seed(),
-                                   withLast ? L_ : L_ - 1, ph, &ready);
+                                   blk_.lb + top, ph, &ready);
     if (!pass1) {
         ph.run(s, 0, (int)ph.ph.size());
         return;
     }
     ph.run(s, 0, done);
     pass1();
-    const int top = k::block_tree_up_levels(nb);
     int up = 0;
     for (int p = done; p < (int)ph.ph.size() || up < top; ++p) {
         BlockPhases::Phase& f = ph.at(p);
@@ -969,7 +969,7 @@ void ScanCore::solve_blocks(hipStream_t s, long nScan, double h, const float* dA
             k::block_start_outputs(ps, blk_, dC, dD, seed(), dU, uDouble, dY);
             if (side) PARODE_HIP(hipEventRecord(side->join, ps));
         }
-        wide_tables(s, dA, dB, dC, dD, dx0, false, nb, [&] {
+        wide_tables(s, dA, dB, dC, dD, dx0, nb, [&] {
             tick(1);
             k::block_pass1(s, blk_, bb_, in, nb, false, block_tiling(1, nb, uDouble));
             tick(2);

@@ -180,7 +180,7 @@ private:
                       const float* dC, const float* dD, const float* dx0, const void* dU,
                       bool uDouble, float* dY, hipEvent_t* marks, const SideStream* side);
     void wide_tables(hipStream_t s, const float* dA, const float* dB, const float* dC,
-                     const float* dD, const float* dx0, bool withLast, long nb,
+                     const float* dD, const float* dx0, long nb,
                      const std::function<void()>& pass1);
     k::BlockInput block_input(const void* dU, bool uDouble, long sL, long nReal) const;
     long blocks_of(long nReal) const { return (nReal + blk_.T - 1) / blk_.T; }
