@@ -164,9 +164,9 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
                 k::g::add_block_scan(P[kUp0 + upSteps - 1], P[kTop], P[kDown0], c.blk_, c.bb_, bin,
                                      nb, c.seed());
             }
-            k::g::add_block_pass1(P[kChunk1], c.blk_, c.bb_, bin, nb, (int)systems.size());
+            k::g::add_block_pass1(P[kChunk1], c.blk_, c.bb_, bin, nb);
             k::g::add_block_pass2(P[kChunk2], c.blk_, c.bb_, bin, nb, s.nScan, c.seed(), q.D,
-                                  yScan, (int)systems.size());
+                                  yScan);
             return;
         }
         const size_t nn = (size_t)n * n, nm = (size_t)n * m, na2 = (size_t)na * na;

@@ -170,9 +170,9 @@ void add_block_elem(Phase& ph, const BlkElem& e);
 void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, const float* D,
                              const double* X0, const double* U, float* Y);
 void add_block_pass1(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb, int group);
+                     long nb);
 void add_block_pass2(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb, long nReal, const double* seed, const float* D, float* Y, int group);
+                     long nb, long nReal, const double* seed, const float* D, float* Y);
 // the scan of a map that is not wide: up and down are used when the blocks go in groups
 void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, const BlockBufs& b,
                     const BlockInput& in, long nb, const double* seed);

@@ -1457,11 +1457,15 @@ static int group_log(long nb)
     return lg;
 }
 // The rule: which systems run as block responses, and with how many steps per
-// block: the fastest by the model below, if it beats the general path's.
-// Covered: inputs and outputs present, horizons from 64 points.  More steps per
-// block make the scan shorter (2 n_a^2 products a block, and its chain of
-// dependent steps), fewer make pass 2 (s m p T / 2 products a step) and the
-// tables (2 n_a^2 (s m + p) T) cheaper.
+// block: the fastest by the model below.  Covered: inputs and outputs present,
+// horizons from 64 points, n up to 1024.  The general path was nowhere faster on
+// either side's edges (us, general against blocks: RK4 n = 65, 64 points 172, 65;
+// n = 1000, 100 points 789, 571; n = 100, 100 inputs and outputs, 5000 points 246,
+// 241; ABM n = 256, 80 points 695, 370; n = 600, 100 points 10531, 10638, the
+// start-up's; n = 17, 2^20 points 660, 261).  More steps per block make the scan
+// shorter (2 n_a^2 products a block, and its chain of dependent steps), fewer make
+// pass 2 (s m p T / 2 products a step) and the tables (2 n_a^2 (s m + p) T)
+// cheaper.
 int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long nScan, long nPad)
 {
     const int na = method == 1 ? 4 * n : n, s = method == 1 ? 1 : 2;
@@ -1503,13 +1507,7 @@ int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long 
             bt = t;
         }
     }
-    if (!best || one) return best;
-    // the general path: two chunk passes (or tree levels) in FP32, FP64 leaves
-    // and outputs, levels
-    const double step = method == 1 ? 8.0 * n * n : 4.0 * n * n;
-    const double general = N * (step / 45e6 + (2.0 * n * m * (method == 1 ? 2 : 3) + 2.0 * p * (n + m)) / 15e6) +
-                           10.0 * std::log2(N) + (n <= 256 ? std::min(N / 512, 256.0) * 1.5 : N * step / 45e6);
-    return bt < general ? best : 0;
+    return best;
 }
 
 BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bool mirror, int lb,
@@ -1929,20 +1927,21 @@ static BlkPass pass_args(const BlockShape& s, const BlockBufs& b, const BlockInp
     return a;
 }
 
-// The tiling of a pass, alone (group 0) or in a launch of `group` systems: 64 x 64
-// tiles from 64 of them (n_a = 48, 2^18 points: 208 us a solve against 262 from
-// 192; n_a = 37, 50 001 points: 135 against 169 from 16), 16 x 16 while those are
-// at most one for each compute unit, K over 16 waves where it is long (or where
-// a work-group of pass 1 squares powers: 6 squarings of 48 x 48 take 10 us with
-// 16 waves, 34 with 4), 32 x 32 between.  Systems launched together fill the
-// GPU between them: the wider tiles from fewer (64 small systems: 785 us from 32
-// and 64, 897 from 64 and 256; 512 systems 43.3 ms against 48).
-static int pass_tiling(const BlkPass& a, bool out, int group)
+// The tiling of a pass, alone or in a grouped launch: 64 x 64 tiles from 64 of
+// them (n_a = 48, 2^18 points: 208 us a solve against 262 from 192; n_a = 37,
+// 50 001 points: 135 against 169 from 16), 16 x 16 while those are at most one
+// for each compute unit, K over 16 waves where it is long (or where a work-group
+// of pass 1 squares powers: 6 squarings of 48 x 48 take 10 us with 16 waves, 34
+// with 4), 32 x 32 between.  Systems launched together fill the GPU between them:
+// the wider tiles from fewer (64 small systems: 785 us from 32 and 64, 897 from 64
+// and 256; 512 systems 43.3 ms against 48), whatever the group, so that a
+// system's results do not depend on it.
+static int pass_tiling(const BlkPass& a, bool out, bool grouped)
 {
     const long tx = (a.cols + kPT - 1) / kPT, ty = (a.nb + kPT - 1) / kPT;
     const long sx = (a.cols + 15) / 16, sy = (a.nb + 15) / 16;
-    if (tx * ty >= (group > 1 ? 32 : 64)) return kBlockTile;
-    if (sx * sy > (group > 1 ? std::max(64, 256 / group) : 256)) return kBlockMid;
+    if (tx * ty >= (grouped ? 32 : 64)) return kBlockTile;
+    if (sx * sy > (grouped ? 64 : 256)) return kBlockMid;
     return (!out && a.na > 16) || ((out ? a.kz : 0) + a.ku) / 4 >= 64 ? kBlockSplit16 : kBlockSplit4;
 }
 static void pass_grid(BlkPass& a, int tiling)
@@ -1956,7 +1955,7 @@ static void pass_grid(BlkPass& a, int tiling)
 template <bool OUT>
 static void launch_pass(hipStream_t st, BlkPass a, bool uDouble, bool powers, int tiling)
 {
-    if (!tiling) tiling = pass_tiling(a, OUT, 0);
+    if (!tiling) tiling = pass_tiling(a, OUT, false);
     pass_grid(a, tiling);
     const dim3 grid((unsigned)(a.gx * a.gy + (powers ? 1 : 0)));
     const long tiles = a.gx * a.gy;
@@ -2245,9 +2244,9 @@ __global__ __launch_bounds__(256) void kg_blk_root(const RootB* __restrict__ arg
     d_blk_root(vb, a.a, a.E);
 }
 
-void add_pass(Phase& ph, BlkPass a, bool out, bool powers, int group)
+void add_pass(Phase& ph, BlkPass a, bool out, bool powers)
 {
-    const int t = pass_tiling(a, out, group);
+    const int t = pass_tiling(a, out, true);
     pass_grid(a, t);
     const float cost = (float)((out ? a.kz : 0) + a.ku);
     append(ph,
@@ -2285,14 +2284,14 @@ void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, con
     append(ph, kBlkStartOut, false, StartOutB{s, C, D, X0, U, Y, 1}, 1);
 }
 void add_block_pass1(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb, int group)
+                     long nb)
 {
-    add_pass(ph, pass1_args(s, b, in, nb), false, !s.wide, group);
+    add_pass(ph, pass1_args(s, b, in, nb), false, !s.wide);
 }
 void add_block_pass2(Phase& ph, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
-                     long nb, long nReal, const double* seed, const float* D, float* Y, int group)
+                     long nb, long nReal, const double* seed, const float* D, float* Y)
 {
-    add_pass(ph, pass2_args(s, b, in, nb, nReal, seed, D, Y), true, false, group);
+    add_pass(ph, pass2_args(s, b, in, nb, nReal, seed, D, Y), true, false);
 }
 void add_block_scan(Phase& up, Phase& all, Phase& down, const BlockShape& s, const BlockBufs& b,
                     const BlockInput& in, long nb, const double* seed)

@@ -4209,7 +4209,7 @@ struct Prep {        // kind 0: out = (double)in; 1: out = v; 2: out[r][c] = in[
     long gx;
 };
 struct Gemm {
-    int r, kk, c;
+    int r, kk, c, t;
     const double *X, *Y;
     double* Z;
     GemmLd ld;
@@ -4358,26 +4358,19 @@ __global__ __launch_bounds__(256) void kg_prep(const Prep* __restrict__ args,
     }
 }
 
-// FP64 products of one phase in one launch: each system's 64 x 64 tiles, or,
-// for a narrow product, its K-split 16 x 16 tiles (the two tilings in separate
-// launches would run one after the other on the stream)
+// FP64 products of one phase in one launch, each in its own tiling (the tilings in
+// separate launches would run one after the other on the stream)
 __global__ __launch_bounds__(256) void kg_gemm(const Gemm* __restrict__ args,
                                                const unsigned* __restrict__ st, int ns)
 {
     PARODE_GROUP(Gemm);
     __shared__ double lds[sizeof(GemmStage) / sizeof(double)];
-    if (gemm_wide(a.r, a.kk, a.c))
+    if (a.t == 64)
         d_gemm_f64_t64<1>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, lds);
+    else if (a.t == 32)
+        d_gemm_f64_w32<4, 2>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, lds);
     else
         d_gemm_f64_mfma<4>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, lds);
-}
-
-__global__ __launch_bounds__(512) void kg_gemm_ks2(const Gemm* __restrict__ args,
-                                                   const unsigned* __restrict__ st, int ns)
-{
-    PARODE_GROUP(Gemm);
-    extern __shared__ double gsm[];
-    d_gemm_f64_ks<2>(vb, a.r, a.kk, a.c, a.X, a.Y, a.Z, a.ld, gsm);
 }
 
 __global__ __launch_bounds__(256) void kg_rk4_combine(const Rk4Comb* __restrict__ args,
@@ -4641,25 +4634,25 @@ void add_gemm_ld(Phase& ph, int r, int kk, int c, const double* X, int ldx, cons
                  int ldy, double* Z, int ldz, const double* add, int shift)
 {
     if (r <= 0 || c <= 0) return;
-    const GemmLd ld{ldx, ldy, ldz, add, ldz, shift};
-    // (a work-group's matrix-core instructions per wave: kk for a 64 x 64 tile,
-    // kk / 16 for a K-split 16 x 16 tile)
-    if (gemm_wide(r, kk, c)) {
-        const long gx = (c + kG64 - 1) / kG64, gy = (r + kG64 - 1) / kG64;
-        append(ph, kGemm, false, Gemm{r, kk, c, X, Y, Z, ld, gx}, gx * gy, 0, (float)kk);
-    } else {
-        const long gx = (c + 15) / 16, gy = (r + 15) / 16;
-        append(ph, kGemm, false, Gemm{r, kk, c, X, Y, Z, ld, gx}, gx * gy, 0, kk / 16.0f);
-    }
+    add_gemm_op(ph, GemmOp{r, kk, c, X, Y, Z, GemmLd{ldx, ldy, ldz, add, ldz, shift}});
 }
 
+// Tiles of 64 from 32 of them (512 systems of up to 1024 states 42.8 ms a batch when
+// every product that they suit takes them, 44.1 from 64 of them: their rate counts),
+// else of 32 (64 systems of up to 256 states 617 us against 733: a tile's time
+// counts).  By the product alone: a system's results do not depend on what it is
+// launched with.
 void add_gemm_op(Phase& ph, const GemmOp& o)
 {
     if (o.r <= 0 || o.c <= 0) return;
-    const int t = gemm_wide(o.r, o.kk, o.c) ? kG64 : 16;
+    const long t64 = (long)((o.r + 63) / 64) * ((o.c + 63) / 64);
+    const long t16 = (long)((o.r + 15) / 16) * ((o.c + 15) / 16);
+    const int t = gemm_wide(o.r, o.kk, o.c) && t64 >= 32 ? 64 : t16 <= 64 ? 16 : 32;
     const long gx = (o.c + t - 1) / t, gy = (o.r + t - 1) / t;
-    append(ph, kGemm, false, Gemm{o.r, o.kk, o.c, o.X, o.Y, o.Z, o.ld, gx}, gx * gy, 0,
-           t == kG64 ? (float)o.kk : o.kk / 16.0f);
+    // (a work-group's matrix-core instructions per wave: kk for a 64 x 64 tile,
+    // kk / 4 for a K-split 32 x 32 tile, kk / 16 for a 16 x 16 one)
+    append(ph, kGemm, false, Gemm{o.r, o.kk, o.c, t, o.X, o.Y, o.Z, o.ld, gx}, gx * gy, 0,
+           (float)o.kk / (t == 64 ? 1 : t == 32 ? 4 : 16));
 }
 
 void add_rk4_combine(Phase& ph, int n, int m, double h, const double* A, const double* A2,
@@ -4958,7 +4951,6 @@ void run(hipStream_t s, const Launch& L, const void* dArgs, const unsigned* dSta
     switch (L.kind) {
     case kPrep: PARODE_RUN(kg_prep, Prep, 256); break;
     case kGemm: PARODE_RUN(kg_gemm, Gemm, 256); break;
-    case kGemmKs2: PARODE_RUN(kg_gemm_ks2, Gemm, 512); break;
     case kRk4Combine: PARODE_RUN(kg_rk4_combine, Rk4Comb, 256); break;
     case kAbmCombine: PARODE_RUN(kg_abm_combine, AbmComb, 256); break;
     case kTranspose: PARODE_RUN(kg_transpose, Transpose, 256); break;
