@@ -10,6 +10,12 @@ class AdamsMoulton : public GPUODESolverFixedStepIterative {
 private:
 	std::vector<vectorf> _UInit;   /* the 9 start-up input samples (h/2 grid) */
 	double _tOrigin;               /* tStart before the start-up shift */
+	/* the start-up states and inputs on their way to pinned memory (null once
+	 * they are taken over) */
+	const double* _pInitStates = nullptr;
+	const void* _pInitInputs = nullptr;
+	bool _bInitInputsDouble = false;
+	void TakeInitialState();
 	void ComputeInitialState(const matrixf& A, const matrixf& B, const vectorf& x0,
 							 double fDeltaT, double tStart, vectorf& x0Scan);
 

@@ -58,6 +58,25 @@ protected:
 	const void* _pSampledInput;
 	bool _bSampledDouble;
 	std::unique_ptr<DeviceBuffer> _BufferSampled;
+	/* blocks of the shared device workspace and pinned staging that this
+	 * simulation holds (given back once the stream has finished) */
+	std::unique_ptr<DeviceBuffer> _BufferSystem;     /* A, B, x0 (C, D) */
+	std::vector<void*> _vectLeased, _vectStaged;
+	const matrixf* _pSystemC;                        /* uploaded beside A, B and x0 when set */
+	const matrixf* _pSystemD;
+
+	/* where the outputs go: the matrix or the array form's result */
+	struct OutputSink;
+	/* bOwnSolver: the solver is one of this library's own, whose start-up values
+	 * and times may be made while the GPU works */
+	ErrorCode Run(const matrixf& A, const matrixf& B, const matrixf& C, const matrixf& D,
+				  double tStart, double tEnd, double tStep, const vectorf& x0,
+				  OutputSink& sink, bool bOwnSolver);
+	bool IsOwnSolver() const;
+	/* a device buffer in the shared workspace, or one of its own */
+	std::unique_ptr<DeviceBuffer> NewBuffer(std::size_t bytes);
+	/* pinned host memory until the simulation ends, or null */
+	void* Stage(std::size_t bytes);
 
 	void SetStrides(int nInputStride, int nStateStride, int nInputOffset = 0, int nStateOffset = 0) {
 		_bStrideSet = true;
@@ -100,6 +119,10 @@ public:
 	virtual ErrorCode SimulateODE(const matrixf& A, const matrixf& B, const matrixf& C, const matrixf& D,
 								  double tStart, double tEnd, double tStep,
 								  const vectorf& x0, vectorf& tVect, matrixf& xVect);
+	/* the array form without the matrix between, for this library's own solvers */
+	virtual ErrorCode SimulateODE(const matrixf& A, const matrixf& B, const matrixf& C, const matrixf& D,
+								  double tStart, double tEnd, double tStep,
+								  const vectorf& x0, fType tVect[], fType xVect[], int& nSteps);
 	using GPUODESolver::SimulateODE;
 
 	/* 0 = plain FP32 (reference parity), 1 = mixed precision, 2 = FP64 scan */

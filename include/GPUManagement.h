@@ -7,8 +7,12 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
+
+namespace parode { class Arena; }
 
 /* A device allocation, owning or a non-owning view (the role of
  * OpenCLMemBuffer, GPUManagement.h:130-160 of the reference). */
@@ -56,6 +60,15 @@ public:
 	/* GPU timer on device 0's stream, milliseconds (GPUManagement.cpp:216-268) */
 	void StartTimer();
 	float StopTimer();
+	/* memory that the simulations of one initialisation share instead of
+	 * allocating on each call: kWorkspaceBytes on the first device and
+	 * kStagingBytes of pinned host memory, made at the first use and given back
+	 * with the devices; thread-safe; null when it cannot be had (callers then
+	 * allocate).  A block goes back only when the work on it is done. */
+	static constexpr std::size_t kWorkspaceBytes = 256u << 20;
+	static constexpr std::size_t kStagingBytes = 8u << 20;
+	parode::Arena* Workspace();
+	parode::Arena* Staging();
 
 private:
 	void Release();
@@ -64,6 +77,8 @@ private:
 	std::vector<hipDeviceProp_t> _props;
 	hipEvent_t _t0 = nullptr, _t1 = nullptr;
 	bool _timerStarted = false;
+	std::mutex _sharedMutex;
+	std::unique_ptr<parode::Arena> _workspace, _staging;
 };
 
 #endif /* PARODE_GPUMANAGEMENT_H_ */

@@ -47,6 +47,8 @@ void GPUManagement::Release()
         (void)hipStreamSynchronize(_streams[i]);
         (void)hipStreamDestroy(_streams[i]);
     }
+    _workspace.reset();
+    _staging.reset();
     if (_t0) (void)hipEventDestroy(_t0);
     if (_t1) (void)hipEventDestroy(_t1);
     _t0 = _t1 = nullptr;
@@ -91,6 +93,34 @@ bool GPUManagement::Initialize(const std::vector<unsigned int>& selected, int)
     PARODE_HIP(hipEventCreate(&_t0));
     PARODE_HIP(hipEventCreate(&_t1));
     return true;
+}
+
+parode::Arena* GPUManagement::Workspace()
+{
+    std::lock_guard<std::mutex> g(_sharedMutex);
+    if (!_workspace && !_devices.empty()) {
+        try {
+            SetCurrent(0);
+            _workspace.reset(new parode::Arena(kWorkspaceBytes, parode::Arena::kDevice));
+        } catch (std::exception&) {
+            (void)hipGetLastError();
+        }
+    }
+    return _workspace.get();
+}
+
+parode::Arena* GPUManagement::Staging()
+{
+    std::lock_guard<std::mutex> g(_sharedMutex);
+    if (!_staging && !_devices.empty()) {
+        try {
+            SetCurrent(0);
+            _staging.reset(new parode::Arena(kStagingBytes, parode::Arena::kPinnedHost));
+        } catch (std::exception&) {
+            (void)hipGetLastError();
+        }
+    }
+    return _staging.get();
 }
 
 std::string GPUManagement::GetDeviceName(unsigned int id)
