@@ -26,8 +26,20 @@ __device__ __forceinline__ doublex4 lds_tile(const double* X, int px, const doub
     const double* xr = X + (i0 + l16) * px + q4;
     const double* yr = YT ? Y + (j0 + l16) * py + q4 : Y + q4 * py + j0 + l16;
     const int ys = YT ? 1 : py;
-    for (int k = 0; k < kk; k += 4)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(xr[k], yr[k * ys], acc, 0, 0, 0);
+    // (kk: whole 16; a chunk's operands are read before its products: one LDS round
+    // trip for four)
+#pragma unroll 1
+    for (int k = 0; k < kk; k += 16) {
+        double x[4], y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            x[u] = xr[k + 4 * u];
+            y[u] = yr[(k + 4 * u) * ys];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[u], y[u], acc, 0, 0, 0);
+    }
     return acc;
 }
 
@@ -1884,24 +1896,33 @@ void block_start_outputs(hipStream_t st, const BlockShape& s, const float* C, co
     check_launch("block start outputs");
 }
 
-// steps of a slice: the largest power of two whose rows fit the LDS
-static int slice_steps(int T, int per)
+// steps of a slice: the largest power of two of at most `rows` rows (at least one
+// step: per rows, which fit the LDS)
+static int slice_steps(int T, int per, int rows)
 {
     int k = 1;
-    while (2 * k <= T && 2 * k * per <= kBN) k *= 2;
+    while (2 * k <= T && 2 * k * per <= rows) k *= 2;
     return k;
 }
 
-static BlkTables table_args(const BlockShape& s, const BlockBufs& b, const float* C)
+static BlkTables table_args(const BlockShape& s, const BlockBufs& b, const float* C, bool grouped)
 {
-    BlkTables a{s, C, b.PT, b.QT, b.OT, b.Ht, slice_steps(s.T, s.p), slice_steps(s.T, s.s * s.m), 0};
-    a.gx = 1 + s.T / a.ni + s.T / a.nq;
+    BlkTables a{s, C, b.PT, b.QT, b.OT, b.Ht, 0, 0, 0};
+    // Short slices while each has its compute unit: a level's time is that of its
+    // products on one (n_a = 48: 20 us for six levels with 64 rows, 15.5 with 16).
+    // Together with other systems the longest, since each slice squares for itself.
+    for (int rows = grouped ? kBN : 16; rows <= kBN; rows *= 2) {
+        a.ni = slice_steps(s.T, s.p, rows);
+        a.nq = slice_steps(s.T, s.s * s.m, rows);
+        a.gx = 1 + s.T / a.ni + s.T / a.nq;
+        if (a.gx <= 256) break;
+    }
     return a;
 }
 
 void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C)
 {
-    const BlkTables a = table_args(s, b, C);
+    const BlkTables a = table_args(s, b, C, false);
     hipLaunchKernelGGL(k_blk_tables, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     check_launch("block_tables");
 }
@@ -2270,7 +2291,7 @@ void add_block_map(Phase& ph, const BlockShape& s, const BlockBufs& b, double h,
 }
 void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, const float* C)
 {
-    const BlkTables a = table_args(s, b, C);
+    const BlkTables a = table_args(s, b, C, true);
     append(ph, kBlkTables, false, a, a.gx, 0, (float)s.na * s.lb);
 }
 void add_block_elem(Phase& ph, const BlkElem& e)
