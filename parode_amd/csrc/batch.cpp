@@ -81,7 +81,7 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
                 blkRest = std::max(blkRest, (int)s.ops.ph.size() - s.ready);
             } else {
                 upSteps = std::max(upSteps, 1);
-                blkSteps = std::max(blkSteps, 2);
+                blkSteps = std::max(blkSteps, 1);
             }
             continue;
         }
@@ -158,9 +158,8 @@ BatchSolve::BatchSolve(const std::vector<BatchSystem>& systems, Arena* arena)
                         k::g::add_gemm_op(P[kDown0 + t], o);
                 k::g::add_block_root(P[kTop], c.blk_, c.bb_, bin, nb, c.seed());
             } else {
-                k::g::add_block_map(P[kBlk0], c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0,
-                                    c.seed());
-                k::g::add_block_tables(P[kBlk0 + 1], c.blk_, c.bb_, q.C);
+                k::g::add_block_tables(P[kBlk0], c.blk_, c.bb_, q.h, q.A, q.B, q.C, q.D, q.x0,
+                                       c.seed());
                 k::g::add_block_scan(P[kUp0 + upSteps - 1], P[kTop], P[kDown0], c.blk_, c.bb_, bin,
                                      nb, c.seed());
             }

@@ -137,16 +137,14 @@ void block_tree_finish(hipStream_t st, const BlockShape& s, const BlockBufs& b,
                        const BlockInput& in, long nb, const double* seed);
 void block_elem(hipStream_t st, const BlkElem& e);
 
-// M, G, the direct terms and (x0 given) the seed: x0, or with the ABM start-up
-// the states x_0..x_3 and their three outputs.  (Maps that are not wide.)
-void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
-               const float* B, const float* C, const float* D, const float* x0, const void* U,
-               bool uDouble, double* seed, float* Y);
+// M, G, the direct terms, the tables (P_0 .. P_lb) and (x0 given) the seed: x0, or
+// the ABM start-up's states x_0..x_3 and its three outputs.  (Maps that are not wide.)
+void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                  const float* B, const float* C, const float* D, const float* x0, const void* U,
+                  bool uDouble, double* seed, float* Y);
 // the outputs of the ABM start-up states (X0: x_0 .. x_3)
 void block_start_outputs(hipStream_t st, const BlockShape& s, const float* C, const float* D,
                          const double* X0, const void* U, bool uDouble, float* Y);
-// PT up to P_lb, QT, OT, Ht
-void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C);
 // the blocks' responses from zero (and, with powers, the rest of PT)
 void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                  long nb, bool powers, int tiling = kBlockAuto);
@@ -163,9 +161,8 @@ void block_pass2(hipStream_t st, const BlockShape& s, const BlockBufs& b, const 
 
 // ---- the same launches for many systems in one grid (FP64 samples)
 namespace g {
-void add_block_map(Phase& ph, const BlockShape& s, const BlockBufs& b, double h, const float* A,
-                   const float* B, const float* C, const float* D, const float* x0, double* seed);
-void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, const float* C);
+void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                      const float* B, const float* C, const float* D, const float* x0, double* seed);
 void add_block_elem(Phase& ph, const BlkElem& e);
 void add_block_start_outputs(Phase& ph, const BlockShape& s, const float* C, const float* D,
                              const double* X0, const double* U, float* Y);

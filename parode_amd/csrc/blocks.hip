@@ -44,17 +44,25 @@ __device__ __forceinline__ doublex4 lds_tile(const double* X, int px, const doub
 }
 
 // ------------------------------------------------------------------- the map
-struct BlkMap {
+struct BlkTables {
     BlockShape s;
     double h;
     Rk4Coef rk;
     AbmCoef ab;
     const float *A, *B, *C, *D, *x0;
     const void* U;
-    double *PT, *QT, *Ht, *DL, *seed;
+    double *PT, *QT, *OT, *Ht, *DL, *seed;
     float* Y;
+    int ni, nq;   // steps of a slice of OT (and Ht), of a slice of QT
     long gx;
 };
+// LDS of a work-group (doubles): P = P_l (transposed power, [n16][kBP]), the rows R of
+// its slice and the input block G ([s m] rows); the map's own arrays lie in R's and
+// G's places (RK4) or behind them (ABM)
+constexpr int kTabR = kBN * kBP, kTabG = 2 * kBN * kBP, kTabMap = 3 * kBN * kBP;
+constexpr int kTabLds = kTabMap + 5280;
+static_assert(2 * kBN * kBP + 4 * kBN * (kBM + 1) <= kTabLds, "room for the RK4 map");
+
 
 // Z = X Y with the reference's rounding: float products, sequential float sums.
 __device__ __forceinline__ void lds_mul_seq(int r, int kk, int c, const float* X, int px,
@@ -72,12 +80,12 @@ __device__ __forceinline__ void lds_mul_seq(int r, int kk, int c, const float* X
     }
 }
 
-// One work-group makes a small system's map (n_a <= 64, m <= 32) in LDS: the
-// step map M, the block input G, the direct terms F and the state's shift D
+// A work-group makes a small system's map (n_a <= 64, m <= 32) in LDS, P_0 and G to
+// its tables' places, and (store) to memory: the step map M, the block input G, the direct terms F and the state's shift D
 // (blocks.h).  RK4 by Horner's scheme, M = I + hA (I + hA/2 (I + hA/3 (I +
 // hA/4))), beside the products A^k B; with the reference's rounding by its own
 // products A^2, A^3, A^4.  A chain of a few dependent 64 x 64 products: latency.
-__device__ __forceinline__ void d_blk_map_rk4(const BlkMap& a, double* lds)
+__device__ __forceinline__ void d_blk_map_rk4(const BlkTables& a, double* lds, bool store)
 {
 #pragma clang fp contract(off)
     const BlockShape& s = a.s;
@@ -206,28 +214,51 @@ __device__ __forceinline__ void d_blk_map_rk4(const BlkMap& a, double* lds)
     }
     // Ts = M; Kb[0], Kb[1], Kb[3] = the three input blocks of a step.
     // G = [B1 + M B3 | B2], the shift and the direct term from B3
-    double* GT = a.QT + (long)s.s * (s.T - 1) * m * n;
-    for (int w = wave; w < nt * mt; w += 16) {
-        const int i0 = w / mt * 16, j0 = w % mt * 16;
-        const doublex4 acc = lds_tile<false>(Ts, kBP, Kb[3], KP, i0, j0, n16);
+    const int gi = wave / mt * 16, gj = wave % mt * 16;
+    const bool mine = wave < nt * mt;   // (at most 4 x 2 tiles)
+    double g1[4], g2[4];
+    if (mine) {
+        const doublex4 acc = lds_tile<false>(Ts, kBP, Kb[3], KP, gi, gj, n16);
         for (int v = 0; v < 4; ++v) {
-            const int i = i0 + 4 * v + q4, j = j0 + l16;
-            if (i >= n || j >= m) continue;
-            GT[(long)j * n + i] = Kb[0][i * KP + j] + acc[v];
-            GT[(long)(m + j) * n + i] = Kb[1][i * KP + j];
+            const int x = (gi + 4 * v + q4) * KP + gj + l16;
+            g1[v] = Kb[0][x] + acc[v];
+            g2[v] = Kb[1][x];
         }
     }
-    for (int t = tid; t < n * n; t += 1024) a.PT[t] = Ts[(t % n) * kBP + t / n];
-    for (int t = tid; t < m * n; t += 1024) a.DL[t] = Kb[3][(t % n) * KP + t / n];
-    double* F = a.Ht + (long)s.s * (s.T - 1) * m * p;
-    for (int t = tid; t < m * p; t += 1024) {
-        const int j = t / p, o = t - j * p;
-        double v = 0.0;
-        if (s.useC)
-            for (int i = 0; i < n; ++i) v = fma((double)a.C[(long)o * n + i], Kb[3][i * KP + j], v);
-        else
-            v = Kb[3][o * KP + j];
-        F[t] = v + (s.useD ? (double)a.D[(long)o * m + j] : 0.0);
+    for (int t = tid; t < n16 * n16; t += 1024) {
+        const int r = t / n16, c = t - r * n16;
+        const double v = r < n && c < n ? Ts[c * kBP + r] : 0.0;
+        As[r * kBP + c] = v;   // (P)
+        if (store && r < n && c < n) a.PT[(long)r * n + c] = v;
+    }
+    if (store) {
+        for (int t = tid; t < m * n; t += 1024) a.DL[t] = Kb[3][(t % n) * KP + t / n];
+        double* F = a.Ht + (long)s.s * (s.T - 1) * m * p;
+        for (int t = tid; t < m * p; t += 1024) {
+            const int j = t / p, o = t - j * p;
+            double v = 0.0;
+            if (s.useC)
+                for (int i = 0; i < n; ++i) v = fma((double)a.C[(long)o * n + i], Kb[3][i * KP + j], v);
+            else
+                v = Kb[3][o * KP + j];
+            F[t] = v + (s.useD ? (double)a.D[(long)o * m + j] : 0.0);
+        }
+    }
+    __syncthreads();
+    double* G = lds + kTabG;
+    double* GT = a.QT + (long)s.s * (s.T - 1) * m * n;
+    for (int t = tid; t < kBN * n16; t += 1024) G[t / n16 * kBP + t % n16] = 0.0;
+    __syncthreads();
+    if (!mine) return;
+    for (int v = 0; v < 4; ++v) {
+        const int i = gi + 4 * v + q4, j = gj + l16;
+        if (i >= n || j >= m) continue;
+        G[j * kBP + i] = g1[v];
+        G[(m + j) * kBP + i] = g2[v];
+        if (store) {
+            GT[(long)j * n + i] = g1[v];
+            GT[(long)(m + j) * n + i] = g2[v];
+        }
     }
 }
 
@@ -235,13 +266,13 @@ __device__ __forceinline__ void d_blk_map_rk4(const BlkMap& a, double* lds)
 // blocks V_0 = B_4, V_t = B_{4-t} + sum_{i < t} M_{4-t+i} V_i (M_b: R's blocks,
 // oldest first; B_q: the step's input blocks), which give
 // G = [V_1; V_2; V_3; V_4], D_r = [0 (r blocks); V_0 .. V_{3-r}], F_r = C V_{3-r}.
-__device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
+__device__ __forceinline__ void d_blk_map_abm(const BlkTables& a, double* lds, bool store)
 {
 #pragma clang fp contract(off)
     const BlockShape& s = a.s;
     const int n = s.n, m = s.m, p = s.p, na = s.na, tid = threadIdx.x;
     constexpr int AP = 17, KP = kBM + 1;
-    double* A1 = lds;                  // [16][AP]
+    double* A1 = lds + kTabMap;        // [16][AP]
     double* A2 = A1 + 16 * AP;
     double* B1 = A2 + 16 * AP;         // [16][KP]
     double* AB = B1 + 16 * KP;
@@ -263,6 +294,7 @@ __device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
             }
             v = f;
         } else {
+#pragma unroll 4
             for (int q = 0; q < n; ++q) v = fma(A1[i * AP + q], y[q * py], v);
         }
         if (j < n)
@@ -293,21 +325,29 @@ __device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
             const int i = t / m, j = t - i * m;
             double v = bq(4 - st, i, j);
             for (int b = 0; b < st; ++b)
+#pragma unroll 4
                 for (int q = 0; q < n; ++q)
                     v = fma(R[i * kBP + (4 - st + b) * n + q], V[(b * 16 + q) * KP + j], v);
             V[(st * 16 + i) * KP + j] = v;
         }
     }
     __syncthreads();
-    for (int t = tid; t < na * na; t += 1024) {
-        const int j = t / na, i = t - j * na;   // PT[j][i] = M[i][j]
-        a.PT[t] = i < 3 * n ? (j == i + n ? 1.0 : 0.0) : R[(i - 3 * n) * kBP + j];
+    const int n16 = (na + 15) & ~15;
+    for (int t = tid; t < n16 * n16; t += 1024) {
+        const int j = t / n16, i = t - j * n16;   // PT[j][i] = M[i][j]
+        double v = 0.0;
+        if (i < na && j < na) v = i < 3 * n ? (j == i + n ? 1.0 : 0.0) : R[(i - 3 * n) * kBP + j];
+        lds[j * kBP + i] = v;
+        if (store && i < na && j < na) a.PT[(long)j * na + i] = v;
     }
     double* GT = a.QT + (long)(s.T - 1) * m * na;
-    for (int t = tid; t < m * na; t += 1024) {
-        const int j = t / na, x = t - j * na, b = x / n, i = x - b * n;
-        GT[t] = V[((b + 1) * 16 + i) * KP + j];
+    for (int t = tid; t < kBN * n16; t += 1024) {
+        const int j = t / n16, x = t - j * n16, b = x / n, i = x - b * n;
+        const double v = j < m && x < na ? V[((b + 1) * 16 + i) * KP + j] : 0.0;
+        lds[kTabG + j * kBP + x] = v;
+        if (store && j < m && x < na) GT[(long)j * na + x] = v;
     }
+    if (!store) return;
     for (int t = tid; t < 4 * m * na; t += 1024) {
         const int rj = t / na, x = t - rj * na, r = rj / m, j = rj - r * m, b = x / n, i = x - b * n;
         a.DL[t] = b >= r ? V[((b - r) * 16 + i) * KP + j] : 0.0;
@@ -316,11 +356,13 @@ __device__ __forceinline__ void d_blk_map_abm(const BlkMap& a, double* lds)
     for (int t = tid; t < 4 * m * p; t += 1024) {
         const int rj = t / p, o = t - rj * p, r = rj / m, j = rj - r * m;
         double v = 0.0;
-        if (s.useC)
+        if (s.useC) {
+#pragma unroll 4
             for (int i = 0; i < n; ++i)
                 v = fma((double)a.C[(long)o * n + i], V[((3 - r) * 16 + i) * KP + j], v);
-        else
+        } else {
             v = V[((3 - r) * 16 + o) * KP + j];
+        }
         F[t] = v + (r == 3 && s.useD ? (double)a.D[(long)o * m + j] : 0.0);
     }
 }
@@ -352,10 +394,10 @@ __global__ __launch_bounds__(1024) void k_blk_start_outputs(BlockShape s, const 
     d_start_outputs<TU>(s, C, D, X0, U, Y);
 }
 
-// The seed of a plan's solve (work-group 1): x0, or the ABM start-up states
+// The seed of a plan's solve (a work-group of its own): x0, or the ABM start-up states
 // and the outputs of the first three (inputs: rows 0, 2, 4 of the h/2 grid).
 template <typename TU>
-__device__ __forceinline__ void d_blk_seed(const BlkMap& a)
+__device__ __forceinline__ void d_blk_seed(const BlkTables& a)
 {
     const BlockShape& s = a.s;
     const TU* U = static_cast<const TU*>(a.U);
@@ -368,35 +410,7 @@ __device__ __forceinline__ void d_blk_seed(const BlkMap& a)
     d_start_outputs<TU>(s, a.C, a.D, a.seed, U, a.Y);
 }
 
-template <typename TU>
-__device__ __forceinline__ void d_blk_map(const VBlock vb, const BlkMap& a, double* lds)
-{
-    if (vb.x == 1)
-        d_blk_seed<TU>(a);
-    else if (a.s.method == 0)
-        d_blk_map_rk4(a, lds);
-    else
-        d_blk_map_abm(a, lds);
-}
-
-constexpr int kMapLds = 2 * kBN * kBP + 4 * kBN * (kBM + 1);   // doubles
-
-template <typename TU>
-__global__ __launch_bounds__(1024) void k_blk_map(const BlkMap a)
-{
-    __shared__ double lds[kMapLds];
-    d_blk_map<TU>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, lds);
-}
-
 // ---------------------------------------------------------------- the tables
-struct BlkTables {
-    BlockShape s;
-    const float* C;
-    double *PT, *QT, *OT, *Ht;
-    int ni, nq;   // steps of a slice of OT (and Ht), of a slice of QT
-    long gx;
-};
-
 // P <- P^2 in LDS (and, with R, the rows of R by P or P^T): every tile from the
 // old values, a barrier, the new values, a barrier.  Sixteen waves, two tiles
 // of P^2 and rows each.  from/to: the rows of R that are read and written.
@@ -435,26 +449,33 @@ __device__ __forceinline__ void lds_step(double* P, int n16, double* R, int from
     __syncthreads();
 }
 
-// Tables of a small system (n_a, p, s m <= 64).  Work-group 0 squares P_0 up
+// Map and tables of a small system (n_a, p, s m <= 64).  Every work-group makes the
+// map for itself (a launch of its own for it cost 5 us more).  Work-group 0 squares P_0 up
 // to P_lb; the others each make a slice of OT and Ht (ni steps) or of QT (nq
 // steps) and square P_l for themselves, since passing it between work-groups
-// would cost a launch per level.  A slice of steps [i0, i0 + 2^a) takes the
-// levels below a by doubling its rows and the others by the bits of i0 (the
-// powers commute).  Time: lb dependent products of 64 x 64 in one compute unit.
-__device__ __forceinline__ void d_blk_tables(const VBlock vb, const BlkTables& a, double* P,
-                                             double* R, double* G)
+// would cost a launch per level; the last, if the solve's start is known, its
+// seed.  A slice of steps [i0, i0 + 2^a) takes the levels below a by doubling its
+// rows and the others by the bits of i0 (the powers commute).  Time: the map and
+// lb dependent products of 64 x 64 in one compute unit.
+template <typename TU>
+__device__ __forceinline__ void d_blk_tables(const VBlock vb, const BlkTables& a, double* lds)
 {
     const BlockShape& s = a.s;
     const int na = s.na, n16 = (na + 15) & ~15, tid = threadIdx.x, m = s.m, p = s.p;
     const int sm = s.s * m, nO = s.T / a.ni;
     const long nn = (long)na * na;
-    const double* GT = a.QT + (long)(s.T - 1) * sm * na;
-    for (int t = tid; t < n16 * n16; t += 1024) {
-        const int r = t / n16, c = t - r * n16;
-        P[r * kBP + c] = (r < na && c < na) ? a.PT[(long)r * na + c] : 0.0;
+    if (a.x0 && vb.x == a.gx - 1) {
+        d_blk_seed<TU>(a);
+        return;
     }
+    if (s.method == 0)
+        d_blk_map_rk4(a, lds, vb.x == 0);
+    else
+        d_blk_map_abm(a, lds, vb.x == 0);
+    __syncthreads();
+    double* P = lds;
+    double* G = lds + kTabG;
     if (vb.x == 0) {
-        __syncthreads();
         for (int l = 0; l < s.lb; ++l) {
             lds_step<false, false>(P, n16, nullptr, 0, 0, 0, true);
             double* out = a.PT + (l + 1) * nn;
@@ -466,18 +487,16 @@ __device__ __forceinline__ void d_blk_tables(const VBlock vb, const BlkTables& a
     const int w = (int)vb.x - 1 - (isO ? 0 : nO);
     const int ns = isO ? a.ni : a.nq, per = isO ? p : sm, i0 = w * ns, rows = ns * per;
     const int off = na - s.n;
-    for (int t = tid; t < kBN * n16; t += 1024) {
-        const int r = t / n16, c = t - r * n16;
-        double v = 0.0;
-        if (r < per) {
-            if (!isO)
-                v = c < na ? GT[(long)r * na + c] : 0.0;
-            else if (c >= off && c < na)
+    // the rows of step 0: those of C E, or G itself
+    double* R = isO ? lds + kTabR : G;
+    if (isO)
+        for (int t = tid; t < kBN * n16; t += 1024) {
+            const int r = t / n16, c = t - r * n16;
+            double v = 0.0;
+            if (r < per && c >= off && c < na)
                 v = s.useC ? (double)a.C[(long)r * s.n + c - off] : (c - off == r ? 1.0 : 0.0);
+            R[r * kBP + c] = v;
         }
-        R[r * kBP + c] = v;
-        if (isO) G[r * kBP + c] = (r < sm && c < na) ? GT[(long)r * na + c] : 0.0;
-    }
     __syncthreads();
     for (int l = 0; l < s.lb; ++l) {
         const bool more = l + 1 < s.lb;
@@ -519,10 +538,11 @@ __device__ __forceinline__ void d_blk_tables(const VBlock vb, const BlkTables& a
     }
 }
 
+template <typename TU>
 __global__ __launch_bounds__(1024) void k_blk_tables(const BlkTables a)
 {
-    __shared__ double P[kBN * kBP], R[kBN * kBP], G[kBN * kBP];
-    d_blk_tables(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, P, R, G);
+    __shared__ double lds[kTabLds];
+    d_blk_tables<TU>(VBlock{(long)blockIdx.x, (long)blockIdx.y, (long)gridDim.x}, a, lds);
 }
 
 // ---------------------------------------------------------------- the passes
@@ -1864,26 +1884,6 @@ long block_groups(int na, long nb)
     return lg ? (nb + (1L << lg) - 1) >> lg : 0;
 }
 
-static BlkMap map_args(const BlockShape& s, const BlockBufs& b, double h, const float* A,
-                       const float* B, const float* C, const float* D, const float* x0,
-                       const void* U, double* seed, float* Y)
-{
-    return BlkMap{s, h, rk4_coefficients(h), abm_coefficients(h), A, B, C, D, x0, U, b.PT, b.QT,
-                  b.Ht, b.DL, seed, Y, x0 ? 2L : 1L};
-}
-
-void block_map(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
-               const float* B, const float* C, const float* D, const float* x0, const void* U,
-               bool uDouble, double* seed, float* Y)
-{
-    const BlkMap a = map_args(s, b, h, A, B, C, D, x0, U, seed, Y);
-    if (uDouble)
-        hipLaunchKernelGGL(k_blk_map<double>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
-    else
-        hipLaunchKernelGGL(k_blk_map<float>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
-    check_launch("block_map");
-}
-
 void block_start_outputs(hipStream_t st, const BlockShape& s, const float* C, const float* D,
                          const double* X0, const void* U, bool uDouble, float* Y)
 {
@@ -1905,9 +1905,12 @@ static int slice_steps(int T, int per, int rows)
     return k;
 }
 
-static BlkTables table_args(const BlockShape& s, const BlockBufs& b, const float* C, bool grouped)
+static BlkTables table_args(const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                            const float* B, const float* C, const float* D, const float* x0,
+                            const void* U, double* seed, float* Y, bool grouped)
 {
-    BlkTables a{s, C, b.PT, b.QT, b.OT, b.Ht, 0, 0, 0};
+    BlkTables a{s, h, rk4_coefficients(h), abm_coefficients(h), A, B, C, D, x0, U, b.PT, b.QT,
+                b.OT, b.Ht, b.DL, seed, Y, 0, 0, 0};
     // Short slices while each has its compute unit: a level's time is that of its
     // products on one (n_a = 48: 20 us for six levels with 64 rows, 15.5 with 16).
     // Together with other systems the longest, since each slice squares for itself.
@@ -1915,15 +1918,21 @@ static BlkTables table_args(const BlockShape& s, const BlockBufs& b, const float
         a.ni = slice_steps(s.T, s.p, rows);
         a.nq = slice_steps(s.T, s.s * s.m, rows);
         a.gx = 1 + s.T / a.ni + s.T / a.nq;
-        if (a.gx <= 256) break;
+        if (a.gx <= 255) break;
     }
+    if (x0) ++a.gx;
     return a;
 }
 
-void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, const float* C)
+void block_tables(hipStream_t st, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                  const float* B, const float* C, const float* D, const float* x0, const void* U,
+                  bool uDouble, double* seed, float* Y)
 {
-    const BlkTables a = table_args(s, b, C, false);
-    hipLaunchKernelGGL(k_blk_tables, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
+    const BlkTables a = table_args(s, b, h, A, B, C, D, x0, U, seed, Y, false);
+    if (uDouble)
+        hipLaunchKernelGGL(k_blk_tables<double>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_blk_tables<float>, dim3((unsigned)a.gx), dim3(1024), 0, st, a);
     check_launch("block_tables");
 }
 
@@ -2191,19 +2200,12 @@ struct RootB {
     long gx;
 };
 
-__global__ __launch_bounds__(1024) void kg_blk_map(const BlkMap* __restrict__ args,
-                                                   const unsigned* __restrict__ st, int ns)
-{
-    PARODE_GROUP(BlkMap);
-    __shared__ double lds[kMapLds];
-    d_blk_map<double>(vb, a, lds);
-}
 __global__ __launch_bounds__(1024) void kg_blk_tables(const BlkTables* __restrict__ args,
                                                       const unsigned* __restrict__ st, int ns)
 {
     PARODE_GROUP(BlkTables);
-    __shared__ double P[kBN * kBP], R[kBN * kBP], G[kBN * kBP];
-    d_blk_tables(vb, a, P, R, G);
+    __shared__ double lds[kTabLds];
+    d_blk_tables<double>(vb, a, lds);
 }
 __global__ __launch_bounds__(256) void kg_blk_elem(const BlkElem* __restrict__ args,
                                                    const unsigned* __restrict__ st, int ns)
@@ -2281,17 +2283,12 @@ void add_pass(Phase& ph, BlkPass a, bool out, bool powers)
 
 }  // namespace
 
-void add_block_map(Phase& ph, const BlockShape& s, const BlockBufs& b, double h, const float* A,
-                   const float* B, const float* C, const float* D, const float* x0, double* seed)
+void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, double h, const float* A,
+                      const float* B, const float* C, const float* D, const float* x0, double* seed)
 {
     // (an ABM start-up reads the input samples: it has a launch of its own)
-    const BlkMap a = map_args(s, b, h, A, B, C, D, s.method == 0 ? x0 : nullptr, nullptr, seed,
-                              nullptr);
-    append(ph, kBlkMap, false, a, a.gx, 0, (float)s.na);
-}
-void add_block_tables(Phase& ph, const BlockShape& s, const BlockBufs& b, const float* C)
-{
-    const BlkTables a = table_args(s, b, C, true);
+    const BlkTables a = table_args(s, b, h, A, B, C, D, s.method == 0 ? x0 : nullptr, nullptr, seed,
+                                   nullptr, true);
     append(ph, kBlkTables, false, a, a.gx, 0, (float)s.na * s.lb);
 }
 void add_block_elem(Phase& ph, const BlkElem& e)
@@ -2343,7 +2340,6 @@ bool run_blocks(hipStream_t s, const Launch& L, const void* dArgs, const unsigne
     hipLaunchKernelGGL((KERNEL), grid, dim3(THREADS), lds, s, static_cast<const T*>(dArgs),   \
                        dStart, ns)
     switch (L.kind) {
-    case kBlkMap: PARODE_RUN(kg_blk_map, BlkMap, 1024); break;
     case kBlkTables: PARODE_RUN(kg_blk_tables, BlkTables, 1024); break;
     case kBlkElem: PARODE_RUN(kg_blk_elem, BlkElem, 256); break;
     case kBlkStartOut: PARODE_RUN(kg_blk_start_outputs, StartOutB, 256); break;

@@ -271,7 +271,7 @@ enum Kind {
     kLevel32, kLevel32W, kLevel32Delta, kLevel32DeltaW, kLevelG, kLevelGDelta, kLevel64, kGather, kTopMfma, kTopSimt, kRoot,
     kOutputsLanes, kOutputsKc8, kOutputsKc16, kOutputsKc24, kOutputsKc32, kOutputsMfma,
     // block responses (flag: pass 2)
-    kBlkMap, kBlkTables, kBlkElem, kBlkStartOut, kBlkTile, kBlkMid, kBlkSplit4, kBlkSplit16, kBlkScanUp,
+    kBlkTables, kBlkElem, kBlkStartOut, kBlkTile, kBlkMid, kBlkSplit4, kBlkSplit16, kBlkScanUp,
     kBlkScanAll, kBlkScanDown, kBlkRoot
 };
 struct Launch {

@@ -252,9 +252,8 @@ void ScanCore::build_powers(hipStream_t s, bool withLast)
             powersDone_ = true;
             return;
         }
-        k::block_map(s, blk_, bb_, h_, dA_, dB_, dC_, dD_, nullptr, nullptr, false, nullptr,
-                     nullptr);
-        k::block_tables(s, blk_, bb_, dC_);
+        k::block_tables(s, blk_, bb_, h_, dA_, dB_, dC_, dD_, nullptr, nullptr, false, nullptr,
+                        nullptr);
         powersDone_ = false;   // the first batch's pass 1 makes the rest of them
         return;
     }
@@ -978,8 +977,7 @@ void ScanCore::solve_blocks(hipStream_t s, long nScan, double h, const float* dA
         if (method_ == kABM && side) PARODE_HIP(hipStreamWaitEvent(s, side->join, 0));
         k::block_tree_finish(s, blk_, bb_, in, nb, seed());
     } else {
-        k::block_map(s, blk_, bb_, h, dA, dB, dC, dD, dx0, dU, uDouble, seed(), dY);
-        k::block_tables(s, blk_, bb_, dC);
+        k::block_tables(s, blk_, bb_, h, dA, dB, dC, dD, dx0, dU, uDouble, seed(), dY);
         tick(1);
         k::block_pass1(s, blk_, bb_, in, nb, true, block_tiling(1, nb, uDouble));
         tick(2);
