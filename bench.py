@@ -14,8 +14,10 @@ Beside it, in the same JSON line:
                one stream (hipEvents), inputs and outputs resident in HBM;
                served_vs_plain = value / plain rate
   group        the same grouped solve through ParODE_GroupExecuteTimed: GPU
-               time of each stage (hipEvents on its stream); `roofline` is the
-               chunk-recurrence stage (the dominant kernels)
+               time of each stage (hipEvents on its stream; of block
+               responses `powers` is the map, tables and squarings,
+               `chunks_pass1` / `chunks_pass2` their passes); `roofline` is
+               the first pass
   served_host  one pass with outputs copied back to host memory
   stream       Poisson arrivals from the same distribution, p50/p99 latency
   accuracy     max relative error vs the FP64 sequential recurrence on a
@@ -46,86 +48,27 @@ METRIC = "state-steps/s at <=1e-6 rel err vs FP64, served vs plain scan; p50/p99
 
 
 # ------------------------------------------------------------ work accounting
-def _pow2(v):
-    p = 1
-    while p < v:
-        p <<= 1
-    return p
-
-
-def scan_shape(method, n, points):
-    """(n_scan, nPad, L, na, chunk log lc, top level lt) as the library plans a
-    mixed-precision solve: chunks of 2^lc elements (lc = min(7, L - 10), at
-    least 2), tree levels [lc, lt), the rest in one work-group."""
-    n_scan = points if method == 0 else points - 3
-    npad = _pow2(n_scan)
-    L = npad.bit_length() - 1
-    na = n if method == 0 else 4 * n
-    pairs = lambda l: (n_scan + (2 << l) - 1) // (2 << l)
-    if npad * na <= 65536:
-        lt = 0
-    elif na >= 64:
-        lt = L
-    else:
-        lt = 0
-        while lt < L and pairs(lt) > 32:
-            lt += 1
-    lc = min(7, L - 10)
-    if lc < 2 or lt <= lc:
-        lc = 0
-    return n_scan, npad, L, na, lc, lt
-
-
-def chunk_flops(method, n, points):
-    """Algorithmic flops of both chunk-recurrence passes: per element and pass,
-    RK4 2 n^2 (the dense map), ABM 4 n^2 (x3 + A w1 + A^2 w2 factored, or
-    x3 + A (w1 + A w2))."""
-    n_scan, _, _, _, lc, _ = scan_shape(method, n, points)
-    if not lc:
-        return 0.0
-    return 2 * n_scan * (2.0 * n * n if method == 0 else 4.0 * n * n)
-
-
-def level_flops(na, n_scan, n_leaf=None, chunk_log=0, factored=False):
-    """Algorithmic flops of one solve's sweeps (both directions): 2 na^2 per
-    pair of every tree level (pairs of level l = ceil(N / 2^(l+1))); levels
-    below chunk_log as two chunk passes per element (ABM: the n x 4n block, or
-    2 n (2n) factored; RK4: 2 na^2); ABM levels 0 and 1 without chunks need
-    fewer products (M's shift rows, the leaves' zero rows).  Returns (flops,
-    tree pairs per sweep)."""
-    L = max(0, (n_scan - 1).bit_length())
-    per = [(n_scan + (2 << l) - 1) // (2 << l) for l in range(L)]
-    if chunk_log:
-        per_step = (2.0 * n_leaf * (2 * n_leaf) if factored else 2.0 * n_leaf * na) \
-            if n_leaf else 2.0 * na * na
-        tree = per[chunk_log:]
-        return 2 * per_step * n_scan + 2 * 2.0 * na * na * sum(tree), sum(tree)
-    pairs = sum(per)
-    flops = 2 * 2.0 * na * na * pairs
-    if n_leaf and L:
-        n = n_leaf
-        flops -= per[0] * (2 * 2.0 * na * na - 2.0 * n * n - 2.0 * n * na)
-        if L > 1:
-            flops -= per[1] * (2 * 2.0 * na * na - 2.0 * (2 * n) * (2 * n) - 2.0 * (2 * n) * na)
-    return flops, pairs
+def pass1_flops(method, n, m, points):
+    """Flops of the first pass of block responses (blocks.h): per step the samples
+    it adds (two of m for RK4, one for ABM) times n_a states."""
+    if method == 0:
+        return points * 2.0 * n * 2 * m
+    return (points - 3) * 2.0 * 4 * n * m
 
 
 def system_bound_seconds(method, n, m, p, points):
-    """Roofline time of one system's mixed-precision solve as built: FP32
-    matrix-core flops (chunk passes and tree levels), FP64 matrix-core flops
-    (the power squarings up to P_{L-1}: 2 n_a^3 each, 56 n^3 for the ABM
-    companion; the leaves, 2 n k m per step with k = 3 for RK4 and 2 for the
-    factored ABM; the outputs, 2 p (n + m) per point), the two kinds sharing
-    the matrix cores, against the compulsory HBM bytes (FP64 samples on the h/2
-    grid in, FP32 outputs out)."""
-    n_scan, _, L, na, lc, _ = scan_shape(method, n, points)
-    f32, _ = level_flops(na, n_scan, n_leaf=n if method else None, chunk_log=lc,
-                         factored=bool(method))
-    sq = 56.0 * n ** 3 if method else 2.0 * na ** 3
-    f64 = max(L - 1, 0) * sq + 2.0 * n * (2 if method else 3) * m * n_scan \
-        + 2.0 * p * (n + m) * points
+    """Roofline time of one system's mixed-precision solve by block responses,
+    whatever the steps of a block: FP64 matrix-core flops (the first pass; the
+    outputs' products with the states and with one step's samples, 2 p (n_a + m)
+    per point; log2 N - 1 squarings of the map, 2 n_a^3 each, 56 n^3 for the ABM
+    companion) against the compulsory HBM bytes (FP64 samples on the h/2 grid in,
+    FP32 outputs out)."""
+    na = 4 * n if method else n
+    squarings = max(0, (points - 1).bit_length() - 1)
+    f64 = pass1_flops(method, n, m, points) + 2.0 * p * (na + m) * points \
+        + squarings * (56.0 * n ** 3 if method else 2.0 * n ** 3)
     hbm = (2 * points + 1) * m * 8.0 + points * p * 4.0
-    return max(f32 / PEAK["fp32"] + f64 / PEAK["fp64"], hbm / PEAK["hbm"])
+    return max(f64 / PEAK["fp64"], hbm / PEAK["hbm"])
 
 
 # ------------------------------------------------------------------- helpers
@@ -410,10 +353,8 @@ def single_legs(args, torch, api, synth, dev):
                               "p99": float(np.percentile(lat, 99))},
                "phases_ms": ph, "autotuned_level_launches": tuned}
         if k == 1 and prec == api.MIXED:
-            na, n_scan, lc = s.n_scan, s.steps - 3, plan.chunk_log
-            flops, _ = level_flops(na, n_scan, s.n, lc, factored=True)
-            sweep_ms = ph["up_sweep"] + ph["down_sweep"]
-            rec["sweeps_tflops"] = flops / (sweep_ms * 1e-3) / 1e12
+            flops = pass1_flops(s.method, s.n, s.m, s.steps)   # (the "leaves" phase)
+            rec["pass1_tflops"] = flops / (ph["leaves"] * 1e-3) / 1e12
         if not args.no_check:
             sys.path.insert(0, os.path.join(ROOT, "oracle"))
             import oracle as orc
@@ -548,10 +489,11 @@ def main():
     log("plain leg")
     plain_ms, y_plain = plain_leg(args, torch, api, systems, dev)
 
-    # roofline: the chunk-recurrence passes (dominant stages of the grouped solve)
-    cflops = sum(chunk_flops(s.method, s.n, s.steps) for s in systems)
-    chunk_ms = grp["stage_ms"]["chunks_pass1"] + grp["stage_ms"]["chunks_pass2"]
-    achieved = cflops / (chunk_ms * 1e-3)
+    # roofline: the first pass of the block responses (its flops do not depend on
+    # the steps of a block)
+    p1flops = sum(pass1_flops(s.method, s.n, s.m, s.steps) for s in systems)
+    p1_ms = grp["stage_ms"]["chunks_pass1"]
+    achieved = p1flops / (p1_ms * 1e-3)
     bound = total / sum(system_bound_seconds(s.method, s.n, s.m, s.p, s.steps) for s in systems)
 
     line = {
@@ -581,14 +523,14 @@ def main():
         "batch_roofline": {
             "bound_state_steps_per_s": bound,
             "frac": value / bound,
-            "model": "sum N_i / sum max(F32_i / 157.3 TF + F64_i / 78.6 TF, B_i / 8 TB/s) with "
-                     "the as-built flops (chunk passes, tree levels, FP64 squarings, leaves, "
-                     "outputs) and the compulsory bytes (FP64 samples in, FP32 outputs out)"},
-        "roofline": {"bound": "mfma", "achieved": achieved / 1e12, "peak": PEAK["fp32"] / 1e12,
-                     "unit": "TFLOP/s", "frac": achieved / PEAK["fp32"], "traffic": None,
-                     "kernel": "grouped chunk recurrences (kg_chunks_fac / kg_chunks_two / "
-                               "kg_chunks_dense), both passes",
-                     "flops_per_pass_pair": cflops, "stage_ms": chunk_ms},
+            "model": "sum N_i / sum max(F64_i / 78.6 TF, B_i / 8 TB/s) with the flops of block "
+                     "responses that do not depend on their length (first pass, outputs, "
+                     "squarings) and the compulsory bytes (FP64 samples in, FP32 outputs out)"},
+        "roofline": {"bound": "mfma", "achieved": achieved / 1e12, "peak": PEAK["fp64"] / 1e12,
+                     "unit": "TFLOP/s", "frac": achieved / PEAK["fp64"], "traffic": None,
+                     "kernel": "grouped first pass of the block responses (kg_blk_tile / "
+                               "kg_blk_split, FP64 matrix cores)",
+                     "flops_per_pass": p1flops, "stage_ms": p1_ms},
     }
     log("stream leg")
     if args.stream_seconds > 0:

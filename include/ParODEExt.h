@@ -28,7 +28,10 @@ void ParODE_SetMaxBatchSteps(long maxSteps);
  * FP32 scan levels on the vector ALUs instead of the matrix cores, bit 1 the
  * FP64 GEMMs of the power table on the vector ALUs, bit 2 launches every level
  * separately instead of finishing the top of the tree in one work-group, bit 3
- * runs the lowest ABM levels as tree levels instead of chunk recurrences. */
+ * runs the lowest ABM levels as tree levels instead of chunk recurrences.  Any
+ * bit also keeps the tree of scan levels where a solve would run as block
+ * responses (several steps at a time as FP64 products); that choice is made when
+ * a plan, a group or a request's solve is set up. */
 void ParODE_SetLevelKernel(int variant);
 
 /* Compiles a UFunc source for a gfx target (e.g. "gfx950") without a GPU.
@@ -90,15 +93,17 @@ int ParODE_PlanLevels(void* plan);
  * own trajectory buffer, on `stream`, and keeps the fastest in a process-wide
  * level schedule that every later solve of the same shape follows (plans,
  * the C ABI, served requests).  Returns the number of level launches tuned
- * (>= 0) or a negative ErrorCode.  Blocks until the timings are done; the
+ * (>= 0) or a negative ErrorCode.  A plan that runs as block responses tunes
+ * the tiling of its two passes instead.  Blocks until the timings are done; the
  * plan's previous outputs are not touched, its trajectory is overwritten.
  * For callers that solve one shape many times.  No counterpart in the
  * reference. */
 int ParODE_PlanAutotune(void* plan, void* stream);
 /* Forgets the autotuned schedule (every level back to the built-in rule). */
 void ParODE_ScheduleClear(void);
-/* Number of the plan's lowest scan levels that run as chunk recurrences
- * (0: all run as tree levels), -1 for a null plan.  For benchmarks that count
+/* Number of the plan's lowest scan levels that run as chunk recurrences where
+ * the plan runs the tree of scan levels (0: all are tree levels), -1 for a
+ * null plan.  For benchmarks that count
  * the work of each path. */
 int ParODE_PlanChunkLog(void* plan);
 int ParODE_PlanDestroy(void* plan);
