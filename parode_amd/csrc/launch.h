@@ -23,6 +23,16 @@ __device__ __forceinline__ void load4(const double* p, double (&r)[4])
     r[2] = b.x;
     r[3] = b.y;
 }
+// four floats at any 4-byte address
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load4(const float* p, double (&r)[4])
+{
+    const float4u a = *reinterpret_cast<const float4u*>(p);
+    r[0] = a.x;
+    r[1] = a.y;
+    r[2] = a.z;
+    r[3] = a.w;
+}
 
 // The block a kernel body works on: (x, y) and the grid's width in x.  A
 // single-system launch passes its own blockIdx and gridDim; a grouped launch
