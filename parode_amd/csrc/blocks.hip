@@ -1602,6 +1602,12 @@ static std::vector<TreeLevel> tree_of(const BlockShape& s, long nb)
         if (n <= tree_top(s)) return t;
     }
 }
+// states from b.Z2 on that all levels take together (tree_of's last place: whole
+// nodes at the top too, up to eight states)
+static size_t tree_states(const std::vector<TreeLevel>& t)
+{
+    return t.size() == 1 ? 0 : t.back().e + (size_t)tree_rows(t.back().n);
+}
 static double* tree_s(const BlockShape& s, const BlockBufs& b, const std::vector<TreeLevel>& t, int k)
 {
     return k == 0 ? b.Z : b.Z2 + t[k].s * s.na;
@@ -1635,8 +1641,7 @@ static size_t state_rows0(const BlockShape& s, long nb)
 size_t block_state_values(const BlockShape& s, long nb)
 {
     if (!s.wide) return (state_rows0(s, nb) + block_groups(s.na, nb) + 1) * s.na;
-    const std::vector<TreeLevel> t = tree_of(s, nb);
-    return (2 * state_rows0(s, nb) + t.back().e + (nb > 1 ? 4 : 0)) * s.na;
+    return (2 * state_rows0(s, nb) + tree_states(tree_of(s, nb))) * s.na;
 }
 
 size_t block_scratch_values(const BlockShape& s)
