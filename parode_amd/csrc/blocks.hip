@@ -1233,9 +1233,11 @@ __device__ __forceinline__ void d_blk_scan_n(const VBlock vb, const BlkScan& a, 
             doublex4 y;
 #pragma unroll
             for (int v = 0; v < 4; ++v) y[v] = cur[(rt * 16 + 4 * v + q4) * pitch + col];
-            y = product(cur, y, 1 << k);
+            // (the first 2^k groups have their start states: a power that has
+            // overflowed would add infinity times their zero neighbours)
+            const doublex4 z = product(cur, y, 1 << k);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) put(nxt, v, y[v]);
+            for (int v = 0; v < 4; ++v) put(nxt, v, rt * 16 + 4 * v + q4 < (1 << k) ? y[v] : z[v]);
             flip();
         }
         if (kAhead) {
