@@ -231,7 +231,7 @@ int ParODE_PlanAutotune(void* plan, void* stream)
     if (!pl) return ParODE_InvalidSystem;
     try {
         PARODE_HIP(hipSetDevice(pl->device));
-        return pl->core->autotune(static_cast<hipStream_t>(stream), pl->nScan, pl->nPad);
+        return pl->core->autotune(static_cast<hipStream_t>(stream), pl->nScan, pl->nPad, pl->uDouble);
     } catch (std::exception& e) {
         parode::last_error() = e.what();
         return ParODE_NotEnoughResources;

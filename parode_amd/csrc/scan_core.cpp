@@ -399,8 +399,8 @@ namespace {
 // The autotuned schedule: (n_a, precision, level, pairs, down) -> path
 std::mutex g_schedMu;
 std::map<std::array<long, 5>, int> g_sched;
-// and of the block passes: (n_a, m, p, T, blocks, FP64 samples, pass) -> tiling
-std::map<std::array<long, 7>, int> g_blockSched;
+// and of the block passes: (method, n_a, m, p, T, blocks, FP64 samples, pass) -> tiling
+std::map<std::array<long, 8>, int> g_blockSched;
 }  // namespace
 
 int ScanCore::scheduled_path(bool down, int l, long np) const
@@ -583,10 +583,10 @@ void ScanCore::zero_trajectory(hipStream_t s, long nPad)
         k::fill_zero_f32(s, nPad * na_, X32_.get());
 }
 
-int ScanCore::autotune(hipStream_t s, long nReal, long nPad)
+int ScanCore::autotune(hipStream_t s, long nReal, long nPad, bool uDouble)
 {
     if (nPad > nPadMax_ || nReal < 1) throw std::invalid_argument("ScanCore::autotune: bad length");
-    if (uses_blocks()) return autotune_blocks(s, nReal);
+    if (uses_blocks()) return autotune_blocks(s, nReal, uDouble);
     const int lt = top_level(nReal, nPad);
     const bool s0 = lt > 0 && structured_level0(nReal, nPad);
     const bool s1 = s0 && structured_level1(nReal, nPad);
@@ -840,20 +840,25 @@ k::BlockInput ScanCore::block_input(const void* dU, bool uDouble, long sL, long 
     return k::BlockInput{dU, uDouble, sL, blk_.s * (nReal - 1) + (method_ == kABM ? 4 : 2)};
 }
 
+// (the method: RK4 with n_a states and ABM with as many have other windows)
+std::array<long, 8> ScanCore::block_key(int pass, long nb, bool uDouble) const
+{
+    return {(long)method_, (long)na_, (long)m_, (long)blk_.p, (long)blk_.T, nb, uDouble ? 1L : 0L,
+            (long)pass};
+}
+
 int ScanCore::block_tiling(int pass, long nb, bool uDouble) const
 {
     std::lock_guard<std::mutex> lk(g_schedMu);
-    auto it = g_blockSched.find({(long)na_, (long)m_, (long)blk_.p, (long)blk_.T, nb,
-                                 uDouble ? 1L : 0L, (long)pass});
+    auto it = g_blockSched.find(block_key(pass, nb, uDouble));
     return it == g_blockSched.end() ? k::kBlockAuto : it->second;
 }
 
 // Times each tiling of the two passes on samples of zeros.
-int ScanCore::autotune_blocks(hipStream_t s, long nReal)
+int ScanCore::autotune_blocks(hipStream_t s, long nReal, bool uDouble)
 {
-    const bool dbl = opt_.precision != kPlain32;
     const long nb = blocks_of(nReal), sL = 2;
-    k::BlockInput in = block_input(nullptr, dbl, sL, nReal);
+    k::BlockInput in = block_input(nullptr, uDouble, sL, nReal);
     const size_t vals = (size_t)(in.last + 1) * (sL / blk_.s) * m_;
     DevArray<double> U(vals);
     DevArray<float> Y((size_t)nReal * blk_.p);
@@ -887,8 +892,7 @@ int ScanCore::autotune_blocks(hipStream_t s, long nReal)
                 }
             }
             std::lock_guard<std::mutex> lk(g_schedMu);
-            g_blockSched[{(long)na_, (long)m_, (long)blk_.p, (long)blk_.T, nb, dbl ? 1L : 0L,
-                          (long)pass}] = best;
+            g_blockSched[block_key(pass, nb, uDouble)] = best;
         }
     } catch (...) {
         (void)hipStreamSynchronize(s);

@@ -19,6 +19,7 @@
 #include "blocks.h"
 #include "hip_util.h"
 
+#include <array>
 #include <functional>
 #include <vector>
 
@@ -153,13 +154,17 @@ public:
     // (K-split tiles, narrow or wide matrix-core tiles, SIMT) on this core's
     // own trajectory buffer (its contents are overwritten) and keeps the
     // fastest per (n_a, precision, level, pairs, sweep) in a process-wide
-    // schedule that every later solve of that shape follows.  Returns the
-    // number of level launches tuned.  Synchronises the stream.
-    int autotune(hipStream_t s, long nReal, long nPad);
+    // schedule that every later solve of that shape follows.  Block responses:
+    // the tilings of their two passes, on samples of the type that the solve
+    // reads.  Returns the number of launches tuned.  Synchronises the stream.
+    int autotune(hipStream_t s, long nReal, long nPad, bool uDouble);
     // Level paths of the schedule (kPathAuto: the built-in rule)
     enum LevelPath { kPathAuto = 0, kPathKs = 1, kPathNarrow = 2, kPathWide = 3, kPathSimt = 4 };
     int scheduled_path(bool down, int l, long np) const;
     static void clear_schedule();
+    // and the tiling of a block pass (1 or 2) over nb blocks (kBlockAuto: the rule)
+    int block_tiling(int pass, long nb, bool uDouble) const;
+    long blocks_of(long nReal) const { return (nReal + blk_.T - 1) / blk_.T; }
 
 private:
     friend class BatchSolve;   // plans grouped launches over the buffers below
@@ -183,9 +188,8 @@ private:
                      const float* dD, const float* dx0, long nb,
                      const std::function<void()>& pass1);
     k::BlockInput block_input(const void* dU, bool uDouble, long sL, long nReal) const;
-    long blocks_of(long nReal) const { return (nReal + blk_.T - 1) / blk_.T; }
-    int block_tiling(int pass, long nb, bool uDouble) const;
-    int autotune_blocks(hipStream_t s, long nReal);
+    std::array<long, 8> block_key(int pass, long nb, bool uDouble) const;
+    int autotune_blocks(hipStream_t s, long nReal, bool uDouble);
     void zero_blocks(hipStream_t s);
 
     int method_, n_, m_, p_, na_;
