@@ -854,7 +854,8 @@ int ScanCore::block_tiling(int pass, long nb, bool uDouble) const
     return it == g_blockSched.end() ? k::kBlockAuto : it->second;
 }
 
-// Times each tiling of the two passes on samples of zeros.
+// Times each tiling of the two passes on samples of zeros, as a solve launches
+// them: a small map's pass 1 squares the powers beside its tiles.
 int ScanCore::autotune_blocks(hipStream_t s, long nReal, bool uDouble)
 {
     const long nb = blocks_of(nReal), sL = 2;
@@ -875,7 +876,7 @@ int ScanCore::autotune_blocks(hipStream_t s, long nReal, bool uDouble)
             for (int t : {k::kBlockTile, k::kBlockMid, k::kBlockSplit4, k::kBlockSplit16}) {
                 auto run = [&] {
                     if (pass == 1)
-                        k::block_pass1(s, blk_, bb_, in, nb, false, t);
+                        k::block_pass1(s, blk_, bb_, in, nb, !blk_.wide, t);
                     else
                         k::block_pass2(s, blk_, bb_, in, nb, nReal, seed(), nullptr, Y.get(), t);
                 };
@@ -910,6 +911,7 @@ void ScanCore::zero_blocks(hipStream_t s)
     k::fill_f64(s, (long)blkTab_.size(), 0.0, blkTab_.get());
     k::fill_f64(s, (long)blkZ_.size(), 0.0, blkZ_.get());
     k::fill_f64(s, na_, 0.0, seed());
+    if (!blk_.wide) k::fill_f64(s, (long)PT64_.size(), 0.0, PT64_.get());
 }
 
 void BlockPhases::run(hipStream_t s, int from, int to) const

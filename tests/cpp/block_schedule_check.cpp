@@ -45,6 +45,14 @@ int main()
     }
     ScanCore::clear_schedule();
     expect(ab.block_tiling(1, nb, false) == k::kBlockAuto, "a cleared schedule is the rule's");
+
+    // pass 1 is timed with the squarings that a small map's runs beside its tiles: on
+    // four waves they take three times as long as its tiles
+    ScanCore sq(kRK4, 48, 6, 6, false, false, 65537, opt);
+    expect(sq.autotune(nullptr, 65537, next_pow2(65537), true) == 2, "two passes tuned");
+    expect(sq.block_tiling(1, sq.blocks_of(65537), true) != k::kBlockSplit4,
+           "squarings on more than four waves");
+    ScanCore::clear_schedule();
     std::printf("ok: 2^%d points, %ld blocks\n", log, nb);
     return 0;
 }
