@@ -1492,6 +1492,12 @@ static int group_log(long nb)
     while (((nb + (1L << lg) - 1) >> lg) > 512) ++lg;
     return lg;
 }
+// Row tiles of the scan's one work-group: 128, 64, 64 and 32 rows at up to 16, 32, 48
+// and 64 states, on 8 waves (12 at 48).  16 waves halve the dependent steps, but all
+// products share one compute unit and each step then takes more than two did (us a
+// solve with 8 and 16: n = 8, 4096 points 34.0, 38.3; n = 24, 9000 points 52.2, 57.5;
+// n = 64, 4000 points 98.3, 114.3).
+static int scan_row_tiles(int na) { return na <= 16 ? 8 : na <= 48 ? 4 : 2; }
 // The rule: which systems run as block responses, and with how many steps per
 // block: the fastest by the model below.  Covered: inputs and outputs present,
 // horizons from 64 points, n up to 1024.  The general path was nowhere faster on
@@ -1524,8 +1530,12 @@ int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long 
         const double pass = pass1 + N * (2.0 * p * na + 2.0 * s * m * p * (T / 2 + 32.0 / p + 2)) / r2;
         double scan, tab;
         if (one) {
-            // k_blk_scan measured: 13 us + 2.4 a step at n_a = 8, 18 + 3.1 at 48;
-            // groups before it 5 + 0.95 a step and 6 + 1.6 (both ways)
+            // k_blk_scan measured: 13 us + 2.4 for each 256 states at n_a = 8, 18 +
+            // 3.1 for each 64 at 48; groups before it 5 + 0.95 a step and 6 + 1.6
+            // (both ways).  (A fit: two of the launch's steps up to 32 states, one up
+            // to 48; at 49 to 64 it is 2.4 us short for each 64 states.  The launch's
+            // own steps and rows in its place: 160 of 702 shapes take another T, from
+            // 9% faster to 14% slower, 0.3% faster on average.)
             const int lg = group_log((long)std::ceil(nb));
             const double rows = na <= 16 ? 256 : na <= 32 ? 128 : 64;
             const double Lg = std::exp2(std::max(0.0, std::ceil(std::log2(nb / (1 << lg) / rows))));
@@ -2100,7 +2110,7 @@ static size_t scan_lds_bytes(const BlkScan& a)
 // over the blocks or the groups.
 static bool scan_plan(BlkScan a0, const BlockBufs& b, BlkScan& u, BlkScan& a, BlkScan& d)
 {
-    const int nct = (a0.na + 15) / 16, lg = group_log(a0.nb);
+    const int lg = group_log(a0.nb);
     a = a0;
     a.R = 1;
     if (lg) {
@@ -2114,8 +2124,8 @@ static bool scan_plan(BlkScan a0, const BlockBufs& b, BlkScan& u, BlkScan& a, Bl
         a.E = b.Z2;
         a.l0 = a0.l0 + lg;
     }
-    // as many row tiles as 16 waves (and 64 KB of LDS) hold, no more than the blocks need
-    while (2 * a.R * nct <= 16 && 2 * scan_lds_bytes(a) <= 65536 && 16L * a.R < a.nb) a.R *= 2;
+    // no more row tiles than the blocks need
+    while (a.R < scan_row_tiles(a.na) && 16L * a.R < a.nb) a.R *= 2;
     a.lg = 0;
     while ((16L * a.R << a.lg) < a.nb) ++a.lg;
     a.gx = 1;
