@@ -82,7 +82,7 @@ BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bo
 // How a pass is tiled (kBlockAuto: by the rule at launch_pass).
 enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit16 = 3, kBlockMid = 4 };
 // Groups of blocks that the scan of nb blocks makes first (0: none).
-long block_groups(int na, long nb);
+long block_groups(long nb);
 
 // doubles in QT, OT, Ht and DL together; in the states for at most nb blocks; in W
 size_t block_table_values(const BlockShape& s);
@@ -148,8 +148,8 @@ void block_start_outputs(hipStream_t st, const BlockShape& s, const float* C, co
 // the blocks' responses from zero (and, with powers, the rest of PT)
 void block_pass1(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                  long nb, bool powers, int tiling = kBlockAuto);
-// the blocks' start states from the seed (in X); Z[nb] is the state after them
-// (wide: tot receives the blocks' response from zero instead, if not null)
+// the blocks' start states from the seed (in X); Z[nb] is the state after them (of a
+// map that is not wide)
 void block_scan(hipStream_t st, const BlockShape& s, const BlockBufs& b, const BlockInput& in,
                 long nb, const double* seed);
 // seedOut = the state (in X) after the blocks

@@ -1069,7 +1069,7 @@ struct BlkScan {
     const double *seed, *DL;
     const void* U;
     bool uDouble;
-    int km, m, gm, gx_;     // taps m; samples skipped after each window row
+    int km, m, gm;          // taps m; samples skipped after each window row
     unsigned magic;
     long last;
     int R;                  // row tiles of a work-group
@@ -1652,7 +1652,7 @@ static size_t state_rows0(const BlockShape& s, long nb)
 }
 size_t block_state_values(const BlockShape& s, long nb)
 {
-    if (!s.wide) return (state_rows0(s, nb) + block_groups(s.na, nb) + 1) * s.na;
+    if (!s.wide) return (state_rows0(s, nb) + block_groups(nb) + 1) * s.na;
     return (2 * state_rows0(s, nb) + tree_states(tree_of(s, nb))) * s.na;
 }
 
@@ -1896,9 +1896,8 @@ std::vector<GemmOp> block_tree_down(const BlockShape& s, const BlockBufs& b, lon
     return ops;
 }
 
-long block_groups(int na, long nb)
+long block_groups(long nb)
 {
-    (void)na;
     const int lg = group_log(nb);
     return lg ? (nb + (1L << lg) - 1) >> lg : 0;
 }
@@ -2117,7 +2116,7 @@ static bool scan_plan(BlkScan a0, const BlockBufs& b, BlkScan& u, BlkScan& a, Bl
         u = a0;
         u.lg = lg;
         u.R = 1;
-        const long groups = block_groups(a0.na, a0.nb);
+        const long groups = block_groups(a0.nb);
         u.gx = (groups + 15) / 16;
         d = u;
         a.nb = groups;

@@ -38,14 +38,13 @@ ScanCore::ScanCore(int method, int n, int m, int p, bool zC, bool zD, long nPadM
             const long nb = nPadMax_ >> lb;
             const size_t tab = k::block_table_values(b), w = k::block_scratch_values(b);
             const size_t z = k::block_state_values(b, nb);
-            if (8 * (na2 * b.slots() + tab + z + w + 3 * na) + 8 * Arena::kAlign > cap) continue;
+            if (8 * (na2 * b.slots() + tab + z + w + 2 * na) + 8 * Arena::kAlign > cap) continue;
             PT64_.alloc(na2 * b.slots(), arena);
             blkTab_.alloc(tab, arena);
             blkZ_.alloc(z, arena);
             if (w) blkW_.alloc(w, arena);
             seed_.alloc(na_, arena);
-            tot_.alloc(na_, arena);
-            seedNext_.alloc(na_, arena);
+            seedNext_.alloc(na_, arena);   // (tot_ is the general path's)
             blk_ = b;
             bb_ = k::block_carve(b, PT64_.get(), blkTab_.get(), blkZ_.get(), nb, blkW_.get());
             return;

@@ -143,7 +143,7 @@ int main()
                 nb_ = nb;
                 what = "scan";
                 in_one("states", b.Z, 0, (nb + 1) * n);
-                in_one("groups", b.Z2, 0, (block_groups(n, nb) + 1) * n);
+                in_one("groups", b.Z2, 0, (block_groups(nb) + 1) * n);
             }
         }
     std::printf("%ld trees inside their buffers\n", trees);
