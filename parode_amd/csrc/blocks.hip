@@ -405,7 +405,7 @@ __device__ __forceinline__ void d_blk_seed(const BlkTables& a)
         for (int i = threadIdx.x; i < s.n; i += 1024) a.seed[i] = (double)a.x0[i];
         return;
     }
-    startup_rows<TU, 16>(s.mirror, s.n, s.m, a.h, a.A, a.B, a.x0, U, a.seed);
+    startup_rows<TU, 4>(s.mirror, s.n, s.m, a.h, a.A, a.B, a.x0, U, a.seed);
     __syncthreads();
     d_start_outputs<TU>(s, a.C, a.D, a.seed, U, a.Y);
 }

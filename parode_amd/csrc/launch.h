@@ -146,9 +146,11 @@ __device__ __forceinline__ void d_abm_startup(const VBlock vb, bool mirror, int 
 
 // The same steps for n, m <= 256 with 1024 threads: four lanes a row, each
 // with NC of the row's columns in registers, so that a derivative is NC
-// products from registers and LDS instead of a chain of n loads (n = 203: 318
-// -> 15 us; n = 64: 56 -> 9 us).  mirror: the row's float sum runs through the
-// four lanes in column order.
+// products from registers and LDS instead of a chain of n loads (us, one lane a
+// row and four: n = 203 286 and 45, n = 64 48 and 13, n = 16 15 and 8, n = 1 6 and
+// 8).  mirror: the row's float sum runs through the four lanes in column order, a
+// chain of n products again (n = 203 286 and 138, n = 64 51 and 43, n = 16 15.7 and
+// 15.6).
 template <typename TU, int NC>
 __device__ __forceinline__ void startup_rows(bool mirror, int n, int m, double h,
                                              const float* __restrict__ A,
@@ -180,7 +182,10 @@ __device__ __forceinline__ void startup_rows(bool mirror, int n, int m, double h
         double y;
         if (mirror) {
             float f = 0.0f;
+            // (segments past the last column or input add nothing)
+#pragma unroll
             for (int seg = 0; seg < 4; ++seg) {
+                if (seg * NC >= n) break;
                 if (q == seg)
 #pragma unroll
                     for (int c = 0; c < NC; ++c) {
@@ -189,7 +194,7 @@ __device__ __forceinline__ void startup_rows(bool mirror, int n, int m, double h
                     }
                 f = __shfl(f, (lane & ~3) + seg);
             }
-            for (int seg = 0; seg < 4; ++seg) {
+            for (int seg = 0; seg < 4 && seg * mq < m; ++seg) {
                 if (q == seg)
                     for (int c = mb; c < me; ++c) {
                         const float pr = Br[c] * (float)u[c];
@@ -242,7 +247,9 @@ __device__ __forceinline__ void d_startup_rows(bool mirror, int n, int m, double
                                                const float* B, const float* x0, const TU* Uh,
                                                double* X0)
 {
-    if (n <= 64)
+    if (n <= 16)
+        startup_rows<TU, 4>(mirror, n, m, h, A, B, x0, Uh, X0);
+    else if (n <= 64)
         startup_rows<TU, 16>(mirror, n, m, h, A, B, x0, Uh, X0);
     else if (n <= 128)
         startup_rows<TU, 32>(mirror, n, m, h, A, B, x0, Uh, X0);
