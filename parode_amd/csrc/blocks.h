@@ -79,7 +79,7 @@ struct BlockInput {
 int block_steps_log(int method, int n, int m, int p, bool useC, bool useD, long nScan, long nPad);
 BlockShape block_shape(int method, int n, int m, int p, bool useC, bool useD, bool mirror, int lb,
                        int L);
-// How a pass is tiled (kBlockAuto: by the rule at launch_pass).
+// How a pass is tiled (kBlockAuto: by the rule at pass_tiling).
 enum BlockTiling { kBlockAuto = 0, kBlockTile = 1, kBlockSplit4 = 2, kBlockSplit16 = 3, kBlockMid = 4 };
 // Groups of blocks that the scan of nb blocks makes first (0: none).
 long block_groups(long nb);
